@@ -6,10 +6,12 @@
 
 Run as `python -m cutlass_flash_atten_fp8_amd.build` or through __graft_entry__.build().
 """
+import concurrent.futures
 import os
 import subprocess
 import sys
 import sysconfig
+import tempfile
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
@@ -19,10 +21,14 @@ LIBFA8 = os.path.join(PKG_DIR, "libfa8.so")
 EXT_NAME = "attention_cutlass_fp8"
 EXT_PATH = os.path.join(PKG_DIR, EXT_NAME + sysconfig.get_config_var("EXT_SUFFIX"))
 
+KERNEL_SOURCES = [os.path.join(CSRC, f) for f in ("fa8_fwd_gfx950.hip", "fa8_shared_rows.hip")]
+
 HIPCC_FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     # never let the compiler form packed fp32 VALU ops
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # matrix results in vector registers, also in kernels whose LDS leaves room for accumulation registers
+    "-mllvm", "-amdgpu-mfma-vgpr-form=1",
 ]
 
 
@@ -35,9 +41,14 @@ def _run(cmd):
 
 
 def build_libfa8():
-    cmd = [os.path.join(ROCM, "bin", "hipcc")] + HIPCC_FLAGS + ["-I", INCLUDE, "-o", LIBFA8,
-                                                               os.path.join(CSRC, "fa8_fwd_gfx950.hip")]
-    _run(cmd)
+    """Compiles the kernel sources side by side, then links them."""
+    hipcc = os.path.join(ROCM, "bin", "hipcc")
+    with tempfile.TemporaryDirectory() as tmp:
+        objects = [os.path.join(tmp, os.path.basename(src) + ".o") for src in KERNEL_SOURCES]
+        with concurrent.futures.ThreadPoolExecutor(4) as pool:
+            list(pool.map(_run, [[hipcc] + HIPCC_FLAGS + ["-I", INCLUDE, "-c", src, "-o", obj]
+                                 for src, obj in zip(KERNEL_SOURCES, objects)]))
+        _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIBFA8] + objects)
     return LIBFA8
 
 

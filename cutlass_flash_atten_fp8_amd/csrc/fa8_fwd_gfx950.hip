@@ -23,13 +23,15 @@
 //     the swizzle being applied on the global-address side of the copy.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdint>
 #include <cstdlib>
 #include <type_traits>
 
-#include "fa8_api.h"
+#include "fa8_device.h"
+#include "fa8_launch.h"
 
 // wavefronts per SIMD the kernels are compiled for: 3 (at most 168 VGPRs per lane) up to head dim 128, 2 (256 VGPRs:
 // the output accumulators alone take 128) for head dim 256; the pipelined loop 2; the dense loop 3 (head dim 64: 4)
@@ -37,135 +39,7 @@
 
 namespace {
 
-typedef int v2i __attribute__((ext_vector_type(2)));
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v8i __attribute__((ext_vector_type(8)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef _Float16 v4h __attribute__((ext_vector_type(4)));
-
-#define LDS_PTR(T, p) ((__attribute__((address_space(3))) T*)(p))
-#define GLOBAL_PTR(T, p) ((__attribute__((address_space(1))) T*)(p))
-
-constexpr int kQBlock = 128;   // query rows per workgroup
-constexpr int kQWave = 32;     // query rows per wavefront
-constexpr int kKvBlock = 64;   // kv rows per online-softmax step
-constexpr int kThreads = 256;  // 4 wavefronts
-constexpr int kVersion = 4;
-// main loops (template parameter LOOP of the kernel)
-constexpr int kLoopRolling = 0, kLoopPipelined = 1, kLoopDense = 2;
-
-struct KernelArgs {
-  const uint8_t* q;
-  const uint8_t* k;
-  const uint8_t* v;
-  void* o;
-  float* lse;  // optional
-  int heads, seqlen_q, seqlen_k, n_qblocks, bh_total;
-  int kv_group;      // q heads per k/v head
-  int interleave;    // causal: how many heads deal their q blocks alternately (see decode_block)
-  int causal_shift;  // key j is visible to query i when j <= i + causal_shift
-  float scale_log2;  // softmax_scale * log2(e)
-  long long q_bs, q_hs, q_rs;
-  long long k_bs, k_hs, k_rs;
-  long long v_bs, v_hs, v_rs;
-  long long o_bs, o_hs, o_rs;
-  long long lse_bs, lse_hs;
-};
-
-// LDS row r (0..63) of a K tile holds kv row kv_of_lds_row(r) of the block.  With this order the 16
-// accumulator registers a lane gets from S^T sub-tile t (rows 8a+4h+b of the 32x32 result, h = lane/32)
-// are kv rows 32h+16t+(4a+b): exactly the bytes 16t..16t+15 of the lane's B operand in the PV MFMA.
-__device__ __forceinline__ int kv_of_lds_row(int r) {
-  const int t = r >> 5, a = (r >> 3) & 3, h = (r >> 2) & 1, b = r & 3;
-  return 32 * h + 16 * t + 4 * a + b;
-}
-
-// Swizzle: a tile is an array of 128-byte lines of eight 16-byte chunks.  A row of D bytes is two lines (D = 256),
-// one line (128), half a line (64) or a quarter (32).  The chunk position inside its line is XORed with a key
-// taken from the row (line) number, chosen so that the eight lanes the LDS serves together (eight consecutive
-// rows, same chunk) fall on eight different positions, for the K reads and for the transposing V reads alike.
-template <int D, bool IS_V>
-__device__ __forceinline__ int tile_offset(int row, int chunk) {
-  if constexpr (D == 256) {
-    const int key = IS_V ? (row & 7) : ((row & 7) ^ ((row >> 3) & 1));
-    return row * 256 + ((chunk >> 3) << 7) + (((chunk & 7) ^ key) << 4);
-  } else if constexpr (D == 128) {
-    const int key = IS_V ? (row & 7) : ((row & 7) ^ ((row >> 3) & 1));
-    return row * 128 + ((chunk ^ key) << 4);
-  } else if constexpr (D == 64) {
-    const int line = row >> 1;
-    const int key = IS_V ? (line & 3) : ((line & 3) ^ ((line >> 2) & 1));
-    return line * 128 + ((((row & 1) << 2) | (chunk ^ key)) << 4);
-  } else {
-    static_assert(D == 32, "head dims: 32, 64, 128, 256");
-    const int line = row >> 2;
-    return line * 128 + ((((row & 3) << 1) | (chunk ^ (line & 1))) << 4);
-  }
-}
-
-// Inverse of tile_offset for the copy engine: which (row, chunk) lives at 16-byte slot `slot`.
-template <int D, bool IS_V>
-__device__ __forceinline__ void tile_slot_decode(int slot, int& row, int& chunk) {
-  if constexpr (D == 256) {
-    row = slot >> 4;
-    const int key = IS_V ? (row & 7) : ((row & 7) ^ ((row >> 3) & 1));
-    chunk = (slot & 8) | ((slot & 7) ^ key);
-  } else if constexpr (D == 128) {
-    row = slot >> 3;
-    const int key = IS_V ? (row & 7) : ((row & 7) ^ ((row >> 3) & 1));
-    chunk = (slot & 7) ^ key;
-  } else if constexpr (D == 64) {
-    const int line = slot >> 3, w = slot & 7;
-    const int key = IS_V ? (line & 3) : ((line & 3) ^ ((line >> 2) & 1));
-    row = line * 2 + (w >> 2);
-    chunk = (w & 3) ^ key;
-  } else {
-    const int line = slot >> 3, w = slot & 7;
-    row = line * 4 + (w >> 1);
-    chunk = (w & 1) ^ (line & 1);
-  }
-}
-
-// v_permlane32_swap exchanges lanes 32-63 of its first operand with lanes 0-31 of its second.  Fed the same
-// value x twice it returns {x of the low half-lane, x of the high half-lane} in every lane of a query.
-typedef unsigned v2u __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float lane32_max(float x) {
-  const v2u r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  // median(a, b, +inf) = max(a, b) in one instruction (fmaxf would first quiet both operands); the +inf is made opaque to
-  // the optimiser, which would otherwise turn the median back into that max
-  float inf = INFINITY;
-  asm("" : "+v"(inf));
-  return __builtin_amdgcn_fmed3f(__uint_as_float(r[0]), __uint_as_float(r[1]), inf);
-}
-__device__ __forceinline__ float lane32_sum(float x) {
-  const v2u r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// max of three floats; the compiler fuses the pair into one v_max3_f32.
-__device__ __forceinline__ float max3(float a, float b, float c) { return __builtin_fmaxf(__builtin_fmaxf(a, b), c); }
-
-template <bool E5M2>
-__device__ __forceinline__ v16f mfma_fp8(const v8i& a, const v8i& b, const v16f& c) {
-  if constexpr (E5M2)
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 1, 1, 0, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
-}
-
-template <bool E5M2>
-__device__ __forceinline__ int pack4_fp8(float a, float b, float c, float d) {
-  int r;
-  asm volatile("" : "=v"(r));  // any value will do (both 16-bit halves are overwritten below): defines r, emits nothing
-  if constexpr (E5M2) {
-    r = __builtin_amdgcn_cvt_pk_bf8_f32(a, b, r, false);
-    r = __builtin_amdgcn_cvt_pk_bf8_f32(c, d, r, true);
-  } else {
-    r = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, r, false);
-    r = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, r, true);
-  }
-  return r;
-}
+using namespace fa8;
 
 // Workgroup id -> (batch*head, q block).  Workgroups are dealt to the 8 XCDs round-robin by id; when
 // batch*heads is a multiple of 8 all q blocks of one head are kept on one XCD so its K/V stay in that
@@ -1081,6 +955,50 @@ int choose_loop(const Fa8FwdParams* p) {
   return small ? FA8_SCHEDULE_PIPELINED : FA8_SCHEDULE_ROLLING;
 }
 
+// How the work of a call is cut (see fa8_fwd_kernel, fa8_shared_rows_kernel).
+struct Plan {
+  int tiles_per_workgroup;  // of 32 query rows
+  int waves_per_tile;       // 1: the loops of this file; 2, 4: wavefronts share a row tile
+};
+
+// The rule, from a sweep over head dims 32 / 64 / 96 / 128 / 160 / 256, 1 - 128 heads, 128 - 8192 keys, full and causal (each plan timed
+// on each shape).  A SIMD with one wavefront issues a vector instruction every 6 - 9 cycles, with three every 3: a launch of few
+// rows is faster if several wavefronts share a row tile, up to the point where the unshared loops have about two wavefronts
+// on every SIMD themselves.  `tiles` counts 32-row tiles (the query rows of a k/v head together), `even` the tiles of the
+// longest tile's length that hold the same work (causal square: half as many): what counts for a launch that starts its longest tiles
+// first.
+//   tiles <= CUs (head dim <= 64: 2 CUs): four wavefronts a tile, one tile a workgroup            1.2x (128 keys) - 2x (8192 keys)
+//   head dim 65 - 128, tiles <= 2 CUs: four wavefronts a tile, two tiles a workgroup (the tiles share the copies of K and V; two
+//     one-tile workgroups do not fit a CU's LDS)                                                  1.25 - 1.7x
+//   even <= 2 CUs (head dim <= 64: 4 CUs; causal: a quarter more): two wavefronts a tile, two tiles a workgroup      1.04 - 1.3x
+Plan choose_plan(const Fa8FwdParams* p) {
+  const Plan unshared = {kQBlock / 32, 1};
+  // the sharing kernels rely on exp2(-inf * scale) = 0 and a finite start of the row max, like the pipelined loop; a schedule hint
+  // asks for a loop of the unshared kernel
+  if (p->schedule != FA8_SCHEDULE_AUTO || !(p->softmax_scale > 0.f && p->softmax_scale < 1.0e6f) || !packable(p)) return unshared;
+  const long long cus = compute_units();
+  const long long group = p->heads_k > 0 ? p->heads / p->heads_k : 1, kv_heads = (long long)p->batch * (p->heads / group);
+  const long long rows = group * p->seqlen_q, tiles = kv_heads * ((rows + 31) / 32);
+  if (tiles > 8 * cus || p->batch > 65535) return unshared;  // (also when the number of compute units is unknown)
+  const long long shift = p->causal_align == FA8_CAUSAL_BOTTOM_RIGHT ? (long long)p->seqlen_k - p->seqlen_q : 0;
+  auto blocks_of = [&](long long q_last) {  // KV blocks that query q_last sees, at least one
+    const long long keys = p->is_causal ? std::min<long long>(p->seqlen_k, q_last + 1 + shift) : p->seqlen_k;
+    return std::max(1LL, (keys + kKvBlock - 1) / kKvBlock);
+  };
+  const long long longest = blocks_of(p->seqlen_q - 1), shortest = blocks_of(std::min<long long>(31 / group, p->seqlen_q - 1));
+  // mean length of the tiles: half way between the first and the last one, but for rows that see every key or none
+  const long long even = tiles * (longest + shortest) / (2 * longest);
+  const int d = p->head_dim;
+  Plan n = unshared;
+  if (tiles <= (d <= 64 ? 2 : 1) * cus)
+    n = {1, 4};
+  else if (d > 64 && d <= 128 && tiles <= 2 * cus && longest > 2)
+    n = {2, 4};
+  else if (4 * even <= (d <= 64 ? 4 : 2) * (p->is_causal ? 5 : 4) * cus)
+    n = {2, 2};
+  return n;
+}
+
 // Tuning aid for measurements only: FA8_CAUSAL_INTERLEAVE=n in the environment (read once) replaces the number of heads of an
 // XCD that take turns at every q block of a causal launch (see decode_block; the results do not depend on it).  0: unset.
 int env_causal_interleave() {
@@ -1153,9 +1071,10 @@ extern "C" int fa8_fwd_validate(const Fa8FwdParams* p) {
   return FA8_OK;
 }
 
-extern "C" int fa8_fwd(const Fa8FwdParams* p, void* hip_stream) {
-  const int rc = fa8_fwd_validate(p);
-  if (rc != FA8_OK) return rc;
+namespace {
+
+// One wavefront per 32 query rows: the kernel of this file.
+int launch_rows(const Fa8FwdParams* p, hipStream_t stream) {
   KernelArgs a;
   a.q = (const uint8_t*)p->q;
   a.k = (const uint8_t*)p->k;
@@ -1177,7 +1096,6 @@ extern "C" int fa8_fwd(const Fa8FwdParams* p, void* hip_stream) {
   a.k_bs = p->k_batch_stride; a.k_hs = p->k_head_stride; a.k_rs = p->k_row_stride;
   a.v_bs = p->v_batch_stride; a.v_hs = p->v_head_stride; a.v_rs = p->v_row_stride;
   a.o_bs = p->o_batch_stride; a.o_hs = p->o_head_stride; a.o_rs = p->o_row_stride;
-  hipStream_t stream = (hipStream_t)hip_stream;
   const int loop = choose_loop(p);
   switch (p->head_dim) {
 #define FA8_HEAD_DIM_CASE(D_) \
@@ -1193,6 +1111,29 @@ extern "C" int fa8_fwd(const Fa8FwdParams* p, void* hip_stream) {
 #undef FA8_HEAD_DIM_CASE
     default: return FA8_ERR_HEAD_DIM;
   }
+}
+
+}  // namespace
+
+extern "C" int fa8_fwd(const Fa8FwdParams* p, void* hip_stream) {
+  const int rc = fa8_fwd_validate(p);
+  if (rc != FA8_OK) return rc;
+  const Plan n = choose_plan(p);
+  const hipStream_t stream = (hipStream_t)hip_stream;
+  return n.waves_per_tile > 1 ? launch_shared(p, n.tiles_per_workgroup, n.waves_per_tile, stream) : launch_rows(p, stream);
+}
+
+extern "C" int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* rows_per_workgroup, int32_t* wavefronts_per_tile,
+                            int32_t* kv_splits) {
+  const int rc = fa8_fwd_validate(p);
+  if (rc != FA8_OK) return rc;
+  if (rows_per_workgroup == nullptr || wavefronts_per_tile == nullptr || kv_splits == nullptr) return FA8_ERR_NULL;
+  (void)with_workspace;
+  const Plan n = choose_plan(p);
+  *rows_per_workgroup = 32 * n.tiles_per_workgroup;
+  *wavefronts_per_tile = n.waves_per_tile;
+  *kv_splits = 1;
+  return FA8_OK;
 }
 
 extern "C" int fa8_fwd_schedule(const Fa8FwdParams* p) {

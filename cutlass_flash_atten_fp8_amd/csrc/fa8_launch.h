@@ -1,0 +1,14 @@
+// Launchers of the kernels that live in source files of their own, called by fa8_fwd.
+#ifndef FA8_LAUNCH_H_
+#define FA8_LAUNCH_H_
+#include <hip/hip_runtime.h>
+
+#include "fa8_api.h"
+
+namespace fa8 {
+
+// r row tiles of 32 query rows per workgroup, w wavefronts per row tile (fa8_shared_rows.h)
+__attribute__((visibility("hidden"))) int launch_shared(const Fa8FwdParams* p, int r, int w, hipStream_t stream);
+
+}  // namespace fa8
+#endif  // FA8_LAUNCH_H_

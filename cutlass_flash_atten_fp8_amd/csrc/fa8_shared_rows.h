@@ -1,0 +1,483 @@
+// Attention for launches with few query rows per compute unit: R tiles of 32 query rows per workgroup, each tile shared by W
+// wavefronts (the kernels of fa8_fwd_gfx950.hip give a tile to one wavefront).
+//
+// W KV blocks of 64 rows are in work at a time.  Wavefront w of a tile computes S^T, the row max and the weights of block w; the
+// row maxima of the W blocks meet in LDS, so every wavefront follows the running max block by block, exactly as one wavefront
+// walking the blocks would.  The fp8 weights go through LDS too, and wavefront w then adds the W blocks, in order, to ITS
+// 32-column tiles of O^T (tiles w, w + W, ...).  Every logit, weight and sum is formed by the same instructions in the same order
+// as in the other kernels: the results are equal bit for bit.
+//
+// One iteration, one group of W blocks (STAGES == 2; the copies fly for an iteration or more):
+//   row max of the group's S -> LDS | barrier 1 | running max; weights of sub-tile 0, PV products of the group before between their
+//   chunks, copy of K two groups ahead | barrier 2 | weights of sub-tile 1, S^T products of the next group between their chunks, copy of
+//   V of the next group; weights and row sums -> LDS
+// Head dims above 128 have LDS for one stage only: the copies of the next group's K and this group's V fly for half an iteration.
+//
+// What bounds it: the issue of vector instructions by the one or two wavefronts of a SIMD (about 200 a wavefront and iteration, each
+// 6 - 9 cycles apart with so few wavefronts) and two barriers an iteration, 3900 cycles at R = 2, W = 4; with fewer stages or all copies
+// of a half iteration started at its beginning the copies are the limit (4100 - 4700).  Measured (us, one wavefront a tile -> shared):
+// 16 heads, 1024 keys, causal: head dim 64 13.3 -> 8.9 (R 1, W 4), 128 17.2 -> 12.4 (2, 4); 8 heads of 2048 keys, head dim 128, full: 28.5 ->
+// 19.5 (2, 4); 512 queries on 16384 keys, 32 heads on 8 k/v heads: 176 -> 100 (2, 4); 16 heads, 2048 keys, head dim 256, causal: 47.1 ->
+// 37.7 (2, 2); 1 query of 32 heads on 8 k/v heads, 16 sequences of 8191 keys: 145 -> 52, the rate of a plain copy (1, 4).
+#ifndef FA8_SHARED_ROWS_H_
+#define FA8_SHARED_ROWS_H_
+#include <type_traits>
+
+#include "fa8_device.h"
+
+namespace fa8 {
+
+constexpr float kMaxStart = -1.0e30f;  // below every possible logit, finite: see m_run in fa8_fwd_kernel
+
+// 112 bytes: a larger argument block makes the launch itself slower on the host (2.75 us up to 112 bytes, 3.4 - 3.6 us from 120 on,
+// an empty kernel in a loop).  Strides are in units of 16 elements (q, k, v) and 4 elements (o); see packable and pack_mode.
+struct SharedArgs {
+  const uint8_t* q;
+  const uint8_t* k;
+  const uint8_t* v;
+  void* o;
+  float* lse;
+  float scale_log2;
+  int seqlen_q, seqlen_k;
+  unsigned mode;  // see pack_mode
+  unsigned q_bs, q_hs, q_rs;
+  unsigned k_bs, k_hs, k_rs;
+  unsigned v_bs, v_hs, v_rs;
+  unsigned o_bs, o_hs, o_rs;
+  unsigned lse_bs, lse_hs;
+};
+static_assert(sizeof(SharedArgs) == 112, "see above");
+
+template <int D, bool E5M2, bool VT, int R, int W, int STAGES>
+__global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2))) void fa8_shared_rows_kernel(const SharedArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int DP = D <= 32 ? 32 : (D <= 64 ? 64 : (D <= 128 ? 128 : 256));
+  constexpr int kTileBytes = kKvBlock * DP;
+  constexpr int kKSteps = (D + 63) / 64;
+  constexpr int kMTiles = D / 32;
+  constexpr int kOwn = (kMTiles + W - 1) / W;     // O^T tiles of a wavefront (the last wavefronts may have one less, or none)
+  constexpr int kSegs = kTileBytes / 1024;        // 1 KB copy segments per K or V tile, shared by the R wavefronts of a block
+  static_assert(kSegs % R == 0, "a block's copy is split evenly over the row tiles");
+  constexpr int kPasses = kSegs / R;
+  // two stages each, separate objects: the compiler then knows that copies in flight do not alias the reads (see fa8_fwd_kernel)
+  __shared__ __attribute__((aligned(1024))) uint8_t k_lds0[W * kTileBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t k_lds1[STAGES == 2 ? W * kTileBytes : 16];
+  __shared__ __attribute__((aligned(1024))) uint8_t v_lds0[W * kTileBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t v_lds1[STAGES == 2 ? W * kTileBytes : 16];
+  __shared__ __attribute__((aligned(1024))) uint8_t p_lds[R * W * 2048];
+  __shared__ float max_lds[R * W * 32];
+  __shared__ float sum_lds[R * W * 64];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = wave / W, w = wave - r * W;  // row tile of the workgroup, block of the group
+  const int qn = lane & 31, h = lane >> 5;
+
+  // grid: k/v heads x batches x row tiles.  Workgroups start in that order (x fastest) and go to the XCDs in turn, so a k/v head
+  // stays on one XCD when there is a multiple of 8 of them; causal: the longest tiles of all heads first.
+  const bool causal = a.mode & kSharedCausal;
+  const int group = (int)(a.mode >> kSharedGroup), group_shift = (int)(a.mode >> kSharedShift) & 31;
+  const int hk = blockIdx.x, b = blockIdx.y;
+  const int tile = causal ? (int)(gridDim.z - 1 - blockIdx.z) : (int)blockIdx.z;
+  // The query rows of a k/v head: row x is query x / group of q head x % group of the group.
+  auto query_of = [&](int x) __attribute__((always_inline)) { return group_shift < 31 ? x >> group_shift : x / group; };
+  const int last_row = group * a.seqlen_q - 1;
+  const int row0 = (tile * R + r) * 32;  // first row of this wavefront's tile
+  const int row = row0 + qn;
+  const int k_rs = (int)a.k_rs * 16, v_rs = (int)a.v_rs * 16;
+  const uint8_t* kp = a.k + ((unsigned long long)a.k_bs * b + (unsigned long long)a.k_hs * hk) * 16;
+  const uint8_t* vp = a.v + ((unsigned long long)a.v_bs * b + (unsigned long long)a.v_hs * hk) * 16;
+  const float c = a.scale_log2;
+
+  // ---- HBM -> LDS copies (see fa8_fwd_kernel): wavefront (r, w) copies segments r, r + R, ... of block w of a group ----
+  constexpr unsigned kNoSource = 0x80000000u;
+  // A lane's offset in a segment depends on the segment number through few of its bits (the swizzle) and otherwise by whole rows:
+  // segments that are kKVar (kVVar) apart differ by a multiple of the row stride.
+  constexpr int kKVar = DP == 256 ? 4 : (DP == 128 ? 2 : 1);
+  constexpr int kVVar = DP == 256 && !VT ? 2 : 1;
+  // row of the block that a segment's rows count from (V^T: row of the tile)
+  auto k_row0 = [](int seg) {
+    if (DP == 256) return 16 * (seg >> 3) + 4 * ((seg >> 1) & 3) + 32 * (seg & 1);
+    if (DP == 128) return 16 * (seg >> 2) + 4 * (seg & 3);
+    return DP == 64 ? 16 * (seg >> 1) + 8 * (seg & 1) : 16 * seg;
+  };
+  auto v_row0 = [](int seg) { return seg * (VT ? 16 : 1024 / DP); };
+  unsigned k_src[kPasses], v_src[kPasses];
+#pragma unroll
+  for (int p = 0; p < kPasses; ++p) {
+    const int seg = p * R + r;
+    constexpr int nk = kKVar > R ? kKVar / R : 1, nv = kVVar > R ? kVVar / R : 1;
+    if (p < nk) {
+      int tr, ch;
+      tile_slot_decode<DP, false>(seg * 64 + lane, tr, ch);
+      k_src[p] = ch * 16 < D ? (unsigned)(kv_of_lds_row(tr) * k_rs + ch * 16) : kNoSource;
+    } else {
+      k_src[p] = k_src[p % nk] + (unsigned)((k_row0(seg) - k_row0(p % nk * R + r)) * k_rs);
+    }
+    if (p < nv) {
+      int tr, ch;
+      tile_slot_decode<VT ? 64 : DP, !VT>(seg * 64 + lane, tr, ch);
+      v_src[p] = VT || ch * 16 < D ? (unsigned)(tr * v_rs + ch * 16) : kNoSource;
+    } else {
+      v_src[p] = v_src[p % nv] + (unsigned)((v_row0(seg) - v_row0(p % nv * R + r)) * v_rs);
+    }
+  }
+  const int kv_last = a.seqlen_k - 1;
+  constexpr int kRsrcFlags = 0x00020000;
+  // Every step starts its copies, also of blocks that do not exist (through a resource of length 0), so that the number of loads
+  // in flight is the same at every step.
+  const int k_bytes = kv_last * k_rs + D;
+  const int v_bytes = VT ? (D - 1) * v_rs + a.seqlen_k : kv_last * v_rs + D;
+  auto issue_k = [&](int j, uint8_t* dst, bool exists, int from, int to) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)kp, 0, exists ? k_bytes : 0, kRsrcFlags);
+    const int base = (int)((unsigned)(exists ? j : 0) * kKvBlock * (unsigned)k_rs);
+#pragma unroll
+    for (int p = from; p < to; ++p)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, dst + w * kTileBytes + (p * R + r) * 1024), 16, k_src[p], base, 0, 0);
+  };
+  auto issue_v = [&](int j, uint8_t* dst, bool exists, int from, int to) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)vp, 0, exists ? v_bytes : 0, kRsrcFlags);
+    const int base = !exists ? 0 : (VT ? j * kKvBlock : (int)((unsigned)j * kKvBlock * (unsigned)v_rs));
+    const bool v_clamp = VT && exists && (j + 1) * kKvBlock > a.seqlen_k;
+#pragma unroll
+    for (int p = from; p < to; ++p) {
+      uint8_t* at = dst + w * kTileBytes + (p * R + r) * 1024;
+      if (v_clamp) {  // transposed v, ragged last block: see fa8_fwd_kernel
+        int tr, ch;
+        tile_slot_decode<64, false>((p * R + r) * 64 + lane, tr, ch);
+        const unsigned off = tr < D ? (unsigned)(tr * v_rs + min(j * kKvBlock + ch * 16, a.seqlen_k - 16)) : kNoSource;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, at), 16, off, 0, 0, 0);
+      } else {
+        // (transposed v: rows of the tile past the head dim lie past the resource or are never read)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, at), 16, v_src[p], base, 0, 0);
+      }
+    }
+  };
+
+  // ---- KV blocks: of this row tile (blocks), of the workgroup (all_blocks), and the leading ones without a mask ----
+  const int shift = (a.mode & kSharedBottomRight) ? a.seqlen_k - a.seqlen_q : 0;
+  auto blocks_of = [&](int first_row) __attribute__((always_inline)) {  // of the 32-row tile that starts at first_row
+    if (!causal) return (a.seqlen_k + kKvBlock - 1) / kKvBlock;
+    return max(1, (min(a.seqlen_k, query_of(min(first_row + 31, last_row)) + 1 + shift) + kKvBlock - 1) / kKvBlock);
+  };
+  const int blocks = blocks_of(row0);
+  const int all_blocks = R == 1 ? blocks : blocks_of((tile * R + R - 1) * 32);
+  const int n_plain = (causal ? max(0, min(query_of(min(row0, last_row)) + shift, a.seqlen_k)) : a.seqlen_k) / kKvBlock;
+  const int rc = min(row, last_row);
+  const int qi = query_of(rc);
+  const int hd = hk * group + (rc - qi * group);
+  const int kv_limit = causal ? min(qi + shift, kv_last) : kv_last;
+
+  // ---- Q fragment ----
+  v8i qf[kKSteps];
+  {
+    const uint8_t* src = a.q + ((unsigned long long)a.q_bs * b + (unsigned long long)a.q_hs * hd + (unsigned long long)a.q_rs * qi) * 16;
+#pragma unroll
+    for (int ks = 0; ks < kKSteps; ++ks) {
+      const bool upper_exists = 64 * ks + 32 < D;
+      const uint8_t* s8 = src + 64 * ks + (upper_exists ? 32 * h : 0);
+      const v4i lo = *(const v4i*)(s8);
+      const v4i hi = *(const v4i*)(s8 + 16);
+      qf[ks] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      if (!upper_exists && h) qf[ks] = v8i{0, 0, 0, 0, 0, 0, 0, 0};
+    }
+  }
+  issue_k(w, k_lds0, w < all_blocks, 0, kPasses);
+  if constexpr (STAGES == 2) issue_k(w + W, k_lds1, w + W < all_blocks, 0, kPasses);
+  issue_v(w, v_lds0, w < all_blocks, 0, kPasses);
+  // ---- LDS read offsets (see fa8_fwd_kernel) ----
+  int k_off[kKSteps][2];
+#pragma unroll
+  for (int ks = 0; ks < kKSteps; ++ks)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) k_off[ks][e] = w * kTileBytes + tile_offset<DP, false>(qn, DP >= 64 ? 4 * ks + 2 * h + e : e);
+  constexpr int kSubTileStride = 32 * DP, kVtTileStride = 32 * 64, kTrStride = 8 * DP;
+  const int tr_j = (lane & 15) >> 1, tr_e = lane & 1, tr_g1 = (lane >> 4) & 1;
+  int v_off[kOwn][VT ? 2 : 1];
+#pragma unroll
+  for (int m = 0; m < kOwn; ++m) {
+    const int mt = min(w + m * W, kMTiles - 1);
+    if constexpr (VT) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) v_off[m][e] = mt * kVtTileStride + tile_offset<64, false>(qn, 2 * h + e);
+    } else {
+      v_off[m][0] = tile_offset<DP, true>(32 * h + tr_j, 2 * mt + tr_g1) + 8 * tr_e;
+    }
+  }
+  auto load_vf = [&](const uint8_t* v_lds, int i, int m) __attribute__((always_inline)) {
+    const uint8_t* vb = v_lds + i * kTileBytes;
+    v8i vf;
+    if constexpr (VT) {
+      const v4i lo = *LDS_PTR(const v4i, vb + v_off[m][0]);
+      const v4i hi = *LDS_PTR(const v4i, vb + v_off[m][VT ? 1 : 0]);
+      vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    } else {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const v2i x = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, vb + v_off[m][0] + g * kTrStride));
+        vf[2 * g] = x[0];
+        vf[2 * g + 1] = x[1];
+      }
+    }
+    return vf;
+  };
+
+  v16f o_acc[kOwn];
+#pragma unroll
+  for (int m = 0; m < kOwn; ++m)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o_acc[m][i] = 0.f;
+  float m_run = kMaxStart, l_run = 0.f;
+  // rescale factors of the group whose PV products are due, and whether any row of the tile needs them
+  float alpha[W];
+  bool changed[W];
+  auto load_kf = [&](const uint8_t* k_lds, int t, int ks) __attribute__((always_inline)) {
+    const v4i lo = *LDS_PTR(const v4i, k_lds + t * kSubTileStride + k_off[ks][0]);
+    const v4i hi = *LDS_PTR(const v4i, k_lds + t * kSubTileStride + k_off[ks][1]);
+    return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  };
+  auto load_pf = [&](int i) __attribute__((always_inline)) {
+    const v4i lo = *LDS_PTR(const v4i, p_lds + (r * W + i) * 2048 + lane * 16);
+    const v4i hi = *LDS_PTR(const v4i, p_lds + (r * W + i) * 2048 + 1024 + lane * 16);
+    return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  };
+  auto s_product = [&](v16f& acc, int ks, const v8i& kf) __attribute__((always_inline)) {
+    if (ks == 0) {
+      v16f z;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) z[i] = 0.f;
+      acc = mfma_fp8<E5M2>(kf, qf[ks], z);
+    } else {
+      acc = mfma_fp8<E5M2>(kf, qf[ks], acc);
+    }
+  };
+  // brings O and l to the running max after block i of the group and adds the block's row sums
+  auto rescale = [&](int i, float sum) __attribute__((always_inline)) {
+#pragma clang fp contract(off)
+    if (changed[i]) {
+      l_run = l_run * alpha[i];
+      if (alpha[i] != 1.f) {
+#pragma unroll
+        for (int m = 0; m < kOwn; ++m)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) o_acc[m][e] *= alpha[i];
+      }
+    }
+    l_run = l_run + sum;
+  };
+  // Barrier once this wavefront's LDS operations are done and all but its latest `copies` tile copies have landed (vmcnt counts a
+  // lane's loads in issue order).  Bare s_barrier: __syncthreads() would wait for all copies.
+  auto sync = [&](auto copies_c) __attribute__((always_inline)) {
+    constexpr int n = decltype(copies_c)::value * kPasses;
+    static_assert(n < 64, "vmcnt has six bits");
+    __builtin_amdgcn_s_waitcnt(0x0070 | (n & 15) | (n >> 4 << 14));
+    __builtin_amdgcn_s_barrier();
+  };
+  constexpr std::integral_constant<int, 0> none{};
+  constexpr bool kAllOwn = kMTiles % W == 0;  // every wavefront has kOwn tiles of O^T
+  auto owns = [&](int m) __attribute__((always_inline)) { return kAllOwn || w + m * W < kMTiles; };
+  constexpr int kPv = W * kOwn, kS = 2 * kKSteps;  // matrix instructions of an iteration
+  v16f sbuf[2][2];
+  v8i p8;
+
+  auto iteration = [&](auto first_c, auto parity_c, int g) __attribute__((always_inline)) {
+    constexpr int PH = decltype(parity_c)::value;
+    v16f(&s)[2] = sbuf[PH];
+    v16f(&sn)[2] = sbuf[PH ^ 1];
+    constexpr bool kTwo = STAGES == 2;
+    uint8_t* const k_this = kTwo && PH ? k_lds1 : k_lds0;
+    uint8_t* const k_next = kTwo && !PH ? k_lds1 : k_lds0;
+    uint8_t* const v_prev = kTwo && !PH ? v_lds1 : v_lds0;
+    constexpr bool kFirst = decltype(first_c)::value;
+    const int j = g * W + w;
+    const bool more = (g + 1) * W < all_blocks;  // workgroup-uniform
+    if (j >= n_plain) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (j * kKvBlock + 32 * h + 16 * t + i > kv_limit) s[t][i] = -INFINITY;
+    }
+    float mx[4];
+#pragma unroll
+    for (int ch = 0; ch < 4; ++ch) mx[ch] = max3(s[0][4 * ch], s[0][4 * ch + 1], s[0][4 * ch + 2]);
+#pragma unroll
+    for (int ch = 0; ch < 4; ++ch) mx[ch] = max3(mx[ch], s[0][4 * ch + 3], s[1][4 * ch]);
+#pragma unroll
+    for (int ch = 0; ch < 4; ++ch) mx[ch] = max3(mx[ch], s[1][4 * ch + 1], s[1][4 * ch + 2]);
+    const float bm = lane32_max(max3(max3(mx[0], s[1][3], s[1][7]), max3(mx[1], s[1][11], s[1][15]), max3(mx[2], mx[3], m_run)));
+    if (h == 0) max_lds[wave * 32 + qn] = bm;
+    sync(std::integral_constant<int, kTwo || kFirst ? 1 : 0>());  // barrier 1: row maxima; weights, row sums and V of group g - 1; K of group g + 1; K of group g has been read
+    v8i vfrag[kPv], pfrag[W], kfrag[kS];
+    float sums[W], maxima[W];
+#pragma unroll
+    for (int i = 0; i < W; ++i) maxima[i] = max_lds[(r * W + i) * 32 + qn];
+    if constexpr (!kFirst) {
+      pfrag[0] = load_pf(0);
+      if (owns(0)) vfrag[0] = load_vf(v_prev, 0, 0);
+#pragma unroll
+      for (int i = 0; i < W; ++i) sums[i] = sum_lds[(r * W + i) * 64 + lane];
+    }
+    float m_after[W], m_own = m_run;
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      m_after[i] = __builtin_fmaxf(i == 0 ? m_run : m_after[i - 1], maxima[i]);
+      if (i == w) m_own = m_after[i];
+    }
+    const float mc = m_own * c;
+    float sum0, sum1;
+    __builtin_amdgcn_sched_barrier(0);
+    // The softmax of 4 weights a chunk, three stages deep so that no instruction waits for the one before it: exponentials of
+    // chunk u, their arguments for chunk u + 1, row sum and fp8 packing of chunk u - 1.  The scheduling barriers keep that order.
+    float y[2][4], x[2][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y[0][i] = __builtin_fmaf(s[0][i], c, -mc);
+    auto pack = [&](int u) __attribute__((always_inline)) {
+      int packed = pack4_fp8<E5M2>(x[u & 1][0], x[u & 1][1], x[u & 1][2], x[u & 1][3]);
+      asm volatile("" : "+v"(packed));
+      p8[u] = packed;
+    };
+    auto add = [&](int u, int i) __attribute__((always_inline)) {
+      float& sum = i & 1 ? sum1 : sum0;
+      sum = (u == 0 && i < 2) ? x[u & 1][i] : sum + x[u & 1][i];
+    };
+    auto chunk = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[u & 1][i] = __builtin_amdgcn_exp2f(y[u & 1][i]);
+        if (u < 7) y[(u + 1) & 1][i] = __builtin_fmaf(s[(u + 1) >> 2][4 * ((u + 1) & 3) + i], c, -mc);
+        if (u > 0) add(u - 1, i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (u > 0) pack(u - 1);
+      if (u == 7) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) add(7, i);
+        pack(7);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if constexpr (kTwo)
+        issue_k(j + 2 * W, k_this, j + 2 * W < all_blocks, u * kPasses / 4, (u + 1) * kPasses / 4);
+      else if (u == 0)
+        issue_k(j + W, k_this, more && j + W < all_blocks, 0, kPasses);
+      chunk(u);
+      if constexpr (!kFirst) {
+#pragma unroll
+        for (int n = u * kPv / 4; n < (u + 1) * kPv / 4; ++n) {
+          const int i = n / kOwn, m = n % kOwn;
+          if (n + 1 < kPv) {  // operands of the next product
+            if ((n + 1) % kOwn == 0) pfrag[(n + 1) / kOwn] = load_pf((n + 1) / kOwn);
+            if (owns((n + 1) % kOwn)) vfrag[n + 1] = load_vf(v_prev, (n + 1) / kOwn, (n + 1) % kOwn);
+          }
+          if (m == 0) rescale(i, sums[i]);
+          if (owns(m)) o_acc[m] = mfma_fp8<E5M2>(vfrag[n], pfrag[i], o_acc[m]);
+        }
+      }
+      if (kTwo && u == 3) kfrag[0] = load_kf(k_next, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      const float before = i == 0 ? m_run : m_after[i - 1];
+      changed[i] = __any(m_after[i] != before);
+      alpha[i] = changed[i] ? __builtin_amdgcn_exp2f((before - m_after[i]) * c) : 1.f;
+    }
+    m_run = m_after[W - 1];
+    // barrier 2: weights, row sums and V of group g - 1 have been read (LDS operations only; one stage: K of group g + 1 has landed)
+    __builtin_amdgcn_s_waitcnt(kTwo ? 0xC07F : 0x0070);
+    __builtin_amdgcn_s_barrier();
+    if constexpr (!kTwo) {
+      if constexpr (!kFirst) issue_v(j, v_prev, j < all_blocks, 0, kPasses);
+      kfrag[0] = load_kf(k_next, 0, 0);
+    }
+#pragma unroll
+    for (int u = 4; u < 8; ++u) {
+      if (more) {
+#pragma unroll
+        for (int n = ((u - 4) * kS + 3) / 4; n < ((u - 3) * kS + 3) / 4; ++n) {
+          if (n + 1 < kS) kfrag[n + 1] = load_kf(k_next, (n + 1) / kKSteps, (n + 1) % kKSteps);
+          s_product(sn[n / kKSteps], n % kKSteps, kfrag[n]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (kTwo) issue_v(j + W, v_prev, j + W < all_blocks, (u - 4) * kPasses / 4, (u - 3) * kPasses / 4);
+      chunk(u);
+      if (u == 4) *LDS_PTR(v4i, p_lds + wave * 2048 + lane * 16) = v4i{p8[0], p8[1], p8[2], p8[3]};
+    }
+    *LDS_PTR(v4i, p_lds + wave * 2048 + 1024 + lane * 16) = v4i{p8[4], p8[5], p8[6], p8[7]};
+    sum_lds[wave * 64 + lane] = sum0 + sum1;
+  };
+
+  using T = std::true_type;
+  using F = std::false_type;
+  constexpr std::integral_constant<int, 0> even{};
+  constexpr std::integral_constant<int, 1> odd{};
+  sync(std::integral_constant<int, STAGES>());  // K of group 0 landed
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int ks = 0; ks < kKSteps; ++ks) s_product(sbuf[0][t], ks, load_kf(k_lds0, t, ks));
+  const int groups = (all_blocks + W - 1) / W;
+  iteration(T(), even, 0);
+  int g = 1;
+  for (; g + 1 < groups; g += 2) {
+    iteration(F(), odd, g);
+    iteration(F(), even, g + 1);
+  }
+  if (g < groups) iteration(F(), odd, g);
+  sync(none);
+  // the PV products of the last group
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    if ((groups - 1) * W + i < blocks) {
+      rescale(i, sum_lds[(r * W + i) * 64 + lane]);
+      const v8i pf = load_pf(i);
+#pragma unroll
+      for (int m = 0; m < kOwn; ++m)
+        if (owns(m)) o_acc[m] = mfma_fp8<E5M2>(load_vf(STAGES == 1 || (groups & 1) ? v_lds0 : v_lds1, i, m), pf, o_acc[m]);
+    }
+  }
+
+  // ---- epilogue (see fa8_fwd_kernel) ----
+  const float l_tot = lane32_sum(l_run);
+  const float inv = (l_tot == 0.f || l_tot != l_tot) ? 1.f : 1.f / l_tot;
+  if (row > last_row) return;
+  if (a.lse != nullptr && h == 0 && w == 0) {
+    const float lse = l_tot > 0.f ? (m_run * c + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f : (l_tot == 0.f ? -INFINITY : l_tot);
+    a.lse[(unsigned long long)a.lse_bs * b + (unsigned long long)a.lse_hs * hd + qi] = lse;
+  }
+  const unsigned long long o_at = ((unsigned long long)a.o_bs * b + (unsigned long long)a.o_hs * hd + (unsigned long long)a.o_rs * qi) * 4 + 4 * h;
+#pragma unroll
+  for (int m = 0; m < kOwn; ++m) {
+    const int mt = w + m * W;
+    if (kMTiles % W != 0 && mt >= kMTiles) break;
+    if (!(a.mode & kSharedFp8Out)) {
+#pragma unroll
+      for (int a2 = 0; a2 < 4; ++a2) {
+        v4h x;
+#pragma unroll
+        for (int b2 = 0; b2 < 4; ++b2) x[b2] = (_Float16)(o_acc[m][4 * a2 + b2] * inv);
+        *(v4h*)((_Float16*)a.o + o_at + 32 * mt + 8 * a2) = x;
+      }
+    } else {
+      constexpr float kMaxFinite = E5M2 ? 57344.f : 448.f;
+#pragma unroll
+      for (int a2 = 0; a2 < 4; ++a2) {
+        float x[4];
+#pragma unroll
+        for (int b2 = 0; b2 < 4; ++b2) {
+          const float y = o_acc[m][4 * a2 + b2] * inv;
+          x[b2] = (y != y) ? y : fminf(fmaxf(y, -kMaxFinite), kMaxFinite);
+        }
+        *(int*)((uint8_t*)a.o + o_at + 32 * mt + 8 * a2) = pack4_fp8<E5M2>(x[0], x[1], x[2], x[3]);
+      }
+    }
+  }
+#endif
+}
+
+}  // namespace fa8
+#endif  // FA8_SHARED_ROWS_H_

@@ -124,7 +124,16 @@ int fa8_fwd_validate(const Fa8FwdParams* p);
 int fa8_fwd(const Fa8FwdParams* p, void* hip_stream);
 
 /*
- * Which main loop fa8_fwd would run for these arguments on the current device: FA8_SCHEDULE_ROLLING,
+ * How a call would be cut on the current device, for benchmarks and tests (nothing is launched): query rows of a workgroup
+ * (grouped q heads counted together), wavefronts that share 32 of them (1: one of the main loops of fa8_fwd_schedule; 2 or 4: shared
+ * rows, for launches with few of them; a schedule hint always gives 1), and into how many parts the keys of a row are split
+ * (more than 1 only with_workspace).  The results of shared and unshared rows are bitwise the same.
+ */
+int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* rows_per_workgroup, int32_t* wavefronts_per_tile,
+                 int32_t* kv_splits);
+
+/*
+ * Which main loop a wavefront that has its 32 query rows to itself (see fa8_fwd_plan) would run for these arguments on the current device: FA8_SCHEDULE_ROLLING,
  * FA8_SCHEDULE_PIPELINED or FA8_SCHEDULE_DENSE (all > 0), or the FA8_ERR_* code fa8_fwd_validate gives.  Launches nothing.  No counterpart in
  * the reference (one kernel, one loop: csrc/flash_attention.cu:468-534); it makes the library's choice visible to
  * benchmarks and tests.

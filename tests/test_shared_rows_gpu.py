@@ -1,0 +1,90 @@
+"""Launches of few query rows: two or four wavefronts share 32 of them (csrc/fa8_shared_rows.h).  Every logit, weight and sum is formed
+in the same order as by one wavefront, so the result must equal the rolling loop's bit for bit, for every feature of the operator, at
+the edges: a single key, a last group of blocks that is not full, row tiles with rows to spare, a workgroup whose second tile is
+empty, masks that end inside a block, grouped q heads packed into one tile."""
+import pytest
+import torch
+
+import cutlass_flash_atten_fp8_amd as fa
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+E4, E5 = torch.float8_e4m3fn, torch.float8_e5m2
+
+
+def _inputs(seed, B, H, Hk, Nq, Nk, d, dtype):
+    g = torch.Generator().manual_seed(seed)
+    spread = 3.0 if seed % 2 else 1.0
+    return tuple((torch.randn(s, generator=g) * spread).to(dtype).to(DEV) for s in ((B, H, Nq, d), (B, Hk, Nk, d), (B, Hk, Nk, d)))
+
+
+CASES = [
+    # B, H, Hk, Nq, Nk, d, causal, bottom_right, vt, dtype, fp8 out, wavefronts per tile, rows per workgroup
+    (1, 1, 1, 1, 1, 128, False, False, False, E4, False, 4, 32),
+    (1, 2, 2, 33, 64, 64, False, False, False, E4, False, 4, 32),
+    (1, 2, 2, 128, 128, 64, True, False, False, E4, True, 4, 32),
+    (1, 2, 2, 300, 257, 128, False, False, False, E4, False, 4, 32),      # one key in the second group's first block
+    (1, 3, 3, 300, 320, 96, True, True, False, E5, True, 4, 32),
+    (1, 2, 2, 700, 100, 128, True, True, False, E4, False, 4, 32),        # queries that see no key
+    (1, 2, 1, 200, 336, 160, False, False, True, E4, False, 4, 32),       # v^T, ragged last block
+    (2, 6, 2, 5, 777, 192, True, True, False, E4, False, 4, 32),          # 15 packed rows, group of 3
+    (1, 16, 2, 9, 1000, 32, True, True, False, E5, False, 4, 32),
+    (1, 8, 8, 64, 1023, 224, True, True, False, E4, True, 4, 32),
+    (1, 4, 2, 100, 513, 256, True, True, False, E5, True, 4, 32),
+    (1, 16, 16, 1024, 1024, 64, True, False, True, E4, True, 4, 32),
+    (1, 16, 16, 1024, 1024, 128, True, False, False, E4, False, 4, 64),
+    (1, 33, 33, 289, 289, 128, False, False, False, E4, False, 4, 64),    # ten tiles: five workgroups; 330 tiles
+    (1, 30, 30, 270, 330, 96, True, True, False, E5, False, 4, 64),       # nine tiles: the last workgroup's second one is empty
+    (1, 32, 8, 512, 2000, 128, True, True, False, E4, False, 4, 64),
+    (1, 64, 64, 128, 128, 128, False, False, False, E4, False, 4, 32),
+    (1, 128, 128, 128, 128, 128, False, False, False, E4, False, 2, 64),  # two blocks only
+    (1, 32, 32, 1000, 1000, 128, True, False, False, E4, False, 2, 64),
+    (4, 16, 16, 500, 500, 64, False, False, False, E5, False, 2, 64),
+    (1, 60, 60, 545, 545, 32, True, False, False, E4, True, 2, 64),       # 18 tiles
+    (1, 16, 16, 1056, 1056, 256, True, False, True, E5, True, 2, 64),
+    (2, 12, 6, 700, 700, 160, True, False, False, E4, False, 2, 64),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "B{}H{}k{}Nq{}Nk{}d{}".format(*c[:6]) + ("c" if c[6] else "f") + ("vt" if c[8] else ""))
+def test_shared_rows_equal_the_rolling_loop_bitwise(case):
+    B, H, Hk, Nq, Nk, d, causal, br, vt, dt, out8, waves, rows = case
+    q, k, v = _inputs(Nq + Nk + d, B, H, Hk, Nq, Nk, d, dt)
+    if vt:
+        v = v.transpose(2, 3).contiguous()
+    kw = dict(v_transposed=vt, return_lse=True, causal_bottom_right=br, out_dtype=dt if out8 else None)
+    want, want_lse = fa.flash_attention_v2_cutlass(q, k, v, causal, d ** -0.5, schedule=fa.FA8_SCHEDULE_ROLLING, **kw)
+    got = torch.full(want.shape, float("nan"), dtype=torch.float16, device=DEV).to(want.dtype)
+    lse = torch.full_like(want_lse, float("nan"))
+    p = fa.make_params(q, k, v, got, causal, d ** -0.5, vt, lse, br)
+    assert fa.plan(p, with_workspace=False) == (rows, waves, 1)
+    import ctypes
+    rc = fa.lib().fa8_fwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, fa.error_string(rc)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+    assert torch.equal(lse, want_lse)
+
+
+def test_strided_tensors_and_guard_bands():
+    """[B,N,H,d] storage (row stride H * d), NaN codes behind the last key, an output whose padding must stay untouched."""
+    import ctypes
+    B, H, n, d, pad = 2, 3, 200, 128, 72
+    kw = {}
+    q, k, v = (t.permute(0, 2, 1, 3).contiguous() for t in _inputs(5, B, H, H, n, n, d, E4))
+
+    def spread_out(t):
+        buf = torch.full((B, n + pad, H, d), 0x7F, dtype=torch.uint8, device=DEV)
+        buf[:, :n] = t.view(torch.uint8)
+        return buf.view(E4)[:, :n].permute(0, 2, 1, 3)
+
+    obuf = torch.full((B, n + pad, H, d), 777.0, dtype=torch.float16, device=DEV)
+    o = obuf[:, :n].permute(0, 2, 1, 3)
+    p = fa.make_params(spread_out(q), spread_out(k), spread_out(v), o, False, 0.09, **kw)
+    assert fa.plan(p)[1] == 4
+    assert fa.lib().fa8_fwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    want = fa.flash_attention_v2_cutlass(*(t.permute(0, 2, 1, 3).contiguous() for t in (q, k, v)), False, 0.09,
+                                         schedule=fa.FA8_SCHEDULE_ROLLING)[0]
+    torch.cuda.synchronize()
+    assert torch.equal(o.contiguous(), want)
+    assert (obuf[:, n:] == 777.0).all()
