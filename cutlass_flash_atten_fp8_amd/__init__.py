@@ -29,7 +29,7 @@ FA8_CAUSAL_TOP_LEFT, FA8_CAUSAL_BOTTOM_RIGHT = 0, 1
 FA8_SCHEDULE_AUTO, FA8_SCHEDULE_ROLLING, FA8_SCHEDULE_PIPELINED, FA8_SCHEDULE_DENSE = 0, 1, 2, 3
 (FA8_QUERY_VERSION, FA8_QUERY_KV_BLOCK, FA8_QUERY_Q_BLOCK, FA8_QUERY_KV_ASCENDING, FA8_QUERY_THREADS,
  FA8_QUERY_PARAMS_SIZE) = range(6)
-FA8_EXPORTS = ("fa8_fwd_validate", "fa8_fwd", "fa8_fwd_plan", "fa8_fwd_schedule", "fa8_query",
+FA8_EXPORTS = ("fa8_fwd_validate", "fa8_fwd", "fa8_fwd_workspace", "fa8_fwd_ws", "fa8_fwd_plan", "fa8_fwd_schedule", "fa8_query",
                "fa8_error_string")
 
 
@@ -67,6 +67,10 @@ def lib():
         L.fa8_fwd_validate.argtypes = [ctypes.POINTER(Fa8FwdParams)]
         L.fa8_fwd.restype = ctypes.c_int
         L.fa8_fwd.argtypes = [ctypes.POINTER(Fa8FwdParams), ctypes.c_void_p]
+        L.fa8_fwd_workspace.restype = ctypes.c_int
+        L.fa8_fwd_workspace.argtypes = [ctypes.POINTER(Fa8FwdParams), ctypes.POINTER(ctypes.c_int64)]
+        L.fa8_fwd_ws.restype = ctypes.c_int
+        L.fa8_fwd_ws.argtypes = [ctypes.POINTER(Fa8FwdParams), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
         L.fa8_fwd_plan.restype = ctypes.c_int
         L.fa8_fwd_plan.argtypes = [ctypes.POINTER(Fa8FwdParams), ctypes.c_int] + [ctypes.POINTER(ctypes.c_int32)] * 3
         L.fa8_fwd_schedule.restype = ctypes.c_int
@@ -188,7 +192,12 @@ def flash_attention_v2_cutlass(q, k, v, is_causal, softmax_scale, *, v_transpose
     p = make_params(q, k, v, o, is_causal, softmax_scale, v_transposed, lse, causal_bottom_right, schedule)
     with torch.cuda.device(q.device):
         stream = torch.cuda.current_stream(q.device).cuda_stream
-        rc = lib().fa8_fwd(ctypes.byref(p), ctypes.c_void_p(stream))
+        need = ctypes.c_int64()
+        rc = lib().fa8_fwd_workspace(ctypes.byref(p), ctypes.byref(need))
+        if rc == 0:
+            # goes back to torch's allocator on return, for later work of this stream
+            workspace = torch.empty(need.value, dtype=torch.uint8, device=q.device) if need.value else None
+            rc = lib().fa8_fwd_ws(ctypes.byref(p), workspace.data_ptr() if need.value else None, need.value, ctypes.c_void_p(stream))
     if rc != 0:
         raise RuntimeError(f"flash_attention_v2_cutlass: {error_string(rc)} (code {rc})")
     return [o, lse] if return_lse else [o]

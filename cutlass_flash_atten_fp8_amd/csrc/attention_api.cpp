@@ -99,7 +99,13 @@ std::vector<torch::Tensor> flash_attention_v2_cutlass(torch::Tensor q, torch::Te
   // PyTorch-ROCm presents HIP devices under the "cuda" device type; these are its guard and stream for them.
   const c10::hip::HIPGuardMasqueradingAsCUDA device_guard(q.device());
   const hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.device().index()).stream();
-  const int rc = fa8_fwd(&p, (void*)stream);
+  int64_t workspace_bytes = 0;
+  torch::Tensor workspace;  // (goes back to torch's allocator on return, for later work of this stream)
+  int rc = fa8_fwd_workspace(&p, &workspace_bytes);
+  if (rc == FA8_OK) {
+    if (workspace_bytes > 0) workspace = torch::empty({workspace_bytes}, q.options().dtype(at::kByte));
+    rc = fa8_fwd_ws(&p, workspace_bytes > 0 ? workspace.data_ptr() : nullptr, workspace_bytes, (void*)stream);
+  }
   TORCH_CHECK(rc == FA8_OK, "flash_attention_v2_cutlass: ", fa8_error_string(rc), " (code ", rc, ")");
   if (return_lse) return {out, lse};
   return {out};

@@ -955,10 +955,11 @@ int choose_loop(const Fa8FwdParams* p) {
   return small ? FA8_SCHEDULE_PIPELINED : FA8_SCHEDULE_ROLLING;
 }
 
-// How the work of a call is cut (see fa8_fwd_kernel, fa8_shared_rows_kernel).
+// How the work of a call is cut (see fa8_fwd_kernel, fa8_shared_rows_kernel, fa8_split_logits_kernel).
 struct Plan {
   int tiles_per_workgroup;  // of 32 query rows
   int waves_per_tile;       // 1: the loops of this file; 2, 4: wavefronts share a row tile
+  int splits;               // > 1: the keys of a row tile dealt to this many workgroups (needs a workspace)
 };
 
 // The rule, from a sweep over head dims 32 / 64 / 96 / 128 / 160 / 256, 1 - 128 heads, 128 - 8192 keys, full and causal (each plan timed
@@ -971,8 +972,10 @@ struct Plan {
 //   head dim 65 - 128, tiles <= 2 CUs: four wavefronts a tile, two tiles a workgroup (the tiles share the copies of K and V; two
 //     one-tile workgroups do not fit a CU's LDS)                                                  1.25 - 1.7x
 //   even <= 2 CUs (head dim <= 64: 4 CUs; causal: a quarter more): two wavefronts a tile, two tiles a workgroup      1.04 - 1.3x
-Plan choose_plan(const Fa8FwdParams* p) {
-  const Plan unshared = {kQBlock / 32, 1};
+// Splitting the keys as well costs a second kernel and a reduction, about 5 us, and spreads the copies over all compute units:
+// taken where the estimate of its time is below the estimate for sharing (per-block times and rates measured; decode steps).
+Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
+  const Plan unshared = {kQBlock / 32, 1, 1};
   // the sharing kernels rely on exp2(-inf * scale) = 0 and a finite start of the row max, like the pipelined loop; a schedule hint
   // asks for a loop of the unshared kernel
   if (p->schedule != FA8_SCHEDULE_AUTO || !(p->softmax_scale > 0.f && p->softmax_scale < 1.0e6f) || !packable(p)) return unshared;
@@ -991,11 +994,22 @@ Plan choose_plan(const Fa8FwdParams* p) {
   const int d = p->head_dim;
   Plan n = unshared;
   if (tiles <= (d <= 64 ? 2 : 1) * cus)
-    n = {1, 4};
+    n = {1, 4, 1};
   else if (d > 64 && d <= 128 && tiles <= 2 * cus && longest > 2)
-    n = {2, 4};
+    n = {2, 4, 1};
   else if (4 * even <= (d <= 64 ? 4 : 2) * (p->is_causal ? 5 : 4) * cus)
-    n = {2, 2};
+    n = {2, 2, 1};
+  if (workspace && n.waves_per_tile == 4 && n.tiles_per_workgroup == 1 && longest >= 16) {
+    const double us_per_block = d <= 64 ? 0.25 : (d <= 128 ? 0.29 : 0.56);
+    const double kv_bytes = 2.0 * kv_heads * longest * kKvBlock * d, live = rows < 32 ? (double)rows : 32.0;
+    const double s_bytes = 8.0 * tiles * live * longest * kKvBlock;
+    const double shared_us = 4.5 + std::max(us_per_block * longest * ((tiles + cus - 1) / cus), kv_bytes / 5.8e6);
+    const double split_us = 8.5 + (kv_bytes + s_bytes) / 5.0e6;
+    const long long splits = std::min({32LL, (cus + tiles - 1) / tiles, longest / 8});
+    if (splits > 1 && split_us < 0.95 * shared_us && s_bytes < 512.0e6 && tiles * splits < 65536 &&
+        longest / (4 * splits) < 65535)
+      n.splits = (int)splits;
+  }
   return n;
 }
 
@@ -1113,14 +1127,32 @@ int launch_rows(const Fa8FwdParams* p, hipStream_t stream) {
   }
 }
 
+int run(const Fa8FwdParams* p, void* workspace, long long bytes, hipStream_t stream) {
+  Plan n = choose_plan(p, workspace != nullptr);
+  if (n.splits > 1 && bytes < split_workspace(p, n.splits)) n = choose_plan(p, false);
+  if (n.splits > 1) return launch_split(p, n.splits, workspace, stream);
+  return n.waves_per_tile > 1 ? launch_shared(p, n.tiles_per_workgroup, n.waves_per_tile, stream) : launch_rows(p, stream);
+}
+
 }  // namespace
 
 extern "C" int fa8_fwd(const Fa8FwdParams* p, void* hip_stream) {
   const int rc = fa8_fwd_validate(p);
+  return rc != FA8_OK ? rc : run(p, nullptr, 0, (hipStream_t)hip_stream);
+}
+
+extern "C" int fa8_fwd_ws(const Fa8FwdParams* p, void* workspace, int64_t bytes, void* hip_stream) {
+  const int rc = fa8_fwd_validate(p);
+  return rc != FA8_OK ? rc : run(p, workspace, bytes, (hipStream_t)hip_stream);
+}
+
+extern "C" int fa8_fwd_workspace(const Fa8FwdParams* p, int64_t* bytes) {
+  const int rc = fa8_fwd_validate(p);
   if (rc != FA8_OK) return rc;
-  const Plan n = choose_plan(p);
-  const hipStream_t stream = (hipStream_t)hip_stream;
-  return n.waves_per_tile > 1 ? launch_shared(p, n.tiles_per_workgroup, n.waves_per_tile, stream) : launch_rows(p, stream);
+  if (bytes == nullptr) return FA8_ERR_NULL;
+  const Plan n = choose_plan(p, true);
+  *bytes = n.splits > 1 ? split_workspace(p, n.splits) : 0;
+  return FA8_OK;
 }
 
 extern "C" int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* rows_per_workgroup, int32_t* wavefronts_per_tile,
@@ -1128,11 +1160,10 @@ extern "C" int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* 
   const int rc = fa8_fwd_validate(p);
   if (rc != FA8_OK) return rc;
   if (rows_per_workgroup == nullptr || wavefronts_per_tile == nullptr || kv_splits == nullptr) return FA8_ERR_NULL;
-  (void)with_workspace;
-  const Plan n = choose_plan(p);
+  const Plan n = choose_plan(p, with_workspace != 0);
   *rows_per_workgroup = 32 * n.tiles_per_workgroup;
   *wavefronts_per_tile = n.waves_per_tile;
-  *kv_splits = 1;
+  *kv_splits = n.splits;
   return FA8_OK;
 }
 

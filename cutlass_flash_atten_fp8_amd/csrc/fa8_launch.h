@@ -10,5 +10,9 @@ namespace fa8 {
 // r row tiles of 32 query rows per workgroup, w wavefronts per row tile (fa8_shared_rows.h)
 __attribute__((visibility("hidden"))) int launch_shared(const Fa8FwdParams* p, int r, int w, hipStream_t stream);
 
+// Keys of every row tile dealt to at most `splits` workgroups (fa8_split_kv.h): workspace bytes, launch.
+__attribute__((visibility("hidden"))) long long split_workspace(const Fa8FwdParams* p, int splits);
+__attribute__((visibility("hidden"))) int launch_split(const Fa8FwdParams* p, int splits, void* workspace, hipStream_t stream);
+
 }  // namespace fa8
 #endif  // FA8_LAUNCH_H_

@@ -1,0 +1,540 @@
+// Attention for few query rows over many keys (decode steps, short chunks): the keys of a k/v head are dealt to `splits` workgroups of
+// four wavefronts, every wavefront walking its own contiguous range of KV blocks without meeting the others.
+//
+// The fp8 weights are taken against the running row max over ALL keys before them (that is what the other kernels do, and it decides how a
+// weight is rounded), so a range cannot start before the row max of the ranges in front of it is known.  Two passes, one kernel each:
+//   logits  reads K, writes S (fp32, masked, live rows only) and the row max of every range
+//   values  starts from the max over the ranges before its own, reads S and V, writes O, l and the max of its range; the workgroup
+//           that ends last for a row tile adds the ranges up (factors exp2((m_range - m_last) * c) <= 1: the maxima only grow)
+// Logits, weights and products are those of the other kernels bit for bit; only the order of the fp32 sums over the ranges is another.
+//
+// Bound: HBM bytes.  K and V are read once; S costs 8 bytes per row and key against 2 * head_dim bytes per key for K and V, which is why
+// the logits are kept instead of read K again (head dim 128: fewer bytes up to 16 rows a tile, and S comes out of the Infinity
+// Cache).  Every wavefront has its own LDS ring, so there is no barrier in either loop.  The rest is latency: two launches, a first
+// memory access in each (kernel arguments and data, 2 us), the parts' way to the last workgroup (stores, a counter, loads: 3 us, with
+// all loads of a step under way together; one by one they took 8).  Measured, 1 query of 32 heads on 8 k/v heads, head dim 128: 32768
+// keys 309 us (one wavefront a head) / 151 (shared rows, no split) -> 21 us, of that 8 logits and 12 values (13 us at the rate of a
+// plain copy); 4 sequences of 4096 keys 23 (shared rows) -> 14 us.
+#ifndef FA8_SPLIT_KV_H_
+#define FA8_SPLIT_KV_H_
+#include <type_traits>
+
+#include "fa8_device.h"
+
+namespace fa8 {
+
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
+constexpr int kSplitWaves = 4;  // wavefronts (key ranges) per workgroup
+constexpr int kSplitMax = 32;   // most splits of a row tile
+
+// The workspace: arrays one after the other, each of the size of all row tiles together (tile index = (batch * k/v heads + head) * tiles
+// + tile).  Offsets in bytes, all multiples of 256.
+struct SplitWorkspace {
+  long long done;       // [1] unsigned: workgroups that have written their part
+  long long range_max;  // [splits * kSplitWaves][32]
+  long long split_max;  // [splits][32]
+  long long part_m;     // [splits][32]
+  long long part_l;     // [splits][32]
+  long long part_o;     // [splits][live rows][head_dim]
+  long long s;          // [live rows][keys]: masked logits, whole KV blocks
+  long long bytes;
+};
+__host__ __device__ inline SplitWorkspace split_layout(long long all_tiles, int splits, int live_rows, int head_dim, int seqlen_k) {
+  auto up = [](long long x) { return (x + 255) / 256 * 256; };
+  const long long keys = ((long long)seqlen_k + kKvBlock - 1) / kKvBlock * kKvBlock, rows32 = all_tiles * splits * 128;
+  SplitWorkspace w;
+  w.done = 0;
+  w.range_max = up(all_tiles * 4);
+  w.split_max = w.range_max + rows32 * kSplitWaves;
+  w.part_m = w.split_max + up(rows32);
+  w.part_l = w.part_m + up(rows32);
+  w.part_o = w.part_l + up(rows32);
+  w.s = w.part_o + up(all_tiles * splits * live_rows * head_dim * 4);
+  w.bytes = w.s + all_tiles * live_rows * keys * 4;
+  return w;
+}
+
+// Two argument blocks of at most 112 bytes (see SharedArgs for the limit, the units of the strides and `mode`).
+struct SplitShape {
+  uint8_t* workspace;
+  float scale_log2;
+  int seqlen_q, seqlen_k;
+  unsigned mode;
+  uint16_t splits, blocks_per_range;  // workgroups per row tile, KV blocks per wavefront
+};
+struct SplitLogitsArgs {
+  SplitShape n;
+  const uint8_t* q;
+  const uint8_t* k;
+  unsigned q_bs, q_hs, q_rs;
+  unsigned k_bs, k_hs, k_rs;
+};
+struct SplitValuesArgs {
+  SplitShape n;
+  const uint8_t* v;
+  void* o;
+  float* lse;
+  unsigned v_bs, v_hs, v_rs;
+  unsigned o_bs, o_hs, o_rs;
+  unsigned lse_bs, lse_hs;
+};
+static_assert(sizeof(SplitLogitsArgs) <= 112 && sizeof(SplitValuesArgs) <= 112, "see above");
+
+// What both passes know about a workgroup: grid = k/v heads x batches x (tiles * splits)
+struct SplitPlace {
+  int hk, b, tile, split, splits;
+  long long at;  // row tile index into the workspace
+  int wave, lane, qn, h;
+  int group, group_shift, shift, live_rows;
+  bool causal;
+  int row, last_row, qi, hd;  // query row of the lane (clamped), its query and q head
+  int first, count;           // KV blocks of this wavefront
+  SplitWorkspace ws;
+  __device__ __forceinline__ int query_of(int x) const { return group_shift < 31 ? x >> group_shift : x / group; }
+};
+
+__device__ __forceinline__ SplitPlace split_place(const SplitShape& n, int head_dim) {
+  SplitPlace p;
+  p.group = (int)(n.mode >> kSharedGroup);
+  p.group_shift = (int)(n.mode >> kSharedShift) & 31;
+  p.causal = n.mode & kSharedCausal;
+  p.shift = (n.mode & kSharedBottomRight) ? n.seqlen_k - n.seqlen_q : 0;
+  p.hk = blockIdx.x;
+  p.b = blockIdx.y;
+  p.splits = n.splits;
+  const int rows = p.group * n.seqlen_q, tiles = (rows + 31) >> 5;
+  p.live_rows = min(rows, 32);
+  p.last_row = rows - 1;
+  p.tile = tiles == 1 ? 0 : (int)blockIdx.z / p.splits;
+  p.split = (int)blockIdx.z - p.tile * p.splits;
+  p.at = ((long long)p.b * gridDim.x + p.hk) * tiles + p.tile;
+  p.ws = split_layout((long long)gridDim.y * gridDim.x * tiles, p.splits, p.live_rows, head_dim, n.seqlen_k);
+  p.lane = threadIdx.x & 63;
+  p.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  p.qn = p.lane & 31;
+  p.h = p.lane >> 5;
+  p.row = p.tile * 32 + p.qn;
+  const int rc = min(p.row, p.last_row);
+  p.qi = p.query_of(rc);
+  p.hd = p.hk * p.group + rc - p.qi * p.group;
+  // blocks that some row of the tile sees
+  const int q_last = p.query_of(min(p.tile * 32 + 31, p.last_row));
+  const int blocks = p.causal ? max(1, (min(n.seqlen_k, q_last + 1 + p.shift) + kKvBlock - 1) / kKvBlock) : (n.seqlen_k + kKvBlock - 1) / kKvBlock;
+  p.first = (p.split * kSplitWaves + p.wave) * n.blocks_per_range;
+  p.count = max(0, min((int)n.blocks_per_range, blocks - p.first));
+  return p;
+}
+
+// Waits until at most N vector memory operations of the wavefront are under way (s_waitcnt immediate, gfx9 layout).
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  static_assert(N < 64, "vmcnt has six bits");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | (N >> 4 << 14));
+}
+
+// ---- pass 1: S and the row max of every range ----
+template <int D, bool E5M2>
+__global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_eu(2))) void fa8_split_logits_kernel(const SplitLogitsArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int DP = D <= 32 ? 32 : (D <= 64 ? 64 : (D <= 128 ? 128 : 256));
+  constexpr int kTileBytes = kKvBlock * DP, kPasses = kTileBytes / 1024, kKSteps = (D + 63) / 64;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds0[kSplitWaves * kTileBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds1[kSplitWaves * kTileBytes];
+  __shared__ float max_lds[kSplitWaves * 32];
+  const SplitPlace p = split_place(a.n, D);
+  const int qn = p.qn, h = p.h, lane = p.lane;
+  const uint8_t* kp = a.k + ((unsigned long long)a.k_bs * p.b + (unsigned long long)a.k_hs * p.hk) * 16;
+  const int k_rs = (int)a.k_rs * 16, seqlen_k = a.n.seqlen_k;
+  constexpr unsigned kNoSource = 0x80000000u;
+  unsigned src[kPasses];
+#pragma unroll
+  for (int i = 0; i < kPasses; ++i) {
+    int r, ch;
+    tile_slot_decode<DP, false>(i * 64 + lane, r, ch);
+    src[i] = ch * 16 < D ? (unsigned)(kv_of_lds_row(r) * k_rs + ch * 16) : kNoSource;
+  }
+  const __amdgpu_buffer_rsrc_t rsrc =
+      __builtin_amdgcn_make_buffer_rsrc((void*)kp, 0, (seqlen_k - 1) * k_rs + D, 0x00020000);
+  auto issue = [&](int j, uint8_t* dst) __attribute__((always_inline)) {
+    const int base = (int)((unsigned)j * kKvBlock * (unsigned)k_rs);
+#pragma unroll
+    for (int i = 0; i < kPasses; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, dst + p.wave * kTileBytes + i * 1024), 16, src[i], base, 0, 0);
+  };
+  v8i qf[kKSteps];
+  {
+    const uint8_t* q8 = a.q + ((unsigned long long)a.q_bs * p.b + (unsigned long long)a.q_hs * p.hd + (unsigned long long)a.q_rs * p.qi) * 16;
+#pragma unroll
+    for (int ks = 0; ks < kKSteps; ++ks) {
+      const bool upper_exists = 64 * ks + 32 < D;
+      const uint8_t* s8 = q8 + 64 * ks + (upper_exists ? 32 * h : 0);
+      const v4i lo = *(const v4i*)(s8);
+      const v4i hi = *(const v4i*)(s8 + 16);
+      qf[ks] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      if (!upper_exists && h) qf[ks] = v8i{0, 0, 0, 0, 0, 0, 0, 0};
+    }
+  }
+  // (the ranges of a tile are added up by the workgroup that counts itself last: the count starts at 0)
+  if (p.split == 0 && threadIdx.x == 0) ((unsigned*)(a.n.workspace + p.ws.done))[p.at] = 0;
+  if (p.count > 0) issue(p.first, lds0);
+  if (p.count > 1) issue(p.first + 1, lds1);
+  int k_off[kKSteps][2];
+#pragma unroll
+  for (int ks = 0; ks < kKSteps; ++ks)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) k_off[ks][e] = p.wave * kTileBytes + tile_offset<DP, false>(qn, DP >= 64 ? 4 * ks + 2 * h + e : e);
+  const int kv_last = seqlen_k - 1;
+  const int kv_limit = p.causal ? min(p.qi + p.shift, kv_last) : kv_last;
+  // leading blocks without a masked logit in any row of the tile
+  const int q_first = p.query_of(min(p.tile * 32, p.last_row));
+  const int n_plain = (p.causal ? max(0, min(q_first + p.shift, seqlen_k)) : seqlen_k) / kKvBlock;
+  const long long keys = (long long)((seqlen_k + kKvBlock - 1) / kKvBlock) * kKvBlock;
+  float* s_out = (float*)(a.n.workspace + p.ws.s) + (p.at * p.live_rows + qn) * keys + 32 * h;
+  const bool live = qn < p.live_rows && p.row <= p.last_row;  // (lane 0 always is: the stores below are never skipped)
+  float m_run = -1.0e30f;
+  // Block i of the range: S, then the copy of block i + 2 into the tile just read, then max and stores.  vmcnt counts loads and stores in
+  // issue order; what is issued after the copy of block i and may still be under way when its S is formed: the stores of block i - 2
+  // (not counted below, they are old by then), the copy of block i + 1 and the stores of block i - 1.
+  constexpr int kStores = 8;
+  auto block = [&](int i, uint8_t* tile) __attribute__((always_inline)) {
+    const int j = p.first + i;
+    if (i + 1 < p.count) {
+      if (i == 0)
+        wait_loads<kPasses>();
+      else
+        wait_loads<kPasses + kStores>();
+    } else {
+      if (i == 0)
+        wait_loads<0>();
+      else
+        wait_loads<kStores>();
+    }
+    v16f s[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[t][e] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < kKSteps; ++ks) {
+        const v4i lo = *LDS_PTR(const v4i, tile + t * 32 * DP + k_off[ks][0]);
+        const v4i hi = *LDS_PTR(const v4i, tile + t * 32 * DP + k_off[ks][1]);
+        s[t] = mfma_fp8<E5M2>(v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}, qf[ks], s[t]);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // the tile has been read
+    if (i + 2 < p.count) issue(j + 2, tile);
+    __builtin_amdgcn_sched_barrier(0);
+    if (j >= n_plain) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (j * kKvBlock + 32 * h + 16 * t + e > kv_limit) s[t][e] = -INFINITY;
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; e += 2) m_run = max3(s[t][e], s[t][e + 1], m_run);
+    if (live) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; e += 4) *(v4f*)(s_out + (long long)j * kKvBlock + 16 * t + e) = v4f{s[t][e], s[t][e + 1], s[t][e + 2], s[t][e + 3]};
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  for (int i = 0; i < p.count; i += 2) {
+    block(i, lds0);
+    if (i + 1 < p.count) block(i + 1, lds1);
+  }
+  m_run = lane32_max(m_run);
+  if (h == 0) {
+    ((float*)(a.n.workspace + p.ws.range_max))[((p.at * p.splits + p.split) * kSplitWaves + p.wave) * 32 + qn] = m_run;
+    max_lds[p.wave * 32 + qn] = m_run;
+  }
+  __syncthreads();
+  if (threadIdx.x < 32) {
+    float m = max_lds[threadIdx.x];
+#pragma unroll
+    for (int x = 1; x < kSplitWaves; ++x) m = __builtin_fmaxf(m, max_lds[x * 32 + threadIdx.x]);
+    ((float*)(a.n.workspace + p.ws.split_max))[(p.at * p.splits + p.split) * 32 + threadIdx.x] = m;
+  }
+#endif
+}
+
+// ---- pass 2: weights and O of every range, and their sum ----
+template <int D, bool E5M2, bool VT>
+__global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2))) void fa8_split_values_kernel(
+    const SplitValuesArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int DP = D <= 32 ? 32 : (D <= 64 ? 64 : (D <= 128 ? 128 : 256));
+  constexpr int kTileBytes = kKvBlock * DP, kPasses = kTileBytes / 1024, kMTiles = D / 32;
+  // (after the loop each ring buffer holds O of two ranges, later the first one the rescale factors and row sums of all splits)
+  constexpr int kRing = kSplitWaves * kTileBytes > kSplitMax * 256 ? kSplitWaves * kTileBytes : kSplitMax * 256;
+  static_assert(kSplitWaves * kTileBytes >= 2 * D * 32 * 4, "O of two ranges fits");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds0[kRing];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds1[kSplitWaves * kTileBytes];
+  __shared__ float m_lds[kSplitWaves * 32], l_lds[kSplitWaves * 32];
+  __shared__ int last_lds;
+  const SplitPlace p = split_place(a.n, D);
+  const int qn = p.qn, h = p.h, lane = p.lane;
+  const float c = a.n.scale_log2;
+  const uint8_t* vp = a.v + ((unsigned long long)a.v_bs * p.b + (unsigned long long)a.v_hs * p.hk) * 16;
+  const int v_rs = (int)a.v_rs * 16, seqlen_k = a.n.seqlen_k;
+  constexpr unsigned kNoSource = 0x80000000u;
+  unsigned src[kPasses];
+#pragma unroll
+  for (int i = 0; i < kPasses; ++i) {
+    int r, ch;
+    tile_slot_decode<VT ? 64 : DP, !VT>(i * 64 + lane, r, ch);
+    src[i] = VT || ch * 16 < D ? (unsigned)(r * v_rs + ch * 16) : kNoSource;
+  }
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)vp, 0, VT ? (D - 1) * v_rs + seqlen_k : (seqlen_k - 1) * v_rs + D, 0x00020000);
+  auto issue = [&](int j, uint8_t* dst) __attribute__((always_inline)) {
+    const int base = VT ? j * kKvBlock : (int)((unsigned)j * kKvBlock * (unsigned)v_rs);
+    const bool v_clamp = VT && (j + 1) * kKvBlock > seqlen_k;
+#pragma unroll
+    for (int i = 0; i < kPasses; ++i) {
+      uint8_t* at = dst + p.wave * kTileBytes + i * 1024;
+      if (v_clamp) {  // transposed v, ragged last block: see fa8_fwd_kernel
+        int r, ch;
+        tile_slot_decode<64, false>(i * 64 + lane, r, ch);
+        const unsigned off = r < D ? (unsigned)(r * v_rs + min(base + ch * 16, seqlen_k - 16)) : kNoSource;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, at), 16, off, 0, 0, 0);
+      } else {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, at), 16, src[i], base, 0, 0);
+      }
+    }
+  };
+  const long long keys = (long long)((seqlen_k + kKvBlock - 1) / kKvBlock) * kKvBlock;
+  const float* s_in = (const float*)(a.n.workspace + p.ws.s) + (p.at * p.live_rows + min(qn, p.live_rows - 1)) * keys + 32 * h;
+  auto load_s = [&](int j, v4f(&s)[8]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s[i] = *(const v4f*)(s_in + (long long)j * kKvBlock + 4 * i);
+  };
+  v4f s0[8], s1[8];
+  // The running max before this range: over the splits before this one and the ranges before this one in the split; all loads under way
+  // together (one after the other they would cost a memory latency each), and before those of the first block.
+  const float* split_max = (const float*)(a.n.workspace + p.ws.split_max) + p.at * p.splits * 32;
+  const float* range_max = (const float*)(a.n.workspace + p.ws.range_max) + (p.at * p.splits + p.split) * kSplitWaves * 32;
+  float before[kSplitMax / 2 + kSplitWaves - 1];
+  if (p.split > 0) {
+#pragma unroll
+    for (int e = 0; e < kSplitMax / 2; ++e) before[e] = split_max[min(2 * e + h, p.split - 1) * 32 + qn];
+  }
+#pragma unroll
+  for (int x = 0; x < kSplitWaves - 1; ++x) before[kSplitMax / 2 + x] = x < p.wave ? range_max[x * 32 + qn] : -1.0e30f;
+  if (p.count > 0) {
+    load_s(p.first, s0);
+    issue(p.first, lds0);
+  }
+  float m_run = -1.0e30f;
+  if (p.split > 0) {
+#pragma unroll
+    for (int e = 0; e < kSplitMax / 2; e += 2) m_run = max3(before[e], before[e + 1], m_run);
+  }
+#pragma unroll
+  for (int x = 0; x < kSplitWaves - 1; ++x) m_run = __builtin_fmaxf(m_run, before[kSplitMax / 2 + x]);
+  m_run = lane32_max(m_run);
+
+  constexpr int kTrStride = 8 * DP;
+  const int tr_j = (lane & 15) >> 1, tr_e = lane & 1, tr_g1 = (lane >> 4) & 1;
+  int v_off[kMTiles], vt_off[2];
+#pragma unroll
+  for (int mt = 0; mt < kMTiles; ++mt) v_off[mt] = p.wave * kTileBytes + tile_offset<DP, true>(32 * h + tr_j, 2 * mt + tr_g1) + 8 * tr_e;
+#pragma unroll
+  for (int e = 0; e < 2; ++e) vt_off[e] = p.wave * kTileBytes + tile_offset<64, false>(qn, 2 * h + e);
+  auto load_vf = [&](const uint8_t* vb, int mt) __attribute__((always_inline)) {
+    v8i vf;
+    if constexpr (VT) {
+      const v4i lo = *LDS_PTR(const v4i, vb + mt * 32 * 64 + vt_off[0]);
+      const v4i hi = *LDS_PTR(const v4i, vb + mt * 32 * 64 + vt_off[1]);
+      vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    } else {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const v2i x = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, vb + v_off[mt] + g * kTrStride));
+        vf[2 * g] = x[0];
+        vf[2 * g + 1] = x[1];
+      }
+    }
+    return vf;
+  };
+  v16f o_acc[kMTiles];
+#pragma unroll
+  for (int mt = 0; mt < kMTiles; ++mt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o_acc[mt][i] = 0.f;
+  float l_run = 0.f;
+  auto block = [&](const uint8_t* vb, const v4f(&s)[8]) __attribute__((always_inline)) {
+    float m = m_run;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m = max3(max3(s[i][0], s[i][1], m), s[i][2], s[i][3]);
+    const float m_new = lane32_max(m);
+    if (__any(m_new != m_run)) {
+      const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * c);
+      l_run *= alpha;
+#pragma unroll
+      for (int mt = 0; mt < kMTiles; ++mt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o_acc[mt][i] *= alpha;
+      m_run = m_new;
+    }
+    const float mc = m_new * c;
+    float sum0 = 0.f, sum1 = 0.f;
+    v8i p8;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float x[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][e], c, -mc));
+      sum0 = sum0 + x[0] + x[2];
+      sum1 = sum1 + x[1] + x[3];
+      p8[i] = pack4_fp8<E5M2>(x[0], x[1], x[2], x[3]);
+    }
+    l_run += sum0 + sum1;
+#pragma unroll
+    for (int mt = 0; mt < kMTiles; ++mt) o_acc[mt] = mfma_fp8<E5M2>(load_vf(vb, mt), p8, o_acc[mt]);
+  };
+  // The next block's logits and V are asked for before a block is worked on: the last kPasses + 8 loads may still fly then.
+  constexpr int kNext = kPasses + 8;
+  for (int i = 0; i < p.count; i += 2) {
+    if (i + 1 < p.count) {
+      load_s(p.first + i + 1, s1);
+      issue(p.first + i + 1, lds1);
+      wait_loads<kNext>();
+    } else {
+      wait_loads<0>();
+    }
+    block(lds0, s0);
+    if (i + 1 < p.count) {
+      if (i + 2 < p.count) {
+        load_s(p.first + i + 2, s0);
+        issue(p.first + i + 2, lds0);
+        wait_loads<kNext>();
+      } else {
+        wait_loads<0>();
+      }
+      block(lds1, s1);
+    }
+  }
+
+  // ---- the four ranges of the workgroup meet in LDS ----
+  if (h == 0) m_lds[p.wave * 32 + qn] = m_run;
+  const float l_wave = lane32_sum(l_run);
+  __syncthreads();
+  const float m_wg = m_lds[(kSplitWaves - 1) * 32 + qn];  // the last range's max is the largest
+  const float f = __builtin_amdgcn_exp2f((m_run - m_wg) * c);
+  if (h == 0) l_lds[p.wave * 32 + qn] = l_wave * f;
+  // [range % 2][row][columns in fours, their number ^ row % 8] in the ring buffer of range / 2: few bank conflicts, no padding
+  constexpr int kFours = D / 4;
+  auto at4 = [](int row, int four) __attribute__((always_inline)) { return row * kFours + (four ^ (row & 7)); };
+  {
+    v4f* o_lds = (v4f*)(p.wave < 2 ? lds0 : lds1) + (p.wave & 1) * 32 * kFours;
+    if (qn < p.live_rows) {
+#pragma unroll
+      for (int mt = 0; mt < kMTiles; ++mt)
+#pragma unroll
+        for (int e = 0; e < 16; e += 4)
+          o_lds[at4(qn, 8 * mt + (e >> 1) + h)] = v4f{o_acc[mt][e] * f, o_acc[mt][e + 1] * f, o_acc[mt][e + 2] * f, o_acc[mt][e + 3] * f};
+    }
+  }
+  __syncthreads();
+  // ---- this workgroup's part goes out.  The workgroups of a tile sit on different XCDs: stores and loads of the parts carry agent
+  // scope (sc1), which passes the XCDs' own L2 caches by ----
+  constexpr int kAgent = 16;  // cache policy of the buffer instructions: sc1
+  const long long parts = p.at * p.splits;
+  const int n = p.live_rows, tid = threadIdx.x, fours = n * kFours;  // of a part
+  const int last_bytes = p.splits * 128;
+  const __amdgpu_buffer_rsrc_t m_rsrc = __builtin_amdgcn_make_buffer_rsrc(a.n.workspace + p.ws.part_m + parts * 128, 0, last_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t l_rsrc = __builtin_amdgcn_make_buffer_rsrc(a.n.workspace + p.ws.part_l + parts * 128, 0, last_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t o_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(a.n.workspace + p.ws.part_o + parts * fours * 16, 0, p.splits * fours * 16, 0x00020000);
+  for (int x = tid; x < fours; x += 64 * kSplitWaves) {
+    const int at = at4(x / kFours, x % kFours);
+    const v4f y = (((const v4f*)lds0)[at] + ((const v4f*)lds0)[32 * kFours + at]) + (((const v4f*)lds1)[at] + ((const v4f*)lds1)[32 * kFours + at]);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, y), o_rsrc, x * 16, p.split * fours * 16, kAgent);
+  }
+  if (tid < 32) {
+    float l = 0.f;
+#pragma unroll
+    for (int x = 0; x < kSplitWaves; ++x) l += l_lds[x * 32 + tid];
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(l), l_rsrc, tid * 4, p.split * 128, kAgent);
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(m_lds[(kSplitWaves - 1) * 32 + tid]), m_rsrc, tid * 4, p.split * 128, kAgent);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores have reached the point where all XCDs see them
+  __syncthreads();
+  if (tid == 0)
+    last_lds = __hip_atomic_fetch_add((unsigned*)(a.n.workspace + p.ws.done) + p.at, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+               (unsigned)p.splits - 1;
+  __syncthreads();
+  if (!last_lds) return;
+  // ---- the last workgroup of the tile adds the parts up ----
+  float* factor = (float*)lds0;                 // [split][32]
+  float* sums = (float*)lds0 + kSplitMax * 32;  // [split][32]
+  {
+    constexpr int kEach = kSplitMax * 32 / (64 * kSplitWaves);
+    const float m_all = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(m_rsrc, (tid & 31) * 4, (p.splits - 1) * 128, kAgent));  // the largest
+    float m[kEach], l[kEach];
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {  // (past the last split: 0)
+      m[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(m_rsrc, (e * 64 * kSplitWaves + tid) * 4, 0, kAgent));
+      l[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(l_rsrc, (e * 64 * kSplitWaves + tid) * 4, 0, kAgent));
+    }
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+      const bool exists = e * 64 * kSplitWaves + tid < p.splits * 32;
+      factor[e * 64 * kSplitWaves + tid] = exists ? __builtin_amdgcn_exp2f((m[e] - m_all) * c) : 0.f;
+      sums[e * 64 * kSplitWaves + tid] = l[e];
+    }
+  }
+  __syncthreads();
+  for (int x = tid; x < fours; x += 64 * kSplitWaves) {
+    const int row_in = x / kFours, col = (x % kFours) * 4, out_row = p.tile * 32 + row_in;
+    v4f y[kSplitMax];  // all parts under way together; past the last split: 0
+#pragma unroll
+    for (int e = 0; e < kSplitMax; ++e)
+      y[e] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(o_rsrc, x * 16, e * fours * 16, kAgent));
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    float l_all = 0.f;
+#pragma unroll
+    for (int e = 0; e < kSplitMax; ++e) {
+      const float g = factor[e * 32 + row_in];
+      l_all = __builtin_fmaf(sums[e * 32 + row_in], g, l_all);
+#pragma unroll
+      for (int z = 0; z < 4; ++z) acc[z] = __builtin_fmaf(y[e][z], g, acc[z]);
+    }
+    if (out_row > p.last_row) continue;
+    const int q_out = p.query_of(out_row), hd_out = p.hk * p.group + out_row - q_out * p.group;
+    const float inv = (l_all == 0.f || l_all != l_all) ? 1.f : 1.f / l_all;
+    if (a.lse != nullptr && col == 0) {
+      const float m_row = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(m_rsrc, row_in * 4, (p.splits - 1) * 128, kAgent));
+      a.lse[(unsigned long long)a.lse_bs * p.b + (unsigned long long)a.lse_hs * hd_out + q_out] =
+          l_all > 0.f ? (m_row * c + __builtin_amdgcn_logf(l_all)) * 0.6931471805599453f : (l_all == 0.f ? -INFINITY : l_all);
+    }
+    const unsigned long long o_at =
+        ((unsigned long long)a.o_bs * p.b + (unsigned long long)a.o_hs * hd_out + (unsigned long long)a.o_rs * q_out) * 4 + col;
+    if (!(a.n.mode & kSharedFp8Out)) {
+      v4h w;
+#pragma unroll
+      for (int z = 0; z < 4; ++z) w[z] = (_Float16)(acc[z] * inv);
+      *(v4h*)((_Float16*)a.o + o_at) = w;
+    } else {
+      constexpr float kMaxFinite = E5M2 ? 57344.f : 448.f;
+      float w[4];
+#pragma unroll
+      for (int z = 0; z < 4; ++z) {
+        const float v = acc[z] * inv;
+        w[z] = (v != v) ? v : fminf(fmaxf(v, -kMaxFinite), kMaxFinite);
+      }
+      *(int*)((uint8_t*)a.o + o_at) = pack4_fp8<E5M2>(w[0], w[1], w[2], w[3]);
+    }
+  }
+#endif
+}
+
+}  // namespace fa8
+#endif  // FA8_SPLIT_KV_H_

@@ -1,0 +1,90 @@
+// Launcher of the split-kv kernels (fa8_split_kv.h): the plan, the workspace and the two launches.
+#include "fa8_launch.h"
+#include "fa8_split_kv.h"
+
+namespace {
+
+using namespace fa8;
+
+template <int D>
+const void* logits_kernel(bool e5m2) {
+  return e5m2 ? (const void*)&fa8_split_logits_kernel<D, true> : (const void*)&fa8_split_logits_kernel<D, false>;
+}
+template <int D>
+const void* values_kernel(bool e5m2, bool vt) {
+  if (e5m2) return vt ? (const void*)&fa8_split_values_kernel<D, true, true> : (const void*)&fa8_split_values_kernel<D, true, false>;
+  return vt ? (const void*)&fa8_split_values_kernel<D, false, true> : (const void*)&fa8_split_values_kernel<D, false, false>;
+}
+
+struct Plan {
+  int heads_k, tiles, live_rows, splits, blocks_per_range;
+};
+
+Plan plan_of(const Fa8FwdParams* p, int splits) {
+  Plan n;
+  n.heads_k = p->heads_k > 0 ? p->heads_k : p->heads;
+  const long long rows = (long long)(p->heads / n.heads_k) * p->seqlen_q;
+  n.tiles = (int)((rows + 31) / 32);
+  n.live_rows = rows < 32 ? (int)rows : 32;
+  // the blocks that the last query sees
+  long long keys = p->seqlen_k;
+  if (p->is_causal && p->causal_align != FA8_CAUSAL_BOTTOM_RIGHT && p->seqlen_q < keys) keys = p->seqlen_q;
+  const int blocks = (int)((keys + kKvBlock - 1) / kKvBlock);
+  n.blocks_per_range = (blocks + splits * kSplitWaves - 1) / (splits * kSplitWaves);
+  n.splits = (blocks + n.blocks_per_range * kSplitWaves - 1) / (n.blocks_per_range * kSplitWaves);
+  return n;
+}
+
+}  // namespace
+
+long long fa8::split_workspace(const Fa8FwdParams* p, int splits) {
+  const Plan n = plan_of(p, splits);
+  return split_layout((long long)p->batch * n.heads_k * n.tiles, n.splits, n.live_rows, p->head_dim, p->seqlen_k).bytes;
+}
+
+int fa8::launch_split(const Fa8FwdParams* p, int splits, void* workspace, hipStream_t stream) {
+  const Plan n = plan_of(p, splits);
+  SplitShape shape;
+  shape.workspace = (uint8_t*)workspace;
+  shape.scale_log2 = p->softmax_scale * 1.4426950408889634f;
+  shape.seqlen_q = p->seqlen_q;
+  shape.seqlen_k = p->seqlen_k;
+  shape.mode = pack_mode(p);
+  shape.splits = (uint16_t)n.splits;
+  shape.blocks_per_range = (uint16_t)n.blocks_per_range;
+  SplitLogitsArgs l;
+  l.n = shape;
+  l.q = (const uint8_t*)p->q;
+  l.k = (const uint8_t*)p->k;
+  l.q_bs = p->q_batch_stride / 16; l.q_hs = p->q_head_stride / 16; l.q_rs = p->q_row_stride / 16;
+  l.k_bs = p->k_batch_stride / 16; l.k_hs = p->k_head_stride / 16; l.k_rs = p->k_row_stride / 16;
+  SplitValuesArgs v;
+  v.n = shape;
+  v.v = (const uint8_t*)p->v;
+  v.o = p->o;
+  v.lse = (float*)p->lse;
+  v.v_bs = p->v_batch_stride / 16; v.v_hs = p->v_head_stride / 16; v.v_rs = p->v_row_stride / 16;
+  v.o_bs = p->o_batch_stride / 4; v.o_hs = p->o_head_stride / 4; v.o_rs = p->o_row_stride / 4;
+  v.lse_bs = p->lse_batch_stride; v.lse_hs = p->lse_head_stride;
+  const bool e5m2 = p->in_dtype == FA8_DTYPE_E5M2, vt = p->v_layout == FA8_V_TRANSPOSED;
+  const void *first = nullptr, *second = nullptr;
+  switch (p->head_dim) {
+#define FA8_HEAD_DIM_CASE(D_) \
+  case D_: first = logits_kernel<D_>(e5m2); second = values_kernel<D_>(e5m2, vt); break
+    FA8_HEAD_DIM_CASE(32);
+    FA8_HEAD_DIM_CASE(64);
+    FA8_HEAD_DIM_CASE(96);
+    FA8_HEAD_DIM_CASE(128);
+    FA8_HEAD_DIM_CASE(160);
+    FA8_HEAD_DIM_CASE(192);
+    FA8_HEAD_DIM_CASE(224);
+    FA8_HEAD_DIM_CASE(256);
+#undef FA8_HEAD_DIM_CASE
+    default: return FA8_ERR_HEAD_DIM;
+  }
+  const dim3 grid((unsigned)n.heads_k, (unsigned)p->batch, (unsigned)(n.tiles * n.splits));
+  void *argv_l[] = {&l}, *argv_v[] = {&v};
+  const hipError_t rc = hipLaunchKernel(first, grid, dim3(64 * kSplitWaves), argv_l, 0, stream);
+  if (rc != hipSuccess) return (int)rc;
+  return (int)hipLaunchKernel(second, grid, dim3(64 * kSplitWaves), argv_v, 0, stream);
+}

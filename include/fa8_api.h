@@ -124,6 +124,17 @@ int fa8_fwd_validate(const Fa8FwdParams* p);
 int fa8_fwd(const Fa8FwdParams* p, void* hip_stream);
 
 /*
+ * The same with device memory to work in.  fa8_fwd_workspace writes the number of bytes that this call can make use of on the
+ * current device (0: none); fa8_fwd_ws runs the call with a workspace of that size (any contents, 256-byte aligned, the caller's
+ * again once the stream has passed the work).  Few query rows over many keys (decode steps) are then spread over the whole GPU by
+ * splitting the keys, which fa8_fwd, without memory for the parts, cannot do.  Without a workspace, or with one that is too
+ * small, fa8_fwd_ws is fa8_fwd.  The weights of a split call are the same bit for bit; its fp32 sums are taken in another order.
+ * (fa8_fwd itself still needs no memory.)  No counterpart in the reference.
+ */
+int fa8_fwd_workspace(const Fa8FwdParams* p, int64_t* bytes);
+int fa8_fwd_ws(const Fa8FwdParams* p, void* workspace, int64_t bytes, void* hip_stream);
+
+/*
  * How a call would be cut on the current device, for benchmarks and tests (nothing is launched): query rows of a workgroup
  * (grouped q heads counted together), wavefronts that share 32 of them (1: one of the main loops of fa8_fwd_schedule; 2 or 4: shared
  * rows, for launches with few of them; a schedule hint always gives 1), and into how many parts the keys of a row are split

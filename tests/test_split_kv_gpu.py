@@ -1,0 +1,112 @@
+"""Few query rows over many keys: the keys of a row tile are dealt to several workgroups (csrc/fa8_split_kv.h; needs the workspace that the
+binding and the ctypes mirror provide).  Weights are those of the rolling loop bit for bit, only the fp32 sums over the keys are taken in
+another order: an output may differ by the rounding of those sums plus one step of the output type."""
+import ctypes
+
+import pytest
+import torch
+
+import cutlass_flash_atten_fp8_amd as fa
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+E4, E5 = torch.float8_e4m3fn, torch.float8_e5m2
+
+
+def _inputs(seed, B, H, Hk, Nq, Nk, d, dtype):
+    g = torch.Generator().manual_seed(seed)
+    spread = 2.0 if seed % 2 else 1.0
+    return tuple((torch.randn(s, generator=g) * spread).to(dtype).to(DEV) for s in ((B, H, Nq, d), (B, Hk, Nk, d), (B, Hk, Nk, d)))
+
+
+def assert_same_up_to_sum_order(got, want, v, n_keys):
+    # Sum of n positive-weighted terms in fp32, two orders: each within n_blocks * 2^-24 (the sums inside a block are the same) of
+    # sum p |v| / sum p <= max |v|, the matrix instruction's cut (2^-22 per step) included; then one rounding to the output type each.
+    step = {torch.float16: 2.0 ** -10, E4: 2.0 ** -3, E5: 2.0 ** -2}[got.dtype]
+    least = {torch.float16: 2.0 ** -24, E4: 2.0 ** -9, E5: 2.0 ** -16}[got.dtype]
+    a, b = got.float(), want.float()
+    bound = step * torch.maximum(a.abs(), b.abs()) + least + 2 * (n_keys / 64 + 8) * 2.0 ** -22 * v.float().abs().max()
+    assert torch.isfinite(a).all()
+    assert ((a - b).abs() <= bound).all(), (a - b).abs().max().item()
+    assert (a != b).float().mean() <= 0.02  # an output moves only if it sits that close to a rounding boundary
+
+
+CASES = [
+    # B, H, Hk, Nq, Nk, d, causal, vt, dtype, fp8 out
+    (1, 8, 2, 1, 6001, 128, True, False, E4, False),
+    (2, 8, 8, 1, 12000, 64, True, False, E4, True),
+    (1, 4, 1, 8, 9999, 128, True, False, E4, False),     # 32 packed rows, masks inside the last block
+    (1, 6, 2, 2, 8191, 96, True, False, E5, False),      # group of 3
+    (1, 8, 1, 5, 7777, 128, True, False, E4, False),     # 40 packed rows: two tiles, the second with 8 rows
+    (1, 8, 2, 1, 8192, 32, True, False, E5, True),
+    (1, 4, 4, 3, 4112, 160, False, True, E4, False),     # v^T, ragged last block
+    (1, 4, 1, 1, 4100, 192, True, False, E4, True),
+    (1, 2, 2, 16, 4096, 224, False, True, E5, False),
+    (1, 8, 2, 1, 20000, 256, True, False, E4, False),
+    (1, 1, 1, 1, 100000, 128, True, False, E4, False),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "B{}H{}k{}Nq{}Nk{}d{}".format(*c[:6]))
+def test_split_keys_against_the_rolling_loop(case):
+    B, H, Hk, Nq, Nk, d, causal, vt, dt, out8 = case
+    q, k, v = _inputs(Nk + d, B, H, Hk, Nq, Nk, d, dt)
+    if vt:
+        v = v.transpose(2, 3).contiguous()
+    kw = dict(v_transposed=vt, return_lse=True, causal_bottom_right=True, out_dtype=dt if out8 else None)
+    want, want_lse = fa.flash_attention_v2_cutlass(q, k, v, causal, d ** -0.5, schedule=fa.FA8_SCHEDULE_ROLLING, **kw)
+    assert fa.plan(fa.make_params(q, k, v, want, causal, d ** -0.5, vt, want_lse, True))[2] > 1
+    got, lse = fa.load_extension().flash_attention_v2_cutlass(q, k, v, causal, d ** -0.5, **kw)
+    again, lse2 = fa.flash_attention_v2_cutlass(q, k, v, causal, d ** -0.5, **kw)
+    torch.cuda.synchronize()
+    assert_same_up_to_sum_order(got, want, v, Nk)
+    assert (lse - want_lse).abs().max() <= 5e-6 * max(1.0, want_lse.abs().max().item())
+    assert torch.equal(got.view(torch.uint8), again.view(torch.uint8)) and torch.equal(lse, lse2)  # whichever part ends last
+
+
+def test_workspace_is_optional_and_its_contents_do_not_matter():
+    q, k, v = _inputs(3, 1, 8, 2, 1, 8000, 128, E4)
+    outs = []
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for fill in (None, 0, 0xFF):
+        o = torch.full(q.shape, float("nan"), dtype=torch.float16, device=DEV)
+        p = fa.make_params(q, k, v, o, True, 0.09, causal_bottom_right=True)
+        need = ctypes.c_int64()
+        assert fa.lib().fa8_fwd_workspace(ctypes.byref(p), ctypes.byref(need)) == 0 and need.value > 0
+        if fill is None:
+            assert fa.plan(p, with_workspace=False)[2] == 1
+            rc = fa.lib().fa8_fwd_ws(ctypes.byref(p), None, 0, stream)
+        else:
+            ws = torch.full((need.value + 512,), fill, dtype=torch.uint8, device=DEV)
+            rc = fa.lib().fa8_fwd_ws(ctypes.byref(p), ws.data_ptr(), need.value, stream)
+            torch.cuda.synchronize()
+            assert (ws[need.value:] == fill).all()
+        assert rc == 0, fa.error_string(rc)
+        outs.append(o)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[1], outs[2])
+    assert_same_up_to_sum_order(outs[1], outs[0], v, 8000)
+
+
+def test_split_keys_in_a_hip_graph():
+    ext = fa.load_extension()
+    q, k, v = _inputs(4, 1, 8, 2, 1, 8000, 128, E4)
+    run = lambda: ext.flash_attention_v2_cutlass(q, k, v, True, 0.09, causal_bottom_right=True)[0]  # noqa: E731
+    eager = run().clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        run()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run()
+    for i in range(4):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), f"replay {i}"
+        q.copy_(_inputs(60 + i, 1, 8, 2, 1, 8, 128, E4)[0])
+        eager = run().clone()
