@@ -29,6 +29,8 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # matrix results in vector registers, also in kernels whose LDS leaves room for accumulation registers
     "-mllvm", "-amdgpu-mfma-vgpr-form=1",
+    # the first kernel arguments arrive in scalar registers (kernels that take their arguments one by one)
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",
 ]
 
 

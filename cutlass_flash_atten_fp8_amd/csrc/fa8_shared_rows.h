@@ -31,26 +31,34 @@ constexpr float kMaxStart = -1.0e30f;  // below every possible logit, finite: se
 
 // 112 bytes: a larger argument block makes the launch itself slower on the host (2.75 us up to 112 bytes, 3.4 - 3.6 us from 120 on,
 // an empty kernel in a loop).  Strides are in units of 16 elements (q, k, v) and 4 elements (o); see packable and pack_mode.
+// The kernel takes the fields one by one in this order: the first 14 dwords then are in scalar registers when a wavefront starts
+// (-amdgpu-kernarg-preload-count), and the first loads need not wait the 800 cycles that the arguments take from host memory.
+#define FA8_SHARED_FIELDS(X)                                                                                                       \
+  X(const uint8_t*, q) X(unsigned, k_hs) X(unsigned, k_rs) X(unsigned, k_bs) X(unsigned, q_hs) X(unsigned, q_rs) X(unsigned, q_bs) \
+  X(int, seqlen_q) X(int, seqlen_k) X(unsigned, mode) X(float, scale_log2) X(const uint8_t*, v) X(void*, o) X(float*, lse)         \
+  X(unsigned, v_bs) X(unsigned, v_hs) X(unsigned, v_rs) X(unsigned, o_bs) X(unsigned, o_hs) X(unsigned, o_rs)                      \
+  X(unsigned, lse_bs) X(unsigned, lse_hs)
 struct SharedArgs {
-  const uint8_t* q;
   const uint8_t* k;
-  const uint8_t* v;
-  void* o;
-  float* lse;
-  float scale_log2;
-  int seqlen_q, seqlen_k;
-  unsigned mode;  // see pack_mode
-  unsigned q_bs, q_hs, q_rs;
-  unsigned k_bs, k_hs, k_rs;
-  unsigned v_bs, v_hs, v_rs;
-  unsigned o_bs, o_hs, o_rs;
-  unsigned lse_bs, lse_hs;
+#define FA8_FIELD(type, name) type name;
+  FA8_SHARED_FIELDS(FA8_FIELD)
+#undef FA8_FIELD
 };
 static_assert(sizeof(SharedArgs) == 112, "see above");
 
 template <int D, bool E5M2, bool VT, int R, int W, int STAGES>
-__global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2))) void fa8_shared_rows_kernel(const SharedArgs a) {
+__global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2))) void fa8_shared_rows_kernel(
+    const uint8_t* k_
+#define FA8_FIELD(type, name) , type name##_
+    FA8_SHARED_FIELDS(FA8_FIELD)
+#undef FA8_FIELD
+) {
 #if defined(__HIP_DEVICE_COMPILE__)
+  const SharedArgs a = {k_
+#define FA8_FIELD(type, name) , name##_
+                        FA8_SHARED_FIELDS(FA8_FIELD)
+#undef FA8_FIELD
+  };
   constexpr int DP = D <= 32 ? 32 : (D <= 64 ? 64 : (D <= 128 ? 128 : 256));
   constexpr int kTileBytes = kKvBlock * DP;
   constexpr int kKSteps = (D + 63) / 64;
@@ -78,7 +86,9 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
   const bool causal = a.mode & kSharedCausal;
   const int group = (int)(a.mode >> kSharedGroup), group_shift = (int)(a.mode >> kSharedShift) & 31;
   const int hk = blockIdx.x, b = blockIdx.y;
-  const int tile = causal ? (int)(gridDim.z - 1 - blockIdx.z) : (int)blockIdx.z;
+  // (gridDim would have to be loaded from memory)
+  const int tiles = (group * a.seqlen_q + 32 * R - 1) / (32 * R);
+  const int tile = causal ? tiles - 1 - (int)blockIdx.z : (int)blockIdx.z;
   // The query rows of a k/v head: row x is query x / group of q head x % group of the group.
   auto query_of = [&](int x) __attribute__((always_inline)) { return group_shift < 31 ? x >> group_shift : x / group; };
   const int last_row = group * a.seqlen_q - 1;

@@ -58,6 +58,10 @@ int fa8::launch_shared(const Fa8FwdParams* p, int r, int w, hipStream_t stream) 
     default: return FA8_ERR_HEAD_DIM;
   }
   if (!fn) return FA8_ERR_UNSUPPORTED;
-  void* argv[] = {&a};
+  void* argv[] = {&a.k
+#define FA8_FIELD(type, name) , &a.name
+                  FA8_SHARED_FIELDS(FA8_FIELD)
+#undef FA8_FIELD
+  };
   return (int)hipLaunchKernel(fn, dim3((unsigned)heads_k, (unsigned)p->batch, (unsigned)tiles), dim3(64 * r * w), argv, 0, stream);
 }

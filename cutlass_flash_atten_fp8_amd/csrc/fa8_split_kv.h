@@ -62,6 +62,7 @@ struct SplitShape {
   int seqlen_q, seqlen_k;
   unsigned mode;
   uint16_t splits, blocks_per_range;  // workgroups per row tile, KV blocks per wavefront
+  int heads_k, all_tiles;             // (gridDim would have to be loaded from elsewhere)
 };
 struct SplitLogitsArgs {
   SplitShape n;
@@ -108,8 +109,8 @@ __device__ __forceinline__ SplitPlace split_place(const SplitShape& n, int head_
   p.last_row = rows - 1;
   p.tile = tiles == 1 ? 0 : (int)blockIdx.z / p.splits;
   p.split = (int)blockIdx.z - p.tile * p.splits;
-  p.at = ((long long)p.b * gridDim.x + p.hk) * tiles + p.tile;
-  p.ws = split_layout((long long)gridDim.y * gridDim.x * tiles, p.splits, p.live_rows, head_dim, n.seqlen_k);
+  p.at = ((long long)p.b * n.heads_k + p.hk) * tiles + p.tile;
+  p.ws = split_layout(n.all_tiles, p.splits, p.live_rows, head_dim, n.seqlen_k);
   p.lane = threadIdx.x & 63;
   p.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   p.qn = p.lane & 31;

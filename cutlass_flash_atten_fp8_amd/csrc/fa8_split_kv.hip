@@ -52,6 +52,8 @@ int fa8::launch_split(const Fa8FwdParams* p, int splits, void* workspace, hipStr
   shape.mode = pack_mode(p);
   shape.splits = (uint16_t)n.splits;
   shape.blocks_per_range = (uint16_t)n.blocks_per_range;
+  shape.heads_k = n.heads_k;
+  shape.all_tiles = p->batch * n.heads_k * n.tiles;
   SplitLogitsArgs l;
   l.n = shape;
   l.q = (const uint8_t*)p->q;
