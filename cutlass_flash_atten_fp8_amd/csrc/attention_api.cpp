@@ -14,11 +14,16 @@
 // (grouped-query attention), `return_lse=True` appends the fp32 log-sum-exp [B,H,Nq] to the returned list, and
 // `causal_bottom_right=True` aligns the causal diagonal with the last key when seqlen_q != seqlen_k.  `schedule`
 // (FA8_SCHEDULE_*, include/fa8_api.h) picks the kernel's main loop by hand: a performance hint, the result is the same.
+//
+// The function is a plain CPython one (vectorcall arguments) and takes its outputs straight from torch's CUDA allocator: argument
+// matching by pybind11 and the dispatcher's empty() were about a quarter of the host time of a call, and a small call is bound by it.
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
 #include <torch/extension.h>
-
-#include <vector>
 
 #include "fa8_api.h"
 
@@ -31,12 +36,17 @@ void check_input(const torch::Tensor& t, const char* name) {
   TORCH_CHECK(t.dim() == 4, name, " must be 4-dimensional [batch, heads, seqlen, head_dim], got ", t.dim(), " dims");
 }
 
-}  // namespace
+torch::Tensor new_tensor(at::IntArrayRef sizes, at::ScalarType type, const torch::Tensor& like) {
+  return torch::Tensor(at::detail::empty_cuda(sizes, type, like.device(), c10::nullopt));
+}
 
-std::vector<torch::Tensor> flash_attention_v2_cutlass(torch::Tensor q, torch::Tensor k, torch::Tensor v, bool is_causal,
-                                                      float softmax_scale, bool v_transposed,
-                                                      c10::optional<at::ScalarType> out_dtype, bool return_lse,
-                                                      bool causal_bottom_right, int64_t schedule) {
+struct Outputs {
+  torch::Tensor o, lse;  // lse: undefined if it was not asked for
+};
+
+Outputs flash_attention_v2_cutlass(const torch::Tensor& q, const torch::Tensor& k, const torch::Tensor& v, bool is_causal,
+                                   float softmax_scale, bool v_transposed, c10::optional<at::ScalarType> out_dtype, bool return_lse,
+                                   bool causal_bottom_right, int64_t schedule) {
   check_input(q, "q");
   check_input(k, "k");
   check_input(v, "v");
@@ -62,9 +72,9 @@ std::vector<torch::Tensor> flash_attention_v2_cutlass(torch::Tensor q, torch::Te
   TORCH_CHECK(o_type == at::kHalf || o_type == in_type,
               "out_dtype must be torch.float16 or the fp8 type of the inputs (the reference's output type), got ", o_type);
 
-  auto out = torch::empty({B, H, Nq, D}, q.options().dtype(o_type));
+  const torch::Tensor out = new_tensor({B, H, Nq, D}, o_type, q);
   torch::Tensor lse;
-  if (return_lse) lse = torch::empty({B, H, Nq}, q.options().dtype(at::kFloat));
+  if (return_lse) lse = new_tensor({B, H, Nq}, at::kFloat, q);
 
   Fa8FwdParams p = {};
   p.q = q.data_ptr();
@@ -103,20 +113,97 @@ std::vector<torch::Tensor> flash_attention_v2_cutlass(torch::Tensor q, torch::Te
   torch::Tensor workspace;  // (goes back to torch's allocator on return, for later work of this stream)
   int rc = fa8_fwd_workspace(&p, &workspace_bytes);
   if (rc == FA8_OK) {
-    if (workspace_bytes > 0) workspace = torch::empty({workspace_bytes}, q.options().dtype(at::kByte));
+    if (workspace_bytes > 0) workspace = new_tensor({workspace_bytes}, at::kByte, q);
     rc = fa8_fwd_ws(&p, workspace_bytes > 0 ? workspace.data_ptr() : nullptr, workspace_bytes, (void*)stream);
   }
   TORCH_CHECK(rc == FA8_OK, "flash_attention_v2_cutlass: ", fa8_error_string(rc), " (code ", rc, ")");
-  if (return_lse) return {out, lse};
-  return {out};
+  return {out, lse};
 }
+
+// ---- the Python function ----
+constexpr int kPositional = 5, kArguments = 10;
+const char* const kNames[kArguments] = {"q", "k", "v", "is_causal", "softmax_scale", "v_transposed", "out_dtype", "return_lse",
+                                        "causal_bottom_right", "schedule"};
+PyObject* interned_names[kArguments];
+
+[[noreturn]] void type_error(const std::string& text) { throw torch::TypeError("flash_attention_v2_cutlass(): " + text); }
+
+const torch::Tensor& tensor_argument(PyObject* v, int i) {
+  if (!THPVariable_Check(v)) type_error(std::string("argument '") + kNames[i] + "' must be a torch.Tensor, not " + Py_TYPE(v)->tp_name);
+  return THPVariable_Unpack(v);
+}
+
+bool bool_argument(PyObject* v, int i) {
+  if (v == Py_True) return true;
+  if (v == nullptr || v == Py_False || v == Py_None) return false;
+  const int x = Py_TYPE(v)->tp_as_number && Py_TYPE(v)->tp_as_number->nb_bool ? PyObject_IsTrue(v) : -1;
+  if (x < 0) {
+    PyErr_Clear();
+    type_error(std::string("argument '") + kNames[i] + "' must be a bool, not " + Py_TYPE(v)->tp_name);
+  }
+  return x != 0;
+}
+
+PyObject* python_flash_attention(PyObject*, PyObject* const* args, Py_ssize_t n_positional, PyObject* keywords) {
+  HANDLE_TH_ERRORS
+  PyObject* v[kArguments] = {};
+  if (n_positional > kPositional)
+    type_error("takes " + std::to_string(kPositional) + " positional arguments but " + std::to_string(n_positional) + " were given");
+  for (Py_ssize_t i = 0; i < n_positional; ++i) v[i] = args[i];
+  const Py_ssize_t n_keywords = keywords ? PyTuple_GET_SIZE(keywords) : 0;
+  for (Py_ssize_t x = 0; x < n_keywords; ++x) {
+    PyObject* const name = PyTuple_GET_ITEM(keywords, x);
+    int i = 0;
+    while (i < kArguments && name != interned_names[i]) ++i;  // keywords written in a program are interned
+    if (i == kArguments)
+      for (i = 0; i < kArguments && PyUnicode_Compare(name, interned_names[i]) != 0;) ++i;
+    if (i == kArguments) type_error(std::string("got an unexpected keyword argument '") + PyUnicode_AsUTF8(name) + "'");
+    if (v[i]) type_error(std::string("got multiple values for argument '") + kNames[i] + "'");
+    v[i] = args[n_positional + x];
+  }
+  for (int i = 0; i < kPositional; ++i)
+    if (!v[i]) type_error(std::string("missing required argument '") + kNames[i] + "'");
+  const torch::Tensor &q = tensor_argument(v[0], 0), &k = tensor_argument(v[1], 1), &value = tensor_argument(v[2], 2);
+  const double scale = PyFloat_AsDouble(v[4]);
+  if (scale == -1.0 && PyErr_Occurred()) {
+    PyErr_Clear();
+    type_error(std::string("argument 'softmax_scale' must be a float, not ") + Py_TYPE(v[4])->tp_name);
+  }
+  c10::optional<at::ScalarType> out_dtype;
+  if (v[6] && v[6] != Py_None) {
+    if (!THPDtype_Check(v[6])) type_error(std::string("argument 'out_dtype' must be a torch.dtype or None, not ") + Py_TYPE(v[6])->tp_name);
+    out_dtype = reinterpret_cast<THPDtype*>(v[6])->scalar_type;
+  }
+  long long schedule = 0;
+  if (v[9]) {
+    schedule = PyFloat_Check(v[9]) ? -1 : PyLong_AsLongLong(v[9]);
+    if (PyFloat_Check(v[9]) || (schedule == -1 && PyErr_Occurred())) {
+      PyErr_Clear();
+      type_error(std::string("argument 'schedule' must be an int, not ") + Py_TYPE(v[9])->tp_name);
+    }
+  }
+  const Outputs out = flash_attention_v2_cutlass(q, k, value, bool_argument(v[3], 3), (float)scale, bool_argument(v[5], 5), out_dtype,
+                                                 bool_argument(v[7], 7), bool_argument(v[8], 8), schedule);
+  PyObject* const list = PyList_New(out.lse.defined() ? 2 : 1);
+  if (!list) throw python_error();
+  PyList_SET_ITEM(list, 0, THPVariable_Wrap(out.o));
+  if (out.lse.defined()) PyList_SET_ITEM(list, 1, THPVariable_Wrap(out.lse));
+  return list;
+  END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef python_method = {
+    "flash_attention_v2_cutlass", (PyCFunction)(void (*)(void))python_flash_attention, METH_FASTCALL | METH_KEYWORDS,
+    "flash_attention_v2_cutlass(q, k, v, is_causal, softmax_scale, *, v_transposed=False, out_dtype=None, return_lse=False, "
+    "causal_bottom_right=False, schedule=0) -> list of torch.Tensor\n\n"
+    "FP8 flash attention forward: fp8 q/k/v [B,H,N,d] -> [O] (fp16 by default), with return_lse=True [O, lse]"};
+
+}  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "FP8 flash-attention forward for AMD MI355X (gfx950)";
-  m.def("flash_attention_v2_cutlass", &flash_attention_v2_cutlass,
-        "FP8 flash attention forward: fp8 q/k/v [B,H,N,d] -> [O] (fp16 by default)", py::arg("q"), py::arg("k"),
-        py::arg("v"), py::arg("is_causal"), py::arg("softmax_scale"), py::kw_only(), py::arg("v_transposed") = false,
-        py::arg("out_dtype") = py::none(), py::arg("return_lse") = false, py::arg("causal_bottom_right") = false,
-        py::arg("schedule") = 0);
+  for (int i = 0; i < kArguments; ++i) interned_names[i] = PyUnicode_InternFromString(kNames[i]);
+  m.add_object("flash_attention_v2_cutlass",
+               py::reinterpret_steal<py::object>(PyCFunction_NewEx(&python_method, nullptr, m.attr("__name__").ptr())));
   m.def("kv_block", []() { return fa8_query(FA8_QUERY_KV_BLOCK); }, "kv rows per online-softmax step of the kernel");
 }
