@@ -968,10 +968,13 @@ struct Plan {
 // on every SIMD themselves.  `tiles` counts 32-row tiles (the query rows of a k/v head together), `even` the tiles of the
 // longest tile's length that hold the same work (causal square: half as many): what counts for a launch that starts its longest tiles
 // first.
-//   tiles <= CUs (head dim <= 64: 2 CUs): four wavefronts a tile, one tile a workgroup            1.2x (128 keys) - 2x (8192 keys)
+//   tiles <= CUs (head dim <= 64: 2 CUs, or a single tile per k/v head and more than 704 keys: bound by HBM): four wavefronts a tile,
+//     one tile a workgroup                                                                        1.2x (128 keys) - 2x (8192 keys)
 //   head dim 65 - 128, tiles <= 2 CUs: four wavefronts a tile, two tiles a workgroup (the tiles share the copies of K and V; two
 //     one-tile workgroups do not fit a CU's LDS)                                                  1.25 - 1.7x
 //   even <= 2 CUs (head dim <= 64: 4 CUs; causal: a quarter more): two wavefronts a tile, two tiles a workgroup      1.04 - 1.3x
+//   1.3 tiles <= wavefronts of the unshared launch (its workgroups have 128 rows of one q head each, which few queries leave idle): the
+//     same; 64 sequences, 8 queries of 64 heads on 8 k/v heads, 700 keys: 108 -> 21 us
 // Splitting the keys as well costs a second kernel and a reduction, about 5 us, and spreads the copies over all compute units:
 // taken where the estimate of its time is below the estimate for sharing (per-block times and rates measured; decode steps).
 Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
@@ -982,7 +985,7 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   const long long cus = compute_units();
   const long long group = p->heads_k > 0 ? p->heads / p->heads_k : 1, kv_heads = (long long)p->batch * (p->heads / group);
   const long long rows = group * p->seqlen_q, tiles = kv_heads * ((rows + 31) / 32);
-  if (tiles > 8 * cus || p->batch > 65535) return unshared;  // (also when the number of compute units is unknown)
+  if (cus == 0 || p->batch > 65535 || rows > 32 * 65535LL) return unshared;
   const long long shift = p->causal_align == FA8_CAUSAL_BOTTOM_RIGHT ? (long long)p->seqlen_k - p->seqlen_q : 0;
   auto blocks_of = [&](long long q_last) {  // KV blocks that query q_last sees, at least one
     const long long keys = p->is_causal ? std::min<long long>(p->seqlen_k, q_last + 1 + shift) : p->seqlen_k;
@@ -993,11 +996,11 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   const long long even = tiles * (longest + shortest) / (2 * longest);
   const int d = p->head_dim;
   Plan n = unshared;
-  if (tiles <= (d <= 64 ? 2 : 1) * cus)
+  if (tiles <= (d <= 64 ? 2 : 1) * cus || (d <= 64 && rows <= 32 && longest >= 12))
     n = {1, 4, 1};
-  else if (d > 64 && d <= 128 && tiles <= 2 * cus && longest > 2)
+  else if (d > 64 && d <= 128 && tiles <= 2 * cus && longest > 2 && rows > 32)
     n = {2, 4, 1};
-  else if (4 * even <= (d <= 64 ? 4 : 2) * (p->is_causal ? 5 : 4) * cus)
+  else if (4 * even <= (d <= 64 ? 4 : 2) * (p->is_causal ? 5 : 4) * cus || 13 * tiles <= 40 * p->batch * p->heads * ((p->seqlen_q + kQBlock - 1LL) / kQBlock))
     n = {2, 2, 1};
   if (workspace && n.waves_per_tile == 4 && n.tiles_per_workgroup == 1 && longest >= 16) {
     const double us_per_block = d <= 64 ? 0.25 : (d <= 128 ? 0.29 : 0.56);
@@ -1005,7 +1008,7 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
     const double s_bytes = 8.0 * tiles * live * longest * kKvBlock;
     const double shared_us = 4.5 + std::max(us_per_block * longest * ((tiles + cus - 1) / cus), kv_bytes / 5.8e6);
     const double split_us = 8.5 + (kv_bytes + s_bytes) / 5.0e6;
-    const long long splits = std::min({32LL, (cus + tiles - 1) / tiles, longest / 8});
+    const long long splits = std::min({32LL, cus / tiles, longest / 8});  // one workgroup more than CUs takes twice as long
     if (splits > 1 && split_us < 0.95 * shared_us && s_bytes < 512.0e6 && tiles * splits < 65536 &&
         longest / (4 * splits) < 65535)
       n.splits = (int)splits;

@@ -43,6 +43,9 @@ CASES = [
     (1, 60, 60, 545, 545, 32, True, False, False, E4, True, 2, 64),       # 18 tiles
     (1, 16, 16, 1056, 1056, 256, True, False, True, E5, True, 2, 64),
     (2, 12, 6, 700, 700, 160, True, False, False, E4, False, 2, 64),
+    (40, 64, 16, 3, 130, 128, True, True, False, E4, False, 2, 64),       # 640 k/v heads of one tile (12 rows): no rows in the second tile
+    (16, 64, 64, 130, 130, 64, True, False, False, E4, False, 2, 64),     # 5120 tiles; 128-row workgroups would be half idle
+    (20, 32, 32, 1, 1000, 32, True, True, False, E5, False, 4, 32),       # 640 tiles of one row
 ]
 
 
