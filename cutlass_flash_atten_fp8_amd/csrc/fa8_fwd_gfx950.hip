@@ -995,6 +995,9 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   // mean length of the tiles: half way between the first and the last one, but for rows that see every key or none
   const long long even = tiles * (longest + shortest) / (2 * longest);
   const int d = p->head_dim;
+  // a single KV block leaves nothing to share but the products, and a wide head's copies have one LDS stage there: 16 heads of 64 keys,
+  // us unshared / shared: head dim 160 4.7 / 6.1, 192 5.0 / 6.4, 224 5.1 / 6.5, 256 5.9 / 6.8 (128 keys: shared is the faster one)
+  if (d > 128 && longest == 1 && p->batch * (long long)p->heads * ((p->seqlen_q + kQBlock - 1) / kQBlock) <= cus) return unshared;
   Plan n = unshared;
   if (tiles <= (d <= 64 ? 2 : 1) * cus || (d <= 64 && rows <= 32 && longest >= 12))
     n = {1, 4, 1};

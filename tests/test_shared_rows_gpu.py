@@ -91,3 +91,10 @@ def test_strided_tensors_and_guard_bands():
     torch.cuda.synchronize()
     assert torch.equal(o.contiguous(), want)
     assert (obuf[:, n:] == 777.0).all()
+
+
+def test_one_block_of_a_wide_head_is_not_shared():
+    for n, waves in ((64, 1), (65, 4)):
+        q, k, v = _inputs(n, 1, 4, 4, n, n, 160, E4)
+        o = torch.empty(q.shape, dtype=torch.float16, device=DEV)
+        assert fa.plan(fa.make_params(q, k, v, o, False, 0.08))[1] == waves
