@@ -18,7 +18,10 @@
 // of a half iteration started at its beginning the copies are the limit (4100 - 4700).  Measured (us, one wavefront a tile -> shared):
 // 16 heads, 1024 keys, causal: head dim 64 13.3 -> 8.9 (R 1, W 4), 128 17.2 -> 12.4 (2, 4); 8 heads of 2048 keys, head dim 128, full: 28.5 ->
 // 19.5 (2, 4); 512 queries on 16384 keys, 32 heads on 8 k/v heads: 176 -> 100 (2, 4); 16 heads, 2048 keys, head dim 256, causal: 47.1 ->
-// 37.7 (2, 2); 1 query of 32 heads on 8 k/v heads, 16 sequences of 8191 keys: 145 -> 52, the rate of a plain copy (1, 4).
+// 37.7 (2, 2); 1 query of 32 heads on 8 k/v heads, 16 sequences of 8191 keys: 137 -> 52, the rate of a plain copy (1, 4).
+// Registers: two wavefronts a SIMD leave a lane 256; head dim 256 with two tiles needs 255 of them (v as rows) and 247 (transposed v, whose
+// copies and fragments take their row differences from scalar and immediate offsets; with a register for each, 31 - 42 of them were
+// spilled at head dims 224 and 256: 16 heads, 2048 keys, causal 76.4 us instead of 36.8, against 51.7 of the unshared loop).
 #ifndef FA8_SHARED_ROWS_H_
 #define FA8_SHARED_ROWS_H_
 #include <type_traits>
@@ -104,15 +107,16 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
   // A lane's offset in a segment depends on the segment number through few of its bits (the swizzle) and otherwise by whole rows:
   // segments that are kKVar (kVVar) apart differ by a multiple of the row stride.
   constexpr int kKVar = DP == 256 ? 4 : (DP == 128 ? 2 : 1);
-  constexpr int kVVar = DP == 256 && !VT ? 2 : 1;
-  // row of the block that a segment's rows count from (V^T: row of the tile)
+  constexpr int kVVar = DP == 256 && !VT ? 2 : 1;  // (transposed v: all segments share one offset, see issue_v)
+  // row of the block that a segment's rows count from
   auto k_row0 = [](int seg) {
     if (DP == 256) return 16 * (seg >> 3) + 4 * ((seg >> 1) & 3) + 32 * (seg & 1);
     if (DP == 128) return 16 * (seg >> 2) + 4 * (seg & 3);
     return DP == 64 ? 16 * (seg >> 1) + 8 * (seg & 1) : 16 * seg;
   };
-  auto v_row0 = [](int seg) { return seg * (VT ? 16 : 1024 / DP); };
-  unsigned k_src[kPasses], v_src[kPasses];
+  auto v_row0 = [](int seg) { return seg * (1024 / DP); };
+  unsigned k_src[kPasses], v_src[VT ? 1 : kPasses];
+  int v_chunk = 0;  // transposed v: the lane's first key of a block
 #pragma unroll
   for (int p = 0; p < kPasses; ++p) {
     const int seg = p * R + r;
@@ -128,7 +132,8 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
       int tr, ch;
       tile_slot_decode<VT ? 64 : DP, !VT>(seg * 64 + lane, tr, ch);
       v_src[p] = VT || ch * 16 < D ? (unsigned)(tr * v_rs + ch * 16) : kNoSource;
-    } else {
+      if (VT) v_chunk = ch * 16;
+    } else if constexpr (!VT) {
       v_src[p] = v_src[p % nv] + (unsigned)((v_row0(seg) - v_row0(p % nv * R + r)) * v_rs);
     }
   }
@@ -147,19 +152,17 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
   };
   auto issue_v = [&](int j, uint8_t* dst, bool exists, int from, int to) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)vp, 0, exists ? v_bytes : 0, kRsrcFlags);
-    const int base = !exists ? 0 : (VT ? j * kKvBlock : (int)((unsigned)j * kKvBlock * (unsigned)v_rs));
-    const bool v_clamp = VT && exists && (j + 1) * kKvBlock > a.seqlen_k;
+    const int v_base = !exists ? 0 : (int)((unsigned)j * kKvBlock * (unsigned)v_rs);
+    // transposed v, ragged last block: chunks past the last key are pulled back onto the last chunk (see fa8_fwd_kernel)
+    const unsigned v_from = VT ? v_src[0] + (unsigned)min(exists ? j * kKvBlock : 0, a.seqlen_k - 16 - v_chunk) : 0;
 #pragma unroll
     for (int p = from; p < to; ++p) {
       uint8_t* at = dst + w * kTileBytes + (p * R + r) * 1024;
-      if (v_clamp) {  // transposed v, ragged last block: see fa8_fwd_kernel
-        int tr, ch;
-        tile_slot_decode<64, false>((p * R + r) * 64 + lane, tr, ch);
-        const unsigned off = tr < D ? (unsigned)(tr * v_rs + min(j * kKvBlock + ch * 16, a.seqlen_k - 16)) : kNoSource;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, at), 16, off, 0, 0, 0);
+      if constexpr (VT) {
+        // segments are 16 rows apart, in the scalar offset; rows of the tile past the head dim lie past the resource
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, at), 16, v_from, (int)((unsigned)(p * R * 16) * (unsigned)v_rs), 0, 0);
       } else {
-        // (transposed v: rows of the tile past the head dim lie past the resource or are never read)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, at), 16, v_src[p], base, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, at), 16, v_src[p], v_base, 0, 0);
       }
     }
   };
@@ -203,28 +206,26 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
     for (int e = 0; e < 2; ++e) k_off[ks][e] = w * kTileBytes + tile_offset<DP, false>(qn, DP >= 64 ? 4 * ks + 2 * h + e : e);
   constexpr int kSubTileStride = 32 * DP, kVtTileStride = 32 * 64, kTrStride = 8 * DP;
   const int tr_j = (lane & 15) >> 1, tr_e = lane & 1, tr_g1 = (lane >> 4) & 1;
-  int v_off[kOwn][VT ? 2 : 1];
+  // (transposed v: the tiles of a wavefront lie W tiles apart, its two offsets serve them all)
+  int v_off[VT ? 2 : kOwn];
+  if constexpr (VT) {
 #pragma unroll
-  for (int m = 0; m < kOwn; ++m) {
-    const int mt = min(w + m * W, kMTiles - 1);
-    if constexpr (VT) {
+    for (int e = 0; e < 2; ++e) v_off[e] = w * kVtTileStride + tile_offset<64, false>(qn, 2 * h + e);
+  } else {
 #pragma unroll
-      for (int e = 0; e < 2; ++e) v_off[m][e] = mt * kVtTileStride + tile_offset<64, false>(qn, 2 * h + e);
-    } else {
-      v_off[m][0] = tile_offset<DP, true>(32 * h + tr_j, 2 * mt + tr_g1) + 8 * tr_e;
-    }
+    for (int m = 0; m < kOwn; ++m) v_off[m] = tile_offset<DP, true>(32 * h + tr_j, 2 * min(w + m * W, kMTiles - 1) + tr_g1) + 8 * tr_e;
   }
   auto load_vf = [&](const uint8_t* v_lds, int i, int m) __attribute__((always_inline)) {
     const uint8_t* vb = v_lds + i * kTileBytes;
     v8i vf;
     if constexpr (VT) {
-      const v4i lo = *LDS_PTR(const v4i, vb + v_off[m][0]);
-      const v4i hi = *LDS_PTR(const v4i, vb + v_off[m][VT ? 1 : 0]);
+      const v4i lo = *LDS_PTR(const v4i, vb + m * W * kVtTileStride + v_off[0]);
+      const v4i hi = *LDS_PTR(const v4i, vb + m * W * kVtTileStride + v_off[VT ? 1 : 0]);
       vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     } else {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const v2i x = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, vb + v_off[m][0] + g * kTrStride));
+        const v2i x = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, vb + v_off[VT ? 0 : m] + g * kTrStride));
         vf[2 * g] = x[0];
         vf[2 * g + 1] = x[1];
       }

@@ -1,0 +1,45 @@
+"""Register use of the compiled kernels, read from the code-object notes of libfa8.so (no GPU): a vector register spilled to scratch costs memory
+traffic in every step of a loop, and the shared-rows kernel of the wide head dims sits close to the 256 registers of a lane."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+import cutlass_flash_atten_fp8_amd as fa
+
+READELF = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-readelf")
+MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
+
+
+def code_objects(path):
+    """The gfx950 code objects bundled in a shared library (one bundle per source file)."""
+    data = open(path, "rb").read()
+    at = data.find(MAGIC)
+    while at >= 0:
+        (count,) = struct.unpack_from("<Q", data, at + len(MAGIC))
+        pos = at + len(MAGIC) + 8
+        for _ in range(count):
+            offset, size, length = struct.unpack_from("<QQQ", data, pos)
+            triple = data[pos + 24:pos + 24 + length].decode()
+            pos += 24 + length
+            if "gfx950" in triple and size:
+                yield data[at + offset:at + offset + size]
+        at = data.find(MAGIC, at + 1)
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="needs llvm-readelf")
+def test_no_kernel_spills_vector_registers(tmp_path):
+    kernels = {}
+    for i, blob in enumerate(code_objects(fa.LIBFA8_PATH)):
+        f = tmp_path / f"{i}.o"
+        f.write_bytes(blob)
+        notes = subprocess.run([READELF, "--notes", str(f)], capture_output=True, text=True, check=True).stdout
+        names = re.findall(r"^\s+\.name:\s+(_Z\S+)$", notes, re.M)
+        spills = re.findall(r"\.vgpr_spill_count:\s+(\d+)", notes)
+        assert len(names) == len(spills)
+        kernels.update(zip(names, map(int, spills)))
+    for part in ("fa8_fwd_kernel", "fa8_shared_rows_kernel", "fa8_split_logits_kernel", "fa8_split_values_kernel"):
+        assert any(part in n for n in kernels), part
+    assert {n: s for n, s in kernels.items() if s} == {}
