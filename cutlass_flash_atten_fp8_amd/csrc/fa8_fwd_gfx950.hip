@@ -962,19 +962,27 @@ struct Plan {
   int splits;               // > 1: the keys of a row tile dealt to this many workgroups (needs a workspace)
 };
 
-// The rule, from a sweep over head dims 32 / 64 / 96 / 128 / 160 / 256, 1 - 128 heads, 128 - 8192 keys, full and causal (each plan timed
-// on each shape).  A SIMD with one wavefront issues a vector instruction every 6 - 9 cycles, with three every 3: a launch of few
-// rows is faster if several wavefronts share a row tile, up to the point where the unshared loops have about two wavefronts
-// on every SIMD themselves.  `tiles` counts 32-row tiles (the query rows of a k/v head together), `even` the tiles of the
-// longest tile's length that hold the same work (causal square: half as many): what counts for a launch that starts its longest tiles
-// first.
-//   tiles <= CUs (head dim <= 64: 2 CUs, or a single tile per k/v head and more than 704 keys: bound by HBM): four wavefronts a tile,
-//     one tile a workgroup                                                                        1.2x (128 keys) - 2x (8192 keys)
-//   head dim 65 - 128, tiles <= 2 CUs: four wavefronts a tile, two tiles a workgroup (the tiles share the copies of K and V; two
-//     one-tile workgroups do not fit a CU's LDS)                                                  1.25 - 1.7x
-//   even <= 2 CUs (head dim <= 64: 4 CUs; causal: a quarter more): two wavefronts a tile, two tiles a workgroup      1.04 - 1.3x
-//   1.3 tiles <= wavefronts of the unshared launch (its workgroups have 128 rows of one q head each, which few queries leave idle): the
-//     same; 64 sequences, 8 queries of 64 heads on 8 k/v heads, 700 keys: 108 -> 21 us
+// The rule, from 18 500 shapes drawn over all head dims, 1 - 10000 row tiles, 1 - 20000 keys, full and causal, grouped or not, every plan
+// timed on every shape.  A SIMD with one wavefront issues a vector instruction every 6 - 9 cycles, with three every 3: a launch of few
+// rows is faster if several wavefronts share a row tile, up to the point where the unshared loops have about two wavefronts on every
+// SIMD themselves; from there on sharing costs (a launch that fills the chip: 1.1 - 1.6x with two wavefronts a tile, 1.5 - 4x with
+// four), unless the unshared launch, whose workgroups have 128 rows of one q head each, would be mostly idle.  `tiles` counts 32-row
+// tiles and `pairs` workgroups of two of them (the query rows of a k/v head together), `wgs` the workgroups of the unshared launch;
+// `longest` is the longest tile's KV blocks, `even` the pairs of that length that hold the same work (causal square: about half as
+// many): what counts for a launch that starts its longest tiles first.  In brackets the median of shared / unshared time.
+//   tiles <= CUs (head dim <= 64: 2 CUs), the most that run at once, and 3 blocks: four wavefronts a tile, one tile a workgroup
+//     (0.75 at 6 blocks, 0.55 from 33 on).  At 2 blocks the exchange costs what it saves, unless the head dim is at most 128 and the
+//     unshared workgroups are well filled (0.95).  Head dim <= 64, a single tile per k/v head, 12 blocks: any number, bound by HBM
+//   head dim 65 - 128, pairs <= CUs (one a CU) and 4 blocks: four wavefronts a tile, two tiles a workgroup, which share the copies of K
+//     and V (0.6 - 0.85)
+//   no more rounds of the CUs with pairs than with unshared workgroups (full and causal, every head dim and number of rounds): two
+//     wavefronts a tile, two tiles a workgroup (0.8 - 0.95; 0.2 - 0.75 where few queries of grouped heads leave half of the unshared
+//     workgroups idle).  One round more costs 1.05 - 1.4, except: rounds of unequal length, even <= CUs (causal: a quarter more; head
+//     dim <= 64: twice as many) and 5 blocks (head dim 32: 2) (0.8 - 1.0); head dim 32 up to 4/3 wgs (0.85 - 1.0); head dim 64 up to
+//     half as many rounds more from 8 blocks on if the tiles are about equally long (0.85 - 0.95)
+//   A single block leaves nothing to share but the products (1.05 - 1.3): only where the rows of grouped q heads fill the tiles that
+//     they would leave idle, 2 pairs <= wgs, and on a full chip (0.2 - 0.8), and under the mask at head dim 32, whose unshared loop is
+//     the rolling one (v as rows: 0.75 - 0.95, transposed 1.0 - 1.4)
 // Splitting the keys as well costs a second kernel and a reduction, about 5 us, and spreads the copies over all compute units:
 // taken where the estimate of its time is below the estimate for sharing (per-block times and rates measured; decode steps).
 Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
@@ -992,18 +1000,22 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
     return std::max(1LL, (keys + kKvBlock - 1) / kKvBlock);
   };
   const long long longest = blocks_of(p->seqlen_q - 1), shortest = blocks_of(std::min<long long>(31 / group, p->seqlen_q - 1));
-  // mean length of the tiles: half way between the first and the last one, but for rows that see every key or none
-  const long long even = tiles * (longest + shortest) / (2 * longest);
   const int d = p->head_dim;
-  // a single KV block leaves nothing to share but the products, and a wide head's copies have one LDS stage there: 16 heads of 64 keys,
-  // us unshared / shared: head dim 160 4.7 / 6.1, 192 5.0 / 6.4, 224 5.1 / 6.5, 256 5.9 / 6.8 (128 keys: shared is the faster one)
-  if (d > 128 && longest == 1 && p->batch * (long long)p->heads * ((p->seqlen_q + kQBlock - 1) / kQBlock) <= cus) return unshared;
+  const long long pairs = kv_heads * ((rows + 63) / 64), wgs = (long long)p->batch * p->heads * ((p->seqlen_q + kQBlock - 1LL) / kQBlock);
+  // mean length of the tiles: half way between the first and the last one, but for rows that see every key or none
+  const long long even = pairs * (longest + shortest) / (2 * longest);
+  const long long pair_rounds = (pairs + cus - 1) / cus, wg_rounds = (wgs + cus - 1) / cus;
+  const bool no_more_rounds = pair_rounds <= wg_rounds || (d == 32 && 3 * pairs <= 4 * wgs) ||
+                              (d == 64 && longest >= 8 && 5 * shortest > 3 * longest && 2 * pair_rounds <= 3 * wg_rounds);
+  const bool few_pairs = (longest >= 5 || d == 32) && 4 * even <= (p->is_causal ? 5 : 4) * (d <= 64 ? 2 : 1) * cus;
+  const bool one_block = (2 * pairs <= wgs && wgs > 2 * cus) || (d == 32 && p->is_causal && p->v_layout == FA8_V_ROWS && pairs <= wgs);
   Plan n = unshared;
-  if (tiles <= (d <= 64 ? 2 : 1) * cus || (d <= 64 && rows <= 32 && longest >= 12))
+  if ((longest >= 3 && tiles <= (d <= 64 ? 2 : 1) * cus) || (longest >= 12 && d <= 64 && rows <= 32) ||
+      (longest == 2 && d <= 128 && tiles <= cus && 8 * wgs < 5 * tiles))
     n = {1, 4, 1};
-  else if (d > 64 && d <= 128 && tiles <= 2 * cus && longest > 2 && rows > 32)
+  else if (d > 64 && d <= 128 && pairs <= cus && longest >= 4 && rows > 32)
     n = {2, 4, 1};
-  else if (4 * even <= (d <= 64 ? 4 : 2) * (p->is_causal ? 5 : 4) * cus || 13 * tiles <= 40 * p->batch * p->heads * ((p->seqlen_q + kQBlock - 1LL) / kQBlock))
+  else if (longest >= 2 ? no_more_rounds || few_pairs : one_block)
     n = {2, 2, 1};
   if (workspace && n.waves_per_tile == 4 && n.tiles_per_workgroup == 1 && longest >= 16) {
     const double us_per_block = d <= 64 ? 0.25 : (d <= 128 ? 0.29 : 0.56);

@@ -1,0 +1,46 @@
+"""How a launch is cut (fa8_fwd_plan): rows of a workgroup, wavefronts per 32 rows, parts of the keys.  Launches that sharing a row tile makes
+slower stay with one wavefront per tile.  Times: us on a MI355X, unshared / shared as the library once chose."""
+import pytest
+import torch
+
+import cutlass_flash_atten_fp8_amd as fa
+
+pytestmark = pytest.mark.gpu
+UNSHARED = (128, 1, 1)
+
+
+def plan_of(B, H, Hk, Nq, Nk, d, causal=False, bottom_right=False, vt=False, with_workspace=True):
+    """Nothing is launched: the parameters of tiny tensors with other sizes and contiguous strides."""
+    t = torch.zeros((1, 1, 1, 256), dtype=torch.float8_e4m3fn, device="cuda:0")
+    p = fa.make_params(t, t, t, torch.zeros((1, 1, 1, 256), dtype=torch.float16, device="cuda:0"), causal, d ** -0.5, vt, None, bottom_right)
+    p.batch, p.heads, p.heads_k, p.seqlen_q, p.seqlen_k, p.head_dim = B, H, Hk, Nq, Nk, d
+    for name, heads, rows, cols in (("q", H, Nq, d), ("k", Hk, Nk, d), ("v", Hk) + ((d, Nk) if vt else (Nk, d)), ("o", H, Nq, d)):
+        setattr(p, name + "_row_stride", cols)
+        setattr(p, name + "_head_stride", rows * cols)
+        setattr(p, name + "_batch_stride", heads * rows * cols)
+    return fa.plan(p, with_workspace)
+
+
+@pytest.mark.parametrize("shape", [
+    (32, 32, 32, 288, 1024, 256),       # 249 / 559
+    (64, 64, 64, 257, 1024, 64),        # 349 / 577
+    (64, 64, 64, 288, 288, 128),        # 241 / 405
+    (64, 64, 64, 96, 96, 96),           # 42 / 65
+    (32, 32, 32, 192, 192, 96),         # 28.8 / 38.7
+    (16, 70, 35, 192, 192, 128),        # 37.4 / 51.4
+    (64, 64, 64, 33, 33, 96),           # 23.8 / 35.7: a single block
+    (8, 32, 32, 64, 64, 64),            # 3.8 / 5.1
+    (1, 1, 1, 1, 1, 128),               # 3.8 / 4.4
+    (8, 12, 12, 157, 157, 128, True),   # 7.0 / 11.5: three blocks, 240 pairs
+    (4, 17, 17, 224, 224, 96, True),    # 7.9 / 10.5
+], ids=lambda s: "B{}H{}k{}Nq{}Nk{}d{}".format(*s[:6]))
+def test_sharing_does_not_take_launches_that_it_slows_down(shape):
+    if shape[4] <= 64 or shape[0] > 8:
+        assert plan_of(*shape) == UNSHARED
+    else:  # two wavefronts a tile: 7.1 and 6.4 us
+        assert plan_of(*shape)[1] <= 2
+
+
+def test_head_counts_beyond_32_bit_products():
+    """65535 sequences of 1024 heads on one k/v head: 40 * batch * heads does not fit 32 bits; one query each leaves 127 of 128 rows idle."""
+    assert plan_of(65535, 1024, 1, 1, 1, 128) == (64, 2, 1)

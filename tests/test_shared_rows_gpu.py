@@ -20,8 +20,10 @@ def _inputs(seed, B, H, Hk, Nq, Nk, d, dtype):
 
 CASES = [
     # B, H, Hk, Nq, Nk, d, causal, bottom_right, vt, dtype, fp8 out, wavefronts per tile, rows per workgroup
-    (1, 1, 1, 1, 1, 128, False, False, False, E4, False, 4, 32),
-    (1, 2, 2, 33, 64, 64, False, False, False, E4, False, 4, 32),
+    (1, 1, 1, 1, 1, 128, False, False, False, E4, False, 1, 128),         # a single block is not shared ...
+    (1, 2, 2, 33, 64, 64, False, False, False, E4, False, 1, 128),
+    (33, 32, 2, 1, 1, 128, False, False, False, E4, False, 2, 64),        # ... unless grouped heads fill the rows
+    (40, 32, 1, 2, 48, 256, True, True, True, E5, True, 2, 64),
     (1, 2, 2, 128, 128, 64, True, False, False, E4, True, 4, 32),
     (1, 2, 2, 300, 257, 128, False, False, False, E4, False, 4, 32),      # one key in the second group's first block
     (1, 3, 3, 300, 320, 96, True, True, False, E5, True, 4, 32),
@@ -44,7 +46,8 @@ CASES = [
     (1, 16, 16, 1056, 1056, 256, True, False, True, E5, True, 2, 64),
     (2, 12, 6, 700, 700, 160, True, False, False, E4, False, 2, 64),
     (40, 64, 16, 3, 130, 128, True, True, False, E4, False, 2, 64),       # 640 k/v heads of one tile (12 rows): no rows in the second tile
-    (16, 64, 64, 130, 130, 64, True, False, False, E4, False, 2, 64),     # 5120 tiles; 128-row workgroups would be half idle
+    (16, 64, 64, 130, 130, 64, True, False, False, E4, False, 1, 128),    # 5 tiles a head: three pairs for two workgroups, not shared
+    (16, 64, 64, 60, 130, 64, True, True, False, E4, False, 2, 64),       # 2 tiles a head: 128-row workgroups would be half idle
     (20, 32, 32, 1, 1000, 32, True, True, False, E5, False, 4, 32),       # 640 tiles of one row
 ]
 
@@ -94,7 +97,7 @@ def test_strided_tensors_and_guard_bands():
 
 
 def test_one_block_of_a_wide_head_is_not_shared():
-    for n, waves in ((64, 1), (65, 4)):
+    for n, waves in ((64, 1), (65, 2)):
         q, k, v = _inputs(n, 1, 4, 4, n, n, 160, E4)
         o = torch.empty(q.shape, dtype=torch.float16, device=DEV)
         assert fa.plan(fa.make_params(q, k, v, o, False, 0.08))[1] == waves
