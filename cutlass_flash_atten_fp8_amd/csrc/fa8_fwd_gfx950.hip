@@ -983,8 +983,12 @@ struct Plan {
 //   A single block leaves nothing to share but the products (1.05 - 1.3): only where the rows of grouped q heads fill the tiles that
 //     they would leave idle, 2 pairs <= wgs, and on a full chip (0.2 - 0.8), and under the mask at head dim 32, whose unshared loop is
 //     the rolling one (v as rows: 0.75 - 0.95, transposed 1.0 - 1.4)
-// Splitting the keys as well costs a second kernel and a reduction, about 5 us, and spreads the copies over all compute units:
-// taken where the estimate of its time is below the estimate for sharing (per-block times and rates measured; decode steps).
+// Splitting the keys as well costs a second kernel, a reduction and the logits' way through memory, and spreads the copies over all
+// compute units: taken where the estimate of its time is below that of four sharing wavefronts.  Both estimates are fits to 2382 drawn
+// launches (split: 5 % of them off by more than a quarter; shared: by more than a tenth): a start and, per block of a wavefront's range, a
+// step, plus K and V, plus the logits written and read (4.6 TB/s).  On those launches the choice is the slower one by more than 5 % in
+// 3 of 100 (17 of 100 with a start of 8.5 us and no step).  One head, 32 queries on 1121 keys, d128: 10.0 us shared, 19.3 split; 1 query
+// of 32 heads on 8 k/v heads, 32768 keys: 151 and 21.
 Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   const Plan unshared = {kQBlock / 32, 1, 1};
   // the sharing kernels rely on exp2(-inf * scale) = 0 and a finite start of the row max, like the pipelined loop; a schedule hint
@@ -1018,13 +1022,13 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   else if (longest >= 2 ? no_more_rounds || few_pairs : one_block)
     n = {2, 2, 1};
   if (workspace && n.waves_per_tile == 4 && n.tiles_per_workgroup == 1 && longest >= 16) {
-    const double us_per_block = d <= 64 ? 0.25 : (d <= 128 ? 0.29 : 0.56);
+    const long long splits = std::max(1LL, std::min({32LL, cus / tiles, longest / 8}));  // one workgroup more than CUs takes twice as long
+    const long long range = (longest + 4 * splits - 1) / (4 * splits);                   // blocks of a wavefront
     const double kv_bytes = 2.0 * kv_heads * longest * kKvBlock * d, live = rows < 32 ? (double)rows : 32.0;
     const double s_bytes = 8.0 * tiles * live * longest * kKvBlock;
-    const double shared_us = 4.5 + std::max(us_per_block * longest * ((tiles + cus - 1) / cus), kv_bytes / 5.8e6);
-    const double split_us = 8.5 + (kv_bytes + s_bytes) / 5.0e6;
-    const long long splits = std::min({32LL, cus / tiles, longest / 8});  // one workgroup more than CUs takes twice as long
-    if (splits > 1 && split_us < 0.95 * shared_us && s_bytes < 512.0e6 && tiles * splits < 65536 &&
+    const double shared_us = 4.3 + std::max((d <= 64 ? 0.25 : (d <= 128 ? 0.29 : 0.53)) * longest, kv_bytes / 5.8e6);
+    const double split_us = 10.5 + 1.34 / 128 * d * range + kv_bytes / 29e6 + s_bytes / 4.6e6;
+    if (splits > 1 && split_us < shared_us && s_bytes < 512.0e6 && tiles * splits < 65536 &&
         longest / (4 * splits) < 65535)
       n.splits = (int)splits;
   }

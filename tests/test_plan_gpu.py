@@ -41,6 +41,24 @@ def test_sharing_does_not_take_launches_that_it_slows_down(shape):
         assert plan_of(*shape)[1] <= 2
 
 
+@pytest.mark.parametrize("shape", [
+    (1, 1, 1, 32, 1121, 128, True, True),    # 10.0 shared, 19.3 split
+    (1, 4, 1, 15, 1244, 64, True, True),     # 9.1, 16.7
+    (1, 2, 1, 1051, 1051, 192, True),        # 15, 26.7
+    (1, 2, 2, 1792, 1792, 160),              # 20.1, 35.5
+    (1, 6, 2, 12, 1245, 128, True, True),    # 10.3, 18
+    (4, 1, 1, 832, 1665, 160),               # 20.1, 34.1
+], ids=lambda s: "B{}H{}k{}Nq{}Nk{}d{}".format(*s[:6]))
+def test_few_keys_are_not_split(shape):
+    assert plan_of(*shape)[1:] == (4, 1)
+
+
+@pytest.mark.parametrize("shape", [(1, 32, 8, 1, 32768, 128, True, True), (4, 32, 8, 1, 4096, 128, True, True), (1, 8, 8, 1, 4096, 64, True, True),
+                                   (1, 2, 2, 16, 4096, 224)], ids=lambda s: "B{}H{}k{}Nq{}Nk{}d{}".format(*s[:6]))
+def test_many_keys_are_split(shape):
+    assert plan_of(*shape)[2] > 1 and plan_of(*shape, with_workspace=False)[2] == 1
+
+
 def test_head_counts_beyond_32_bit_products():
     """65535 sequences of 1024 heads on one k/v head: 40 * batch * heads does not fit 32 bits; one query each leaves 127 of 128 rows idle."""
     assert plan_of(65535, 1024, 1, 1, 1, 128) == (64, 2, 1)
