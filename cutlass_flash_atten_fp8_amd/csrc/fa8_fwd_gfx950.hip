@@ -182,23 +182,26 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
   // Start the asynchronous copy of the K rows / the V rows of KV block j into the LDS buffer kb / vb.  The pipelined loops
   // start two tile copies in every step, also when the block no longer exists (so that one s_waitcnt constant fits every
   // step): such a copy (exists = false, wave-uniform) goes through a resource of length 0, every lane of it is out of range,
-  // zeros land in LDS and no memory is touched.
+  // zeros land in LDS and no memory is touched.  Its scalar offset is 0: a lane is out of range if its own offset is not below
+  // length - scalar offset, a difference that must not be negative.
   // (Dense loop: the second pass of a copy differs from the first by a whole number of rows, 16 kv rows of K and 32 (64) rows
   // of V (V^T): the difference sits in the scalar offset and both passes share one vector register.)
   const int k_bytes = (int)(kv_last * a.k_rs + D);
   const int v_bytes = VT ? (int)((D - 1) * a.v_rs + a.seqlen_k) : (int)(kv_last * a.v_rs + D);
   auto issue_k = [&](int j, uint8_t* kb, bool exists) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)kp, 0, exists ? k_bytes : 0, kRsrcFlags);
-    const int k_base = (int)((unsigned)j * kKvBlock * (unsigned)a.k_rs);  // below 2^32 (fa8_fwd_validate)
+    const int k_rs = exists ? (int)a.k_rs : 0;
+    const int k_base = (int)((unsigned)j * kKvBlock * (unsigned)k_rs);  // below 2^32 (fa8_fwd_validate)
 #pragma unroll
     for (int p = 0; p < kPasses; ++p)
       if (!kSplitPass || wave < 2)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, kb + copy_segment(p) * 1024), 16, DENSE ? k_src[0] : k_src[p],
-                                                 DENSE ? k_base + p * 16 * (int)a.k_rs : k_base, 0, 0);
+                                                 DENSE ? k_base + p * 16 * k_rs : k_base, 0, 0);
   };
   auto issue_v = [&](int j, uint8_t* vb, bool exists) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)vp, 0, exists ? v_bytes : 0, kRsrcFlags);
-    const int v_base = VT ? j * kKvBlock : (int)((unsigned)j * kKvBlock * (unsigned)a.v_rs);
+    const int v_rs = exists ? (int)a.v_rs : 0;
+    const int v_base = VT ? (exists ? j * kKvBlock : 0) : (int)((unsigned)j * kKvBlock * (unsigned)v_rs);
     // transposed v, ragged last block: the 16-byte chunks past the last kv column would read the start of the next
     // head-dim row (or run off the tensor); they are pulled back onto the last chunk instead (and masked later)
     const bool v_clamp = VT && (j + 1) * kKvBlock > a.seqlen_k;
@@ -213,7 +216,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, vb + seg), 16, off, 0, 0, 0);
         } else {
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, vb + seg), 16, DENSE ? v_src[0] : v_src[p],
-                                                   DENSE ? v_base + p * (VT ? 64 : 32) * (int)a.v_rs : v_base, 0, 0);
+                                                   DENSE ? v_base + p * (VT ? 64 : 32) * v_rs : v_base, 0, 0);
         }
       }
     }

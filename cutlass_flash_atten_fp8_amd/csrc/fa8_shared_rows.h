@@ -159,8 +159,11 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
     for (int p = from; p < to; ++p) {
       uint8_t* at = dst + w * kTileBytes + (p * R + r) * 1024;
       if constexpr (VT) {
-        // segments are 16 rows apart, in the scalar offset; rows of the tile past the head dim lie past the resource
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, at), 16, v_from, (int)((unsigned)(p * R * 16) * (unsigned)v_rs), 0, 0);
+        // Segments are 16 rows apart, in the scalar offset.  A lane is out of range if its offset is not below length - scalar offset,
+        // which must not be negative: rows of the tile past the head dim, like blocks that do not exist, take length 0 and scalar offset 0.
+        const bool there = exists && (16 * (p * R + R - 1) < D || 16 * (p * R + r) < D);
+        const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc((void*)vp, 0, there ? v_bytes : 0, kRsrcFlags);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, LDS_PTR(void, at), 16, v_from, there ? (int)((unsigned)(p * R * 16) * (unsigned)v_rs) : 0, 0, 0);
       } else {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, at), 16, v_src[p], v_base, 0, 0);
       }
