@@ -964,6 +964,7 @@ struct Plan {
   int waves_per_tile;       // 1: the loops of this file; 2, 4: wavefronts share a row tile
   int splits;               // > 1: the keys of a row tile dealt to this many workgroups (needs a workspace)
 };
+constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask for
 
 // The rule, from 18 500 shapes drawn over all head dims, 1 - 10000 row tiles, 1 - 20000 keys, full and causal, grouped or not, every plan
 // timed on every shape.  A SIMD with one wavefront issues a vector instruction every 6 - 9 cycles, with three every 3: a launch of few
@@ -1031,8 +1032,8 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
     const double s_bytes = 8.0 * tiles * live * longest * kKvBlock;
     const double shared_us = 4.3 + std::max((d <= 64 ? 0.25 : (d <= 128 ? 0.29 : 0.53)) * longest, kv_bytes / 5.8e6);
     const double split_us = 10.5 + 1.34 / 128 * d * range + kv_bytes / 29e6 + s_bytes / 4.6e6;
-    if (splits > 1 && split_us < shared_us && s_bytes < 512.0e6 && tiles * splits < 65536 &&
-        longest / (4 * splits) < 65535)
+    if (splits > 1 && split_us < shared_us && tiles * splits < 65536 && longest / (4 * splits) < 65535 &&
+        split_workspace(p, (int)splits) <= kMaxWorkspace)
       n.splits = (int)splits;
   }
   return n;

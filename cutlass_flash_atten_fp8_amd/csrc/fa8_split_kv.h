@@ -37,13 +37,19 @@ struct SplitWorkspace {
   long long part_m;     // [splits][32]
   long long part_l;     // [splits][32]
   long long part_o;     // [splits][live rows][head_dim]
-  long long s;          // [live rows][keys]: masked logits, whole KV blocks
+  long long s;          // [live rows][keys]: masked logits of the keys that some query sees, whole KV blocks
+  long long keys;
   long long bytes;
 };
-__host__ __device__ inline SplitWorkspace split_layout(long long all_tiles, int splits, int live_rows, int head_dim, int seqlen_k) {
+// Keys that some query sees: a mask aligned with the first key hides those past the last query.
+__host__ __device__ inline int split_visible_keys(int seqlen_q, int seqlen_k, bool causal, bool bottom_right) {
+  return causal && !bottom_right && seqlen_q < seqlen_k ? seqlen_q : seqlen_k;
+}
+__host__ __device__ inline SplitWorkspace split_layout(long long all_tiles, int splits, int live_rows, int head_dim, int visible_keys) {
   auto up = [](long long x) { return (x + 255) / 256 * 256; };
-  const long long keys = ((long long)seqlen_k + kKvBlock - 1) / kKvBlock * kKvBlock, rows32 = all_tiles * splits * 128;
+  const long long keys = ((long long)visible_keys + kKvBlock - 1) / kKvBlock * kKvBlock, rows32 = all_tiles * splits * 128;
   SplitWorkspace w;
+  w.keys = keys;
   w.done = 0;
   w.range_max = up(all_tiles * 4);
   w.split_max = w.range_max + rows32 * kSplitWaves;
@@ -110,7 +116,8 @@ __device__ __forceinline__ SplitPlace split_place(const SplitShape& n, int head_
   p.tile = tiles == 1 ? 0 : (int)blockIdx.z / p.splits;
   p.split = (int)blockIdx.z - p.tile * p.splits;
   p.at = ((long long)p.b * n.heads_k + p.hk) * tiles + p.tile;
-  p.ws = split_layout(n.all_tiles, p.splits, p.live_rows, head_dim, n.seqlen_k);
+  p.ws = split_layout(n.all_tiles, p.splits, p.live_rows, head_dim,
+                      split_visible_keys(n.seqlen_q, n.seqlen_k, p.causal, n.mode & kSharedBottomRight));
   p.lane = threadIdx.x & 63;
   p.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   p.qn = p.lane & 31;
@@ -190,8 +197,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_e
   // leading blocks without a masked logit in any row of the tile
   const int q_first = p.query_of(min(p.tile * 32, p.last_row));
   const int n_plain = (p.causal ? max(0, min(q_first + p.shift, seqlen_k)) : seqlen_k) / kKvBlock;
-  const long long keys = (long long)((seqlen_k + kKvBlock - 1) / kKvBlock) * kKvBlock;
-  float* s_out = (float*)(a.n.workspace + p.ws.s) + (p.at * p.live_rows + qn) * keys + 32 * h;
+  float* s_out = (float*)(a.n.workspace + p.ws.s) + (p.at * p.live_rows + qn) * p.ws.keys + 32 * h;
   const bool live = qn < p.live_rows && p.row <= p.last_row;  // (lane 0 always is: the stores below are never skipped)
   float m_run = -1.0e30f;
   // Block i of the range: S, then the copy of block i + 2 into the tile just read, then max and stores.  vmcnt counts loads and stores in
@@ -310,8 +316,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_e
       }
     }
   };
-  const long long keys = (long long)((seqlen_k + kKvBlock - 1) / kKvBlock) * kKvBlock;
-  const float* s_in = (const float*)(a.n.workspace + p.ws.s) + (p.at * p.live_rows + min(qn, p.live_rows - 1)) * keys + 32 * h;
+  const float* s_in = (const float*)(a.n.workspace + p.ws.s) + (p.at * p.live_rows + min(qn, p.live_rows - 1)) * p.ws.keys + 32 * h;
   auto load_s = [&](int j, v4f(&s)[8]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) s[i] = *(const v4f*)(s_in + (long long)j * kKvBlock + 4 * i);

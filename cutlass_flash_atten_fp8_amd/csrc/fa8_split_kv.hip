@@ -17,7 +17,7 @@ const void* values_kernel(bool e5m2, bool vt) {
 }
 
 struct Plan {
-  int heads_k, tiles, live_rows, splits, blocks_per_range;
+  int heads_k, tiles, live_rows, keys, splits, blocks_per_range;
 };
 
 Plan plan_of(const Fa8FwdParams* p, int splits) {
@@ -26,10 +26,8 @@ Plan plan_of(const Fa8FwdParams* p, int splits) {
   const long long rows = (long long)(p->heads / n.heads_k) * p->seqlen_q;
   n.tiles = (int)((rows + 31) / 32);
   n.live_rows = rows < 32 ? (int)rows : 32;
-  // the blocks that the last query sees
-  long long keys = p->seqlen_k;
-  if (p->is_causal && p->causal_align != FA8_CAUSAL_BOTTOM_RIGHT && p->seqlen_q < keys) keys = p->seqlen_q;
-  const int blocks = (int)((keys + kKvBlock - 1) / kKvBlock);
+  n.keys = split_visible_keys(p->seqlen_q, p->seqlen_k, p->is_causal, p->causal_align == FA8_CAUSAL_BOTTOM_RIGHT);
+  const int blocks = (int)(((long long)n.keys + kKvBlock - 1) / kKvBlock);
   n.blocks_per_range = (blocks + splits * kSplitWaves - 1) / (splits * kSplitWaves);
   n.splits = (blocks + n.blocks_per_range * kSplitWaves - 1) / (n.blocks_per_range * kSplitWaves);
   return n;
@@ -39,7 +37,7 @@ Plan plan_of(const Fa8FwdParams* p, int splits) {
 
 long long fa8::split_workspace(const Fa8FwdParams* p, int splits) {
   const Plan n = plan_of(p, splits);
-  return split_layout((long long)p->batch * n.heads_k * n.tiles, n.splits, n.live_rows, p->head_dim, p->seqlen_k).bytes;
+  return split_layout((long long)p->batch * n.heads_k * n.tiles, n.splits, n.live_rows, p->head_dim, n.keys).bytes;
 }
 
 int fa8::launch_split(const Fa8FwdParams* p, int splits, void* workspace, hipStream_t stream) {

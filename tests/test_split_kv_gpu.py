@@ -88,6 +88,24 @@ def test_workspace_is_optional_and_its_contents_do_not_matter():
     assert_same_up_to_sum_order(outs[1], outs[0], v, 8000)
 
 
+def test_workspace_is_for_the_keys_that_some_query_sees():
+    """A mask aligned with the first key hides all keys past the last query: 131072 keys of which 2048 count (the others hold NaN codes)."""
+    nq, nk, d = 2048, 131072, 160
+    q, k, v = _inputs(7, 1, 1, 1, nq, nk, d, E4)
+    k.view(torch.uint8)[:, :, nq:] = 0x7F
+    v.view(torch.uint8)[:, :, nq:] = 0x7F
+    want, want_lse = fa.flash_attention_v2_cutlass(q, k, v, True, d ** -0.5, return_lse=True, schedule=fa.FA8_SCHEDULE_ROLLING)
+    p = fa.make_params(q, k, v, want, True, d ** -0.5, False, want_lse)
+    splits, need = fa.plan(p)[2], ctypes.c_int64()
+    assert splits > 1 and fa.lib().fa8_fwd_workspace(ctypes.byref(p), ctypes.byref(need)) == 0
+    parts = 64 * splits * 32 * (d + 8) * 4  # 64 row tiles: O, the row sums and the maxima of every part
+    assert 0 < need.value <= nq * nq * 4 + parts + 8192
+    got, lse = fa.flash_attention_v2_cutlass(q, k, v, True, d ** -0.5, return_lse=True)
+    torch.cuda.synchronize()
+    assert_same_up_to_sum_order(got, want, v[:, :, :nq], nq)
+    assert (lse - want_lse).abs().max() <= 5e-6 * max(1.0, want_lse.abs().max().item())
+
+
 def test_split_keys_in_a_hip_graph():
     ext = fa.load_extension()
     q, k, v = _inputs(4, 1, 8, 2, 1, 8000, 128, E4)
