@@ -196,8 +196,13 @@ def flash_attention_v2_cutlass(q, k, v, is_causal, softmax_scale, *, v_transpose
         rc = lib().fa8_fwd_workspace(ctypes.byref(p), ctypes.byref(need))
         if rc == 0:
             # goes back to torch's allocator on return, for later work of this stream
-            workspace = torch.empty(need.value, dtype=torch.uint8, device=q.device) if need.value else None
-            rc = lib().fa8_fwd_ws(ctypes.byref(p), workspace.data_ptr() if need.value else None, need.value, ctypes.c_void_p(stream))
+            workspace = None
+            if need.value:
+                try:
+                    workspace = torch.empty(need.value, dtype=torch.uint8, device=q.device)
+                except torch.OutOfMemoryError:  # the call needs none, it only takes longer
+                    pass
+            rc = lib().fa8_fwd_ws(ctypes.byref(p), None if workspace is None else workspace.data_ptr(), need.value, ctypes.c_void_p(stream))
     if rc != 0:
         raise RuntimeError(f"flash_attention_v2_cutlass: {error_string(rc)} (code {rc})")
     return [o, lse] if return_lse else [o]

@@ -113,8 +113,13 @@ Outputs flash_attention_v2_cutlass(const torch::Tensor& q, const torch::Tensor& 
   torch::Tensor workspace;  // (goes back to torch's allocator on return, for later work of this stream)
   int rc = fa8_fwd_workspace(&p, &workspace_bytes);
   if (rc == FA8_OK) {
-    if (workspace_bytes > 0) workspace = new_tensor({workspace_bytes}, at::kByte, q);
-    rc = fa8_fwd_ws(&p, workspace_bytes > 0 ? workspace.data_ptr() : nullptr, workspace_bytes, (void*)stream);
+    if (workspace_bytes > 0) {
+      try {
+        workspace = new_tensor({workspace_bytes}, at::kByte, q);
+      } catch (const c10::OutOfMemoryError&) {  // the call needs none, it only takes longer
+      }
+    }
+    rc = workspace.defined() ? fa8_fwd_ws(&p, workspace.data_ptr(), workspace_bytes, (void*)stream) : fa8_fwd(&p, (void*)stream);
   }
   TORCH_CHECK(rc == FA8_OK, "flash_attention_v2_cutlass: ", fa8_error_string(rc), " (code ", rc, ")");
   return {out, lse};

@@ -88,6 +88,28 @@ def test_workspace_is_optional_and_its_contents_do_not_matter():
     assert_same_up_to_sum_order(outs[1], outs[0], v, 8000)
 
 
+@pytest.mark.parametrize("call", [lambda *a, **kw: fa.load_extension().flash_attention_v2_cutlass(*a, **kw), fa.flash_attention_v2_cutlass],
+                         ids=["binding", "ctypes"])
+def test_no_memory_for_the_workspace(call):
+    """The allocator refuses another segment: the call goes on without a workspace."""
+    q, k, v = _inputs(9, 1, 32, 8, 1, 131072, 32, E4)
+    want = torch.empty(q.shape, dtype=torch.float16, device=DEV)
+    p = fa.make_params(q, k, v, want, True, 0.09, causal_bottom_right=True)
+    need = ctypes.c_int64()
+    assert fa.plan(p)[2] > 1 and fa.lib().fa8_fwd_workspace(ctypes.byref(p), ctypes.byref(need)) == 0
+    assert fa.lib().fa8_fwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction(1e-6)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(need.value, dtype=torch.uint8, device=DEV)
+        got = call(q, k, v, True, 0.09, causal_bottom_right=True)[0]
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(got, want)
+
+
 def test_workspace_is_for_the_keys_that_some_query_sees():
     """A mask aligned with the first key hides all keys past the last query: 131072 keys of which 2048 count (the others hold NaN codes)."""
     nq, nk, d = 2048, 131072, 160
