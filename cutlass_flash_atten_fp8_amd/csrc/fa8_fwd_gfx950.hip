@@ -1156,7 +1156,7 @@ int launch_rows(const Fa8FwdParams* p, hipStream_t stream) {
 int run(const Fa8FwdParams* p, void* workspace, long long bytes, hipStream_t stream) {
   Plan n = choose_plan(p, workspace != nullptr);
   if (n.splits > 1 && bytes < split_workspace(p, n.splits)) n = choose_plan(p, false);
-  if (n.splits > 1) return launch_split(p, n.splits, workspace, stream);
+  if (n.splits > 1) return (uintptr_t)workspace % 16 != 0 ? FA8_ERR_ALIGN : launch_split(p, n.splits, workspace, stream);
   return n.waves_per_tile > 1 ? launch_shared(p, n.tiles_per_workgroup, n.waves_per_tile, stream) : launch_rows(p, stream);
 }
 
@@ -1218,7 +1218,7 @@ extern "C" const char* fa8_error_string(int code) {
     case FA8_ERR_SHAPE: return "bad shape (a size < 1, too many workgroups, heads not a multiple of heads_k, or k/v of one head spanning 2 GiB or more)";
     case FA8_ERR_HEAD_DIM: return "head_dim must be a multiple of 32, at most 256";
     case FA8_ERR_STRIDE: return "a stride is smaller than the extent it spans";
-    case FA8_ERR_ALIGN: return "q/k/v rows must be 16-byte aligned and o rows 8-byte aligned";
+    case FA8_ERR_ALIGN: return "q/k/v rows and a workspace must be 16-byte aligned and o rows 8-byte aligned";
     case FA8_ERR_DTYPE: return "unknown in_dtype / out_dtype / v_layout / causal_align code";
     case FA8_ERR_UNSUPPORTED: return "this build has no kernel for the requested combination";
     case FA8_ERR_SCALE: return "softmax_scale must be finite";

@@ -125,8 +125,8 @@ int fa8_fwd(const Fa8FwdParams* p, void* hip_stream);
 
 /*
  * The same with device memory to work in.  fa8_fwd_workspace writes the number of bytes that this call can make use of on the
- * current device (0: none); fa8_fwd_ws runs the call with a workspace of that size (any contents, 256-byte aligned, the caller's
- * again once the stream has passed the work).  Few query rows over many keys (decode steps) are then spread over the whole GPU by
+ * current device (0: none); fa8_fwd_ws runs the call with a workspace of that size (any contents, 16-byte aligned or the call that would
+ * use it returns FA8_ERR_ALIGN, the caller's again once the stream has passed the work).  Few query rows over many keys (decode steps) are then spread over the whole GPU by
  * splitting the keys, which fa8_fwd, without memory for the parts, cannot do.  Without a workspace, or with one that is too
  * small, fa8_fwd_ws is fa8_fwd.  The weights of a split call are the same bit for bit; its fp32 sums are taken in another order.
  * (fa8_fwd itself still needs no memory.)  No counterpart in the reference.

@@ -88,6 +88,22 @@ def test_workspace_is_optional_and_its_contents_do_not_matter():
     assert_same_up_to_sum_order(outs[1], outs[0], v, 8000)
 
 
+def test_workspace_alignment_and_size():
+    """16-byte vector accesses: a workspace off that alignment is refused before anything is launched; one that is too small is not used."""
+    q, k, v = _inputs(3, 1, 8, 2, 1, 8000, 128, E4)
+    outs = [torch.full(q.shape, float("nan"), dtype=torch.float16, device=DEV) for _ in range(3)]
+    params = [fa.make_params(q, k, v, o, True, 0.09, causal_bottom_right=True) for o in outs]
+    need = ctypes.c_int64()
+    assert fa.lib().fa8_fwd_workspace(ctypes.byref(params[0]), ctypes.byref(need)) == 0 and need.value > 0
+    ws = torch.full((need.value + 512,), 0xFF, dtype=torch.uint8, device=DEV)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert fa.lib().fa8_fwd_ws(ctypes.byref(params[0]), ws.data_ptr() + 8, need.value, stream) == -5  # FA8_ERR_ALIGN
+    assert fa.lib().fa8_fwd_ws(ctypes.byref(params[1]), ws.data_ptr(), need.value - 1, stream) == 0
+    assert fa.lib().fa8_fwd(ctypes.byref(params[2]), stream) == 0
+    torch.cuda.synchronize()
+    assert torch.isnan(outs[0]).all() and torch.equal(outs[1], outs[2]) and (ws == 0xFF).all()
+
+
 @pytest.mark.parametrize("call", [lambda *a, **kw: fa.load_extension().flash_attention_v2_cutlass(*a, **kw), fa.flash_attention_v2_cutlass],
                          ids=["binding", "ctypes"])
 def test_no_memory_for_the_workspace(call):
