@@ -162,7 +162,10 @@ PyObject* python_flash_attention(PyObject*, PyObject* const* args, Py_ssize_t n_
     while (i < kArguments && name != interned_names[i]) ++i;  // keywords written in a program are interned
     if (i == kArguments)
       for (i = 0; i < kArguments && PyUnicode_Compare(name, interned_names[i]) != 0;) ++i;
-    if (i == kArguments) type_error(std::string("got an unexpected keyword argument '") + PyUnicode_AsUTF8(name) + "'");
+    if (i == kArguments) {  // (a name need not have a UTF-8 form)
+      PyErr_Format(PyExc_TypeError, "flash_attention_v2_cutlass(): got an unexpected keyword argument '%U'", name);
+      return nullptr;
+    }
     if (v[i]) type_error(std::string("got multiple values for argument '") + kNames[i] + "'");
     v[i] = args[n_positional + x];
   }

@@ -176,6 +176,18 @@ def test_compiled_binding_mirrors_reference_errors():
     assert ext.kv_block() == fa.query(fa.FA8_QUERY_KV_BLOCK)
 
 
+@pytest.mark.parametrize("name", ["foo", "v_transpose", "\u00fc", "\ud800"], ids=["ascii", "near", "latin", "surrogate"])
+def test_compiled_binding_refuses_unknown_keywords(name):
+    """Any str can be a keyword of a ** call, also one without a UTF-8 form (a lone surrogate); in a process of its own: it used to crash."""
+    import subprocess
+    import sys
+    code = ("import torch, attention_cutlass_fp8 as m\nq = torch.zeros(1, 1, 1, 32)\ntry:\n"
+            f"    m.flash_attention_v2_cutlass(q, q, q, False, 0.1, **{{{ascii(name)}: 1}})\n"
+            f"except TypeError as e:\n    assert {ascii(name)} in str(e), ascii(e)\n    print('refused')\n")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and "refused" in r.stdout, (r.returncode, r.stderr[-500:])
+
+
 def test_schedule_query_follows_explicit_hints_without_a_gpu():
     """fa8_fwd_schedule: an explicit hint is answered without touching the GPU; it holds only where the loop it names exists."""
     sched = fa.lib().fa8_fwd_schedule
