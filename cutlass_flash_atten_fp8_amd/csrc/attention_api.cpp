@@ -185,6 +185,11 @@ PyObject* python_flash_attention(PyObject*, PyObject* const* args, Py_ssize_t n_
   long long schedule = 0;
   if (v[9]) {
     schedule = PyFloat_Check(v[9]) ? -1 : PyLong_AsLongLong(v[9]);
+    if (schedule == -1 && !PyFloat_Check(v[9]) && PyErr_Occurred() && PyNumber_Check(v[9])) {  // no __index__: __int__, as pybind11 does
+      PyErr_Clear();
+      const py::object whole = py::reinterpret_steal<py::object>(PyNumber_Long(v[9]));
+      if (whole) schedule = PyLong_AsLongLong(whole.ptr());
+    }
     if (PyFloat_Check(v[9]) || (schedule == -1 && PyErr_Occurred())) {
       PyErr_Clear();
       type_error(std::string("argument 'schedule' must be an int, not ") + Py_TYPE(v[9])->tp_name);

@@ -176,6 +176,21 @@ def test_compiled_binding_mirrors_reference_errors():
     assert ext.kv_block() == fa.query(fa.FA8_QUERY_KV_BLOCK)
 
 
+def test_compiled_binding_takes_every_number_as_a_schedule():
+    """What pybind11's int conversion takes: whatever has __index__ or __int__ and is no float."""
+    from decimal import Decimal
+
+    import numpy as np
+    ext = fa.load_extension()
+    q = torch.zeros(1, 1, 1, 32)  # (the arguments are converted first, then the CPU tensors are refused)
+    for taken in (0, True, np.int64(3), np.float32(1), Decimal(2), torch.tensor(1), torch.tensor(1.0), 77):
+        with pytest.raises(RuntimeError, match="GPU tensor"):
+            ext.flash_attention_v2_cutlass(q, q, q, False, 0.1, schedule=taken)
+    for refused in (1.0, np.float64(1), "1", None, 1 << 70, 1j, [1], torch.zeros(2)):
+        with pytest.raises(TypeError):
+            ext.flash_attention_v2_cutlass(q, q, q, False, 0.1, schedule=refused)
+
+
 @pytest.mark.parametrize("name", ["foo", "v_transpose", "\u00fc", "\ud800"], ids=["ascii", "near", "latin", "surrogate"])
 def test_compiled_binding_refuses_unknown_keywords(name):
     """Any str can be a keyword of a ** call, also one without a UTF-8 form (a lone surrogate); in a process of its own: it used to crash."""
