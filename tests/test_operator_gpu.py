@@ -245,11 +245,12 @@ def test_capturable_in_a_hip_graph(schedule, causal):
         eager = ext.flash_attention_v2_cutlass(q, k, v, causal, 0.09, schedule=schedule)[0].clone()
 
 
-@pytest.mark.parametrize("nk,causal,schedule", [(99968, False, fa.FA8_SCHEDULE_AUTO), (100000, False, fa.FA8_SCHEDULE_PIPELINED),
+@pytest.mark.parametrize("nk,causal,schedule", [(99968, False, fa.FA8_SCHEDULE_AUTO), (99968, False, fa.FA8_SCHEDULE_DENSE),
+                                                (100000, False, fa.FA8_SCHEDULE_PIPELINED),
                                                 (100000, True, fa.FA8_SCHEDULE_ROLLING), (100000, True, fa.FA8_SCHEDULE_PIPELINED)])
 def test_long_kv_with_rows_far_apart(nk, causal, schedule):
     """100 000 keys whose rows lie 20 480 bytes apart: the kernel's 32-bit byte offsets into k and v run up to 2.05e9, just
-    under the 2^31 the library accepts.  The gaps between the rows hold NaN codes, so a misplaced read shows.  Bit for bit the
+    under the 2^31 the library accepts; in all loops, and in the shared-rows kernel (without a hint).  The gaps between the rows hold NaN codes, so a misplaced read shows.  Bit for bit the
     result of the same call on contiguous copies, and a few rows against the oracle."""
     d, nq, stride = 128, 200, 20480
     q, k, v = (rand_fp8((1, 1, n, d), s).to(DEV) for n, s in ((nq, 31), (nk, 32), (nk, 33)))
@@ -265,6 +266,8 @@ def test_long_kv_with_rows_far_apart(nk, causal, schedule):
     for kk, vv in ((kw, vw), (k, v)):
         o = torch.empty((1, 1, nq, d), dtype=torch.float16, device=DEV)
         p = fa.make_params(q, kk, vv, o, causal, scale, causal_bottom_right=True, schedule=schedule)
+        assert fa.plan(p, with_workspace=False)[1] == (4 if schedule == fa.FA8_SCHEDULE_AUTO else 1)
+        assert schedule == fa.FA8_SCHEDULE_AUTO or fa.lib().fa8_fwd_schedule(ctypes.byref(p)) == schedule
         rc = fa.lib().fa8_fwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
         assert rc == 0, fa.error_string(rc)
         outs.append(o)

@@ -86,7 +86,8 @@ def test_strided_tensors_and_guard_bands():
 
     obuf = torch.full((B, n + pad, H, d), 777.0, dtype=torch.float16, device=DEV)
     o = obuf[:, :n].permute(0, 2, 1, 3)
-    p = fa.make_params(spread_out(q), spread_out(k), spread_out(v), o, False, 0.09, **kw)
+    wide = spread_out(q), spread_out(k), spread_out(v)  # (kept: the parameters hold pointers only)
+    p = fa.make_params(*wide, o, False, 0.09, **kw)
     assert fa.plan(p)[1] == 4
     assert fa.lib().fa8_fwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
     want = fa.flash_attention_v2_cutlass(*(t.permute(0, 2, 1, 3).contiguous() for t in (q, k, v)), False, 0.09,
@@ -94,6 +95,26 @@ def test_strided_tensors_and_guard_bands():
     torch.cuda.synchronize()
     assert torch.equal(o.contiguous(), want)
     assert (obuf[:, n:] == 777.0).all()
+
+
+@pytest.mark.parametrize("shape", [(1, 4, 2, 40, 700, 64), (1, 16, 16, 256, 700, 128), (1, 40, 40, 700, 700, 64), (1, 8, 8, 300, 700, 256)],
+                         ids=lambda s: "B{}H{}k{}Nq{}Nk{}d{}".format(*s))
+@pytest.mark.parametrize("where", ["q", "k", "v"])
+@pytest.mark.parametrize("code", [0x7C, 0x7F], ids=["inf", "nan"])  # of e5m2
+def test_infinity_and_nan_reach_the_rows_that_they_reach_in_the_rolling_loop(shape, where, code):
+    """One element of one head, full attention.  An infinite key gives a row a logit of +inf (NaN row), or of -inf (the key is not seen)."""
+    q, k, v = _inputs(2, *shape, E5)
+    t = {"q": q, "k": k, "v": v}[where]
+    t.view(torch.uint8)[0, 1, 33 if where == "q" else 432, 17] = code
+    outs = []
+    for schedule in (fa.FA8_SCHEDULE_ROLLING, fa.FA8_SCHEDULE_AUTO):
+        outs += fa.flash_attention_v2_cutlass(q, k, v, False, 0.125, return_lse=True, schedule=schedule)
+    want, want_lse, got, lse = outs
+    assert fa.plan(fa.make_params(q, k, v, got, False, 0.125, lse=lse))[1:] in ((2, 1), (4, 1))
+    torch.cuda.synchronize()
+    assert not torch.isfinite(want).all() and torch.isfinite(want).any()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got[~torch.isnan(got)], want[~torch.isnan(want)])
+    assert torch.equal(torch.isnan(lse), torch.isnan(want_lse)) and torch.equal(lse[~torch.isnan(lse)], want_lse[~torch.isnan(want_lse)])
 
 
 def test_one_block_of_a_wide_head_is_not_shared():

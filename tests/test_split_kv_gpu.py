@@ -44,6 +44,9 @@ CASES = [
     (1, 2, 2, 16, 4096, 224, False, True, E5, False),
     (1, 8, 2, 1, 20000, 256, True, False, E4, False),
     (1, 1, 1, 1, 100000, 128, True, False, E4, False),
+    (1, 4, 2, 7, 6007, 128, False, False, E4, False),    # no mask, ragged last block
+    (2, 2, 2, 1, 8192, 64, False, False, E5, True),      # no mask, whole blocks
+    (1, 4, 2, 50, 12345, 128, True, False, E4, False),   # 100 packed rows: four tiles, the last with 4 rows
 ]
 
 
@@ -62,6 +65,83 @@ def test_split_keys_against_the_rolling_loop(case):
     assert_same_up_to_sum_order(got, want, v, Nk)
     assert (lse - want_lse).abs().max() <= 5e-6 * max(1.0, want_lse.abs().max().item())
     assert torch.equal(got.view(torch.uint8), again.view(torch.uint8)) and torch.equal(lse, lse2)  # whichever part ends last
+
+
+def _with_workspace(p):
+    need = ctypes.c_int64()
+    assert fa.lib().fa8_fwd_workspace(ctypes.byref(p), ctypes.byref(need)) == 0 and need.value > 0
+    ws = torch.full((need.value,), 0xFF, dtype=torch.uint8, device=DEV)
+    rc = fa.lib().fa8_fwd_ws(ctypes.byref(p), ws.data_ptr(), need.value, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, fa.error_string(rc)
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("vt", [False, True], ids=["rows", "vt"])
+def test_strided_tensors_and_guard_bands(vt):
+    """[B,N,H,d] storage, NaN codes behind the last key (transposed v: behind every row of keys), an output whose padding must stay untouched."""
+    B, H, Hk, nq, nk, d, pad = 2, 4, 2, 3, 6000, 96, 80
+    q, k, v = _inputs(5, B, H, Hk, nq, nk, d, E4)
+
+    def spread_out(t, rows_first):
+        t = t.permute(0, 2, 1, 3) if rows_first else t
+        shape = list(t.shape)
+        shape[1 if rows_first else 3] += pad
+        buf = torch.full(shape, 0x7F, dtype=torch.uint8, device=DEV)
+        at = buf[:, :t.shape[1]] if rows_first else buf[..., :t.shape[3]]
+        at.copy_(t.view(torch.uint8))
+        return at.permute(0, 2, 1, 3).view(E4) if rows_first else at.view(E4)
+
+    vv = v.transpose(2, 3).contiguous() if vt else v
+    obuf = torch.full((B, nq + pad, H, d), 777.0, dtype=torch.float16, device=DEV)
+    o = obuf[:, :nq].permute(0, 2, 1, 3)
+    wide = spread_out(q, True), spread_out(k, True), spread_out(vv, not vt)  # (kept: the parameters hold pointers only)
+    p = fa.make_params(*wide, o, True, 0.1, vt, causal_bottom_right=True)
+    assert fa.plan(p)[2] > 1
+    _with_workspace(p)
+    want = fa.flash_attention_v2_cutlass(q, k, vv, True, 0.1, v_transposed=vt, causal_bottom_right=True)[0]
+    assert torch.equal(o.contiguous(), want)  # the same plan: the same bits
+    assert (obuf[:, nq:] == 777.0).all()
+    rolling = fa.flash_attention_v2_cutlass(q, k, vv, True, 0.1, v_transposed=vt, causal_bottom_right=True, schedule=fa.FA8_SCHEDULE_ROLLING)[0]
+    assert_same_up_to_sum_order(want, rolling, v, nk)
+
+
+def test_long_kv_with_rows_far_apart():
+    """100 000 keys 20 480 bytes apart: 32-bit byte offsets into k and v up to 2.05e9; the gaps between the rows hold NaN codes."""
+    d, nk, stride = 128, 100000, 20480
+    q, k, v = _inputs(8, 1, 1, 1, 4, nk, d, E4)
+    wide = []
+    for t in (k, v):
+        big = torch.full((nk, stride), 0x7F, dtype=torch.uint8, device=DEV)
+        big[:, :d] = t.view(torch.uint8)[0, 0]
+        wide.append(big[:, :d].view(E4)[None, None])
+    o = torch.full(q.shape, float("nan"), dtype=torch.float16, device=DEV)
+    p = fa.make_params(q, wide[0], wide[1], o, True, 0.09, causal_bottom_right=True)
+    assert fa.plan(p)[2] > 1
+    _with_workspace(p)
+    assert torch.equal(o, fa.flash_attention_v2_cutlass(q, k, v, True, 0.09, causal_bottom_right=True)[0])
+
+
+@pytest.mark.parametrize("where", ["q", "k", "v"])
+@pytest.mark.parametrize("code", [0x7C, 0x7F], ids=["inf", "nan"])  # of e5m2
+def test_infinity_and_nan_reach_the_rows_that_they_reach_in_the_rolling_loop(where, code):
+    """One element of one head, full attention.  An infinite key gives a row a logit of +inf (NaN row), or of -inf (the key is not seen)."""
+    q, k, v = _inputs(2, 1, 4, 2, 6, 6001, 64, E5)
+    t = {"q": q, "k": k, "v": v}[where]
+    t.view(torch.uint8)[0, 1, 3 if where == "q" else 4321, 17] = code
+    outs = []
+    for schedule in (fa.FA8_SCHEDULE_ROLLING, fa.FA8_SCHEDULE_AUTO):
+        outs += fa.flash_attention_v2_cutlass(q, k, v, False, 0.125, return_lse=True, schedule=schedule)
+    want, want_lse, got, lse = outs
+    assert fa.plan(fa.make_params(q, k, v, got, False, 0.125, lse=lse))[2] > 1
+    torch.cuda.synchronize()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    assert not torch.isfinite(want).all() and torch.isfinite(want).any()
+    fine = torch.isfinite(want)
+    least = torch.where(torch.isfinite(v.float()), v.float(), torch.zeros_like(v.float()))
+    assert_same_up_to_sum_order(got[fine], want[fine], least, 6001)
+    assert torch.equal(torch.isnan(lse), torch.isnan(want_lse))
+    seen = ~torch.isnan(want_lse)
+    assert (lse - want_lse)[seen].abs().max() <= 5e-6 * max(1.0, want_lse[seen].abs().max().item())
 
 
 def test_workspace_is_optional_and_its_contents_do_not_matter():
