@@ -165,8 +165,8 @@ def flash_attention_v2_cutlass(q, k, v, is_causal, softmax_scale, *, v_transpose
     RuntimeError on bad arguments, like the reference's TORCH_CHECKs (include/attention_api.cuh:12-18).
     Beyond the reference: k/v may have fewer heads than q (grouped-query attention), return_lse=True returns
     [O, lse] with lse the float32 [B,H,Nq] log-sum-exp of the scaled logits, causal_bottom_right=True aligns the
-    causal diagonal with the last key when seqlen_q != seqlen_k; schedule (FA8_SCHEDULE_*) is a performance hint that
-    never changes the result.
+    causal diagonal with the last key when seqlen_q != seqlen_k; schedule (FA8_SCHEDULE_*) is a performance hint: 0 lets the
+    library choose, and is the only value with which it may split the keys of a few query rows (other order of the fp32 sums).
     """
     import torch
     for name, t in (("q", q), ("k", k), ("v", v)):

@@ -17,13 +17,12 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 
 #define LDS_PTR(T, p) ((__attribute__((address_space(3))) T*)(p))
-#define GLOBAL_PTR(T, p) ((__attribute__((address_space(1))) T*)(p))
 
 constexpr int kQBlock = 128;   // query rows per workgroup
 constexpr int kQWave = 32;     // query rows per wavefront
 constexpr int kKvBlock = 64;   // kv rows per online-softmax step
 constexpr int kThreads = 256;  // 4 wavefronts
-constexpr int kVersion = 4;
+constexpr int kVersion = 5;
 // main loops (template parameter LOOP of the kernel)
 constexpr int kLoopRolling = 0, kLoopPipelined = 1, kLoopDense = 2;
 

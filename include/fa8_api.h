@@ -38,8 +38,9 @@ extern "C" {
 #define FA8_CAUSAL_TOP_LEFT 0     /* key j <= query i: the reference's rule (csrc/flash_attention.cu:62-64, loop bound :458) */
 #define FA8_CAUSAL_BOTTOM_RIGHT 1 /* key j <= i + seqlen_k - seqlen_q: the last query sees every key (decode, chunked prefill) */
 
-/* which main loop the kernel runs: a performance hint, the results are bitwise the same
- *   AUTO      the library chooses from the shape of the launch
+/* which main loop the kernel runs: a performance hint.  The three loops and shared rows (fa8_fwd_plan) give bitwise the same results.
+ *   AUTO      the library chooses from the shape of the launch.  The only value with which fa8_fwd_ws may split the keys of a call, and
+ *             so sum in another order (fa8_fwd_plan tells); any hint, and any call without a workspace, keeps the unsplit order
  *   ROLLING   one KV block after the other, three wavefronts per SIMD: for masked launches that fill the chip
  *   PIPELINED software-pipelined over neighbouring KV blocks, two wavefronts per SIMD: for small masked launches
  *   DENSE     the same pipeline in three wavefronts per SIMD, for launches without any masked logit: full (non-causal)
@@ -100,7 +101,7 @@ typedef struct Fa8FwdParams {
   int32_t heads_k;
   int32_t causal_align; /* FA8_CAUSAL_* */
   /* ---- library version 3; all-zero = the library chooses ---- */
-  int32_t schedule;  /* FA8_SCHEDULE_*: a performance hint, never changes the result */
+  int32_t schedule;  /* FA8_SCHEDULE_*: a performance hint; fa8_fwd gives the same bits for all of them */
   int32_t reserved0; /* must be 0 (anything else: FA8_ERR_UNSUPPORTED) */
 } Fa8FwdParams;
 
@@ -124,18 +125,19 @@ int fa8_fwd_validate(const Fa8FwdParams* p);
 int fa8_fwd(const Fa8FwdParams* p, void* hip_stream);
 
 /*
- * The same with device memory to work in.  fa8_fwd_workspace writes the number of bytes that this call can make use of on the
- * current device (0: none); fa8_fwd_ws runs the call with a workspace of that size (any contents, 16-byte aligned or the call that would
- * use it returns FA8_ERR_ALIGN, the caller's again once the stream has passed the work).  Few query rows over many keys (decode steps) are then spread over the whole GPU by
- * splitting the keys, which fa8_fwd, without memory for the parts, cannot do.  Without a workspace, or with one that is too
- * small, fa8_fwd_ws is fa8_fwd.  The weights of a split call are the same bit for bit; its fp32 sums are taken in another order.
- * (fa8_fwd itself still needs no memory.)  No counterpart in the reference.
+ * The same with device memory to work in (library version 5).  fa8_fwd_workspace writes the number of bytes that this call can make
+ * use of on the current device (0: none, at most 256 MB); fa8_fwd_ws runs the call with a workspace of that size (any contents; 16-byte
+ * aligned, or a call that would use it returns FA8_ERR_ALIGN; the caller's again once the stream has passed the work).  Few query rows
+ * over many keys (decode steps) are then spread over the whole GPU by splitting the keys, which fa8_fwd, without memory for the parts,
+ * cannot do.  Without a workspace, or with one that is too small, fa8_fwd_ws is fa8_fwd.  The weights of a split call are the same bit
+ * for bit; its fp32 sums are taken in another order, and since the cut depends on the whole launch, the last bits of a row of O can then
+ * depend on the batch size and the number of compute units.  (fa8_fwd itself still needs no memory.)  No counterpart in the reference.
  */
 int fa8_fwd_workspace(const Fa8FwdParams* p, int64_t* bytes);
 int fa8_fwd_ws(const Fa8FwdParams* p, void* workspace, int64_t bytes, void* hip_stream);
 
 /*
- * How a call would be cut on the current device, for benchmarks and tests (nothing is launched): query rows of a workgroup
+ * How a call would be cut on the current device, for benchmarks and tests (library version 5; nothing is launched): query rows of a workgroup
  * (grouped q heads counted together), wavefronts that share 32 of them (1: one of the main loops of fa8_fwd_schedule; 2 or 4: shared
  * rows, for launches with few of them; a schedule hint always gives 1), and into how many parts the keys of a row are split
  * (more than 1 only with_workspace).  The results of shared and unshared rows are bitwise the same.
@@ -144,10 +146,10 @@ int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* rows_per_wo
                  int32_t* kv_splits);
 
 /*
- * Which main loop a wavefront that has its 32 query rows to itself (see fa8_fwd_plan) would run for these arguments on the current device: FA8_SCHEDULE_ROLLING,
- * FA8_SCHEDULE_PIPELINED or FA8_SCHEDULE_DENSE (all > 0), or the FA8_ERR_* code fa8_fwd_validate gives.  Launches nothing.  No counterpart in
- * the reference (one kernel, one loop: csrc/flash_attention.cu:468-534); it makes the library's choice visible to
- * benchmarks and tests.
+ * Which main loop a wavefront that has its 32 query rows to itself would run for these arguments on the current device:
+ * FA8_SCHEDULE_ROLLING, FA8_SCHEDULE_PIPELINED or FA8_SCHEDULE_DENSE (all > 0), or the FA8_ERR_* code fa8_fwd_validate gives; whether
+ * the call has such wavefronts, fa8_fwd_plan tells.  Launches nothing.  No counterpart in the reference (one kernel, one loop:
+ * csrc/flash_attention.cu:468-534); it makes the library's choice visible to benchmarks and tests.
  */
 int fa8_fwd_schedule(const Fa8FwdParams* p);
 

@@ -33,6 +33,10 @@ def test_library_exports_every_declared_symbol():
         assert getattr(lib, name) is not None
 
 
+def test_library_version_tells_of_the_workspace_entry_points():
+    assert fa.query(fa.FA8_QUERY_VERSION) >= 5  # fa8_fwd_workspace, fa8_fwd_ws, fa8_fwd_plan
+
+
 def test_query_values():
     assert fa.query(fa.FA8_QUERY_VERSION) >= 1
     assert fa.query(fa.FA8_QUERY_KV_BLOCK) in (64, 128)
