@@ -100,8 +100,8 @@ def shape_sweep(ext, fa, torch):
             q, k, v = (torch.randn((bsz, heads, n, d), generator=g).to(torch.float8_e4m3fn).cuda() for _ in range(3))
             for causal in (False, True):
                 scale = 1.0 / math.sqrt(d)
-                plan = fa.lib().fa8_fwd_schedule(ctypes.byref(fa.make_params(
-                    q, k, v, ext.flash_attention_v2_cutlass(q, k, v, causal, scale)[0], causal, scale)))
+                main_loop = loop_name(fa, fa.make_params(
+                    q, k, v, ext.flash_attention_v2_cutlass(q, k, v, causal, scale)[0], causal, scale))
                 t0 = time.perf_counter()
                 while time.perf_counter() - t0 < 0.1:
                     for _ in range(10):
@@ -117,7 +117,7 @@ def shape_sweep(ext, fa, torch):
                 avg = sum(ms) / len(ms)
                 flops = 4.0 * bsz * heads * n * n * d * (0.5 if causal else 1.0)
                 rows.append({"batch": bsz, "heads": heads, "seq_len": n, "head_dim": d, "causal": causal,
-                             "main_loop": MAIN_LOOPS.get(plan, str(plan)), "kernel_ms_avg": round(avg, 5),
+                             "main_loop": main_loop, "kernel_ms_avg": round(avg, 5),
                              "tflops": round(flops / (avg * 1e-3) / 1e12, 1),
                              "pct_fp8_mfma_peak": round(100.0 * flops / (avg * 1e-3) / 1e12 / FP8_MFMA_PEAK_TFLOPS, 2)})
     print(json.dumps({"metric": "fp8_attention_fwd_shape_sweep", "unit": "TFLOP/s", "rows": rows}), flush=True)
@@ -209,7 +209,7 @@ def time_other_workload(name, ext, fa, inputs, torch, launches=20, settle_second
 
     def step():
         return ext.flash_attention_v2_cutlass(q, k, v, causal, scale)[0]
-    plan = fa.lib().fa8_fwd_schedule(ctypes.byref(fa.make_params(q, k, v, step(), causal, scale)))
+    main_loop = loop_name(fa, fa.make_params(q, k, v, step(), causal, scale))
     t0 = time.perf_counter()
     while time.perf_counter() - t0 < settle_seconds:
         for _ in range(20):
@@ -226,7 +226,7 @@ def time_other_workload(name, ext, fa, inputs, torch, launches=20, settle_second
     flops, alg = inputs.flops(cfg), inputs.algorithmic_bytes(cfg)
     traffic = MEASURED_TRAFFIC_BYTES.get(name)
     return {"workload": f"{name}: B={cfg['B']} H={cfg['H']} N={cfg['N']} d={cfg['d']} {'causal' if causal else 'non-causal'}",
-            "main_loop": MAIN_LOOPS.get(plan, f"error {plan}"),
+            "main_loop": main_loop,
             "kernel_ms_avg": round(avg, 5), "kernel_ms_min": round(ms[0], 5),
             "tflops": round(flops / (avg * 1e-3) / 1e12, 1),
             "pct_fp8_mfma_peak": round(100.0 * flops / (avg * 1e-3) / 1e12 / FP8_MFMA_PEAK_TFLOPS, 2),
@@ -237,6 +237,17 @@ def time_other_workload(name, ext, fa, inputs, torch, launches=20, settle_second
 
 
 MAIN_LOOPS = {1: "rolling", 2: "pipelined", 3: "dense"}  # FA8_SCHEDULE_* (include/fa8_api.h)
+
+
+def loop_name(fa, p):
+    """What the library runs for a call through the binding: split keys, shared rows, or one of the three main loops."""
+    _, waves, splits = fa.plan(p)
+    if splits > 1:
+        return f"split keys ({splits} parts)"
+    if waves > 1:
+        return f"shared rows ({waves} wavefronts)"
+    loop = fa.lib().fa8_fwd_schedule(ctypes.byref(p))
+    return MAIN_LOOPS.get(loop, f"error {loop}")
 
 
 def main():
@@ -332,10 +343,7 @@ def main():
     def step():
         return ext.flash_attention_v2_cutlass(q, k, v, causal, scale, v_transposed=args.v_transposed, schedule=hint)[0]
 
-    # which of the kernel's main loops the library runs for this launch (include/fa8_api.h, FA8_SCHEDULE_*)
-    plan = fa.lib().fa8_fwd_schedule(ctypes.byref(fa.make_params(q, k, v, step(), causal, scale, v_transposed=args.v_transposed,
-                                                                 schedule=hint)))
-    main_loop = MAIN_LOOPS.get(plan, f"error {plan}")
+    main_loop = loop_name(fa, fa.make_params(q, k, v, step(), causal, scale, v_transposed=args.v_transposed, schedule=hint))
     for _ in range(args.warmup):
         step()
     torch.cuda.synchronize()
