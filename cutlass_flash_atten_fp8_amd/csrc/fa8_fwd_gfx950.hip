@@ -988,11 +988,12 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 //     they would leave idle, 2 pairs <= wgs, and on a full chip (0.2 - 0.8), and under the mask at head dim 32, whose unshared loop is
 //     the rolling one (v as rows: 0.75 - 0.95, transposed 1.0 - 1.4)
 // Splitting the keys as well costs a second kernel, a reduction and the logits' way through memory, and spreads the copies over all
-// compute units: taken where the estimate of its time is below that of four sharing wavefronts.  Both estimates are fits to 2382 drawn
-// launches (split: 5 % of them off by more than a quarter; shared: by more than a tenth): a start and, per block of a wavefront's range, a
-// step, plus K and V, plus the logits written and read (4.6 TB/s).  On those launches the choice is the slower one by more than 5 % in
-// 3 of 100 (17 of 100 with a start of 8.5 us and no step).  One head, 32 queries on 1121 keys, d128: 10.0 us shared, 19.3 split; 1 query
-// of 32 heads on 8 k/v heads, 32768 keys: 151 and 21.
+// compute units: taken where the estimate of its time is below that of four sharing wavefronts.  Both estimates are fits to 3003 drawn
+// launches whose K and V come from HBM and 1725 whose K and V the Infinity Cache still holds: a start, a step per block of a wavefront's
+// range, K and V, and the logits written and read; neither is below the rate at which it moves its bytes.  On these launches the choice is
+// the slower one by more than 5 % in 2 of 100, from HBM as from the cache.  (Fitted on repeated inputs alone and without a bound by the
+// bytes, K and V seemed to pass at 29 TB/s: 16 sequences of 8191 keys, 1 query of 32 heads on 8 k/v heads, d128 were split, 69 us instead
+// of 53.)  One head, 32 queries on 1121 keys, d128: 10.0 us shared, 19.3 split; one sequence of 32768 keys: 151 and 21.
 Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   const Plan unshared = {kQBlock / 32, 1, 1};
   // the sharing kernels rely on exp2(-inf * scale) = 0 and a finite start of the row max, like the pipelined loop; a schedule hint
@@ -1030,8 +1031,8 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
     const long long range = (longest + 4 * splits - 1) / (4 * splits);                   // blocks of a wavefront
     const double kv_bytes = 2.0 * kv_heads * longest * kKvBlock * d, live = rows < 32 ? (double)rows : 32.0;
     const double s_bytes = 8.0 * tiles * live * longest * kKvBlock;
-    const double shared_us = 4.3 + std::max((d <= 64 ? 0.25 : (d <= 128 ? 0.29 : 0.53)) * longest, kv_bytes / 5.8e6);
-    const double split_us = 10.5 + 1.34 / 128 * d * range + kv_bytes / 29e6 + s_bytes / 4.6e6;
+    const double shared_us = 5.4 + std::max((d <= 64 ? 0.23 : (d <= 128 ? 0.30 : 0.63)) * longest, kv_bytes / 5.6e6);
+    const double split_us = std::max(10.0 + 1.6 / 128 * d * range + kv_bytes / 30e6 + s_bytes / 4.0e6, 2.6 + (kv_bytes + s_bytes) / 5.2e6);
     if (splits > 1 && split_us < shared_us && tiles * splits < 65536 && longest / (4 * splits) < 65535 &&
         split_workspace(p, (int)splits) <= kMaxWorkspace)
       n.splits = (int)splits;
