@@ -202,7 +202,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_e
   float m_run = -1.0e30f;
   // Block i of the range: S, then the copy of block i + 2 into the tile just read, then max and stores.  vmcnt counts loads and stores in
   // issue order; what is issued after the copy of block i and may still be under way when its S is formed: the stores of block i - 2
-  // (not counted below, they are old by then), the copy of block i + 1 and the stores of block i - 1.
+  // (not counted below, they are old by then), the copy of block i + 1 and the stores of block i - 1.  That is what the odd blocks wait
+  // for; in front of the even ones' reads the compiler, which does not see that no copy under way writes lds0, waits for everything.
   constexpr int kStores = 8;
   auto block = [&](int i, uint8_t* tile) __attribute__((always_inline)) {
     const int j = p.first + i;
@@ -322,8 +323,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_e
     for (int i = 0; i < 8; ++i) s[i] = *(const v4f*)(s_in + (long long)j * kKvBlock + 4 * i);
   };
   v4f s0[8], s1[8];
-  // The running max before this range: over the splits before this one and the ranges before this one in the split; all loads under way
-  // together (one after the other they would cost a memory latency each), and before those of the first block.
+  // The running max before this range: over the splits before this one (their loads under way together; the compiler takes their max
+  // inside this branch, so a split > 0 waits for them before the loads below start) and the ranges before this one in the split.
   const float* split_max = (const float*)(a.n.workspace + p.ws.split_max) + p.at * p.splits * 32;
   const float* range_max = (const float*)(a.n.workspace + p.ws.range_max) + (p.at * p.splits + p.split) * kSplitWaves * 32;
   float before[kSplitMax / 2 + kSplitWaves - 1];
@@ -405,7 +406,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
     for (int mt = 0; mt < kMTiles; ++mt) o_acc[mt] = mfma_fp8<E5M2>(load_vf(vb, mt), p8, o_acc[mt]);
   };
-  // The next block's logits and V are asked for before a block is worked on: the last kPasses + 8 loads may still fly then.
+  // The next block's logits and V are asked for before a block is worked on: the last kPasses + 8 loads may still fly then.  (So they do
+  // in front of the blocks in lds0; in front of the V reads from lds1 the compiler waits for everything, as in the logits kernel.)
   constexpr int kNext = kPasses + 8;
   for (int i = 0; i < p.count; i += 2) {
     if (i + 1 < p.count) {
