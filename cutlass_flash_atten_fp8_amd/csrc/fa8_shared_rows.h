@@ -18,7 +18,7 @@
 // of a half iteration started at its beginning the copies are the limit (4100 - 4700).  Measured (us, one wavefront a tile -> shared):
 // 16 heads, 1024 keys, causal: head dim 64 13.3 -> 8.9 (R 1, W 4), 128 17.2 -> 12.4 (2, 4); 8 heads of 2048 keys, head dim 128, full: 28.5 ->
 // 19.5 (2, 4); 512 queries on 16384 keys, 32 heads on 8 k/v heads: 176 -> 100 (2, 4); 16 heads, 2048 keys, head dim 256, causal: 47.1 ->
-// 37.7 (2, 2); 1 query of 32 heads on 8 k/v heads, 16 sequences of 8191 keys: 137 -> 52, the rate of a plain copy (1, 4).
+// 36.4 (2, 2); 1 query of 32 heads on 8 k/v heads, 16 sequences of 8191 keys: 137 -> 52, the rate of a plain copy (1, 4).
 // Registers: two wavefronts a SIMD leave a lane 256; head dim 256 with two tiles needs 255 of them (v as rows) and 247 (transposed v, whose
 // copies and fragments take their row differences from scalar and immediate offsets; with a register for each, 31 - 42 of them were
 // spilled at head dims 224 and 256: 16 heads, 2048 keys, causal 76.4 us instead of 36.8, against 51.7 of the unshared loop).
