@@ -142,6 +142,13 @@ __device__ __forceinline__ float lane32_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// max of two floats that are no signalling NaN (fmaxf first quiets operands that come from memory, an instruction each)
+__device__ __forceinline__ float max2(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
 // max of three floats; the compiler fuses the pair into one v_max3_f32.
 __device__ __forceinline__ float max3(float a, float b, float c) { return __builtin_fmaxf(__builtin_fmaxf(a, b), c); }
 

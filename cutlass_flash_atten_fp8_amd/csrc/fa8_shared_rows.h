@@ -13,15 +13,21 @@
 //   V of the next group; weights and row sums -> LDS
 // Head dims above 128 have LDS for one stage only: the copies of the next group's K and this group's V fly for half an iteration.
 //
-// What bounds it: the issue of vector instructions by the one or two wavefronts of a SIMD (about 200 a wavefront and iteration, each
-// 6 - 9 cycles apart with so few wavefronts) and two barriers an iteration, 3900 cycles at R = 2, W = 4; with fewer stages or all copies
-// of a half iteration started at its beginning the copies are the limit (4100 - 4700).  Measured (us, one wavefront a tile -> shared):
+// What bounds it: the one or two wavefronts of a SIMD walk one chain (row max - LDS - barrier - weights - LDS - barrier), about 310
+// instructions a wavefront and iteration, each 5 cycles or more apart within a wavefront whatever its kind; 3500 cycles at R = 2, W = 4.
+// Not the LDS (its reads run at 29 % of the cycles), not the copies alone (10 % without them), not the exponentials (10 %).
+// With fewer stages or all copies of a half iteration started at its beginning the copies are the limit (4100 - 4700).
+// S^T of the next group is formed also where no group follows (a stale tile, never used): behind a branch, the wait counts of the
+// two paths met at every chunk and each one waited for the LDS reads just issued; with the additions of the row sums pinned to their
+// chunks (the compiler moved all 32 to the end, with the weights alive until then) the registers went from 194 to 153 (R 2, W 4, head dim
+// 128) and from 255 to 215 (R 2, W 2, head dim 256).  16 sequences of 8191 keys, K and V from the cache, 42.9 -> 41.1 us; 512 queries on 16384
+// keys 102.1 -> 100.5; 16 heads, 2048 keys, head dim 256, causal 39.2 -> 38.4 (in a captured graph).  Measured (us, one wavefront a tile -> shared):
 // 16 heads, 1024 keys, causal: head dim 64 13.3 -> 8.9 (R 1, W 4), 128 17.2 -> 12.4 (2, 4); 8 heads of 2048 keys, head dim 128, full: 28.5 ->
-// 19.5 (2, 4); 512 queries on 16384 keys, 32 heads on 8 k/v heads: 176 -> 100 (2, 4); 16 heads, 2048 keys, head dim 256, causal: 47.1 ->
+// 19.5 (2, 4); 512 queries on 16384 keys, 32 heads on 8 k/v heads: 176 -> 100 (2, 4); 8 heads, 3000 keys, head dim 160, causal: (2, 2) 43.5 -> (2, 4) 37.1; 16 heads, 2048 keys, head dim 256, causal: 47.1 ->
 // 36.4 (2, 2); 1 query of 32 heads on 8 k/v heads, 16 sequences of 8191 keys: 137 -> 52, the rate of a plain copy (1, 4).
-// Registers: two wavefronts a SIMD leave a lane 256; head dim 256 with two tiles needs 255 of them (v as rows) and 247 (transposed v, whose
-// copies and fragments take their row differences from scalar and immediate offsets; with a register for each, 31 - 42 of them were
-// spilled at head dims 224 and 256: 16 heads, 2048 keys, causal 76.4 us instead of 36.8, against 51.7 of the unshared loop).
+// Registers: two wavefronts a SIMD leave a lane 256, of which head dims 224 and 256 with two tiles take about 220.  (Transposed v: copies and
+// fragments take their row differences from scalar and immediate offsets; with a register for each, 31 - 42 were once spilled there:
+// 16 heads, 2048 keys, causal 76.4 us instead of 36.8, against 51.7 of the unshared loop.)
 #ifndef FA8_SHARED_ROWS_H_
 #define FA8_SHARED_ROWS_H_
 #include <type_traits>
@@ -335,7 +341,7 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
     float m_after[W], m_own = m_run;
 #pragma unroll
     for (int i = 0; i < W; ++i) {
-      m_after[i] = __builtin_fmaxf(i == 0 ? m_run : m_after[i - 1], maxima[i]);
+      m_after[i] = max2(i == 0 ? m_run : m_after[i - 1], maxima[i]);
       if (i == w) m_own = m_after[i];
     }
     const float mc = m_own * c;
@@ -363,7 +369,10 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
         if (u > 0) add(u - 1, i);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (u > 0) pack(u - 1);
+      if (u > 0) {
+        pack(u - 1);
+        asm volatile("" : "+v"(sum0), "+v"(sum1));  // keeps the additions in their chunk
+      }
       if (u == 7) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) add(7, i);
@@ -409,12 +418,11 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
     }
 #pragma unroll
     for (int u = 4; u < 8; ++u) {
-      if (more) {
+      // (after the last group this is the product of a stale tile: never used)
 #pragma unroll
-        for (int n = ((u - 4) * kS + 3) / 4; n < ((u - 3) * kS + 3) / 4; ++n) {
-          if (n + 1 < kS) kfrag[n + 1] = load_kf(k_next, (n + 1) / kKSteps, (n + 1) % kKSteps);
-          s_product(sn[n / kKSteps], n % kKSteps, kfrag[n]);
-        }
+      for (int n = ((u - 4) * kS + 3) / 4; n < ((u - 3) * kS + 3) / 4; ++n) {
+        if (n + 1 < kS) kfrag[n + 1] = load_kf(k_next, (n + 1) / kKSteps, (n + 1) % kKSteps);
+        s_product(sn[n / kKSteps], n % kKSteps, kfrag[n]);
       }
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (kTwo) issue_v(j + W, v_prev, j + W < all_blocks, (u - 4) * kPasses / 4, (u - 3) * kPasses / 4);
