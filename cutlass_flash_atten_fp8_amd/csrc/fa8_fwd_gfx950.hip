@@ -979,6 +979,8 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 //     unshared workgroups are well filled (0.95).  Head dim <= 64, a single tile per k/v head, 12 blocks: any number, bound by HBM
 //   head dim 65 - 128, pairs <= CUs (one a CU) and 4 blocks: four wavefronts a tile, two tiles a workgroup, which share the copies of K
 //     and V (0.6 - 0.85)
+//   head dim above 128: the same from 16 blocks on (one LDS stage; 1.0 - 1.1 at 6 - 12 blocks, 0.95 at 16 - 24, 0.86 from 64 on, against two
+//     wavefronts a tile).  Tiles of unequal length: also more pairs, from 24 blocks and even <= 3/4 CUs on (0.85 - 0.95; 1.0 - 1.1 at even = CUs)
 //   no more rounds of the CUs with pairs than with unshared workgroups (full and causal, every head dim and number of rounds): two
 //     wavefronts a tile, two tiles a workgroup (0.8 - 0.95; 0.2 - 0.75 where few queries of grouped heads leave half of the unshared
 //     workgroups idle).  One round more costs 1.05 - 1.4, except: rounds of unequal length, even <= CUs (causal: a quarter more; head
@@ -1022,7 +1024,7 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   if ((longest >= 3 && tiles <= (d <= 64 ? 2 : 1) * cus) || (longest >= 12 && d <= 64 && rows <= 32) ||
       (longest == 2 && d <= 128 && tiles <= cus && 8 * wgs < 5 * tiles))
     n = {1, 4, 1};
-  else if (d > 64 && d <= 128 && pairs <= cus && longest >= 4 && rows > 32)
+  else if (d > 64 && rows > 32 && ((pairs <= cus && longest >= (d <= 128 ? 4 : 16)) || (d > 128 && 4 * even <= 3 * cus && longest >= 24)))
     n = {2, 4, 1};
   else if (longest >= 2 ? no_more_rounds || few_pairs : one_block)
     n = {2, 2, 1};

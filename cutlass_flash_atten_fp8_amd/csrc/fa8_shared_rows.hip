@@ -16,8 +16,8 @@ const void* pick_rw(int r, int w, bool e5m2, bool vt) {
   constexpr int S = D > 128 ? 1 : 2;
   if (r == 1 && w == 4) return pick<D, 1, 4, S>(e5m2, vt);
   if (r == 2 && w == 2) return pick<D, 2, 2, S>(e5m2, vt);
-  if constexpr (D > 64 && D <= 128)
-    if (r == 2 && w == 4) return pick<D, 2, 4, 2>(e5m2, vt);
+  if constexpr (D > 64)
+    if (r == 2 && w == 4) return pick<D, 2, 4, S>(e5m2, vt);
   return nullptr;
 }
 

@@ -48,6 +48,10 @@ CASES = [
     (40, 64, 16, 3, 130, 128, True, True, False, E4, False, 2, 64),       # 640 k/v heads of one tile (12 rows): no rows in the second tile
     (16, 64, 64, 130, 130, 64, True, False, False, E4, False, 1, 128),    # 5 tiles a head: three pairs for two workgroups, not shared
     (16, 64, 64, 60, 130, 64, True, True, False, E4, False, 2, 64),       # 2 tiles a head: 128-row workgroups would be half idle
+    (2, 16, 16, 450, 961, 160, False, False, False, E4, False, 4, 64),    # wide heads, 256 pairs; 16 blocks, the last of one key
+    (1, 90, 30, 100, 1500, 192, True, True, False, E5, True, 4, 64),      # 300 packed rows: the last workgroup's second tile is not full
+    (1, 14, 14, 1540, 1540, 256, True, False, False, E4, False, 4, 64),   # 350 pairs of unequal length
+    (1, 9, 9, 1040, 1040, 224, True, False, True, E5, False, 4, 64),
     (20, 32, 32, 1, 1000, 32, True, True, False, E5, False, 4, 32),       # 640 tiles of one row
 ]
 
