@@ -24,7 +24,7 @@ constexpr int kKvBlock = 64;   // kv rows per online-softmax step
 constexpr int kThreads = 256;  // 4 wavefronts
 constexpr int kVersion = 5;
 // main loops (template parameter LOOP of the kernel)
-constexpr int kLoopRolling = 0, kLoopPipelined = 1, kLoopDense = 2;
+constexpr int kLoopRolling = 0, kLoopPipelined = 1, kLoopDense = 2, kLoopDenseRagged = 3;
 
 struct KernelArgs {
   const uint8_t* q;

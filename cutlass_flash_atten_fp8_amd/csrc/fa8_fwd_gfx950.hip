@@ -35,7 +35,7 @@
 
 // wavefronts per SIMD the kernels are compiled for: 3 (at most 168 VGPRs per lane) up to head dim 128, 2 (256 VGPRs:
 // the output accumulators alone take 128) for head dim 256; the pipelined loop 2; the dense loop 3 (head dim 64: 4)
-#define FA8_WAVES_PER_EU(D, LOOP) ((LOOP) == 1 ? 2 : ((LOOP) == 2 ? ((D) == 64 ? 4 : 3) : ((D) > 128 ? 2 : 3)))
+#define FA8_WAVES_PER_EU(D, LOOP) ((LOOP) == 1 ? 2 : ((LOOP) >= 2 ? ((D) == 64 ? 4 : 3) : ((D) > 128 ? 2 : 3)))
 
 namespace {
 
@@ -87,14 +87,16 @@ __device__ __forceinline__ void decode_block(const KernelArgs& a, int id, int& b
 // kLoopDense: the same pipeline squeezed into 168 VGPRs (three wavefronts per SIMD, three LDS stages) for launches
 // in which no block needs a mask (full attention over a whole number of KV blocks): one logits buffer, whose halves are
 // refilled by the S^T products of block j+1 as soon as the softmax of block j has turned them into weights.
+// kLoopDenseRagged: the same for full attention over keys that end inside a block: the last steps mask.  (A form of its own: as a
+// branch of the dense loop's last steps it cost launches of whole blocks 0.5 - 1 %.)
 template <int D, bool CAUSAL, bool E5M2, int OUT, bool VT, int LOOP>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WAVES_PER_EU(D, LOOP)))) void fa8_fwd_kernel(
     const KernelArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only types (buffer resources); the host pass only needs the stub
   static_assert(D % 32 == 0 && D >= 32 && D <= 256, "head dims: multiples of 32 up to 256");
-  constexpr bool PIPE = LOOP == kLoopPipelined, DENSE = LOOP == kLoopDense;
+  constexpr bool PIPE = LOOP == kLoopPipelined, RAGGED = LOOP == kLoopDenseRagged, DENSE = LOOP == kLoopDense || RAGGED;
   static_assert(LOOP == kLoopRolling || D == 64 || D == 128, "the pipelined loops are built for head dims 64 and 128");
-  static_assert(!DENSE || !CAUSAL, "the dense loop has no masks");
+  static_assert(!DENSE || !CAUSAL, "the dense loop masks nothing but the keys past the end");
   // LDS tiles are laid out for the next power of two: rows of DP bytes, of which the first D are used
   constexpr int DP = D <= 32 ? 32 : (D <= 64 ? 64 : (D <= 128 ? 128 : 256));
   constexpr int kTileBytes = kKvBlock * DP;  // one K or V tile
@@ -185,9 +187,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
   // zeros land in LDS and no memory is touched.  Its scalar offset is 0: a lane is out of range if its own offset is not below
   // length - scalar offset, a difference that must not be negative.
   // (Dense loop: the second pass of a copy differs from the first by a whole number of rows, 16 kv rows of K and 32 (64) rows
-  // of V (V^T): the difference sits in the scalar offset and both passes share one vector register.)
+  // of V (V^T): the difference sits in the scalar offset and both passes share one vector register.  In a ragged last block that
+  // scalar offset may lie past the last row: it stops at the resource's length, where every lane is out of range.)
   const int k_bytes = (int)(kv_last * a.k_rs + D);
   const int v_bytes = VT ? (int)((D - 1) * a.v_rs + a.seqlen_k) : (int)(kv_last * a.v_rs + D);
+  auto segment_offset = [&](int base, int rows, int length) __attribute__((always_inline)) {
+    return RAGGED ? (int)min((unsigned)base + (unsigned)rows, (unsigned)length) : base + rows;
+  };
   auto issue_k = [&](int j, uint8_t* kb, bool exists) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)kp, 0, exists ? k_bytes : 0, kRsrcFlags);
     const int k_rs = exists ? (int)a.k_rs : 0;
@@ -196,7 +202,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
     for (int p = 0; p < kPasses; ++p)
       if (!kSplitPass || wave < 2)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, kb + copy_segment(p) * 1024), 16, DENSE ? k_src[0] : k_src[p],
-                                                 DENSE ? k_base + p * 16 * k_rs : k_base, 0, 0);
+                                                 DENSE ? segment_offset(k_base, p * 16 * k_rs, k_bytes) : k_base, 0, 0);
   };
   auto issue_v = [&](int j, uint8_t* vb, bool exists) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)vp, 0, exists ? v_bytes : 0, kRsrcFlags);
@@ -216,7 +222,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, vb + seg), 16, off, 0, 0, 0);
         } else {
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(void, vb + seg), 16, DENSE ? v_src[0] : v_src[p],
-                                                   DENSE ? v_base + p * (VT ? 64 : 32) * v_rs : v_base, 0, 0);
+                                                   DENSE ? segment_offset(v_base, p * (VT ? 64 : 32) * v_rs, v_bytes) : v_base, 0, 0);
         }
       }
     }
@@ -265,11 +271,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
   for (int mt = 0; mt < kMTiles; ++mt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o_acc[mt][i] = 0.f;
-  // running row max of raw S (both half-lanes of a query hold the same value).  The pipelined loop starts it at a finite value
+  // running row max of raw S (both half-lanes of a query hold the same value).  The loops that mask without a special case start it at a finite value
   // below every possible logit (|s| <= 57344^2 * 256 < 1e12) instead of -inf: a row that has not seen a key yet then needs no
   // special case (its rescale factor exp2((m_run - m_new) * c) is 0 or multiplies zeros, m_new * c stays finite, and a masked
-  // logit -inf still gives exp2(-inf) = 0 for the positive scales this loop runs with); the results are the same bit for bit.
-  float m_run = PIPE ? -1.0e30f : -INFINITY;
+  // logit -inf still gives exp2(-inf) = 0 for the positive scales these loops run with); the results are the same bit for bit.
+  float m_run = PIPE || RAGGED ? -1.0e30f : -INFINITY;
   float l_run = 0.f;        // this lane's share of the running row sum
 
   // K fragment of S^T sub-tile t, k-step ks, and V^T fragment of O^T tile mt, from the tiles in kb / vb
@@ -407,12 +413,23 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
     v8i p8;
     constexpr int kPvEvery = 4 / kMTiles;  // the PV product of tile mt goes in front of chunk mt * kPvEvery
     constexpr int kSEvery = 2 / kKSteps;   // the S^T product (sub-tile 0, k-step ks) in front of chunk 4 + ks * kSEvery
-    auto iteration = [&](auto first_c, int j, const uint8_t* kb_next, const uint8_t* vb_prev, uint8_t* k_dst, uint8_t* v_dst)
+    auto iteration = [&](auto first_c, auto tail_c, int j, const uint8_t* kb_next, const uint8_t* vb_prev, uint8_t* k_dst, uint8_t* v_dst)
                          __attribute__((always_inline)) {
       constexpr bool kFirst = decltype(first_c)::value;
+      constexpr bool kTail = RAGGED && decltype(tail_c)::value;  // block j may be the last one, with keys that do not exist
       v8i vfrag[kMTiles];
       v8i kfrag[2][kKSteps];
       if constexpr (!kFirst) vfrag[0] = load_vf(vb_prev, 0);
+      if constexpr (kTail) {
+        if (j >= n_plain) {  // wave-uniform; the block has a key, so the row max stays finite
+          const int left = kv_last - j * kKvBlock - 32 * h;
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+              if (16 * t + i > left) s[t][i] = -INFINITY;
+        }
+      }
       float mx[4];
 #pragma unroll
       for (int ch = 0; ch < 4; ++ch) mx[ch] = max3(s[0][4 * ch], s[0][4 * ch + 1], s[0][4 * ch + 2]);
@@ -531,26 +548,30 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
     }
     __builtin_amdgcn_s_barrier();  // every wavefront has read K(0): step 0 may overwrite its stage
     // One step with compile-time LDS stages (PH = j % 3).
-    auto step = [&](auto first_c, auto ph_c, int j) __attribute__((always_inline)) {
+    auto step = [&](auto first_c, auto tail_c, auto ph_c, int j) __attribute__((always_inline)) {
       constexpr int PH = decltype(ph_c)::value;
       uint8_t* const kst[3] = {k_lds0, k_lds1, k_lds2};
       uint8_t* const vst[3] = {v_lds0, v_lds1, v_lds2};
-      iteration(first_c, j, kst[(PH + 1) % 3], vst[(PH + 2) % 3], kst[PH], vst[(PH + 1) % 3]);
+      iteration(first_c, tail_c, j, kst[(PH + 1) % 3], vst[(PH + 2) % 3], kst[PH], vst[(PH + 1) % 3]);
       wait_in_flight(std::integral_constant<int, 2>());  // the two copies of this step may stay in flight
     };
     constexpr std::integral_constant<int, 0> ph0{};
     constexpr std::integral_constant<int, 1> ph1{};
     constexpr std::integral_constant<int, 2> ph2{};
-    step(T(), ph0, 0);
+    step(T(), T(), ph0, 0);
     int j = 1;
-    for (; j + 2 < n_tiles; j += 3) {
-      step(F(), ph1, j);
-      step(F(), ph2, j + 1);
-      step(F(), ph0, j + 2);
+    for (; j + 2 < (RAGGED ? n_plain : n_tiles); j += 3) {
+      step(F(), F(), ph1, j);
+      step(F(), F(), ph2, j + 1);
+      step(F(), F(), ph0, j + 2);
     }
+    // up to two more whole blocks, and a ragged one
     if (j < n_tiles) {
-      step(F(), ph1, j);
-      if (j + 1 < n_tiles) step(F(), ph2, j + 1);
+      step(F(), T(), ph1, j);
+      if (j + 1 < n_tiles) {
+        step(F(), T(), ph2, j + 1);
+        if (RAGGED && j + 2 < n_tiles) step(F(), T(), ph0, j + 2);
+      }
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // the last copies (of nothing) must not outlive the workgroup's LDS
     // the PV product of the last block
@@ -884,6 +905,9 @@ int launch(const KernelArgs& a, bool v_transposed, int loop, hipStream_t stream)
       if (loop == FA8_SCHEDULE_DENSE)
         fn = v_transposed ? (const void*)&fa8_fwd_kernel<D, false, E5M2, OUT, true, kLoopDense>
                           : (const void*)&fa8_fwd_kernel<D, false, E5M2, OUT, false, kLoopDense>;
+      if (loop == FA8_SCHEDULE_DENSE && a.seqlen_k % kKvBlock != 0)
+        fn = v_transposed ? (const void*)&fa8_fwd_kernel<D, false, E5M2, OUT, true, kLoopDenseRagged>
+                          : (const void*)&fa8_fwd_kernel<D, false, E5M2, OUT, false, kLoopDenseRagged>;
     }
   }
   return (int)hipLaunchKernel(fn, grid, dim3(kThreads), argv, 0, stream);
@@ -940,17 +964,20 @@ int compute_units() {
 // Dense: full (non-causal) attention over a whole number of KV blocks, where no logit is ever masked; measured 1 - 2 % faster
 // than the rolling loop on launches that fill the chip and 3 - 5 % faster than the pipelined loop on small ones, so it is
 // the choice wherever it applies.  A hint for it that does not apply falls back to the automatic choice.
+// ragged_dense: also over keys that end inside a block (what launch_rows runs; fa8_fwd_schedule reports such calls as the loop
+// they would take without it).  Head dim 128, new / old time: 0.90 - 0.95 where the pipelined loop ran (2 sequences, 16 heads, 2999 keys
+// 96.0 -> 91.8 us; 8, 40, 777: 102 -> 92), 0.97 - 0.98 where the rolling one did (2, 32, 4097: 346 -> 336); head dim 64 0.95 - 0.99 above
+// three workgroups a compute unit, 1.00 - 1.02 below, where the pipelined loop stays.
 // Pipelined: launches that cannot keep three wavefronts on every SIMD for most of their run: at most four workgroups per
 // compute unit (two resident at a time), or little work per compute unit (then filling and draining the chip, and for
 // causal launches the thinning out of the workgroups, is a large share of the run).  Measured 5 - 15 % faster than the
 // rolling loop there; the rolling loop is equal or up to 5 % faster elsewhere.
-int choose_loop(const Fa8FwdParams* p) {
+int choose_loop(const Fa8FwdParams* p, bool ragged_dense) {
   if ((p->head_dim != 64 && p->head_dim != 128) || !(p->softmax_scale > 0.f && p->softmax_scale < 1.0e6f)) return FA8_SCHEDULE_ROLLING;
-  const bool dense_ok = !p->is_causal && p->seqlen_k % kKvBlock == 0;
   if (p->schedule == FA8_SCHEDULE_ROLLING || p->schedule == FA8_SCHEDULE_PIPELINED) return p->schedule;
-  if (dense_ok) return FA8_SCHEDULE_DENSE;
   const long long cus = compute_units();
   const long long wgs = (long long)p->batch * p->heads * ((p->seqlen_q + kQBlock - 1) / kQBlock);
+  if (!p->is_causal && (p->seqlen_k % kKvBlock == 0 || (ragged_dense && (p->head_dim == 128 || wgs > 3 * cus)))) return FA8_SCHEDULE_DENSE;
   // KV blocks per compute unit below which the pipelined loop was measured to win (head dim 64 has half the matrix work
   // per block)
   const long long few_blocks = p->head_dim == 64 ? 264 : 144;
@@ -1139,7 +1166,7 @@ int launch_rows(const Fa8FwdParams* p, hipStream_t stream) {
   a.k_bs = p->k_batch_stride; a.k_hs = p->k_head_stride; a.k_rs = p->k_row_stride;
   a.v_bs = p->v_batch_stride; a.v_hs = p->v_head_stride; a.v_rs = p->v_row_stride;
   a.o_bs = p->o_batch_stride; a.o_hs = p->o_head_stride; a.o_rs = p->o_row_stride;
-  const int loop = choose_loop(p);
+  const int loop = choose_loop(p, true);
   switch (p->head_dim) {
 #define FA8_HEAD_DIM_CASE(D_) \
   case D_: return p->is_causal ? launch_types<D_, true>(p, a, loop, stream) : launch_types<D_, false>(p, a, loop, stream)
@@ -1199,7 +1226,7 @@ extern "C" int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* 
 extern "C" int fa8_fwd_schedule(const Fa8FwdParams* p) {
   const int rc = fa8_fwd_validate(p);
   if (rc != FA8_OK) return rc;
-  return choose_loop(p);
+  return choose_loop(p, false);
 }
 
 extern "C" int fa8_query(int what) {

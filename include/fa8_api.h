@@ -148,7 +148,8 @@ int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* rows_per_wo
 /*
  * Which main loop a wavefront that has its 32 query rows to itself would run for these arguments on the current device:
  * FA8_SCHEDULE_ROLLING, FA8_SCHEDULE_PIPELINED or FA8_SCHEDULE_DENSE (all > 0), or the FA8_ERR_* code fa8_fwd_validate gives; whether
- * the call has such wavefronts, fa8_fwd_plan tells.  Launches nothing.  No counterpart in the reference (one kernel, one loop:
+ * the call has such wavefronts, fa8_fwd_plan tells.  (Full attention over keys that end inside a block may run the dense loop, its last
+ * block masked, where this reports one of the other two: those are what a launch of that size takes under a causal mask.)  Launches nothing.  No counterpart in the reference (one kernel, one loop:
  * csrc/flash_attention.cu:468-534); it makes the library's choice visible to benchmarks and tests.
  */
 int fa8_fwd_schedule(const Fa8FwdParams* p);
