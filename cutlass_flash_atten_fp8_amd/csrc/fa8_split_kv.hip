@@ -1,4 +1,7 @@
-// Launcher of the split-kv kernels (fa8_split_kv.h): the plan, the workspace and the two launches.
+// Launcher of the split-kv kernels (fa8_split_kv.h): the plan, the workspace and the launches.
+#include <atomic>
+#include <cstdlib>
+
 #include "fa8_launch.h"
 #include "fa8_split_kv.h"
 
@@ -14,6 +17,37 @@ template <int D>
 const void* values_kernel(bool e5m2, bool vt) {
   if (e5m2) return vt ? (const void*)&fa8_split_values_kernel<D, true, true> : (const void*)&fa8_split_values_kernel<D, true, false>;
   return vt ? (const void*)&fa8_split_values_kernel<D, false, true> : (const void*)&fa8_split_values_kernel<D, false, false>;
+}
+
+template <int D>
+const void* fused_kernel(bool e5m2, bool vt) {
+  if (e5m2) return vt ? (const void*)&fa8_split_fused_kernel<D, true, true> : (const void*)&fa8_split_fused_kernel<D, true, false>;
+  return vt ? (const void*)&fa8_split_fused_kernel<D, false, true> : (const void*)&fa8_split_fused_kernel<D, false, false>;
+}
+
+// A number that no other launch has (SplitFusedArgs::tag): a bijection (splitmix64's) of a count.  Halves of zeros or ones are left out:
+// a workspace may be full of them.
+unsigned long long next_tag() {
+  static std::atomic<unsigned long long> count{0};
+  for (;;) {
+    unsigned long long x = (count.fetch_add(1, std::memory_order_relaxed) + 1) * 0x9e3779b97f4a7c15ull;
+    x = (x ^ x >> 30) * 0xbf58476d1ce4e5b9ull;
+    x = (x ^ x >> 27) * 0x94d049bb133111ebull;
+    x ^= x >> 31;
+    const unsigned lo = (unsigned)x, hi = (unsigned)(x >> 32);
+    if (lo != 0 && hi != 0 && ~lo != 0 && ~hi != 0) return x;
+  }
+}
+
+// For tests: FA8_SPLIT_POLLS in the environment (read once) replaces how often a workgroup looks at another one's maximum before it
+// forms that itself (the results do not depend on it).
+int polls() {
+  static const int n = [] {
+    const char* e = std::getenv("FA8_SPLIT_POLLS");
+    const int x = e ? std::atoi(e) : -1;
+    return x >= 0 && x <= 1 << 16 ? x : 2048;
+  }();
+  return n;
 }
 
 struct Plan {
@@ -52,6 +86,41 @@ int fa8::launch_split(const Fa8FwdParams* p, int splits, void* workspace, hipStr
   shape.blocks_per_range = (uint16_t)n.blocks_per_range;
   shape.heads_k = n.heads_k;
   shape.all_tiles = p->batch * n.heads_k * n.tiles;
+  const bool e5m2 = p->in_dtype == FA8_DTYPE_E5M2, vt = p->v_layout == FA8_V_TRANSPOSED;
+  const dim3 grid((unsigned)n.heads_k, (unsigned)p->batch, (unsigned)(n.tiles * n.splits));
+  if (split_fused_fits(p->head_dim, n.live_rows, n.blocks_per_range)) {
+    SplitFusedArgs f;
+    f.n = shape;
+    f.q = (const uint8_t*)p->q;
+    f.k = (const uint8_t*)p->k;
+    f.v = (const uint8_t*)p->v;
+    f.o = p->o;
+    f.lse = (float*)p->lse;
+    f.tag = next_tag();
+    f.polls = polls();
+    f.q_bs = p->q_batch_stride / 16; f.q_hs = p->q_head_stride / 16; f.q_rs = p->q_row_stride / 16;
+    f.k_bs = p->k_batch_stride / 16; f.k_hs = p->k_head_stride / 16; f.k_rs = p->k_row_stride / 16;
+    f.v_bs = p->v_batch_stride / 16; f.v_hs = p->v_head_stride / 16; f.v_rs = p->v_row_stride / 16;
+    f.o_bs = p->o_batch_stride / 4; f.o_hs = p->o_head_stride / 4; f.o_rs = p->o_row_stride / 4;
+    f.lse_bs = p->lse_batch_stride; f.lse_hs = p->lse_head_stride;
+    const void* fn = nullptr;
+    switch (p->head_dim) {
+#define FA8_HEAD_DIM_CASE(D_) \
+  case D_: fn = fused_kernel<D_>(e5m2, vt); break
+      FA8_HEAD_DIM_CASE(32);
+      FA8_HEAD_DIM_CASE(64);
+      FA8_HEAD_DIM_CASE(96);
+      FA8_HEAD_DIM_CASE(128);
+      FA8_HEAD_DIM_CASE(160);
+      FA8_HEAD_DIM_CASE(192);
+      FA8_HEAD_DIM_CASE(224);
+      FA8_HEAD_DIM_CASE(256);
+#undef FA8_HEAD_DIM_CASE
+      default: return FA8_ERR_HEAD_DIM;
+    }
+    void* argv[] = {&f};
+    return (int)hipLaunchKernel(fn, grid, dim3(64 * kSplitWaves), argv, 0, stream);
+  }
   SplitLogitsArgs l;
   l.n = shape;
   l.q = (const uint8_t*)p->q;
@@ -66,7 +135,6 @@ int fa8::launch_split(const Fa8FwdParams* p, int splits, void* workspace, hipStr
   v.v_bs = p->v_batch_stride / 16; v.v_hs = p->v_head_stride / 16; v.v_rs = p->v_row_stride / 16;
   v.o_bs = p->o_batch_stride / 4; v.o_hs = p->o_head_stride / 4; v.o_rs = p->o_row_stride / 4;
   v.lse_bs = p->lse_batch_stride; v.lse_hs = p->lse_head_stride;
-  const bool e5m2 = p->in_dtype == FA8_DTYPE_E5M2, vt = p->v_layout == FA8_V_TRANSPOSED;
   const void *first = nullptr, *second = nullptr;
   switch (p->head_dim) {
 #define FA8_HEAD_DIM_CASE(D_) \
@@ -82,7 +150,6 @@ int fa8::launch_split(const Fa8FwdParams* p, int splits, void* workspace, hipStr
 #undef FA8_HEAD_DIM_CASE
     default: return FA8_ERR_HEAD_DIM;
   }
-  const dim3 grid((unsigned)n.heads_k, (unsigned)p->batch, (unsigned)(n.tiles * n.splits));
   void *argv_l[] = {&l}, *argv_v[] = {&v};
   const hipError_t rc = hipLaunchKernel(first, grid, dim3(64 * kSplitWaves), argv_l, 0, stream);
   if (rc != hipSuccess) return (int)rc;

@@ -1,0 +1,97 @@
+"""Split keys in one kernel (fa8_split_fused_kernel): workgroups take the row max of those before them from the workspace.  What the other tests
+of split keys do not reach: a workgroup that stops waiting and forms that max itself, workspaces with the state of earlier calls, several
+streams, ranges of every length up to the two-kernel form."""
+import ctypes
+import os
+import subprocess
+import sys
+
+import pytest
+import torch
+
+import cutlass_flash_atten_fp8_amd as fa
+from test_split_kv_gpu import DEV, E4, E5, _inputs, assert_same_up_to_sum_order
+
+pytestmark = pytest.mark.gpu
+
+# B, H, Hk, Nq, Nk, d, causal, vt, dtype
+CASES = [
+    (1, 8, 2, 1, 6001, 128, True, False, E4),
+    (1, 6, 2, 2, 8191, 96, True, False, E5),
+    (1, 8, 1, 5, 7777, 128, True, False, E4),    # two row tiles, the second with 8 rows
+    (1, 8, 2, 1, 8192, 32, True, False, E5),
+    (1, 4, 4, 3, 4112, 160, False, True, E4),    # v^T, ragged last block
+    (1, 8, 2, 1, 20000, 256, True, False, E4),
+    (1, 4, 2, 50, 12345, 64, True, False, E4),   # masks in several blocks, four tiles
+]
+
+
+def outputs():
+    res = []
+    for B, H, Hk, Nq, Nk, d, causal, vt, dt in CASES:
+        q, k, v = _inputs(Nk + d, B, H, Hk, Nq, Nk, d, dt)
+        k.view(torch.uint8)[0, 0, 70, 3] = 0x7C if dt == E5 else 0x7E  # infinity, the largest finite number
+        v = v.transpose(2, 3).contiguous() if vt else v
+        o, lse = fa.flash_attention_v2_cutlass(q, k, v, causal, d ** -0.5, v_transposed=vt, return_lse=True, causal_bottom_right=True)
+        assert fa.plan(fa.make_params(q, k, v, o, causal, d ** -0.5, vt, lse, True))[2] > 1
+        res += [o.view(torch.int16).cpu(), lse.view(torch.int32).cpu()]
+    return res
+
+
+def test_a_workgroup_that_does_not_wait_forms_the_maximum_itself(tmp_path):
+    """No looks at all at the other workgroups' maxima (the setting is read once, so in a process of its own): the same bits."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    code = (f"import sys; sys.path[:0] = [{here!r}, {os.path.dirname(here)!r}]\n"
+            f"import torch, test_split_fused_gpu as t\ntorch.save(t.outputs(), {str(tmp_path / 'o.pt')!r})\n")
+    env = dict(os.environ, FA8_SPLIT_POLLS="0")
+    r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+    for want, got in zip(outputs(), torch.load(tmp_path / "o.pt", weights_only=True)):
+        assert torch.equal(want, got)
+
+
+def test_a_workspace_with_the_state_of_earlier_calls():
+    """The same workspace for calls with other keys, other lengths, other splits: no value of an earlier call is taken."""
+    ws = torch.zeros(64 << 20, dtype=torch.uint8, device=DEV)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for seed, nk in enumerate((8000, 8000, 5000, 16000, 8000)):
+        q, k, v = _inputs(seed, 1, 8, 2, 1, nk, 128, E4)
+        if seed % 2 == 0:
+            k = (k.float() * 0.25).to(E4)
+        o = torch.full(q.shape, float("nan"), dtype=torch.float16, device=DEV)
+        p = fa.make_params(q, k, v, o, True, 0.09, causal_bottom_right=True)
+        need = ctypes.c_int64()
+        assert fa.lib().fa8_fwd_workspace(ctypes.byref(p), ctypes.byref(need)) == 0 and 0 < need.value <= ws.numel()
+        assert fa.lib().fa8_fwd_ws(ctypes.byref(p), ws.data_ptr(), need.value, stream) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(o, fa.flash_attention_v2_cutlass(q, k, v, True, 0.09, causal_bottom_right=True)[0])
+
+
+@pytest.mark.parametrize("group", [1, 4, 8, 16, 32])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_ranges_up_to_the_two_kernel_form(d, group):
+    """One to about thirty blocks a wavefront; the logits of the longer ones do not fit in LDS."""
+    for nk in (4096, 9000, 30011, 120001):
+        q, k, v = _inputs(nk + group, 1, group, 1, 1, nk, d, E4)
+        if 2 * nk * d > 40e6:
+            continue
+        want = fa.flash_attention_v2_cutlass(q, k, v, True, d ** -0.5, causal_bottom_right=True, schedule=fa.FA8_SCHEDULE_ROLLING)[0]
+        got = fa.flash_attention_v2_cutlass(q, k, v, True, d ** -0.5, causal_bottom_right=True)[0]
+        torch.cuda.synchronize()
+        assert_same_up_to_sum_order(got, want, v, nk)
+
+
+def test_two_streams():
+    """Calls side by side on two streams, each with more workgroups than half the compute units."""
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    ins = [_inputs(i, 2, 32, 8, 1, 20000, 128, E4) for i in range(2)]
+    want = [fa.flash_attention_v2_cutlass(*t, True, 0.09, causal_bottom_right=True)[0] for t in ins]
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(10):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                got[i].append(fa.flash_attention_v2_cutlass(*ins[i], True, 0.09, causal_bottom_right=True)[0])
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(o, want[i]) for o in got[i])
