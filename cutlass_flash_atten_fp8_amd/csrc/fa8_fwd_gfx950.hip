@@ -1016,13 +1016,15 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 //   A single block leaves nothing to share but the products (1.05 - 1.3): only where the rows of grouped q heads fill the tiles that
 //     they would leave idle, 2 pairs <= wgs, and on a full chip (0.2 - 0.8), and under the mask at head dim 32, whose unshared loop is
 //     the rolling one (v as rows: 0.75 - 0.95, transposed 1.0 - 1.4)
-// Splitting the keys as well costs a second kernel, a reduction and the logits' way through memory, and spreads the copies over all
-// compute units: taken where the estimate of its time is below that of four sharing wavefronts.  Both estimates are fits to 3003 drawn
-// launches whose K and V come from HBM and 1725 whose K and V the Infinity Cache still holds: a start, a step per block of a wavefront's
-// range, K and V, and the logits written and read; neither is below the rate at which it moves its bytes.  On these launches the choice is
-// the slower one by more than 5 % in 2 of 100, from HBM as from the cache.  (Fitted on repeated inputs alone and without a bound by the
-// bytes, K and V seemed to pass at 29 TB/s: 16 sequences of 8191 keys, 1 query of 32 heads on 8 k/v heads, d128 were split, 69 us instead
-// of 53.)  One head, 32 queries on 1121 keys, d128: 10.0 us shared, 19.3 split; one sequence of 32768 keys: 151 and 21.
+// Splitting the keys as well costs an exchange of maxima and a reduction (where the logits do not fit in LDS a second kernel and their way
+// through memory), and spreads the copies over all compute units: taken where the estimate of its time is below that of four sharing
+// wavefronts, and then as fine as the compute units allow, down to one block a wavefront.  The estimates are fits (shared rows: 3003 drawn
+// launches whose K and V come from HBM and 1725 whose K and V the Infinity Cache still holds; split: 1663 pairs of 306 drawn launches and a
+// number of splits, K and V mostly from HBM): a start, a step per block of a wavefront's range, K and V, the parts of O, and the logits
+// written and read; neither is below the rate at which it moves its bytes.  On the 306 launches the choice takes 0.5 % longer than the best
+// of all numbers of splits on average; two blocks a wavefront at least, and the estimate for two kernels, took 6.5 % longer.  One head, 32
+// queries on 1121 keys, d128: 10.0 us shared, 19.3 split; one sequence of 32768 keys: 151 and 18; 2 sequences of 6881 keys, 8 queries of 3 k/v heads,
+// group of 4, d128: 25.2 in 13 parts, 16.1 in 27.
 Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   const Plan unshared = {kQBlock / 32, 1, 1};
   // the sharing kernels rely on exp2(-inf * scale) = 0 and a finite start of the row max, like the pipelined loop; a schedule hint
@@ -1056,12 +1058,18 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   else if (longest >= 2 ? no_more_rounds || few_pairs : one_block)
     n = {2, 2, 1};
   if (workspace && n.waves_per_tile == 4 && n.tiles_per_workgroup == 1 && longest >= 16) {
-    const long long splits = std::max(1LL, std::min({32LL, cus / tiles, longest / 8}));  // one workgroup more than CUs takes twice as long
-    const long long range = (longest + 4 * splits - 1) / (4 * splits);                   // blocks of a wavefront
+    const long long most = std::max(1LL, std::min({32LL, cus / tiles, longest / 4}));  // one workgroup more than CUs takes twice as long
+    const SplitForm form = split_form(p, (int)most);
+    const long long splits = form.splits;
+    const double range = form.blocks_per_range, row_bytes = d <= 32 ? 32 : (d <= 64 ? 64 : (d <= 128 ? 128 : 256));  // of an LDS tile
     const double kv_bytes = 2.0 * kv_heads * longest * kKvBlock * d, live = rows < 32 ? (double)rows : 32.0;
     const double s_bytes = 8.0 * tiles * live * longest * kKvBlock;
     const double shared_us = 5.4 + std::max((d <= 64 ? 0.23 : (d <= 128 ? 0.30 : 0.63)) * longest, kv_bytes / 5.6e6);
-    const double split_us = std::max(10.0 + 1.6 / 128 * d * range + kv_bytes / 30e6 + s_bytes / 4.0e6, 2.6 + (kv_bytes + s_bytes) / 5.2e6);
+    const double split_us =
+        form.one_kernel
+            ? std::max(7.7 + (0.53 + 0.0057 * row_bytes) * range + kv_bytes / 23.5e6 + 1.34e-3 * d * live + 0.07 * splits, 5.4 + kv_bytes / 5.6e6)
+            : std::max(7.5 + (0.6 + 0.0054 * row_bytes) * range + kv_bytes / 9.3e6 + 0.9e-3 * d * live + 0.16 * splits + 0.063 * range * live +
+                           s_bytes / 11e6, 2.3 + (kv_bytes + s_bytes) / 5.8e6);
     if (splits > 1 && split_us < shared_us && tiles * splits < 65536 && longest / (4 * splits) < 65535 &&
         split_workspace(p, (int)splits) <= kMaxWorkspace)
       n.splits = (int)splits;

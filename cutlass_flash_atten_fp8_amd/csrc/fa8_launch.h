@@ -10,7 +10,13 @@ namespace fa8 {
 // r row tiles of 32 query rows per workgroup, w wavefronts per row tile (fa8_shared_rows.h)
 __attribute__((visibility("hidden"))) int launch_shared(const Fa8FwdParams* p, int r, int w, hipStream_t stream);
 
-// Keys of every row tile dealt to at most `splits` workgroups (fa8_split_kv.h): workspace bytes, launch.
+// Keys of every row tile dealt to at most `splits` workgroups (fa8_split_kv.h): how (workgroups, KV blocks of a wavefront, whether one kernel does
+// it), workspace bytes, launch.
+struct SplitForm {
+  int splits, blocks_per_range;
+  bool one_kernel;
+};
+__attribute__((visibility("hidden"))) SplitForm split_form(const Fa8FwdParams* p, int splits);
 __attribute__((visibility("hidden"))) long long split_workspace(const Fa8FwdParams* p, int splits);
 __attribute__((visibility("hidden"))) int launch_split(const Fa8FwdParams* p, int splits, void* workspace, hipStream_t stream);
 

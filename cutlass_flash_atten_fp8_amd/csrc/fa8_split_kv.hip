@@ -69,6 +69,11 @@ Plan plan_of(const Fa8FwdParams* p, int splits) {
 
 }  // namespace
 
+fa8::SplitForm fa8::split_form(const Fa8FwdParams* p, int splits) {
+  const Plan n = plan_of(p, splits);
+  return {n.splits, n.blocks_per_range, split_fused_fits(p->head_dim, n.live_rows, n.blocks_per_range)};
+}
+
 long long fa8::split_workspace(const Fa8FwdParams* p, int splits) {
   const Plan n = plan_of(p, splits);
   return split_layout((long long)p->batch * n.heads_k * n.tiles, n.splits, n.live_rows, p->head_dim, n.keys).bytes;
