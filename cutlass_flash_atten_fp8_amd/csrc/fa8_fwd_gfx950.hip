@@ -990,6 +990,7 @@ struct Plan {
   int tiles_per_workgroup;  // of 32 query rows
   int waves_per_tile;       // 1: the loops of this file; 2, 4: wavefronts share a row tile
   int splits;               // > 1: the keys of a row tile dealt to this many workgroups (needs a workspace)
+  int stages = 1;           // LDS stages, where sharing wavefronts have the choice
 };
 constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask for
 
@@ -1004,6 +1005,12 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 //   tiles <= CUs (head dim <= 64: 2 CUs), the most that run at once, and 3 blocks: four wavefronts a tile, one tile a workgroup
 //     (0.75 at 6 blocks, 0.55 from 33 on).  At 2 blocks the exchange costs what it saves, unless the head dim is at most 128 and the
 //     unshared workgroups are well filled (0.95).  Head dim <= 64, a single tile per k/v head, 12 blocks: any number, bound by HBM
+//   More of them where the tiles differ in length (shortest < 3/5 longest), so that two or three share a CU with one LDS stage each and do not
+//     wait for each other's barriers.  Work of the tiles / (CUs x longest): head dim <= 64 from 6 blocks on up to 1.5 (0.85 - 0.97), 16 blocks
+//     1.75 (0.84 - 0.94), 24 blocks 2 (0.9); head dim 65 - 128 8 blocks 1 (0.90 - 0.93), 24 blocks 1.25 (0.86), 32 blocks 1.5 (0.82).  Equal
+//     tiles: head dim <= 64, 16 blocks, up to the three a CU that run at once (0.85 - 0.97).  (13 400 drawn launches; beyond these lines 1.0 - 1.4)
+//   LDS stages of one tile, four wavefronts: with one workgroup a CU (head dim 64: two) one stage takes 0.96 - 0.98 of the time of two below 16
+//     blocks, the same at 16 - 24, 1.0 - 1.3 above; two stages of head dim 128 have no room for a second workgroup (0.7 - 0.8)
 //   head dim 65 - 128, pairs <= CUs (one a CU) and 4 blocks: four wavefronts a tile, two tiles a workgroup, which share the copies of K
 //     and V (0.6 - 0.85)
 //   head dim above 128: the same from 16 blocks on (one LDS stage; 1.0 - 1.1 at 6 - 12 blocks, 0.95 at 16 - 24, 0.86 from 64 on, against two
@@ -1044,6 +1051,10 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   const long long pairs = kv_heads * ((rows + 63) / 64), wgs = (long long)p->batch * p->heads * ((p->seqlen_q + kQBlock - 1LL) / kQBlock);
   // mean length of the tiles: half way between the first and the last one, but for rows that see every key or none
   const long long even = pairs * (longest + shortest) / (2 * longest);
+  // the same for workgroups of one tile, in quarters of the compute units; only lengths that differ make room for more than run at once
+  const bool unequal = 5 * shortest < 3 * longest;
+  const long long quarters = (tiles * (longest + shortest) / (2 * longest) * 4 + cus - 1) / cus;
+  const long long most_quarters = d <= 64 ? (longest < 16 ? 6 : (longest < 24 ? 7 : 8)) : (d > 128 ? 0 : (longest < 24 ? 4 : (longest < 32 ? 5 : 6)));
   const long long pair_rounds = (pairs + cus - 1) / cus, wg_rounds = (wgs + cus - 1) / cus;
   const bool no_more_rounds = pair_rounds <= wg_rounds || (d == 32 && 3 * pairs <= 4 * wgs) ||
                               (d == 64 && longest >= 8 && 5 * shortest > 3 * longest && 2 * pair_rounds <= 3 * wg_rounds);
@@ -1052,6 +1063,8 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   Plan n = unshared;
   if ((longest >= 3 && tiles <= (d <= 64 ? 2 : 1) * cus) || (longest >= 12 && d <= 64 && rows <= 32) ||
       (longest == 2 && d <= 128 && tiles <= cus && 8 * wgs < 5 * tiles))
+    n = {1, 4, 1, longest >= 24 && tiles <= (d <= 64 ? 2 : 1) * cus ? 2 : 1};
+  else if (longest >= (d <= 64 ? 6 : 8) && (unequal ? quarters <= most_quarters : d <= 64 && tiles <= 3 * cus && longest >= 16))
     n = {1, 4, 1};
   else if (d > 64 && rows > 32 && ((pairs <= cus && longest >= (d <= 128 ? 4 : 16)) || (d > 128 && 4 * even <= 3 * cus && longest >= 24)))
     n = {2, 4, 1};
@@ -1195,7 +1208,7 @@ int run(const Fa8FwdParams* p, void* workspace, long long bytes, hipStream_t str
   Plan n = choose_plan(p, workspace != nullptr);
   if (n.splits > 1 && bytes < split_workspace(p, n.splits)) n = choose_plan(p, false);
   if (n.splits > 1) return (uintptr_t)workspace % 16 != 0 ? FA8_ERR_ALIGN : launch_split(p, n.splits, workspace, stream);
-  return n.waves_per_tile > 1 ? launch_shared(p, n.tiles_per_workgroup, n.waves_per_tile, stream) : launch_rows(p, stream);
+  return n.waves_per_tile > 1 ? launch_shared(p, n.tiles_per_workgroup, n.waves_per_tile, n.stages, stream) : launch_rows(p, stream);
 }
 
 }  // namespace

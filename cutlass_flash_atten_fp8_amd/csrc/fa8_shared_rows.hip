@@ -12,9 +12,12 @@ const void* pick(bool e5m2, bool vt) {
   return vt ? (const void*)&fa8_shared_rows_kernel<D, false, true, R, W, STAGES> : (const void*)&fa8_shared_rows_kernel<D, false, false, R, W, STAGES>;
 }
 template <int D>
-const void* pick_rw(int r, int w, bool e5m2, bool vt) {
+const void* pick_rw(int r, int w, int stages, bool e5m2, bool vt) {
   constexpr int S = D > 128 ? 1 : 2;
-  if (r == 1 && w == 4) return pick<D, 1, 4, S>(e5m2, vt);
+  // (1, 4): see choose_plan for the stages; head dim 32 has no use for two (0.97 - 1.01)
+  if constexpr (D > 32 && D <= 128)
+    if (r == 1 && w == 4 && stages == 2) return pick<D, 1, 4, 2>(e5m2, vt);
+  if (r == 1 && w == 4) return pick<D, 1, 4, 1>(e5m2, vt);
   if (r == 2 && w == 2) return pick<D, 2, 2, S>(e5m2, vt);
   if constexpr (D > 64)
     if (r == 2 && w == 4) return pick<D, 2, 4, S>(e5m2, vt);
@@ -23,7 +26,7 @@ const void* pick_rw(int r, int w, bool e5m2, bool vt) {
 
 }  // namespace
 
-int fa8::launch_shared(const Fa8FwdParams* p, int r, int w, hipStream_t stream) {
+int fa8::launch_shared(const Fa8FwdParams* p, int r, int w, int stages, hipStream_t stream) {
   SharedArgs a;
   a.q = (const uint8_t*)p->q;
   a.k = (const uint8_t*)p->k;
@@ -45,7 +48,7 @@ int fa8::launch_shared(const Fa8FwdParams* p, int r, int w, hipStream_t stream) 
   const void* fn = nullptr;
   switch (p->head_dim) {
 #define FA8_HEAD_DIM_CASE(D_) \
-  case D_: fn = pick_rw<D_>(r, w, e5m2, vt); break
+  case D_: fn = pick_rw<D_>(r, w, stages, e5m2, vt); break
     FA8_HEAD_DIM_CASE(32);
     FA8_HEAD_DIM_CASE(64);
     FA8_HEAD_DIM_CASE(96);

@@ -1,0 +1,43 @@
+"""One tile of 32 query rows a workgroup, four wavefronts, one or two LDS stages (csrc/fa8_shared_rows.h): the stages and the launches of more
+tiles than compute units are chosen by length and number of the tiles.  Results equal the rolling loop's bit for bit on both sides of each line."""
+import pytest
+import torch
+
+import cutlass_flash_atten_fp8_amd as fa
+from test_shared_rows_gpu import E4, E5, _inputs
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # B, H, Hk, Nq, Nk, d, causal, bottom_right, vt, dtype, fp8 out
+    (1, 2, 2, 100, 1472, 128, False, False, False, E4, False),   # 23 blocks: one stage
+    (1, 2, 2, 100, 1473, 128, False, False, False, E4, False),   # 24: two
+    (1, 2, 1, 70, 1600, 64, True, True, True, E5, True),         # two, v^T
+    (1, 2, 2, 97, 3000, 96, True, True, False, E5, False),
+    (1, 4, 4, 130, 130, 32, True, False, False, E4, False),
+    (1, 3, 3, 200, 190, 64, False, False, False, E4, False),     # one stage, 3 blocks: no group is full
+    (1, 14, 14, 960, 960, 128, True, False, False, E4, False),   # 420 tiles of unequal length
+    (1, 14, 7, 944, 944, 96, True, False, True, E5, True),
+    (1, 9, 9, 1990, 1990, 128, True, False, False, E4, False),   # 567 tiles, 32 blocks
+    (1, 24, 24, 720, 720, 64, True, False, False, E5, False),    # 552 tiles, 12 blocks
+    (1, 20, 20, 1200, 1200, 64, True, False, True, E4, True),    # 760 tiles
+    (1, 24, 24, 700, 700, 32, True, False, False, E4, False),
+    (1, 24, 12, 700, 1030, 64, False, False, False, E4, False),  # equal tiles, 528 of them, ragged last block
+    (2, 12, 12, 992, 1024, 32, False, False, False, E5, True),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "B{}H{}k{}Nq{}Nk{}d{}".format(*c[:6]))
+def test_one_tile_a_workgroup_equals_the_rolling_loop_bitwise(case):
+    B, H, Hk, Nq, Nk, d, causal, br, vt, dt, out8 = case
+    q, k, v = _inputs(Nq + Nk + d, B, H, Hk, Nq, Nk, d, dt)
+    v = v.transpose(2, 3).contiguous() if vt else v
+    kw = dict(v_transposed=vt, return_lse=True, causal_bottom_right=br, out_dtype=dt if out8 else None)
+    want, want_lse = fa.flash_attention_v2_cutlass(q, k, v, causal, d ** -0.5, schedule=fa.FA8_SCHEDULE_ROLLING, **kw)
+    got, lse = torch.empty_like(want), torch.empty_like(want_lse)
+    p = fa.make_params(q, k, v, got, causal, d ** -0.5, vt, lse, br)
+    assert fa.plan(p, with_workspace=False) == (32, 4, 1)
+    import ctypes
+    assert fa.lib().fa8_fwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)) and torch.equal(lse, want_lse)
