@@ -1020,6 +1020,12 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 //     workgroups idle).  One round more costs 1.05 - 1.4, except: rounds of unequal length, even <= CUs (causal: a quarter more; head
 //     dim <= 64: twice as many) and 5 blocks (head dim 32: 2) (0.8 - 1.0); head dim 32 up to 4/3 wgs (0.85 - 1.0); head dim 64 up to
 //     half as many rounds more from 8 blocks on if the tiles are about equally long (0.85 - 0.95)
+//   LDS stages of two tiles, two wavefronts a tile (423 drawn launches, head dims 64 - 128): with one stage a CU holds four workgroups of head dim
+//     64 instead of three, three of 96 and 128 instead of two.  Where there are as many, one stage takes 0.90 - 0.96 of the time of
+//     two (head dim 64) and 0.82 - 0.95 (96, 128); where there are fewer, 0.97 below 16 (8) blocks, 1.0 - 1.03 above, where two stay
+//     (head dims 96, 128, tiles of unequal length, 24 blocks: up to 2.4 pairs a CU; one stage takes 1.05 - 1.07 there)
+//   head dim 65 - 128, 8 blocks, more than two pairs a CU and up to the three that one stage lets run at once (causal, 16 blocks: 3.5): two
+//     wavefronts a tile, two tiles, though the unshared launch has fewer rounds (median 0.92, 0.82 - 1.0; beyond 1.03 - 1.4)
 //   A single block leaves nothing to share but the products (1.05 - 1.3): only where the rows of grouped q heads fill the tiles that
 //     they would leave idle, 2 pairs <= wgs, and on a full chip (0.2 - 0.8), and under the mask at head dim 32, whose unshared loop is
 //     the rolling one (v as rows: 0.75 - 0.95, transposed 1.0 - 1.4)
@@ -1059,6 +1065,8 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   const bool no_more_rounds = pair_rounds <= wg_rounds || (d == 32 && 3 * pairs <= 4 * wgs) ||
                               (d == 64 && longest >= 8 && 5 * shortest > 3 * longest && 2 * pair_rounds <= 3 * wg_rounds);
   const bool few_pairs = (longest >= 5 || d == 32) && 4 * even <= (p->is_causal ? 5 : 4) * (d <= 64 ? 2 : 1) * cus;
+  const bool three_a_cu = d > 64 && d <= 128 && longest >= 8 && pairs > 2 * cus &&
+                          (pairs <= 3 * cus || (unequal && longest >= 16 && 2 * pairs <= 7 * cus));
   const bool one_block = (2 * pairs <= wgs && wgs > 2 * cus) || (d == 32 && p->is_causal && p->v_layout == FA8_V_ROWS && pairs <= wgs);
   Plan n = unshared;
   if ((longest >= 3 && tiles <= (d <= 64 ? 2 : 1) * cus) || (longest >= 12 && d <= 64 && rows <= 32) ||
@@ -1068,8 +1076,9 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
     n = {1, 4, 1};
   else if (d > 64 && rows > 32 && ((pairs <= cus && longest >= (d <= 128 ? 4 : 16)) || (d > 128 && 4 * even <= 3 * cus && longest >= 24)))
     n = {2, 4, 1};
-  else if (longest >= 2 ? no_more_rounds || few_pairs : one_block)
-    n = {2, 2, 1};
+  else if (longest >= 2 ? no_more_rounds || few_pairs || three_a_cu : one_block)
+    n = {2, 2, 1, d == 32 || (d == 64 && longest >= 16 && pairs <= 3 * cus) ||
+                          (d > 64 && d <= 128 && longest >= 8 && (pairs <= 2 * cus || (unequal && longest >= 24 && 5 * pairs <= 12 * cus))) ? 2 : 1};
   if (workspace && n.waves_per_tile == 4 && n.tiles_per_workgroup == 1 && longest >= 16) {
     const long long most = std::max(1LL, std::min({32LL, cus / tiles, longest / 4}));  // one workgroup more than CUs takes twice as long
     const SplitForm form = split_form(p, (int)most);

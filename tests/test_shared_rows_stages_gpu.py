@@ -1,5 +1,7 @@
-"""One tile of 32 query rows a workgroup, four wavefronts, one or two LDS stages (csrc/fa8_shared_rows.h): the stages and the launches of more
-tiles than compute units are chosen by length and number of the tiles.  Results equal the rolling loop's bit for bit on both sides of each line."""
+"""One or two LDS stages (csrc/fa8_shared_rows.h), for one tile of 32 query rows a workgroup and four wavefronts and for two tiles and two wavefronts
+each: the stages, and the launches that fill the compute units more than once, are chosen by length and number of the tiles.  Results equal the rolling loop's bit for bit on both sides of each line."""
+import ctypes
+
 import pytest
 import torch
 
@@ -26,9 +28,32 @@ CASES = [
     (2, 12, 12, 992, 1024, 32, False, False, False, E5, True),
 ]
 
+TWO_TILES = [
+    (1, 56, 56, 519, 519, 64, False, False, False, E4, False),    # 504 workgroups, 9 blocks: one stage
+    (1, 56, 56, 512, 528, 64, False, False, True, E5, True),      # the same, v^T, a block of 16 keys
+    (1, 14, 14, 2432, 2432, 64, False, False, False, E4, False),  # 532, 38 blocks: two
+    (1, 25, 25, 2112, 2112, 64, True, False, True, E5, True),     # 825, more than three a compute unit: one
+    (1, 104, 104, 320, 320, 96, True, False, False, E4, False),   # 520, 5 blocks: one
+    (1, 17, 17, 1600, 1600, 128, True, False, False, E5, False),  # 425, 25 blocks: two
+    (1, 45, 45, 705, 705, 128, False, False, False, E4, False),   # 540, 12 blocks, the last with one key
+    (1, 26, 26, 1217, 1232, 128, False, False, True, E5, True),
+    (1, 20, 20, 2496, 2496, 96, True, False, True, E4, True),     # 780, 39 blocks
+    (8, 32, 8, 180, 600, 128, False, False, False, E5, False),    # 768 with the rows of four q heads together: three a compute unit
+    (8, 32, 8, 180, 600, 128, True, True, False, E4, False),
+]
+
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "B{}H{}k{}Nq{}Nk{}d{}".format(*c[:6]))
 def test_one_tile_a_workgroup_equals_the_rolling_loop_bitwise(case):
+    check(case, (32, 4, 1))
+
+
+@pytest.mark.parametrize("case", TWO_TILES, ids=lambda c: "B{}H{}k{}Nq{}Nk{}d{}c{:d}".format(*c[:7]))
+def test_two_tiles_a_workgroup_equal_the_rolling_loop_bitwise(case):
+    check(case, (64, 2, 1))
+
+
+def check(case, plan):
     B, H, Hk, Nq, Nk, d, causal, br, vt, dt, out8 = case
     q, k, v = _inputs(Nq + Nk + d, B, H, Hk, Nq, Nk, d, dt)
     v = v.transpose(2, 3).contiguous() if vt else v
@@ -36,8 +61,7 @@ def test_one_tile_a_workgroup_equals_the_rolling_loop_bitwise(case):
     want, want_lse = fa.flash_attention_v2_cutlass(q, k, v, causal, d ** -0.5, schedule=fa.FA8_SCHEDULE_ROLLING, **kw)
     got, lse = torch.empty_like(want), torch.empty_like(want_lse)
     p = fa.make_params(q, k, v, got, causal, d ** -0.5, vt, lse, br)
-    assert fa.plan(p, with_workspace=False) == (32, 4, 1)
-    import ctypes
+    assert fa.plan(p, with_workspace=False) == plan
     assert fa.lib().fa8_fwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)) and torch.equal(lse, want_lse)
