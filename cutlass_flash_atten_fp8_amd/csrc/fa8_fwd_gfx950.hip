@@ -1023,6 +1023,7 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 //   LDS stages of two tiles, two wavefronts a tile (423 drawn launches, head dims 64 - 128): with one stage a CU holds four workgroups of head dim
 //     64 instead of three, three of 96 and 128 instead of two.  Where there are as many, one stage takes 0.90 - 0.96 of the time of
 //     two (head dim 64) and 0.82 - 0.95 (96, 128); where there are fewer, 0.97 below 16 (8) blocks, 1.0 - 1.03 above, where two stay
+//     (head dim 64, tiles of unequal length: from 8 blocks on; 40 heads, 704 keys: 9.0 us with two, 9.7 - 10.0 with one)
 //     (head dims 96, 128, tiles of unequal length, 24 blocks: up to 2.4 pairs a CU; one stage takes 1.05 - 1.07 there)
 //   head dim 65 - 128, 8 blocks, more than two pairs a CU and up to the three that one stage lets run at once (causal, 16 blocks: 3.5): two
 //     wavefronts a tile, two tiles, though the unshared launch has fewer rounds (median 0.92, 0.82 - 1.0; beyond 1.03 - 1.4)
@@ -1077,7 +1078,7 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   else if (d > 64 && rows > 32 && ((pairs <= cus && longest >= (d <= 128 ? 4 : 16)) || (d > 128 && 4 * even <= 3 * cus && longest >= 24)))
     n = {2, 4, 1};
   else if (longest >= 2 ? no_more_rounds || few_pairs || three_a_cu : one_block)
-    n = {2, 2, 1, d == 32 || (d == 64 && longest >= 16 && pairs <= 3 * cus) ||
+    n = {2, 2, 1, d == 32 || (d == 64 && longest >= (unequal ? 8 : 16) && pairs <= 3 * cus) ||
                           (d > 64 && d <= 128 && longest >= 8 && (pairs <= 2 * cus || (unequal && longest >= 24 && 5 * pairs <= 12 * cus))) ? 2 : 1};
   if (workspace && n.waves_per_tile == 4 && n.tiles_per_workgroup == 1 && longest >= 16) {
     const long long most = std::max(1LL, std::min({32LL, cus / tiles, longest / 4}));  // one workgroup more than CUs takes twice as long
