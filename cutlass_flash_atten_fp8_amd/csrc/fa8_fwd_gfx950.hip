@@ -961,23 +961,23 @@ int compute_units() {
 // The pipelined loops exist for head dims 64 and 128 and for a softmax scale in (0, 1e6) (the pipelined loop relies on
 // exp2(-inf * scale) = 0 for masked logits and on its finite stand-in for a row max of -inf times the scale staying finite);
 // elsewhere every hint is ignored and the rolling loop runs.
-// Dense: full (non-causal) attention over a whole number of KV blocks, where no logit is ever masked; measured 1 - 2 % faster
-// than the rolling loop on launches that fill the chip and 3 - 5 % faster than the pipelined loop on small ones, so it is
-// the choice wherever it applies.  A hint for it that does not apply falls back to the automatic choice.
-// ragged_dense: also over keys that end inside a block (what launch_rows runs; fa8_fwd_schedule reports such calls as the loop
-// they would take without it).  Head dim 128, new / old time: 0.90 - 0.95 where the pipelined loop ran (2 sequences, 16 heads, 2999 keys
-// 96.0 -> 91.8 us; 8, 40, 777: 102 -> 92), 0.97 - 0.98 where the rolling one did (2, 32, 4097: 346 -> 336); head dim 64 0.95 - 0.99 above
-// three workgroups a compute unit, 1.00 - 1.02 below, where the pipelined loop stays.
+// Dense: full (non-causal) attention.  Over a whole number of KV blocks no logit is ever masked: measured 1 - 2 % faster than the rolling
+// loop on launches that fill the chip and 3 - 5 % faster than the pipelined loop on small ones, so it is the choice wherever it applies.
+// Over keys that end inside a block (kLoopDenseRagged) head dim 128, new / old time: 0.90 - 0.95 where the pipelined loop ran (2 sequences,
+// 16 heads, 2999 keys 96.0 -> 91.8 us; 8, 40, 777: 102 -> 92), 0.97 - 0.98 where the rolling one did (2, 32, 4097: 346 -> 336); head dim 64
+// 0.95 - 0.99 above three workgroups a compute unit, 1.00 - 1.02 below, where the pipelined loop stays.  A hint for the dense loop
+// that does not apply falls back to the automatic choice.
 // Pipelined: launches that cannot keep three wavefronts on every SIMD for most of their run: at most four workgroups per
 // compute unit (two resident at a time), or little work per compute unit (then filling and draining the chip, and for
 // causal launches the thinning out of the workgroups, is a large share of the run).  Measured 5 - 15 % faster than the
 // rolling loop there; the rolling loop is equal or up to 5 % faster elsewhere.
-int choose_loop(const Fa8FwdParams* p, bool ragged_dense) {
+int choose_loop(const Fa8FwdParams* p) {
   if ((p->head_dim != 64 && p->head_dim != 128) || !(p->softmax_scale > 0.f && p->softmax_scale < 1.0e6f)) return FA8_SCHEDULE_ROLLING;
   if (p->schedule == FA8_SCHEDULE_ROLLING || p->schedule == FA8_SCHEDULE_PIPELINED) return p->schedule;
+  if (!p->is_causal && (p->head_dim == 128 || p->seqlen_k % kKvBlock == 0)) return FA8_SCHEDULE_DENSE;
   const long long cus = compute_units();
   const long long wgs = (long long)p->batch * p->heads * ((p->seqlen_q + kQBlock - 1) / kQBlock);
-  if (!p->is_causal && (p->seqlen_k % kKvBlock == 0 || (ragged_dense && (p->head_dim == 128 || wgs > 3 * cus)))) return FA8_SCHEDULE_DENSE;
+  if (!p->is_causal && cus > 0 && wgs > 3 * cus) return FA8_SCHEDULE_DENSE;
   // KV blocks per compute unit below which the pipelined loop was measured to win (head dim 64 has half the matrix work
   // per block)
   const long long few_blocks = p->head_dim == 64 ? 264 : 144;
@@ -1197,7 +1197,7 @@ int launch_rows(const Fa8FwdParams* p, hipStream_t stream) {
   a.k_bs = p->k_batch_stride; a.k_hs = p->k_head_stride; a.k_rs = p->k_row_stride;
   a.v_bs = p->v_batch_stride; a.v_hs = p->v_head_stride; a.v_rs = p->v_row_stride;
   a.o_bs = p->o_batch_stride; a.o_hs = p->o_head_stride; a.o_rs = p->o_row_stride;
-  const int loop = choose_loop(p, true);
+  const int loop = choose_loop(p);
   switch (p->head_dim) {
 #define FA8_HEAD_DIM_CASE(D_) \
   case D_: return p->is_causal ? launch_types<D_, true>(p, a, loop, stream) : launch_types<D_, false>(p, a, loop, stream)
@@ -1257,7 +1257,7 @@ extern "C" int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* 
 extern "C" int fa8_fwd_schedule(const Fa8FwdParams* p) {
   const int rc = fa8_fwd_validate(p);
   if (rc != FA8_OK) return rc;
-  return choose_loop(p, false);
+  return choose_loop(p);
 }
 
 extern "C" int fa8_query(int what) {

@@ -43,8 +43,8 @@ extern "C" {
  *             so sum in another order (fa8_fwd_plan tells); any hint, and any call without a workspace, keeps the unsplit order
  *   ROLLING   one KV block after the other, three wavefronts per SIMD: for masked launches that fill the chip
  *   PIPELINED software-pipelined over neighbouring KV blocks, two wavefronts per SIMD: for small masked launches
- *   DENSE     the same pipeline in three wavefronts per SIMD, for launches without any masked logit: full (non-causal)
- *             attention with seqlen_k a multiple of 64; asked for elsewhere, the library chooses as for AUTO
+ *   DENSE     the same pipeline in three wavefronts per SIMD, for full (non-causal) attention: head dim 128, or seqlen_k a multiple of
+ *             64, or more than three workgroups per compute unit; asked for elsewhere, the library chooses as for AUTO
  *   (PIPELINED and DENSE are built for head dims 64 and 128 and a softmax scale in (0, 1e6); ignored elsewhere) */
 #define FA8_SCHEDULE_AUTO 0
 #define FA8_SCHEDULE_ROLLING 1
@@ -148,8 +148,7 @@ int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* rows_per_wo
 /*
  * Which main loop a wavefront that has its 32 query rows to itself would run for these arguments on the current device:
  * FA8_SCHEDULE_ROLLING, FA8_SCHEDULE_PIPELINED or FA8_SCHEDULE_DENSE (all > 0), or the FA8_ERR_* code fa8_fwd_validate gives; whether
- * the call has such wavefronts, fa8_fwd_plan tells.  (Full attention over keys that end inside a block may run the dense loop, its last
- * block masked, where this reports one of the other two: those are what a launch of that size takes under a causal mask.)  Launches nothing.  No counterpart in the reference (one kernel, one loop:
+ * the call has such wavefronts, fa8_fwd_plan tells.  Launches nothing.  No counterpart in the reference (one kernel, one loop:
  * csrc/flash_attention.cu:468-534); it makes the library's choice visible to benchmarks and tests.
  */
 int fa8_fwd_schedule(const Fa8FwdParams* p);

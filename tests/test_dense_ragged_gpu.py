@@ -1,6 +1,8 @@
 """Full attention over keys that end inside a KV block: the dense loop with a masked last block.  The same arithmetic in the same order as
 the rolling loop, so the results are compared bit for bit: every number of blocks up to two trips of its unrolled loop, ends on both sides
 of the rows that the two passes of a tile copy take, both v layouts, guard bands behind the last key, infinities and NaN."""
+import ctypes
+
 import pytest
 import torch
 
@@ -20,12 +22,12 @@ def _guarded(t, rows):
 
 
 def _both(q, k, v, vt, out_dtype=torch.float16):
-    import ctypes
     res = []
     for schedule in (fa.FA8_SCHEDULE_ROLLING, fa.FA8_SCHEDULE_DENSE):
         o = torch.empty(q.shape, dtype=out_dtype, device=DEV)
         lse = torch.empty(q.shape[:3], device=DEV)
         p = fa.make_params(q, k, v, o, False, 0.125, vt, lse, False, schedule)
+        assert fa.lib().fa8_fwd_schedule(ctypes.byref(p)) == schedule  # over keys that end inside a block: the masked form
         rc = fa.lib().fa8_fwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
         assert rc == 0, fa.error_string(rc)
         res.append((o.float(), lse))
