@@ -59,6 +59,24 @@ def test_transposed_v(d, heads, keys):
     _assert_same(_both(q, _guarded(k, keys), vt, True, E5))
 
 
+@pytest.mark.parametrize("keys,stride", [(65, 22486736), (79, 20950000), (100, 19004272)])
+def test_rows_so_far_apart_that_a_second_copy_lies_past_31_bits(keys, stride):
+    """The largest row strides that the library takes for so few keys: with 65 of them the second copy of the last block's V would start at
+    2.16e9 bytes.  Between the rows lie NaN codes."""
+    g = torch.Generator(device=DEV).manual_seed(keys)
+    q, k, v = ((3 * torch.randn(1, 1, n, 128, device=DEV, generator=g)).to(E4) for n in (45, keys, keys))
+    far = []
+    for t in (k, v):
+        buf = torch.full(((keys - 1) * stride + 128,), 0x7F, dtype=torch.uint8, device=DEV)
+        rows = buf.as_strided((1, 1, keys, 128), (keys * stride, keys * stride, stride, 1))
+        rows.copy_(t.view(torch.uint8))
+        far.append(rows.view(E4))
+    res = _both(q, *far, False)
+    _assert_same(res)
+    for want, got in zip(_both(q, k, v, False)[1], res[1]):
+        assert torch.isfinite(got).all() and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("where", ["q", "k", "v"])
 @pytest.mark.parametrize("row", [3, 68, 199])
 @pytest.mark.parametrize("code", [0x7C, 0x7F], ids=["inf", "nan"])  # of e5m2

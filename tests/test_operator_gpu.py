@@ -246,11 +246,13 @@ def test_capturable_in_a_hip_graph(schedule, causal):
 
 
 @pytest.mark.parametrize("nk,causal,schedule", [(99968, False, fa.FA8_SCHEDULE_AUTO), (99968, False, fa.FA8_SCHEDULE_DENSE),
-                                                (100000, False, fa.FA8_SCHEDULE_PIPELINED),
+                                                (99973, False, fa.FA8_SCHEDULE_DENSE), (99988, False, fa.FA8_SCHEDULE_DENSE),
+                                                (100008, False, fa.FA8_SCHEDULE_DENSE), (100000, False, fa.FA8_SCHEDULE_PIPELINED),
                                                 (100000, True, fa.FA8_SCHEDULE_ROLLING), (100000, True, fa.FA8_SCHEDULE_PIPELINED)])
 def test_long_kv_with_rows_far_apart(nk, causal, schedule):
     """100 000 keys whose rows lie 20 480 bytes apart: the kernel's 32-bit byte offsets into k and v run up to 2.05e9, just
-    under the 2^31 the library accepts; in all loops, and in the shared-rows kernel (without a hint).  The gaps between the rows hold NaN codes, so a misplaced read shows.  Bit for bit the
+    under the 2^31 the library accepts; in all loops (the dense one also with 5, 20 and 40 keys in its last block: in front of, between and
+    behind the first rows of the second copy of K and of V), and in the shared-rows kernel (without a hint).  The gaps between the rows hold NaN codes, so a misplaced read shows.  Bit for bit the
     result of the same call on contiguous copies, and a few rows against the oracle."""
     d, nq, stride = 128, 200, 20480
     q, k, v = (rand_fp8((1, 1, n, d), s).to(DEV) for n, s in ((nq, 31), (nk, 32), (nk, 33)))
