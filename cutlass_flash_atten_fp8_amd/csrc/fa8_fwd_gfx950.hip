@@ -1214,10 +1214,10 @@ int launch_rows(const Fa8FwdParams* p, hipStream_t stream) {
   }
 }
 
-int run(const Fa8FwdParams* p, void* workspace, long long bytes, hipStream_t stream) {
+int run(const Fa8FwdParams* p, void* workspace, long long bytes, unsigned late, hipStream_t stream) {
   Plan n = choose_plan(p, workspace != nullptr);
   if (n.splits > 1 && bytes < split_workspace(p, n.splits)) n = choose_plan(p, false);
-  if (n.splits > 1) return (uintptr_t)workspace % 16 != 0 ? FA8_ERR_ALIGN : launch_split(p, n.splits, workspace, stream);
+  if (n.splits > 1) return (uintptr_t)workspace % 16 != 0 ? FA8_ERR_ALIGN : launch_split(p, n.splits, workspace, late, stream);
   return n.waves_per_tile > 1 ? launch_shared(p, n.tiles_per_workgroup, n.waves_per_tile, n.stages, stream) : launch_rows(p, stream);
 }
 
@@ -1225,12 +1225,17 @@ int run(const Fa8FwdParams* p, void* workspace, long long bytes, hipStream_t str
 
 extern "C" int fa8_fwd(const Fa8FwdParams* p, void* hip_stream) {
   const int rc = fa8_fwd_validate(p);
-  return rc != FA8_OK ? rc : run(p, nullptr, 0, (hipStream_t)hip_stream);
+  return rc != FA8_OK ? rc : run(p, nullptr, 0, 0, (hipStream_t)hip_stream);
 }
 
 extern "C" int fa8_fwd_ws(const Fa8FwdParams* p, void* workspace, int64_t bytes, void* hip_stream) {
   const int rc = fa8_fwd_validate(p);
-  return rc != FA8_OK ? rc : run(p, workspace, bytes, (hipStream_t)hip_stream);
+  return rc != FA8_OK ? rc : run(p, workspace, bytes, 0, (hipStream_t)hip_stream);
+}
+
+extern "C" int fa8_fwd_ws_late(const Fa8FwdParams* p, void* workspace, int64_t bytes, uint32_t late_parts, void* hip_stream) {
+  const int rc = fa8_fwd_validate(p);
+  return rc != FA8_OK ? rc : run(p, workspace, bytes, late_parts, (hipStream_t)hip_stream);
 }
 
 extern "C" int fa8_fwd_workspace(const Fa8FwdParams* p, int64_t* bytes) {

@@ -11,14 +11,15 @@ namespace fa8 {
 __attribute__((visibility("hidden"))) int launch_shared(const Fa8FwdParams* p, int r, int w, int stages, hipStream_t stream);
 
 // Keys of every row tile dealt to at most `splits` workgroups (fa8_split_kv.h): how (workgroups, KV blocks of a wavefront, whether one kernel does
-// it), workspace bytes, launch.
+// it), workspace bytes, launch (late: see fa8_fwd_ws_late).
 struct SplitForm {
   int splits, blocks_per_range;
   bool one_kernel;
 };
 __attribute__((visibility("hidden"))) SplitForm split_form(const Fa8FwdParams* p, int splits);
 __attribute__((visibility("hidden"))) long long split_workspace(const Fa8FwdParams* p, int splits);
-__attribute__((visibility("hidden"))) int launch_split(const Fa8FwdParams* p, int splits, void* workspace, hipStream_t stream);
+__attribute__((visibility("hidden"))) int launch_split(const Fa8FwdParams* p, int splits, void* workspace, unsigned late,
+                                                            hipStream_t stream);
 
 }  // namespace fa8
 #endif  // FA8_LAUNCH_H_

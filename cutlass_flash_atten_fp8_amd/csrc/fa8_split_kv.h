@@ -32,6 +32,7 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 constexpr int kSplitWaves = 4;  // wavefronts (key ranges) per workgroup
 constexpr int kSplitMax = 32;   // most splits of a row tile
+constexpr int kSplitLooks = 2048;  // most looks at the maximum of another workgroup
 
 // The workspace: arrays one after the other, each of the size of all row tiles together (tile index = (batch * k/v heads + head) * tiles
 // + tile).  Offsets in bytes, all multiples of 256.
@@ -586,7 +587,7 @@ struct SplitFusedArgs {
   unsigned v_bs, v_hs, v_rs;
   unsigned o_bs, o_hs, o_rs;
   unsigned lse_bs, lse_hs;
-  int polls;  // most looks at the maximum of another workgroup
+  unsigned late;  // splits (a bit each) that do not hand on their maximum, for tests
 };
 // LDS bytes for the logits of the four ranges: what the ring of two tiles a wavefront leaves of 160 KB.  (Rings of three and four: 20.3 and
 // 20.6 us for 32768 keys of 8 k/v heads instead of 18.8, head dim 64 1 - 3 % slower: ranges are rounded up to whole rounds of the ring, and
@@ -760,7 +761,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_e
   const unsigned tag0 = (unsigned)a.tag, tag1 = (unsigned)(a.tag >> 32);
   u64* const maxima = (u64*)(a.n.workspace + p.ws.range_max) + p.at * p.splits * 64;  // [split][row][2]
   u64* const done = (u64*)(a.n.workspace + p.ws.split_max) + p.at * p.splits;         // [split]
-  if (tid < live && p.split + 1 < p.splits) {
+  if (tid < live && p.split + 1 < p.splits && !(a.late >> p.split & 1)) {
     float m = max_lds[tid];
 #pragma unroll
     for (int x = 1; x < kSplitWaves; ++x) m = __builtin_fmaxf(m, max_lds[x * 32 + tid]);
@@ -775,7 +776,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_e
     const u64* const at = maxima + (split * 32 + row) * 2;
     u64 x = 0, y = 0;
     bool there = false;
-    for (int n = a.polls; n > 0 && !there; --n) {
+    for (int n = kSplitLooks; n > 0 && !there; --n) {
       x = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       y = __hip_atomic_load(at + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       there = (unsigned)x == tag0 && (unsigned)y == tag1 && x >> 32 == y >> 32;

@@ -1,6 +1,5 @@
 // Launcher of the split-kv kernels (fa8_split_kv.h): the plan, the workspace and the launches.
 #include <atomic>
-#include <cstdlib>
 
 #include "fa8_launch.h"
 #include "fa8_split_kv.h"
@@ -39,17 +38,6 @@ unsigned long long next_tag() {
   }
 }
 
-// For tests: FA8_SPLIT_POLLS in the environment (read once) replaces how often a workgroup looks at another one's maximum before it
-// forms that itself (the results do not depend on it).
-int polls() {
-  static const int n = [] {
-    const char* e = std::getenv("FA8_SPLIT_POLLS");
-    const int x = e ? std::atoi(e) : -1;
-    return x >= 0 && x <= 1 << 16 ? x : 2048;
-  }();
-  return n;
-}
-
 struct Plan {
   int heads_k, tiles, live_rows, keys, splits, blocks_per_range;
 };
@@ -79,7 +67,7 @@ long long fa8::split_workspace(const Fa8FwdParams* p, int splits) {
   return split_layout((long long)p->batch * n.heads_k * n.tiles, n.splits, n.live_rows, p->head_dim, n.keys).bytes;
 }
 
-int fa8::launch_split(const Fa8FwdParams* p, int splits, void* workspace, hipStream_t stream) {
+int fa8::launch_split(const Fa8FwdParams* p, int splits, void* workspace, unsigned late, hipStream_t stream) {
   const Plan n = plan_of(p, splits);
   SplitShape shape;
   shape.workspace = (uint8_t*)workspace;
@@ -102,7 +90,7 @@ int fa8::launch_split(const Fa8FwdParams* p, int splits, void* workspace, hipStr
     f.o = p->o;
     f.lse = (float*)p->lse;
     f.tag = next_tag();
-    f.polls = polls();
+    f.late = late;
     f.q_bs = p->q_batch_stride / 16; f.q_hs = p->q_head_stride / 16; f.q_rs = p->q_row_stride / 16;
     f.k_bs = p->k_batch_stride / 16; f.k_hs = p->k_head_stride / 16; f.k_rs = p->k_row_stride / 16;
     f.v_bs = p->v_batch_stride / 16; f.v_hs = p->v_head_stride / 16; f.v_rs = p->v_row_stride / 16;

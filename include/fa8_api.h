@@ -137,6 +137,13 @@ int fa8_fwd_workspace(const Fa8FwdParams* p, int64_t* bytes);
 int fa8_fwd_ws(const Fa8FwdParams* p, void* workspace, int64_t bytes, void* hip_stream);
 
 /*
+ * fa8_fwd_ws for tests (library version 6).  Where the parts of split keys run in one kernel, each takes the row maxima of the parts before
+ * it from the workspace and, after a number of looks, forms those that have not come itself; the parts in late_parts (a bit each) do not
+ * hand theirs on.  The results are those of fa8_fwd_ws bit for bit.
+ */
+int fa8_fwd_ws_late(const Fa8FwdParams* p, void* workspace, int64_t bytes, uint32_t late_parts, void* hip_stream);
+
+/*
  * How a call would be cut on the current device, for benchmarks and tests (library version 5; nothing is launched): query rows of a workgroup
  * (grouped q heads counted together), wavefronts that share 32 of them (1: one of the main loops of fa8_fwd_schedule; 2 or 4: shared
  * rows, for launches with few of them; a schedule hint always gives 1), and into how many parts the keys of a row are split

@@ -2,9 +2,6 @@
 of split keys do not reach: a workgroup that stops waiting and forms that max itself, workspaces with the state of earlier calls, several
 streams, ranges of every length up to the two-kernel form."""
 import ctypes
-import os
-import subprocess
-import sys
 
 import pytest
 import torch
@@ -26,28 +23,31 @@ CASES = [
 ]
 
 
-def outputs():
-    res = []
-    for B, H, Hk, Nq, Nk, d, causal, vt, dt in CASES:
-        q, k, v = _inputs(Nk + d, B, H, Hk, Nq, Nk, d, dt)
-        k.view(torch.uint8)[0, 0, 70, 3] = 0x7C if dt == E5 else 0x7E  # infinity, the largest finite number
-        v = v.transpose(2, 3).contiguous() if vt else v
-        o, lse = fa.flash_attention_v2_cutlass(q, k, v, causal, d ** -0.5, v_transposed=vt, return_lse=True, causal_bottom_right=True)
-        assert fa.plan(fa.make_params(q, k, v, o, causal, d ** -0.5, vt, lse, True))[2] > 1
-        res += [o.view(torch.int16).cpu(), lse.view(torch.int32).cpu()]
-    return res
+def call(q, k, v, o, causal, vt=False, lse=None, late=0):
+    """One call through fa8_fwd_ws_late on a workspace of the size asked for."""
+    p = fa.make_params(q, k, v, o, causal, q.shape[3] ** -0.5, vt, lse, True)
+    assert fa.plan(p)[2] > 1
+    need = ctypes.c_int64()
+    assert fa.lib().fa8_fwd_workspace(ctypes.byref(p), ctypes.byref(need)) == 0
+    ws = torch.empty(need.value, dtype=torch.uint8, device=DEV)
+    rc = fa.lib().fa8_fwd_ws_late(ctypes.byref(p), ws.data_ptr(), need.value, late, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, fa.error_string(rc)
+    torch.cuda.synchronize()
 
 
-def test_a_workgroup_that_does_not_wait_forms_the_maximum_itself(tmp_path):
-    """No looks at all at the other workgroups' maxima (the setting is read once, so in a process of its own): the same bits."""
-    here = os.path.dirname(os.path.abspath(__file__))
-    code = (f"import sys; sys.path[:0] = [{here!r}, {os.path.dirname(here)!r}]\n"
-            f"import torch, test_split_fused_gpu as t\ntorch.save(t.outputs(), {str(tmp_path / 'o.pt')!r})\n")
-    env = dict(os.environ, FA8_SPLIT_POLLS="0")
-    r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
-    assert r.returncode == 0, r.stderr[-2000:]
-    for want, got in zip(outputs(), torch.load(tmp_path / "o.pt", weights_only=True)):
-        assert torch.equal(want, got)
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "B{}H{}k{}Nq{}Nk{}d{}".format(*c[:6]))
+def test_a_workgroup_that_does_not_wait_forms_the_maximum_itself(case):
+    """No workgroup hands on its maximum, or the first, the second, the last but one or every other one does not: the same bits."""
+    B, H, Hk, Nq, Nk, d, causal, vt, dt = case
+    q, k, v = _inputs(Nk + d, B, H, Hk, Nq, Nk, d, dt)
+    k.view(torch.uint8)[0, 0, 70, 3] = 0x7C if dt == E5 else 0x7E  # infinity, the largest finite number
+    v = v.transpose(2, 3).contiguous() if vt else v
+    want, want_lse = fa.flash_attention_v2_cutlass(q, k, v, causal, d ** -0.5, v_transposed=vt, return_lse=True, causal_bottom_right=True)
+    splits = fa.plan(fa.make_params(q, k, v, want, causal, d ** -0.5, vt, want_lse, True))[2]
+    for late in (0, 0xFFFFFFFF, 1, 2, 1 << splits - 2, 0x55555555):
+        got, lse = torch.full_like(want, float("nan")), torch.full_like(want_lse, float("nan"))
+        call(q, k, v, got, causal, vt, lse, late)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and torch.equal(lse.view(torch.int32), want_lse.view(torch.int32))
 
 
 def test_a_workspace_with_the_state_of_earlier_calls():
