@@ -9,7 +9,7 @@
 // Both are one kernel where the logits of a range fit in LDS (fa8_split_fused_kernel): the workgroups exchange their maxima through the
 // workspace while their first tiles of V are on the way, S never goes through memory and one launch, its start and its first accesses
 // are saved.  A workgroup waits for those before it in the grid, which start earlier or at the same time; if another stream keeps them off
-// the chip it stops waiting after a number of looks and forms their maximum itself.  Where the logits do not fit, one kernel each.
+// the chip it stops waiting after a number of looks and forms the maxima that have not come itself.  Where the logits do not fit, one kernel each.
 // Logits, weights and products are those of the other kernels bit for bit; only the order of the fp32 sums over the ranges is another.
 //
 // Bound: HBM bytes.  K and V are read once; S costs 8 bytes per row and key against 2 * head_dim bytes per key for K and V, which is why
@@ -32,7 +32,10 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 constexpr int kSplitWaves = 4;  // wavefronts (key ranges) per workgroup
 constexpr int kSplitMax = 32;   // most splits of a row tile
-constexpr int kSplitLooks = 2048;  // most looks at the maximum of another workgroup
+// Most looks that a thread takes at the maxima of the workgroups before its own until they have all come, 0.17 us each: 45 us, about what
+// forming a few of them from K takes (1 us a block of a wavefront's range; 32768 keys of 8 k/v heads, head dim 128, one late part: 70 us in all, every
+// part late: 182; with 2048 looks at each and all K before the workgroup read for a single late one: 470 and 452).
+constexpr int kSplitLooks = 256;
 
 // The workspace: arrays one after the other, each of the size of all row tiles together (tile index = (batch * k/v heads + head) * tiles
 // + tile).  Offsets in bytes, all multiples of 256.
@@ -612,7 +615,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_e
   __shared__ __attribute__((aligned(1024))) uint8_t s_lds[kSBytes];
   __shared__ float max_lds[kSplitWaves * 32], m_lds[kSplitWaves * 32], l_lds[kSplitWaves * 32];
   __shared__ int before_lds[32];  // max over the splits before this one, as an integer of the same order
-  __shared__ int late_lds, last_lds;
+  __shared__ unsigned late_lds;  // splits whose maximum has not come, a bit each
+  __shared__ int last_lds;
   const SplitPlace p = split_place(a.n, D);
   const int qn = p.qn, h = p.h, lane = p.lane, tid = threadIdx.x, live = p.live_rows;
   const float c = a.n.scale_log2;
@@ -771,47 +775,53 @@ __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_e
   }
   // (signed integers of the order of the floats; no NaN comes out of the maxima)
   auto ordered = [](float x) __attribute__((always_inline)) { const int i = __float_as_int(x); return i ^ ((i >> 31) & 0x7fffffff); };
+  int looks = kSplitLooks;  // of this thread, at all the maxima that it takes
   for (int e = tid; e < p.split * live; e += 64 * kSplitWaves) {
     const int split = e / live, row = e - split * live;
     const u64* const at = maxima + (split * 32 + row) * 2;
     u64 x = 0, y = 0;
     bool there = false;
-    for (int n = kSplitLooks; n > 0 && !there; --n) {
+    do {  // (one look at each, also when the others have used them up)
       x = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       y = __hip_atomic_load(at + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       there = (unsigned)x == tag0 && (unsigned)y == tag1 && x >> 32 == y >> 32;
-    }
+    } while (!there && --looks > 0);
     if (there)
       atomicMax(before_lds + row, ordered(__uint_as_float((unsigned)(x >> 32))));
     else
-      late_lds = 1;
+      atomicOr(&late_lds, 1u << split);
   }
   sync();
-  if (late_lds) {
-    // A workgroup before this one has not run yet (the chip is busy with something else): its maximum is formed here, from K in memory.
+  const unsigned late = __builtin_amdgcn_readfirstlane(late_lds);
+  if (late) {
+    // Workgroups before this one have not run yet (the chip is busy with something else): their maxima are formed here, from K in memory.
     float m = -1.0e30f;
-    for (int j = p.wave; j < p.split * kSplitWaves * a.n.blocks_per_range; j += kSplitWaves) {
-      v16f s[2];
+    const int blocks = kSplitWaves * a.n.blocks_per_range;  // of a split
+    for (unsigned left = late; left != 0; left &= left - 1) {
+      const int first = __builtin_ctz(left) * blocks;
+      for (int j = first + p.wave; j < first + blocks; j += kSplitWaves) {
+        v16f s[2];
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const uint8_t* row = kp + (long long)min(j * kKvBlock + kv_of_lds_row(32 * t + qn), kv_last) * k_rs;
+        for (int t = 0; t < 2; ++t) {
+          const uint8_t* row = kp + (long long)min(j * kKvBlock + kv_of_lds_row(32 * t + qn), kv_last) * k_rs;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) s[t][e] = 0.f;
+          for (int e = 0; e < 16; ++e) s[t][e] = 0.f;
 #pragma unroll
-        for (int ks = 0; ks < kKSteps; ++ks) {
-          const uint8_t* k8 = row + 64 * ks + (64 * ks + 32 < D ? 32 * h : 0);  // (past the head dim Q is 0)
-          const v4i lo = *(const v4i*)(k8);
-          const v4i hi = *(const v4i*)(k8 + 16);
-          v8i kf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-          if (64 * ks + 32 >= D && h) kf = v8i{0, 0, 0, 0, 0, 0, 0, 0};  // (nor may a NaN meet that 0)
-          s[t] = mfma_fp8<E5M2>(kf, qf[ks], s[t]);
+          for (int ks = 0; ks < kKSteps; ++ks) {
+            const uint8_t* k8 = row + 64 * ks + (64 * ks + 32 < D ? 32 * h : 0);  // (past the head dim Q is 0)
+            const v4i lo = *(const v4i*)(k8);
+            const v4i hi = *(const v4i*)(k8 + 16);
+            v8i kf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            if (64 * ks + 32 >= D && h) kf = v8i{0, 0, 0, 0, 0, 0, 0, 0};  // (nor may a NaN meet that 0)
+            s[t] = mfma_fp8<E5M2>(kf, qf[ks], s[t]);
+          }
         }
+        mask(j, s);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int e = 0; e < 16; e += 2) m = max3(s[t][e], s[t][e + 1], m);
       }
-      mask(j, s);
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int e = 0; e < 16; e += 2) m = max3(s[t][e], s[t][e + 1], m);
     }
     m = lane32_max(m);
     if (h == 0) atomicMax(before_lds + qn, ordered(m));

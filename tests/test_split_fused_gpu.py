@@ -50,6 +50,25 @@ def test_a_workgroup_that_does_not_wait_forms_the_maximum_itself(case):
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and torch.equal(lse.view(torch.int32), want_lse.view(torch.int32))
 
 
+def test_one_late_part_costs_its_own_keys_alone():
+    """16 blocks a wavefront in 32 parts: with one maximum late a workgroup reads the keys of that part again, not those of all before it."""
+    q, k, v = _inputs(1, 1, 8, 2, 1, 131072, 128, E4)
+    o = torch.empty(q.shape, dtype=torch.float16, device=DEV)
+
+    def microseconds(late):
+        times = []
+        for _ in range(5):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            call(q, k, v, o, True, late=late)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(begin.elapsed_time(end) * 1e3)
+        return sorted(times)[2]
+    one, all_of_them = microseconds(1), microseconds(0xFFFFFFFF)
+    assert 2 * one < all_of_them, (one, all_of_them)
+
+
 def test_a_workspace_with_the_state_of_earlier_calls():
     """The same workspace for calls with other keys, other lengths, other splits: no value of an earlier call is taken."""
     ws = torch.zeros(64 << 20, dtype=torch.uint8, device=DEV)
