@@ -599,8 +599,12 @@ constexpr int split_fused_s_bytes(int d) {
   const int dp = d <= 32 ? 32 : (d <= 64 ? 64 : (d <= 128 ? 128 : 256));
   return (160 * 1024 - 2048 - 2 * kSplitWaves * kKvBlock * dp) / 4096 * 4096;
 }
+// What a launch asks for.  (Held whatever the ranges needed, 161 KB a workgroup, a call had to wait for compute units that another stream's
+// kernel left empty: 4 sequences of 8192 keys, 8 k/v heads, head dim 64, beside full attention over 4096 keys of 64 heads, head dim 128: 295 us
+// a call, 30 so (the two kernels before: 92); alone 11.7 either way.)
+inline long long split_fused_s_used(int live_rows, int blocks_per_range) { return (long long)blocks_per_range * live_rows * kKvBlock * 4 * kSplitWaves; }
 inline bool split_fused_fits(int d, int live_rows, int blocks_per_range) {
-  return (long long)blocks_per_range * live_rows * kKvBlock * 4 * kSplitWaves <= split_fused_s_bytes(d);
+  return split_fused_s_used(live_rows, blocks_per_range) <= split_fused_s_bytes(d);
 }
 
 template <int D, bool E5M2, bool VT>
@@ -608,11 +612,11 @@ __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_e
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int DP = D <= 32 ? 32 : (D <= 64 ? 64 : (D <= 128 ? 128 : 256));
   constexpr int kTileBytes = kKvBlock * DP, kPasses = kTileBytes / 1024, kKSteps = (D + 63) / 64, kMTiles = D / 32;
-  constexpr int R = 2, kSBytes = split_fused_s_bytes(D);
+  constexpr int R = 2;
   static_assert(kSplitWaves * kTileBytes >= 2 * D * 32 * 4 && kSplitWaves * kTileBytes >= kSplitMax * 256, "see split_merge");
   __shared__ __attribute__((aligned(1024))) uint8_t lds0[kSplitWaves * kTileBytes];
   __shared__ __attribute__((aligned(1024))) uint8_t lds1[kSplitWaves * kTileBytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t s_lds[kSBytes];
+  extern __shared__ __attribute__((aligned(1024))) uint8_t s_lds[];  // split_fused_s_used() bytes
   __shared__ float max_lds[kSplitWaves * 32], m_lds[kSplitWaves * 32], l_lds[kSplitWaves * 32];
   __shared__ int before_lds[32];  // max over the splits before this one, as an integer of the same order
   __shared__ unsigned late_lds;  // splits whose maximum has not come, a bit each
@@ -696,7 +700,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_e
           if (j * kKvBlock + 32 * h + 16 * t + e > kv_limit) s[t][e] = -INFINITY;
     }
   };
-  uint8_t* const s_at = s_lds + p.wave * (kSBytes / kSplitWaves) + (h * live + min(qn, live - 1)) * 16;
+  uint8_t* const s_at = s_lds + p.wave * a.n.blocks_per_range * live * (kKvBlock * 4) + (h * live + min(qn, live - 1)) * 16;
   float m_run = -1.0e30f;
   const int groups = max(1, (p.count + R - 1) / R);
   // Q has arrived.  (Left to the compiler, which waits in front of the loop, this would be a wait for all copies.)

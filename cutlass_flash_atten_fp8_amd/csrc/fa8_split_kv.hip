@@ -112,7 +112,7 @@ int fa8::launch_split(const Fa8FwdParams* p, int splits, void* workspace, unsign
       default: return FA8_ERR_HEAD_DIM;
     }
     void* argv[] = {&f};
-    return (int)hipLaunchKernel(fn, grid, dim3(64 * kSplitWaves), argv, 0, stream);
+    return (int)hipLaunchKernel(fn, grid, dim3(64 * kSplitWaves), argv, (size_t)split_fused_s_used(n.live_rows, n.blocks_per_range), stream);
   }
   SplitLogitsArgs l;
   l.n = shape;

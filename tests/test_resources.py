@@ -1,4 +1,4 @@
-"""Register use of the compiled kernels, read from the code-object notes of libfa8.so (no GPU): a vector register spilled to scratch costs memory
+"""Register and LDS use of the compiled kernels, read from the code-object notes of libfa8.so (no GPU): a vector register spilled to scratch costs memory
 traffic in every step of a loop, and the shared-rows kernel of the wide head dims sits close to the 256 registers of a lane."""
 import os
 import re
@@ -29,17 +29,35 @@ def code_objects(path):
         at = data.find(MAGIC, at + 1)
 
 
-@pytest.mark.skipif(not os.path.exists(READELF), reason="needs llvm-readelf")
-def test_no_kernel_spills_vector_registers(tmp_path):
+def kernel_notes(tmp_path, key):
+    """{mangled kernel name: the number that its code object notes under .key}"""
     kernels = {}
     for i, blob in enumerate(code_objects(fa.LIBFA8_PATH)):
         f = tmp_path / f"{i}.o"
         f.write_bytes(blob)
         notes = subprocess.run([READELF, "--notes", str(f)], capture_output=True, text=True, check=True).stdout
         names = re.findall(r"^\s+\.name:\s+(_Z\S+)$", notes, re.M)
-        spills = re.findall(r"\.vgpr_spill_count:\s+(\d+)", notes)
-        assert len(names) == len(spills)
-        kernels.update(zip(names, map(int, spills)))
-    for part in ("fa8_fwd_kernel", "fa8_shared_rows_kernel", "fa8_split_logits_kernel", "fa8_split_values_kernel"):
+        values = re.findall(rf"\.{key}:\s+(\d+)", notes)
+        assert len(names) == len(values)
+        kernels.update(zip(names, map(int, values)))
+    return kernels
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="needs llvm-readelf")
+def test_no_kernel_spills_vector_registers(tmp_path):
+    kernels = kernel_notes(tmp_path, "vgpr_spill_count")
+    for part in ("fa8_fwd_kernel", "fa8_shared_rows_kernel", "fa8_split_fused_kernel", "fa8_split_logits_kernel", "fa8_split_values_kernel"):
         assert any(part in n for n in kernels), part
     assert {n: s for n, s in kernels.items() if s} == {}
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="needs llvm-readelf")
+def test_split_keys_in_one_kernel_hold_no_lds_that_their_ranges_do_not_need(tmp_path):
+    """Every workgroup holds its ring of two tiles a wavefront and 2 KB; LDS for the logits is asked for by length at the launch, so that a
+    call with short ranges does not need compute units that are empty."""
+    lds = {n: x for n, x in kernel_notes(tmp_path, "group_segment_fixed_size").items() if "fa8_split_fused_kernel" in n}
+    assert len(lds) == 8 * 4
+    for name, x in lds.items():
+        d = int(re.search(r"kernelILi(\d+)E", name)[1])
+        row = 32 if d <= 32 else 64 if d <= 64 else 128 if d <= 128 else 256
+        assert x <= 2 * 4 * 64 * row + 2048, name
