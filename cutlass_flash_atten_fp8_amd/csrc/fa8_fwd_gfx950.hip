@@ -1009,8 +1009,12 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 //     wait for each other's barriers.  Work of the tiles / (CUs x longest): head dim <= 64 from 6 blocks on up to 1.5 (0.85 - 0.97), 16 blocks
 //     1.75 (0.84 - 0.94), 24 blocks 2 (0.9); head dim 65 - 128 8 blocks 1 (0.90 - 0.93), 24 blocks 1.25 (0.86), 32 blocks 1.5 (0.82).  Equal
 //     tiles: head dim <= 64, 16 blocks, up to the three a CU that run at once (0.85 - 0.97).  (13 400 drawn launches; beyond these lines 1.0 - 1.4)
-//   LDS stages of one tile, four wavefronts: with one workgroup a CU (head dim 64: two) one stage takes 0.96 - 0.98 of the time of two below 16
-//     blocks, the same at 16 - 24, 1.0 - 1.3 above; two stages of head dim 128 have no room for a second workgroup (0.7 - 0.8)
+//   LDS stages of one tile, four wavefronts: with one workgroup a CU (head dim <= 64: two) one stage takes 0.94 - 0.98 of the time of two below 16
+//     blocks, the same at 16 - 24, 1.0 - 1.3 above (head dim 32: 0.98 at every length).  Where K and V come from memory for a tile or two alone
+//     (decode steps), it takes more from fewer blocks on: head dims 96, 128 1.01 - 1.25 from 4 blocks a CU (of all k/v heads together), head dim 64 1.03 -
+//     1.08 from 12 with a tile a CU at most (0.95 - 1.0 with more, below 24 blocks a head), head dim 32 1.07 - 1.26 from 32 (more than two tiles a k/v head: 64; 192 heads, 42244 keys, head dim 32: 177 us with two, 223 with one; 128 heads, 1457
+//     keys, head dim 128: 13.7, 17.2).  Two stages of head dim 128 have no room for a second workgroup (0.7 - 0.8), of 64 and 32 for a third
+//     (0.8 - 0.88, up to the 4 a CU that take two rounds either way: 1.02 - 1.13 from 24 blocks)
 //   head dim 65 - 128, pairs <= CUs (one a CU) and 4 blocks: four wavefronts a tile, two tiles a workgroup, which share the copies of K
 //     and V (0.6 - 0.85)
 //   head dim above 128: the same from 16 blocks on (one LDS stage; 1.0 - 1.1 at 6 - 12 blocks, 0.95 at 16 - 24, 0.86 from 64 on, against two
@@ -1069,10 +1073,14 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   const bool three_a_cu = d > 64 && d <= 128 && longest >= 8 && pairs > 2 * cus &&
                           (pairs <= 3 * cus || (unequal && longest >= 16 && 2 * pairs <= 7 * cus));
   const bool one_block = (2 * pairs <= wgs && wgs > 2 * cus) || (d == 32 && p->is_causal && p->v_layout == FA8_V_ROWS && pairs <= wgs);
+  // one tile a workgroup, two LDS stages: they run at once, or in no more rounds than with one stage; and K and V come from memory for a tile or two
+  const bool two_fit = d <= 128 && (tiles <= (d <= 64 ? 2 : 1) * cus || (d <= 64 && longest >= 24 && tiles > 3 * cus && tiles <= 4 * cus));
+  const long long own_blocks = d == 32 ? (rows <= 64 ? 32 : 64) : (rows > 64 || (d == 64 && tiles > cus) ? 1LL << 40 : (d == 64 ? 12 : 4));
+  const bool own_kv = kv_heads * longest >= own_blocks * cus;
   Plan n = unshared;
   if ((longest >= 3 && tiles <= (d <= 64 ? 2 : 1) * cus) || (longest >= 12 && d <= 64 && rows <= 32) ||
       (longest == 2 && d <= 128 && tiles <= cus && 8 * wgs < 5 * tiles))
-    n = {1, 4, 1, longest >= 24 && tiles <= (d <= 64 ? 2 : 1) * cus ? 2 : 1};
+    n = {1, 4, 1, two_fit && ((longest >= 24 && d > 32) || own_kv) ? 2 : 1};
   else if (longest >= (d <= 64 ? 6 : 8) && (unequal ? quarters <= most_quarters : d <= 64 && tiles <= 3 * cus && longest >= 16))
     n = {1, 4, 1};
   else if (d > 64 && rows > 32 && ((pairs <= cus && longest >= (d <= 128 ? 4 : 16)) || (d > 128 && 4 * even <= 3 * cus && longest >= 24)))

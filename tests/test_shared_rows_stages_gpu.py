@@ -26,6 +26,14 @@ CASES = [
     (1, 24, 24, 700, 700, 32, True, False, False, E4, False),
     (1, 24, 12, 700, 1030, 64, False, False, False, E4, False),  # equal tiles, 528 of them, ragged last block
     (2, 12, 12, 992, 1024, 32, False, False, False, E5, True),
+    # K and V for one tile or two alone: two stages from fewer blocks on
+    (64, 2, 1, 3, 8129, 32, True, True, False, E4, False),       # 64 heads of 128 blocks
+    (64, 2, 1, 3, 8100, 32, True, True, False, E4, False),       # of 127: one stage
+    (16, 64, 64, 1, 1536, 32, False, False, True, E5, True),     # 1024 tiles, 24 blocks
+    (1, 24, 24, 90, 43777, 32, True, True, False, E5, False),    # three tiles a head, 685 blocks
+    (32, 16, 8, 2, 777, 64, True, True, False, E4, True),        # 256 heads of 13 blocks
+    (16, 16, 8, 20, 512, 128, True, True, False, E5, False),     # 128 heads, two tiles each, 8 blocks
+    (16, 8, 8, 1, 449, 96, True, True, False, E4, False),
 ]
 
 TWO_TILES = [
