@@ -1028,9 +1028,11 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 //     64 instead of three, three of 96 and 128 instead of two.  Where there are as many, one stage takes 0.90 - 0.96 of the time of
 //     two (head dim 64) and 0.82 - 0.95 (96, 128); where there are fewer, 0.97 below 16 (8) blocks, 1.0 - 1.03 above, where two stay
 //     (head dim 64, tiles of unequal length: from 8 blocks on; 40 heads, 704 keys: 9.0 us with two, 9.7 - 10.0 with one)
-//     (head dims 96, 128, tiles of unequal length, 24 blocks: up to 2.4 pairs a CU; one stage takes 1.05 - 1.07 there)
-//   head dim 65 - 128, 8 blocks, more than two pairs a CU and up to the three that one stage lets run at once (causal, 16 blocks: 3.5): two
-//     wavefronts a tile, two tiles, though the unshared launch has fewer rounds (median 0.92, 0.82 - 1.0; beyond 1.03 - 1.4)
+//     (head dims 96, 128, tiles of unequal length: 17 blocks up to 2.4 pairs a CU and even <= 5/4 CUs, 24 blocks 7/5 CUs, 28 blocks 2.5 pairs; one
+//     stage takes 1.02 - 1.13 there, 0.9 - 0.93 beyond)
+//   head dim 65 - 128, 8 blocks, more than two pairs a CU and up to the three that one stage lets run at once (causal, 16 blocks: 3.5, if
+//     even <= 2 CUs): two wavefronts a tile, two tiles, though the unshared launch has fewer rounds (median 0.92, 0.82 - 1.0; beyond 1.02 - 1.4,
+//     as with a mask aligned to the last key: 64 heads, 895 queries on 1841 keys, even 2.7 CUs, head dim 128: 36.9 us, 43.0 shared)
 //   A single block leaves nothing to share but the products (1.05 - 1.3): only where the rows of grouped q heads fill the tiles that
 //     they would leave idle, 2 pairs <= wgs, and on a full chip (0.2 - 0.8), and under the mask at head dim 32, whose unshared loop is
 //     the rolling one (v as rows: 0.75 - 0.95, transposed 1.0 - 1.4)
@@ -1071,7 +1073,9 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
                               (d == 64 && longest >= 8 && 5 * shortest > 3 * longest && 2 * pair_rounds <= 3 * wg_rounds);
   const bool few_pairs = (longest >= 5 || d == 32) && 4 * even <= (p->is_causal ? 5 : 4) * (d <= 64 ? 2 : 1) * cus;
   const bool three_a_cu = d > 64 && d <= 128 && longest >= 8 && pairs > 2 * cus &&
-                          (pairs <= 3 * cus || (unequal && longest >= 16 && 2 * pairs <= 7 * cus));
+                          (pairs <= 3 * cus || (unequal && longest >= 16 && 2 * pairs <= 7 * cus && even <= 2 * cus));
+  const bool unequal_pairs = unequal && (longest >= 24 ? 5 * even <= 7 * cus : longest >= 17 && 4 * even <= 5 * cus) &&
+                             (longest >= 28 ? 2 * pairs < 5 * cus : 5 * pairs <= 12 * cus);
   const bool one_block = (2 * pairs <= wgs && wgs > 2 * cus) || (d == 32 && p->is_causal && p->v_layout == FA8_V_ROWS && pairs <= wgs);
   // one tile a workgroup, two LDS stages: they run at once, or in no more rounds than with one stage; and K and V come from memory for a tile or two
   const bool two_fit = d <= 128 && (tiles <= (d <= 64 ? 2 : 1) * cus || (d <= 64 && longest >= 24 && tiles > 3 * cus && tiles <= 4 * cus));
@@ -1087,7 +1091,7 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
     n = {2, 4, 1};
   else if (longest >= 2 ? no_more_rounds || few_pairs || three_a_cu : one_block)
     n = {2, 2, 1, d == 32 || (d == 64 && longest >= (unequal ? 8 : 16) && pairs <= 3 * cus) ||
-                          (d > 64 && d <= 128 && longest >= 8 && (pairs <= 2 * cus || (unequal && longest >= 24 && 5 * pairs <= 12 * cus))) ? 2 : 1};
+                          (d > 64 && d <= 128 && longest >= 8 && (pairs <= 2 * cus || unequal_pairs)) ? 2 : 1};
   if (workspace && n.waves_per_tile == 4 && n.tiles_per_workgroup == 1 && longest >= 16) {
     const long long most = std::max(1LL, std::min({32LL, cus / tiles, longest / 4}));  // one workgroup more than CUs takes twice as long
     const SplitForm form = split_form(p, (int)most);

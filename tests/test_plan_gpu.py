@@ -42,6 +42,15 @@ def test_sharing_does_not_take_launches_that_it_slows_down(shape):
 
 
 @pytest.mark.parametrize("shape", [
+    (1, 64, 64, 895, 1841, 128, True, True),   # 36.9 / 43.0: 3.5 pairs a compute unit, work of 2.7
+    (1, 64, 64, 884, 1271, 128, True, True),   # 27.8 / 31.9
+    (1, 32, 32, 1757, 3649, 96, True, True),   # 60.7 / 67.7
+], ids=lambda s: "B{}H{}k{}Nq{}Nk{}d{}".format(*s[:6]))
+def test_chunks_whose_tiles_are_long_throughout_are_not_shared(shape):
+    assert plan_of(*shape) == UNSHARED
+
+
+@pytest.mark.parametrize("shape", [
     (1, 1, 1, 32, 1121, 128, True, True),    # 10.0 shared, 19.3 split
     (1, 4, 1, 15, 1244, 64, True, True),     # 9.1, 16.7
     (1, 2, 1, 1051, 1051, 192, True),        # 15, 26.7

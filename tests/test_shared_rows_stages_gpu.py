@@ -46,6 +46,8 @@ TWO_TILES = [
     (1, 45, 45, 705, 705, 128, False, False, False, E4, False),   # 540, 12 blocks, the last with one key
     (1, 26, 26, 1217, 1232, 128, False, False, True, E5, True),
     (1, 20, 20, 2496, 2496, 96, True, False, True, E4, True),     # 780, 39 blocks
+    (1, 32, 32, 1152, 1152, 128, True, False, False, E4, False),  # 576 of unequal length, 18 blocks: two
+    (1, 32, 32, 1094, 1786, 128, True, True, False, E5, False),   # the work of 1.6 a compute unit: one
     (8, 32, 8, 180, 600, 128, False, False, False, E5, False),    # 768 with the rows of four q heads together: three a compute unit
     (8, 32, 8, 180, 600, 128, True, True, False, E4, False),
 ]
