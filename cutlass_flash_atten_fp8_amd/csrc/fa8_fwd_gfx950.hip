@@ -1041,8 +1041,12 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 // wavefronts, and then as fine as the compute units allow, down to one block a wavefront.  The estimates are fits (shared rows: 3003 drawn
 // launches whose K and V come from HBM and 1725 whose K and V the Infinity Cache still holds; split: 1663 pairs of 306 drawn launches and a
 // number of splits, K and V mostly from HBM): a start, a step per block of a wavefront's range, K and V, the parts of O, and the logits
-// written and read; neither is below the rate at which it moves its bytes.  On the 306 launches the choice takes 0.5 % longer than the best
-// of all numbers of splits on average; two blocks a wavefront at least, and the estimate for two kernels, took 6.5 % longer.  One head, 32
+// written and read; neither is below the rate at which it moves its bytes.  On the 306 launches the choice takes 0.5 % longer than
+// the best of all numbers of splits on average; two blocks a wavefront at least, and the estimate for two kernels, took 6.5 % longer.  Of 5700 more
+// launches, each measured with and without splitting, the choice is the slower one by more than 3 % in 2 of 100.  They set three things: head
+// dims above 128 (one LDS stage) take K and V at 3.6 - 4.4 TB/s, from 24 blocks on added to the steps (at the 5.6 of the others 128 tiles of head dim 192, 7695 keys,
+// were not split: 105 us, 82 in two parts), and two kernels 5 - 10 % longer than the fit; head dims 32 and 64 take 0.255 us a block from 56 on; and below 20 blocks head dims up to 128 are not
+// split (4 heads, 974 keys, head dim 128: 8.8 us, 9.9 in four parts; 16 - 19 blocks 1.03 - 1.11).  One head, 32
 // queries on 1121 keys, d128: 10.0 us shared, 19.3 split; one sequence of 32768 keys: 151 and 18; 2 sequences of 6881 keys, 8 queries of 3 k/v heads,
 // group of 4, d128: 25.2 in 13 parts, 16.1 in 27.
 Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
@@ -1092,19 +1096,21 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   else if (longest >= 2 ? no_more_rounds || few_pairs || three_a_cu : one_block)
     n = {2, 2, 1, d == 32 || (d == 64 && longest >= (unequal ? 8 : 16) && pairs <= 3 * cus) ||
                           (d > 64 && d <= 128 && longest >= 8 && (pairs <= 2 * cus || unequal_pairs)) ? 2 : 1};
-  if (workspace && n.waves_per_tile == 4 && n.tiles_per_workgroup == 1 && longest >= 16) {
+  if (workspace && n.waves_per_tile == 4 && n.tiles_per_workgroup == 1 && longest >= (d <= 128 ? 20 : 16)) {
     const long long most = std::max(1LL, std::min({32LL, cus / tiles, longest / 4}));  // one workgroup more than CUs takes twice as long
     const SplitForm form = split_form(p, (int)most);
     const long long splits = form.splits;
     const double range = form.blocks_per_range, row_bytes = d <= 32 ? 32 : (d <= 64 ? 64 : (d <= 128 ? 128 : 256));  // of an LDS tile
     const double kv_bytes = 2.0 * kv_heads * longest * kKvBlock * d, live = rows < 32 ? (double)rows : 32.0;
     const double s_bytes = 8.0 * tiles * live * longest * kKvBlock;
-    const double shared_us = 5.4 + std::max((d <= 64 ? 0.23 : (d <= 128 ? 0.30 : 0.63)) * longest, kv_bytes / 5.6e6);
+    const double shared_us = std::max({5.4 + (d <= 64 ? 0.23 : (d <= 128 ? 0.30 : 0.63)) * longest, 5.4 + kv_bytes / 5.6e6,
+                                       d <= 64 ? 4.0 + 0.255 * longest : (d <= 128 || longest < 24 ? 0.0 : 4.1 + (d <= 192 ? 0.59 : 0.65) * longest + kv_bytes / 13.6e6)});
     const double split_us =
         form.one_kernel
             ? std::max(7.7 + (0.53 + 0.0057 * row_bytes) * range + kv_bytes / 23.5e6 + 1.34e-3 * d * live + 0.07 * splits, 5.4 + kv_bytes / 5.6e6)
-            : std::max(7.5 + (0.6 + 0.0054 * row_bytes) * range + kv_bytes / 9.3e6 + 0.9e-3 * d * live + 0.16 * splits + 0.063 * range * live +
-                           s_bytes / 11e6, 2.3 + (kv_bytes + s_bytes) / 5.8e6);
+            : (d <= 128 ? 1.0 : (d <= 192 ? 1.05 : 1.1)) *
+                  std::max(7.5 + (0.6 + 0.0054 * row_bytes) * range + kv_bytes / 9.3e6 + 0.9e-3 * d * live + 0.16 * splits +
+                               0.063 * range * live + s_bytes / 11e6, 2.3 + (kv_bytes + s_bytes) / 5.8e6);
     if (splits > 1 && split_us < shared_us && tiles * splits < 65536 && longest / (4 * splits) < 65535 &&
         split_workspace(p, (int)splits) <= kMaxWorkspace)
       n.splits = (int)splits;

@@ -57,6 +57,8 @@ def test_chunks_whose_tiles_are_long_throughout_are_not_shared(shape):
     (1, 2, 2, 1792, 1792, 160),              # 20.1, 35.5
     (1, 6, 2, 12, 1245, 128, True, True),    # 10.3, 18
     (4, 1, 1, 832, 1665, 160),               # 20.1, 34.1
+    (4, 4, 4, 1, 974, 128, True, True),      # 8.8, 9.9: 16 blocks
+    (1, 12, 6, 2, 999, 128, True, True),     # 8.6, 9.6
 ], ids=lambda s: "B{}H{}k{}Nq{}Nk{}d{}".format(*s[:6]))
 def test_few_keys_are_not_split(shape):
     assert plan_of(*shape)[1:] == (4, 1)
@@ -68,7 +70,10 @@ def test_keys_are_not_split_where_their_bytes_bound_both():
 
 
 @pytest.mark.parametrize("shape", [(1, 32, 8, 1, 32768, 128, True, True), (4, 32, 8, 1, 4096, 128, True, True), (1, 8, 8, 1, 4096, 64, True, True),
-                                   (1, 2, 2, 16, 4096, 224)], ids=lambda s: "B{}H{}k{}Nq{}Nk{}d{}".format(*s[:6]))
+                                   (1, 2, 2, 16, 4096, 224),
+                                   # K and V bound by few bytes under way with one LDS stage: 105 us shared, 82 split; 129, 101; 156, 132; 173, 151
+                                   (64, 4, 2, 1, 7695, 192, True, True), (2, 64, 64, 2, 9601, 192, True, True),
+                                   (16, 12, 6, 2, 11470, 256, True, True), (8, 12, 12, 2, 42156, 64, True, True)], ids=lambda s: "B{}H{}k{}Nq{}Nk{}d{}".format(*s[:6]))
 def test_many_keys_are_split(shape):
     assert plan_of(*shape)[2] > 1 and plan_of(*shape, with_workspace=False)[2] == 1
 
