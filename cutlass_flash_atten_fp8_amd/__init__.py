@@ -29,8 +29,8 @@ FA8_CAUSAL_TOP_LEFT, FA8_CAUSAL_BOTTOM_RIGHT = 0, 1
 FA8_SCHEDULE_AUTO, FA8_SCHEDULE_ROLLING, FA8_SCHEDULE_PIPELINED, FA8_SCHEDULE_DENSE = 0, 1, 2, 3
 (FA8_QUERY_VERSION, FA8_QUERY_KV_BLOCK, FA8_QUERY_Q_BLOCK, FA8_QUERY_KV_ASCENDING, FA8_QUERY_THREADS,
  FA8_QUERY_PARAMS_SIZE) = range(6)
-FA8_EXPORTS = ("fa8_fwd_validate", "fa8_fwd", "fa8_fwd_workspace", "fa8_fwd_ws", "fa8_fwd_ws_late", "fa8_fwd_plan", "fa8_fwd_schedule",
-               "fa8_query", "fa8_error_string")
+FA8_EXPORTS = ("fa8_fwd_validate", "fa8_fwd", "fa8_fwd_workspace", "fa8_fwd_ws", "fa8_fwd_ws_late", "fa8_fwd_plan", "fa8_fwd_form",
+               "fa8_fwd_schedule", "fa8_query", "fa8_error_string")
 
 
 class Fa8FwdParams(ctypes.Structure):
@@ -75,6 +75,8 @@ def lib():
         L.fa8_fwd_ws_late.argtypes = [ctypes.POINTER(Fa8FwdParams), ctypes.c_void_p, ctypes.c_int64, ctypes.c_uint32, ctypes.c_void_p]
         L.fa8_fwd_plan.restype = ctypes.c_int
         L.fa8_fwd_plan.argtypes = [ctypes.POINTER(Fa8FwdParams), ctypes.c_int] + [ctypes.POINTER(ctypes.c_int32)] * 3
+        L.fa8_fwd_form.restype = ctypes.c_int
+        L.fa8_fwd_form.argtypes = [ctypes.POINTER(Fa8FwdParams), ctypes.c_int] + [ctypes.POINTER(ctypes.c_int32)] * 2
         L.fa8_fwd_schedule.restype = ctypes.c_int
         L.fa8_fwd_schedule.argtypes = [ctypes.POINTER(Fa8FwdParams)]
         L.fa8_query.restype = ctypes.c_int
@@ -99,6 +101,15 @@ def plan(p, with_workspace=True):
     rc = lib().fa8_fwd_plan(ctypes.byref(p), int(with_workspace), *(ctypes.byref(x) for x in v))
     if rc != 0:
         raise RuntimeError(f"fa8_fwd_plan: {error_string(rc)} (code {rc})")
+    return tuple(x.value for x in v)
+
+
+def form(p, with_workspace=True):
+    """(LDS stages of shared rows or 0, kernels launched) of a call with these parameters."""
+    v = [ctypes.c_int32() for _ in range(2)]
+    rc = lib().fa8_fwd_form(ctypes.byref(p), int(with_workspace), *(ctypes.byref(x) for x in v))
+    if rc != 0:
+        raise RuntimeError(f"fa8_fwd_form: {error_string(rc)} (code {rc})")
     return tuple(x.value for x in v)
 
 

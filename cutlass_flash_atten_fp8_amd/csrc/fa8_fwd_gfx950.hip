@@ -990,7 +990,7 @@ struct Plan {
   int tiles_per_workgroup;  // of 32 query rows
   int waves_per_tile;       // 1: the loops of this file; 2, 4: wavefronts share a row tile
   int splits;               // > 1: the keys of a row tile dealt to this many workgroups (needs a workspace)
-  int stages = 1;           // LDS stages, where sharing wavefronts have the choice
+  int stages = 1;           // LDS stages of sharing wavefronts
 };
 constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask for
 
@@ -1092,7 +1092,7 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
   else if (longest >= (d <= 64 ? 6 : 8) && (unequal ? quarters <= most_quarters : d <= 64 && tiles <= 3 * cus && longest >= 16))
     n = {1, 4, 1};
   else if (d > 64 && rows > 32 && ((pairs <= cus && longest >= (d <= 128 ? 4 : 16)) || (d > 128 && 4 * even <= 3 * cus && longest >= 24)))
-    n = {2, 4, 1};
+    n = {2, 4, 1, d <= 128 ? 2 : 1};
   else if (longest >= 2 ? no_more_rounds || few_pairs || three_a_cu : one_block)
     n = {2, 2, 1, d == 32 || (d == 64 && longest >= (unequal ? 8 : 16) && pairs <= 3 * cus) ||
                           (d > 64 && d <= 128 && longest >= 8 && (pairs <= 2 * cus || unequal_pairs)) ? 2 : 1};
@@ -1274,6 +1274,16 @@ extern "C" int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* 
   *rows_per_workgroup = 32 * n.tiles_per_workgroup;
   *wavefronts_per_tile = n.waves_per_tile;
   *kv_splits = n.splits;
+  return FA8_OK;
+}
+
+extern "C" int fa8_fwd_form(const Fa8FwdParams* p, int with_workspace, int32_t* lds_stages, int32_t* kernels) {
+  const int rc = fa8_fwd_validate(p);
+  if (rc != FA8_OK) return rc;
+  if (lds_stages == nullptr || kernels == nullptr) return FA8_ERR_NULL;
+  const Plan n = choose_plan(p, with_workspace != 0);
+  *lds_stages = n.waves_per_tile > 1 && n.splits == 1 ? n.stages : 0;
+  *kernels = n.splits > 1 && !split_form(p, n.splits).one_kernel ? 2 : 1;
   return FA8_OK;
 }
 

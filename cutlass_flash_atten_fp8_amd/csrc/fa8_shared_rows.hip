@@ -13,16 +13,16 @@ const void* pick(bool e5m2, bool vt) {
 }
 template <int D>
 const void* pick_rw(int r, int w, int stages, bool e5m2, bool vt) {
-  constexpr int S = D > 128 ? 1 : 2;
-  // see choose_plan for the stages; head dim 32 has no use for one with (2, 2) (1.0 - 1.2)
-  if constexpr (D <= 128)
+  // what choose_plan takes; head dim 32 has no use for one stage with (2, 2) (1.0 - 1.2)
+  if (r == 1 && w == 4 && stages == 1) return pick<D, 1, 4, 1>(e5m2, vt);
+  if constexpr (D <= 128) {
     if (r == 1 && w == 4 && stages == 2) return pick<D, 1, 4, 2>(e5m2, vt);
-  if (r == 1 && w == 4) return pick<D, 1, 4, 1>(e5m2, vt);
-  if constexpr (D > 32 && D <= 128)
+    if (r == 2 && w == 2 && stages == 2) return pick<D, 2, 2, 2>(e5m2, vt);
+  }
+  if constexpr (D > 32)
     if (r == 2 && w == 2 && stages == 1) return pick<D, 2, 2, 1>(e5m2, vt);
-  if (r == 2 && w == 2) return pick<D, 2, 2, S>(e5m2, vt);
   if constexpr (D > 64)
-    if (r == 2 && w == 4) return pick<D, 2, 4, S>(e5m2, vt);
+    if (r == 2 && w == 4 && stages == (D <= 128 ? 2 : 1)) return pick<D, 2, 4, D <= 128 ? 2 : 1>(e5m2, vt);
   return nullptr;
 }
 

@@ -153,6 +153,12 @@ int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* rows_per_wo
                  int32_t* kv_splits);
 
 /*
+ * More of the same (library version 6): the LDS stages of shared rows (1 or 2; 0: the call does not share rows or splits its keys), and the
+ * kernels that the call launches (1; 2 where the logits of split keys do not fit in LDS).
+ */
+int fa8_fwd_form(const Fa8FwdParams* p, int with_workspace, int32_t* lds_stages, int32_t* kernels);
+
+/*
  * Which main loop a wavefront that has its 32 query rows to itself would run for these arguments on the current device:
  * FA8_SCHEDULE_ROLLING, FA8_SCHEDULE_PIPELINED or FA8_SCHEDULE_DENSE (all > 0), or the FA8_ERR_* code fa8_fwd_validate gives; whether
  * the call has such wavefronts, fa8_fwd_plan tells.  Launches nothing.  No counterpart in the reference (one kernel, one loop:

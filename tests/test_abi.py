@@ -34,7 +34,7 @@ def test_library_exports_every_declared_symbol():
 
 
 def test_library_version_tells_of_the_workspace_entry_points():
-    assert fa.query(fa.FA8_QUERY_VERSION) >= 5  # fa8_fwd_workspace, fa8_fwd_ws, fa8_fwd_plan; from 6 on fa8_fwd_ws_late
+    assert fa.query(fa.FA8_QUERY_VERSION) >= 5  # fa8_fwd_workspace, fa8_fwd_ws, fa8_fwd_plan; from 6 on fa8_fwd_form, fa8_fwd_ws_late
 
 
 def test_query_values():

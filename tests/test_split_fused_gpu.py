@@ -26,7 +26,7 @@ CASES = [
 def call(q, k, v, o, causal, vt=False, lse=None, late=0):
     """One call through fa8_fwd_ws_late on a workspace of the size asked for."""
     p = fa.make_params(q, k, v, o, causal, q.shape[3] ** -0.5, vt, lse, True)
-    assert fa.plan(p)[2] > 1
+    assert fa.plan(p)[2] > 1 and fa.form(p) == (0, 1)
     need = ctypes.c_int64()
     assert fa.lib().fa8_fwd_workspace(ctypes.byref(p), ctypes.byref(need)) == 0
     ws = torch.empty(need.value, dtype=torch.uint8, device=DEV)
@@ -80,6 +80,7 @@ def test_a_workspace_with_the_state_of_earlier_calls():
         o = torch.full(q.shape, float("nan"), dtype=torch.float16, device=DEV)
         p = fa.make_params(q, k, v, o, True, 0.09, causal_bottom_right=True)
         need = ctypes.c_int64()
+        assert fa.form(p) == (0, 1)
         assert fa.lib().fa8_fwd_workspace(ctypes.byref(p), ctypes.byref(need)) == 0 and 0 < need.value <= ws.numel()
         assert fa.lib().fa8_fwd_ws(ctypes.byref(p), ws.data_ptr(), need.value, stream) == 0
         torch.cuda.synchronize()
@@ -88,8 +89,8 @@ def test_a_workspace_with_the_state_of_earlier_calls():
 
 @pytest.mark.parametrize("group", [1, 4, 8, 16, 32])
 @pytest.mark.parametrize("d", [64, 128, 256])
-def test_ranges_up_to_the_two_kernel_form(d, group):
-    """One to about thirty blocks a wavefront; the logits of the longer ones do not fit in LDS."""
+def test_ranges_of_many_lengths(d, group):
+    """One to fifteen blocks a wavefront, in one kernel and, where the logits of many rows do not fit in LDS, in two."""
     for nk in (4096, 9000, 30011, 120001):
         q, k, v = _inputs(nk + group, 1, group, 1, 1, nk, d, E4)
         if 2 * nk * d > 40e6:
@@ -97,6 +98,21 @@ def test_ranges_up_to_the_two_kernel_form(d, group):
         want = fa.flash_attention_v2_cutlass(q, k, v, True, d ** -0.5, causal_bottom_right=True, schedule=fa.FA8_SCHEDULE_ROLLING)[0]
         got = fa.flash_attention_v2_cutlass(q, k, v, True, d ** -0.5, causal_bottom_right=True)[0]
         torch.cuda.synchronize()
+        assert fa.plan(fa.make_params(q, k, v, got, True, d ** -0.5, causal_bottom_right=True))[2] > 1
+        assert_same_up_to_sum_order(got, want, v, nk)
+
+
+# the blocks of a wavefront whose logits just fit in LDS, for head dim and rows
+@pytest.mark.parametrize("d,rows,fit", [(32, 16, 8), (64, 8, 15), (96, 16, 5), (128, 4, 23), (160, 8, 3), (256, 4, 7)])
+def test_the_longest_ranges_of_one_kernel(d, rows, fit):
+    """32 parts of four ranges that are all as long as fits, the last one a key shorter, and one block more, which takes two kernels."""
+    for nk, kernels in ((32 * 4 * fit * 64 - 1, 1), (32 * 4 * fit * 64 + 1, 2)):
+        q, k, v = _inputs(nk + rows, 1, rows, 1, 1, nk, d, E4)
+        want = fa.flash_attention_v2_cutlass(q, k, v, True, d ** -0.5, causal_bottom_right=True, schedule=fa.FA8_SCHEDULE_ROLLING)[0]
+        got = fa.flash_attention_v2_cutlass(q, k, v, True, d ** -0.5, causal_bottom_right=True)[0]
+        torch.cuda.synchronize()
+        p = fa.make_params(q, k, v, got, True, d ** -0.5, causal_bottom_right=True)
+        assert fa.plan(p)[2] > 1 and fa.form(p) == (0, kernels)
         assert_same_up_to_sum_order(got, want, v, nk)
 
 
