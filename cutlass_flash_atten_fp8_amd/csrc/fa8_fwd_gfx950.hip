@@ -963,10 +963,10 @@ int compute_units() {
 // elsewhere every hint is ignored and the rolling loop runs.
 // Dense: full (non-causal) attention.  Over a whole number of KV blocks no logit is ever masked: measured 1 - 2 % faster than the rolling
 // loop on launches that fill the chip and 3 - 5 % faster than the pipelined loop on small ones, so it is the choice wherever it applies.
-// Over keys that end inside a block (kLoopDenseRagged) head dim 128, new / old time: 0.90 - 0.95 where the pipelined loop ran (2 sequences,
-// 16 heads, 2999 keys 96.0 -> 91.8 us; 8, 40, 777: 102 -> 92), 0.97 - 0.98 where the rolling one did (2, 32, 4097: 346 -> 336); head dim 64
-// 0.95 - 0.99 above three workgroups a compute unit, 1.00 - 1.02 below, where the pipelined loop stays.  A hint for the dense loop
-// that does not apply falls back to the automatic choice.
+// Over keys that end inside a block (kLoopDenseRagged) head dim 128, new / old time: 0.87 - 0.98 where the pipelined loop ran (2 sequences,
+// 16 heads, 2999 keys 96.0 -> 91.8 us; 8, 40, 777: 102 -> 92), 0.90 - 1.0 where the rolling one did (2, 32, 4097: 346 -> 336), 1.01 - 1.04 up to
+// one workgroup a compute unit (1, 4, 8096: 93.7 -> 96.6), where the pipelined loop stays; head dim 64 0.91 - 1.0 above three workgroups a compute
+// unit, 1.00 - 1.02 below, where it stays too.  A hint for the dense loop under a mask falls back to the automatic choice.
 // Pipelined: launches that cannot keep three wavefronts on every SIMD for most of their run: at most four workgroups per
 // compute unit (two resident at a time), or little work per compute unit (then filling and draining the chip, and for
 // causal launches the thinning out of the workgroups, is a large share of the run).  Measured 5 - 15 % faster than the
@@ -974,10 +974,10 @@ int compute_units() {
 int choose_loop(const Fa8FwdParams* p) {
   if ((p->head_dim != 64 && p->head_dim != 128) || !(p->softmax_scale > 0.f && p->softmax_scale < 1.0e6f)) return FA8_SCHEDULE_ROLLING;
   if (p->schedule == FA8_SCHEDULE_ROLLING || p->schedule == FA8_SCHEDULE_PIPELINED) return p->schedule;
-  if (!p->is_causal && (p->head_dim == 128 || p->seqlen_k % kKvBlock == 0)) return FA8_SCHEDULE_DENSE;
+  if (!p->is_causal && (p->schedule == FA8_SCHEDULE_DENSE || p->seqlen_k % kKvBlock == 0)) return FA8_SCHEDULE_DENSE;
   const long long cus = compute_units();
   const long long wgs = (long long)p->batch * p->heads * ((p->seqlen_q + kQBlock - 1) / kQBlock);
-  if (!p->is_causal && cus > 0 && wgs > 3 * cus) return FA8_SCHEDULE_DENSE;
+  if (!p->is_causal && cus > 0 && wgs > (p->head_dim == 128 ? 1 : 3) * cus) return FA8_SCHEDULE_DENSE;
   // KV blocks per compute unit below which the pipelined loop was measured to win (head dim 64 has half the matrix work
   // per block)
   const long long few_blocks = p->head_dim == 64 ? 264 : 144;

@@ -43,8 +43,8 @@ extern "C" {
  *             so sum in another order (fa8_fwd_plan tells); any hint, and any call without a workspace, keeps the unsplit order
  *   ROLLING   one KV block after the other, three wavefronts per SIMD: for masked launches that fill the chip
  *   PIPELINED software-pipelined over neighbouring KV blocks, two wavefronts per SIMD: for small masked launches
- *   DENSE     the same pipeline in three wavefronts per SIMD, for full (non-causal) attention: head dim 128, or seqlen_k a multiple of
- *             64, or more than three workgroups per compute unit; asked for elsewhere, the library chooses as for AUTO
+ *   DENSE     the same pipeline in three wavefronts per SIMD, for full (non-causal) attention; asked for under a mask, the library
+ *             chooses as for AUTO
  *   (PIPELINED and DENSE are built for head dims 64 and 128 and a softmax scale in (0, 1e6); ignored elsewhere) */
 #define FA8_SCHEDULE_AUTO 0
 #define FA8_SCHEDULE_ROLLING 1

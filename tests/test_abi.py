@@ -220,10 +220,11 @@ def test_schedule_query_follows_explicit_hints_without_a_gpu():
         q, k, v, o = cpu_tensors(d=d)
         p = fa.make_params(q, k, v, o, True, scale, schedule=hint)
         assert sched(ctypes.byref(p)) == want, (d, scale, hint)
-    # the dense loop: full attention, head dim 128 or seqlen_k a multiple of the KV block, positive scale; chosen without a hint
+    # the dense loop: full attention, head dim 64 / 128, positive scale; chosen without a hint where seqlen_k is a multiple of the KV block
     for d, n, scale, hint, want in ((128, 128, 0.1, fa.FA8_SCHEDULE_AUTO, fa.FA8_SCHEDULE_DENSE),
                                     (64, 64, 0.1, fa.FA8_SCHEDULE_DENSE, fa.FA8_SCHEDULE_DENSE),
-                                    (128, 65, 0.1, fa.FA8_SCHEDULE_AUTO, fa.FA8_SCHEDULE_DENSE),
+                                    (128, 65, 0.1, fa.FA8_SCHEDULE_DENSE, fa.FA8_SCHEDULE_DENSE),
+                                    (64, 65, 0.1, fa.FA8_SCHEDULE_DENSE, fa.FA8_SCHEDULE_DENSE),
                                     (128, 1, 0.1, fa.FA8_SCHEDULE_DENSE, fa.FA8_SCHEDULE_DENSE),
                                     (128, 65, 0.1, fa.FA8_SCHEDULE_ROLLING, fa.FA8_SCHEDULE_ROLLING),
                                     (96, 65, 0.1, fa.FA8_SCHEDULE_DENSE, fa.FA8_SCHEDULE_ROLLING),

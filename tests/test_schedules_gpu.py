@@ -2,8 +2,7 @@
 arithmetic in the same order: their outputs must be bitwise equal, for every feature of the operator.  The parity of the
 result itself is the business of the parity tests; they reach the dense loop through the library's own choice (full
 attention), the pipelined loop through small masked launches and the rolling loop through the large
-causal configurations.  A dense hint that does not apply (causal; ragged seqlen_k in a small launch of head dim 64) is answered with
-the automatic choice, so asking for it is always valid."""
+causal configurations.  A dense hint under a causal mask is answered with the automatic choice, so asking for it is always valid."""
 import numpy as np
 import pytest
 import torch
@@ -99,8 +98,8 @@ def test_non_positive_scale_and_other_head_dims_ignore_the_hint():
 
 
 def test_library_choice_by_launch_size():
-    """fa8_fwd_schedule on a GPU: full attention takes the dense loop (over keys that end inside a block only head dim 128, and 64 above
-    three workgroups a compute unit); of the others, small launches take the pipelined loop and launches that fill the chip the rolling one."""
+    """fa8_fwd_schedule on a GPU: full attention takes the dense loop (over keys that end inside a block only above one workgroup
+    a compute unit, head dim 64 three); of the others, small launches take the pipelined loop and launches that fill the chip the rolling one."""
     import ctypes
 
     def plan(B, H, N, d, causal):
@@ -115,6 +114,7 @@ def test_library_choice_by_launch_size():
     assert plan(2, 32, 4096, 128, False) == fa.FA8_SCHEDULE_DENSE         # the headline shape
     assert plan(2, 32, 4097, 128, False) == fa.FA8_SCHEDULE_DENSE         # ... with a ragged last block
     assert plan(2, 16, 2999, 128, False) == fa.FA8_SCHEDULE_DENSE
+    assert plan(1, 4, 8096, 128, False) == fa.FA8_SCHEDULE_PIPELINED      # 256 workgroups with a ragged last block
     assert plan(8, 16, 1000, 64, False) == fa.FA8_SCHEDULE_DENSE          # 1024 workgroups with a ragged last block
     assert plan(6, 16, 1000, 64, False) == fa.FA8_SCHEDULE_PIPELINED      # 768, three a compute unit
     assert plan(1, 32, 8192, 128, True) == fa.FA8_SCHEDULE_ROLLING        # cfg4
