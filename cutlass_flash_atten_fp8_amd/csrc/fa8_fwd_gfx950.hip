@@ -1029,7 +1029,8 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 //     two (head dim 64) and 0.82 - 0.95 (96, 128); where there are fewer, 0.97 below 16 (8) blocks, 1.0 - 1.03 above, where two stay
 //     (head dim 64, tiles of unequal length: from 8 blocks on; 40 heads, 704 keys: 9.0 us with two, 9.7 - 10.0 with one)
 //     (head dims 96, 128, tiles of unequal length: 17 blocks up to 2.4 pairs a CU and even <= 5/4 CUs, 24 blocks 7/5 CUs, 28 blocks 2.5 pairs; one
-//     stage takes 1.02 - 1.13 there, 0.9 - 0.93 beyond)
+//     stage takes 1.02 - 1.13 there, 0.9 - 0.93 beyond; a pair a k/v head, 10 blocks: also the 3 - 4 pairs a CU that take two rounds either way,
+//     1.02 - 1.13: 1024 heads, 2097 keys, head dim 96, 80.8 us with two, 91.7 with one)
 //   head dim 65 - 128, 8 blocks, more than two pairs a CU and up to the three that one stage lets run at once (causal, 16 blocks: 3.5, if
 //     even <= 2 CUs): two wavefronts a tile, two tiles, though the unshared launch has fewer rounds (median 0.92, 0.82 - 1.0; beyond 1.02 - 1.4,
 //     as with a mask aligned to the last key: 64 heads, 895 queries on 1841 keys, even 2.7 CUs, head dim 128: 36.9 us, 43.0 shared)
@@ -1080,6 +1081,7 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
                           (pairs <= 3 * cus || (unequal && longest >= 16 && 2 * pairs <= 7 * cus && even <= 2 * cus));
   const bool unequal_pairs = unequal && (longest >= 24 ? 5 * even <= 7 * cus : longest >= 17 && 4 * even <= 5 * cus) &&
                              (longest >= 28 ? 2 * pairs < 5 * cus : 5 * pairs <= 12 * cus);
+  const bool two_rounds = rows <= 64 && longest >= 10 && pairs > 3 * cus && pairs <= 4 * cus;
   const bool one_block = (2 * pairs <= wgs && wgs > 2 * cus) || (d == 32 && p->is_causal && p->v_layout == FA8_V_ROWS && pairs <= wgs);
   // one tile a workgroup, two LDS stages: they run at once, or in no more rounds than with one stage; and K and V come from memory for a tile or two
   const bool two_fit = d <= 128 && (tiles <= (d <= 64 ? 2 : 1) * cus || (d <= 64 && longest >= 24 && tiles > 3 * cus && tiles <= 4 * cus));
@@ -1095,7 +1097,7 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
     n = {2, 4, 1, d <= 128 ? 2 : 1};
   else if (longest >= 2 ? no_more_rounds || few_pairs || three_a_cu : one_block)
     n = {2, 2, 1, d == 32 || (d == 64 && longest >= (unequal ? 8 : 16) && pairs <= 3 * cus) ||
-                          (d > 64 && d <= 128 && longest >= 8 && (pairs <= 2 * cus || unequal_pairs)) ? 2 : 1};
+                          (d > 64 && d <= 128 && longest >= 8 && (pairs <= 2 * cus || unequal_pairs || two_rounds)) ? 2 : 1};
   if (workspace && n.waves_per_tile == 4 && n.tiles_per_workgroup == 1 && longest >= (d <= 128 ? 20 : 16)) {
     const long long most = std::max(1LL, std::min({32LL, cus / tiles, longest / 4}));  // one workgroup more than CUs takes twice as long
     const SplitForm form = split_form(p, (int)most);

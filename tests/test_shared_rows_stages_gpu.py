@@ -48,6 +48,8 @@ TWO_TILES = [
     (1, 20, 20, 2496, 2496, 96, True, False, True, E4, True, 1),     # 780, 39 blocks
     (1, 32, 32, 1152, 1152, 128, True, False, False, E4, False, 2),  # 576 of unequal length, 18 blocks
     (1, 32, 32, 1094, 1786, 128, True, True, False, E5, False, 1),   # the work of 1.6 a compute unit
+    (32, 32, 32, 1, 640, 128, True, True, False, E4, False, 2),      # 1024 heads, 10 blocks
+    (32, 32, 32, 2, 576, 96, True, True, True, E5, True, 1),         # 9
     (8, 32, 8, 180, 600, 128, False, False, False, E5, False, 1),    # 768 with the rows of four q heads together: three a compute unit
     (8, 32, 8, 180, 600, 128, True, True, False, E4, False, 1),
 ]
