@@ -995,7 +995,7 @@ struct Plan {
 constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask for
 
 // The rule, from 18 500 shapes drawn over all head dims, 1 - 10000 row tiles, 1 - 20000 keys, full and causal, grouped or not, every plan
-// timed on every shape.  A SIMD with one wavefront issues a vector instruction every 6 - 9 cycles, with three every 3: a launch of few
+// timed on every shape, and 9000 of `draw` in perf/cases.py.  A SIMD with one wavefront issues a vector instruction every 6 - 9 cycles, with three every 3: a launch of few
 // rows is faster if several wavefronts share a row tile, up to the point where the unshared loops have about two wavefronts on every
 // SIMD themselves; from there on sharing costs (a launch that fills the chip: 1.1 - 1.6x with two wavefronts a tile, 1.5 - 4x with
 // four), unless the unshared launch, whose workgroups have 128 rows of one q head each, would be mostly idle.  `tiles` counts 32-row
@@ -1012,9 +1012,10 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 //   LDS stages of one tile, four wavefronts: with one workgroup a CU (head dim <= 64: two) one stage takes 0.94 - 0.98 of the time of two below 16
 //     blocks, the same at 16 - 24, 1.0 - 1.3 above (head dim 32: 0.98 at every length).  Where K and V come from memory for a tile or two alone
 //     (decode steps), it takes more from fewer blocks on: head dims 96, 128 1.01 - 1.25 from 4 blocks a CU (of all k/v heads together), head dim 64 1.03 -
-//     1.08 from 12 with a tile a CU at most (0.95 - 1.0 with more, below 24 blocks a head), head dim 32 1.07 - 1.26 from 32 (more than two tiles a k/v head: 64; 192 heads, 42244 keys, head dim 32: 177 us with two, 223 with one; 128 heads, 1457
-//     keys, head dim 128: 13.7, 17.2).  Two stages of head dim 128 have no room for a second workgroup (0.7 - 0.8), of 64 and 32 for a third
-//     (0.8 - 0.88, up to the 4 a CU that take two rounds either way: 1.02 - 1.13 from 24 blocks)
+//     1.08 from 12 with a tile a CU at most (0.95 - 1.0 with more, below 24 blocks a head), head dim 32 1.07 - 1.26 from 32 (more than two tiles a
+//     k/v head: 64).  192 heads, 42244 keys, head dim 32: 176 us with two, 222 with one; 128 heads, 1457 keys, head dim 128: 13.4, 16.9.  Two
+//     stages of head dim 128 have no room for a second workgroup (0.7 - 0.8), of 64 and 32 for a third (0.8 - 0.88, up to the 4 a CU that take
+//     two rounds either way: 1.02 - 1.13 from 24 blocks)
 //   head dim 65 - 128, pairs <= CUs (one a CU) and 4 blocks: four wavefronts a tile, two tiles a workgroup, which share the copies of K
 //     and V (0.6 - 0.85)
 //   head dim above 128: the same from 16 blocks on (one LDS stage; 1.0 - 1.1 at 6 - 12 blocks, 0.95 at 16 - 24, 0.86 from 64 on, against two

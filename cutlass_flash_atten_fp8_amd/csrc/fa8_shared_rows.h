@@ -12,10 +12,9 @@
 //   chunks, copy of K two groups ahead | barrier 2 | weights of sub-tile 1, S^T products of the next group between their chunks, copy of
 //   V of the next group; weights and row sums -> LDS
 // One stage (STAGES == 1): the copies of the next group's K and this group's V fly for half an iteration.  Head dims above 128 have LDS for no more;
-// one tile a workgroup takes it so that two or three workgroups fit on a compute unit, each with barriers of its own: the one works
-// while the other waits (16 heads, 1024 keys, head dim 128, causal: 12.98 us with two tiles a workgroup, 11.73 so; 12, 1000: 12.4, 11.3).
-// Likewise two tiles, two wavefronts a tile: four workgroups of head dim 64 a compute unit instead of three, three of 96 and 128 instead of two (45
-// heads, 705 keys, head dim 128, full: 22.8 us with two stages, 19.9 with one; 104, 320, head dim 96, causal: 10.6, 8.6).
+// up to 128 it lets two to four workgroups share a compute unit, each with barriers of its own: the one works while the other waits (16
+// heads, 1024 keys, head dim 128, causal: 12.98 us with two tiles a workgroup, 11.73 with one and one stage).  Half an iteration is too short a
+// flight where K and V come from memory for a tile or two alone.  choose_plan has the lines between the two and both sides of each.
 //
 // What bounds it: the one or two wavefronts of a SIMD walk one chain (row max - LDS - barrier - weights - LDS - barrier), about 310
 // instructions a wavefront and iteration, each 5 cycles or more apart within a wavefront whatever its kind; 3500 cycles at R = 2, W = 4.

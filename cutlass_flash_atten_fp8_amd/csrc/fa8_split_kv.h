@@ -12,14 +12,15 @@
 // the chip it stops waiting after a number of looks and forms the maxima that have not come itself.  Where the logits do not fit, one kernel each.
 // Logits, weights and products are those of the other kernels bit for bit; only the order of the fp32 sums over the ranges is another.
 //
-// Bound: HBM bytes.  K and V are read once; S costs 8 bytes per row and key against 2 * head_dim bytes per key for K and V, which is why
-// the logits are kept instead of read K again (head dim 128: fewer bytes up to 16 rows a tile, and S comes out of the Infinity
-// Cache).  Every wavefront has its own LDS ring, so there is no barrier in either loop.  The rest is latency: two launches, a first
-// memory access in each (kernel arguments and data, 2 us), the parts' way to the last workgroup (stores, a counter, loads: 3 us, with
-// all loads of a step under way together; one by one they took 8).  Measured, 1 query of 32 heads on 8 k/v heads, head dim 128: 32768
-// keys 309 us (one wavefront a head) / 151 (shared rows, no split) / 21.7 (two kernels, of that 8 logits and 12 values) -> 18.8 us (13 us at
-// the rate of a plain copy); 4 sequences of 32768 keys 71.3 (two kernels) -> 55.4, of 4096 keys 23 (shared rows) / 15.9 -> 13.9; 4 queries,
-// 16384 keys 22.7 -> 18.1; 2 sequences of 60000 keys, 8 k/v heads, head dim 64: 39.8 -> 29.5.
+// Bound: HBM bytes.  K and V are read once; in two kernels S costs 8 bytes per row and key against 2 * head_dim bytes per key for K and V,
+// which is why the logits are kept instead of read K again (head dim 128: fewer bytes up to 16 rows a tile, and S comes out of the Infinity
+// Cache).  Every wavefront has its own LDS ring, so there is no barrier in either loop.  The rest is latency: a launch and a first memory
+// access (kernel arguments and data, 2 us), both twice in two kernels, the exchange of the maxima in one, and the parts' way to the last
+// workgroup (stores, a counter, loads: 3 us, with all loads of a step under way together; one by one they took 8).  Measured among other
+// calls, inputs rotating, 1 query of 32 heads on 8 k/v heads, head dim 128: 32768 keys 309 us (one wavefront a head) / 151 (shared rows, no
+// split) / 20.7 (two kernels, of that 8 logits and 12 values) -> 17.9 us (13 us at the rate of a plain copy).  In a loop of single calls: 4
+// sequences of 32768 keys 71.3 (two kernels) -> 55.4, of 4096 keys 23 (shared rows) / 15.9 -> 13.9; 4 queries, 16384 keys 22.7 -> 18.1; 2
+// sequences of 60000 keys, 8 k/v heads, head dim 64: 39.8 -> 29.5.
 #ifndef FA8_SPLIT_KV_H_
 #define FA8_SPLIT_KV_H_
 #include <type_traits>
@@ -592,8 +593,8 @@ struct SplitFusedArgs {
   unsigned lse_bs, lse_hs;
   unsigned late;  // splits (a bit each) that do not hand on their maximum, for tests
 };
-// LDS bytes for the logits of the four ranges: what the ring of two tiles a wavefront leaves of 160 KB.  (Rings of three and four: 20.3 and
-// 20.6 us for 32768 keys of 8 k/v heads instead of 18.8, head dim 64 1 - 3 % slower: ranges are rounded up to whole rounds of the ring, and
+// Most LDS bytes for the logits of the four ranges: what the ring of two tiles a wavefront leaves of 160 KB.  (Rings of three and four: 20.3
+// and 20.6 us for 32768 keys of 8 k/v heads instead of 18.8 in a loop of single calls, head dim 64 1 - 3 % slower: ranges are rounded up to whole rounds of the ring, and
 // the logits have less room.)
 constexpr int split_fused_s_bytes(int d) {
   const int dp = d <= 32 ? 32 : (d <= 64 ? 64 : (d <= 128 ? 128 : 256));
