@@ -27,10 +27,11 @@ FA8_OUT_FP16, FA8_OUT_E4M3, FA8_OUT_E5M2 = 0, 1, 2
 FA8_V_ROWS, FA8_V_TRANSPOSED = 0, 1
 FA8_CAUSAL_TOP_LEFT, FA8_CAUSAL_BOTTOM_RIGHT = 0, 1
 FA8_SCHEDULE_AUTO, FA8_SCHEDULE_ROLLING, FA8_SCHEDULE_PIPELINED, FA8_SCHEDULE_DENSE = 0, 1, 2, 3
+FA8_PLAN_ANY_ORDER = 2  # with_workspace of plan and form: what fa8_fwd_any_order (and both bindings) would run
 (FA8_QUERY_VERSION, FA8_QUERY_KV_BLOCK, FA8_QUERY_Q_BLOCK, FA8_QUERY_KV_ASCENDING, FA8_QUERY_THREADS,
  FA8_QUERY_PARAMS_SIZE) = range(6)
-FA8_EXPORTS = ("fa8_fwd_validate", "fa8_fwd", "fa8_fwd_workspace", "fa8_fwd_ws", "fa8_fwd_ws_late", "fa8_fwd_plan", "fa8_fwd_form",
-               "fa8_fwd_schedule", "fa8_query", "fa8_error_string")
+FA8_EXPORTS = ("fa8_fwd_validate", "fa8_fwd", "fa8_fwd_workspace", "fa8_fwd_ws", "fa8_fwd_any_order", "fa8_fwd_apart", "fa8_fwd_ws_late",
+               "fa8_fwd_plan", "fa8_fwd_form", "fa8_fwd_schedule", "fa8_query", "fa8_error_string")
 
 
 class Fa8FwdParams(ctypes.Structure):
@@ -72,6 +73,10 @@ def lib():
         L.fa8_fwd_ws.restype = ctypes.c_int
         L.fa8_fwd_ws.argtypes = [ctypes.POINTER(Fa8FwdParams), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
         L.fa8_fwd_ws_late.restype = ctypes.c_int
+        L.fa8_fwd_any_order.restype = ctypes.c_int
+        L.fa8_fwd_any_order.argtypes = L.fa8_fwd_ws.argtypes
+        L.fa8_fwd_apart.restype = ctypes.c_int
+        L.fa8_fwd_apart.argtypes = [ctypes.POINTER(Fa8FwdParams)]
         L.fa8_fwd_ws_late.argtypes = [ctypes.POINTER(Fa8FwdParams), ctypes.c_void_p, ctypes.c_int64, ctypes.c_uint32, ctypes.c_void_p]
         L.fa8_fwd_plan.restype = ctypes.c_int
         L.fa8_fwd_plan.argtypes = [ctypes.POINTER(Fa8FwdParams), ctypes.c_int] + [ctypes.POINTER(ctypes.c_int32)] * 3
@@ -179,7 +184,7 @@ def flash_attention_v2_cutlass(q, k, v, is_causal, softmax_scale, *, v_transpose
     Beyond the reference: k/v may have fewer heads than q (grouped-query attention), return_lse=True returns
     [O, lse] with lse the float32 [B,H,Nq] log-sum-exp of the scaled logits, causal_bottom_right=True aligns the
     causal diagonal with the last key when seqlen_q != seqlen_k; schedule (FA8_SCHEDULE_*) is a performance hint: 0 lets the
-    library choose, and is the only value with which it may split the keys of a few query rows (other order of the fp32 sums).
+    library choose, and is the only value with which it may split the keys of a row over workgroups or wavefronts (other order of the fp32 sums).
     """
     import torch
     for name, t in (("q", q), ("k", k), ("v", v)):
@@ -215,7 +220,7 @@ def flash_attention_v2_cutlass(q, k, v, is_causal, softmax_scale, *, v_transpose
                     workspace = torch.empty(need.value, dtype=torch.uint8, device=q.device)
                 except torch.OutOfMemoryError:  # the call needs none, it only takes longer
                     pass
-            rc = lib().fa8_fwd_ws(ctypes.byref(p), None if workspace is None else workspace.data_ptr(), need.value, ctypes.c_void_p(stream))
+            rc = lib().fa8_fwd_any_order(ctypes.byref(p), None if workspace is None else workspace.data_ptr(), need.value, ctypes.c_void_p(stream))
     if rc != 0:
         raise RuntimeError(f"flash_attention_v2_cutlass: {error_string(rc)} (code {rc})")
     return [o, lse] if return_lse else [o]

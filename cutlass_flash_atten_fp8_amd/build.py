@@ -21,7 +21,7 @@ LIBFA8 = os.path.join(PKG_DIR, "libfa8.so")
 EXT_NAME = "attention_cutlass_fp8"
 EXT_PATH = os.path.join(PKG_DIR, EXT_NAME + sysconfig.get_config_var("EXT_SUFFIX"))
 
-KERNEL_SOURCES = [os.path.join(CSRC, f) for f in ("fa8_fwd_gfx950.hip", "fa8_shared_rows.hip", "fa8_split_kv.hip")]
+KERNEL_SOURCES = [os.path.join(CSRC, f) for f in ("fa8_fwd_gfx950.hip", "fa8_shared_rows.hip", "fa8_apart_rows.hip", "fa8_split_kv.hip")]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

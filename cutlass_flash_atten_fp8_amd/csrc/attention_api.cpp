@@ -120,7 +120,8 @@ Outputs flash_attention_v2_cutlass(const torch::Tensor& q, const torch::Tensor& 
       } catch (const c10::OutOfMemoryError&) {  // the call needs none, it only takes longer
       }
     }
-    rc = workspace.defined() ? fa8_fwd_ws(&p, workspace.data_ptr(), workspace_bytes, (void*)stream) : fa8_fwd(&p, (void*)stream);
+    rc = workspace.defined() ? fa8_fwd_any_order(&p, workspace.data_ptr(), workspace_bytes, (void*)stream)
+                             : fa8_fwd_any_order(&p, nullptr, 0, (void*)stream);
   }
   TORCH_CHECK(rc == FA8_OK, "flash_attention_v2_cutlass: ", fa8_error_string(rc), " (code ", rc, ")");
   return {out, lse};

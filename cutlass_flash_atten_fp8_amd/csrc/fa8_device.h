@@ -22,7 +22,7 @@ constexpr int kQBlock = 128;   // query rows per workgroup
 constexpr int kQWave = 32;     // query rows per wavefront
 constexpr int kKvBlock = 64;   // kv rows per online-softmax step
 constexpr int kThreads = 256;  // 4 wavefronts
-constexpr int kVersion = 6;
+constexpr int kVersion = 7;
 // main loops (template parameter LOOP of the kernel)
 constexpr int kLoopRolling = 0, kLoopPipelined = 1, kLoopDense = 2, kLoopDenseRagged = 3;
 

@@ -991,6 +991,7 @@ struct Plan {
   int waves_per_tile;       // 1: the loops of this file; 2, 4: wavefronts share a row tile
   int splits;               // > 1: the keys of a row tile dealt to this many workgroups (needs a workspace)
   int stages = 1;           // LDS stages of sharing wavefronts
+  bool apart = false;       // sharing wavefronts each keep the sums of their own blocks
 };
 constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask for
 
@@ -1051,7 +1052,43 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 // split (4 heads, 974 keys, head dim 128: 8.8 us, 9.9 in four parts; 16 - 19 blocks 1.03 - 1.11).  One head, 32
 // queries on 1121 keys, d128: 10.0 us shared, 19.3 split; one sequence of 32768 keys: 151 and 18; 2 sequences of 6881 keys, 8 queries of 3 k/v heads,
 // group of 4, d128: 25.2 in 13 parts, 16.1 in 27.
-Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
+// Sums apart (fa8_shared_rows_kernel with APART, head dims up to 128), where the caller leaves the order of the sums open: it replaces what the rules above
+// give from the number of blocks on where its groups, with half the exchange, repay a longer start and the sum of the parts at the end.  24 000 drawn
+// launches, K and V from HBM, median and 95th percentile of its time / theirs:
+//   four wavefronts a tile, one tile: head dim 32 0.80, 0.96 and 64 0.85, 0.97 from 12 blocks on, up to two tiles a CU (below 12: 0.97 - 1.02; up to three a
+//     CU 0.79 - 0.88 at head dim 32, 0.93 from 48 blocks on at 64, unless a k/v head has few rows and its bytes bound both: 1.1 - 1.3); head dim 96 0.89,
+//     0.98 from 12 blocks and 128 0.94, 1.0 from 20 on, up to a tile a CU and more than one tile a k/v head (one: 0.98 - 1.05, bytes)
+//   four wavefronts a tile, two tiles: 0.88, 1.0 (head dim 96, 12 blocks), 0.90, 0.99 (128, 20 blocks)
+//   two wavefronts a tile, two tiles, instead of the same with sums together or of the unshared loops: head dim 32 0.90, 0.97 and 0.80, 0.92 (12 blocks, unequal
+//     tiles 24; up to three pairs a CU); head dim 64 0.94, 0.99 instead of the former alone (16 blocks up to two pairs a CU, 32 up to three); head
+//     dim 96 0.86, 0.95 and 0.87, 0.96 (12 blocks), 128 0.92, 0.98 and 0.90, 1.0 (24 blocks, instead of the unshared loops 32), up to the two pairs a CU that run
+//     at once, k/v heads of more than 128 rows (fewer: up to 1.23, bytes); unequal tiles, 48 blocks: up to three pairs (head dim 32 from 12
+//     blocks eight, 64 five), 0.87 - 0.93
+void keep_sums_apart(const Fa8FwdParams* p, long long cus, long long rows, long long tiles, long long pairs, long long longest, bool unequal, Plan& n) {
+  const int d = p->head_dim;
+  if (n.splits > 1 || d > 128 || d % 32 != 0) return;
+  const bool many_rows = rows > 128;
+  bool apart;
+  if (n.waves_per_tile == 4 && n.tiles_per_workgroup == 1) {
+    apart = d <= 64 ? longest >= 12 && (tiles <= 2 * cus || (tiles <= 3 * cus && many_rows && (d == 32 || longest >= 48)))
+                    : longest >= (d == 96 ? 12 : 20) && tiles <= cus && rows > 32;
+  } else if (n.waves_per_tile == 4) {
+    apart = longest >= (d == 96 ? 12 : 20);
+  } else {
+    const bool shared = n.waves_per_tile == 2;
+    const long long least = d == 32 ? (unequal ? 24 : 12) : (d == 64 ? (pairs <= 2 * cus ? 16 : 32) : (d == 96 ? 12 : (shared ? 24 : 32)));
+    const long long most_unequal = d == 32 ? 8 : (d == 64 ? 5 : 3);
+    apart = (d != 64 || shared) && longest >= least && pairs <= (d <= 64 ? 3 : 2) * cus && (d == 64 ? rows > 32 : many_rows);
+    apart |= unequal && longest >= (d == 32 ? 24 : 48) && pairs <= most_unequal * cus && many_rows;
+    if (apart) n = {2, 2, 1};
+  }
+  if (apart) {
+    n.stages = 2;
+    n.apart = true;
+  }
+}
+
+Plan choose_plan(const Fa8FwdParams* p, bool workspace, bool any_order) {
   const Plan unshared = {kQBlock / 32, 1, 1};
   // the sharing kernels rely on exp2(-inf * scale) = 0 and a finite start of the row max, like the pipelined loop; a schedule hint
   // asks for a loop of the unshared kernel
@@ -1118,6 +1155,7 @@ Plan choose_plan(const Fa8FwdParams* p, bool workspace) {
         split_workspace(p, (int)splits) <= kMaxWorkspace)
       n.splits = (int)splits;
   }
+  if (any_order) keep_sums_apart(p, cus, rows, tiles, pairs, longest, unequal, n);
   return n;
 }
 
@@ -1235,35 +1273,45 @@ int launch_rows(const Fa8FwdParams* p, hipStream_t stream) {
   }
 }
 
-int run(const Fa8FwdParams* p, void* workspace, long long bytes, unsigned late, hipStream_t stream) {
-  Plan n = choose_plan(p, workspace != nullptr);
-  if (n.splits > 1 && bytes < split_workspace(p, n.splits)) n = choose_plan(p, false);
+int run(const Fa8FwdParams* p, void* workspace, long long bytes, unsigned late, bool any_order, hipStream_t stream) {
+  Plan n = choose_plan(p, workspace != nullptr, any_order);
+  if (n.splits > 1 && bytes < split_workspace(p, n.splits)) n = choose_plan(p, false, any_order);
   if (n.splits > 1) return (uintptr_t)workspace % 16 != 0 ? FA8_ERR_ALIGN : launch_split(p, n.splits, workspace, late, stream);
-  return n.waves_per_tile > 1 ? launch_shared(p, n.tiles_per_workgroup, n.waves_per_tile, n.stages, stream) : launch_rows(p, stream);
+  return n.waves_per_tile > 1 ? launch_shared(p, n.tiles_per_workgroup, n.waves_per_tile, n.stages, n.apart, stream) : launch_rows(p, stream);
 }
 
 }  // namespace
 
 extern "C" int fa8_fwd(const Fa8FwdParams* p, void* hip_stream) {
   const int rc = fa8_fwd_validate(p);
-  return rc != FA8_OK ? rc : run(p, nullptr, 0, 0, (hipStream_t)hip_stream);
+  return rc != FA8_OK ? rc : run(p, nullptr, 0, 0, false, (hipStream_t)hip_stream);
 }
 
 extern "C" int fa8_fwd_ws(const Fa8FwdParams* p, void* workspace, int64_t bytes, void* hip_stream) {
   const int rc = fa8_fwd_validate(p);
-  return rc != FA8_OK ? rc : run(p, workspace, bytes, 0, (hipStream_t)hip_stream);
+  return rc != FA8_OK ? rc : run(p, workspace, bytes, 0, false, (hipStream_t)hip_stream);
 }
 
 extern "C" int fa8_fwd_ws_late(const Fa8FwdParams* p, void* workspace, int64_t bytes, uint32_t late_parts, void* hip_stream) {
   const int rc = fa8_fwd_validate(p);
-  return rc != FA8_OK ? rc : run(p, workspace, bytes, late_parts, (hipStream_t)hip_stream);
+  return rc != FA8_OK ? rc : run(p, workspace, bytes, late_parts, false, (hipStream_t)hip_stream);
+}
+
+extern "C" int fa8_fwd_any_order(const Fa8FwdParams* p, void* workspace, int64_t bytes, void* hip_stream) {
+  const int rc = fa8_fwd_validate(p);
+  return rc != FA8_OK ? rc : run(p, workspace, bytes, 0, true, (hipStream_t)hip_stream);
+}
+
+extern "C" int fa8_fwd_apart(const Fa8FwdParams* p) {
+  const int rc = fa8_fwd_validate(p);
+  return rc != FA8_OK ? rc : (int)choose_plan(p, true, true).apart;
 }
 
 extern "C" int fa8_fwd_workspace(const Fa8FwdParams* p, int64_t* bytes) {
   const int rc = fa8_fwd_validate(p);
   if (rc != FA8_OK) return rc;
   if (bytes == nullptr) return FA8_ERR_NULL;
-  const Plan n = choose_plan(p, true);
+  const Plan n = choose_plan(p, true, false);  // (the same bytes for fa8_fwd_any_order: it changes no call that splits its keys)
   *bytes = n.splits > 1 ? split_workspace(p, n.splits) : 0;
   return FA8_OK;
 }
@@ -1273,7 +1321,7 @@ extern "C" int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* 
   const int rc = fa8_fwd_validate(p);
   if (rc != FA8_OK) return rc;
   if (rows_per_workgroup == nullptr || wavefronts_per_tile == nullptr || kv_splits == nullptr) return FA8_ERR_NULL;
-  const Plan n = choose_plan(p, with_workspace != 0);
+  const Plan n = choose_plan(p, with_workspace != 0, with_workspace == FA8_PLAN_ANY_ORDER);
   *rows_per_workgroup = 32 * n.tiles_per_workgroup;
   *wavefronts_per_tile = n.waves_per_tile;
   *kv_splits = n.splits;
@@ -1284,7 +1332,7 @@ extern "C" int fa8_fwd_form(const Fa8FwdParams* p, int with_workspace, int32_t* 
   const int rc = fa8_fwd_validate(p);
   if (rc != FA8_OK) return rc;
   if (lds_stages == nullptr || kernels == nullptr) return FA8_ERR_NULL;
-  const Plan n = choose_plan(p, with_workspace != 0);
+  const Plan n = choose_plan(p, with_workspace != 0, with_workspace == FA8_PLAN_ANY_ORDER);
   *lds_stages = n.waves_per_tile > 1 && n.splits == 1 ? n.stages : 0;
   *kernels = n.splits > 1 && !split_form(p, n.splits).one_kernel ? 2 : 1;
   return FA8_OK;

@@ -31,6 +31,20 @@
 // Registers: two wavefronts a SIMD leave a lane 256, of which head dims 224 and 256 with two tiles take about 220.  (Transposed v: copies and
 // fragments take their row differences from scalar and immediate offsets; with a register for each, 31 - 42 were once spilled there:
 // 16 heads, 2048 keys, causal 76.4 us instead of 36.8, against 51.7 of the unshared loop.)
+//
+// APART (two LDS stages, head dims up to 128): the wavefronts of a tile exchange row maxima only.  Wavefront w takes every W-th block, its weights against
+// the running max after that block as before, and adds the products to an O and an l of its own, brought to its own running max; at the end the W
+// O's meet in the LDS of K and V and are added in order.  Logits and weights are the same bit for bit, the fp32 sums are taken in another order.
+//   softmax of group g, chunks 0 - 5: S^T products of group g + 1 between them, copy of V of group g; row max of group g + 1 -> LDS | barrier 1 |
+//   O to the max of group g - 1; chunks 6 and 7: PV products of group g - 1 between them, copy of K of group g + 3 | R > 1: barrier 2
+// No weights go through LDS, no wavefront is without a column tile (head dims 32 and 64), every wavefront reads one block of K and V, and the latency of
+// the exchange lies under chunks 6 and 7: without the barriers it takes 0.98 of the time.  What bounds it: the 211 vector instructions of a block (64 of them
+// the rescaling of O, needed in two thirds of the groups, four blocks apart: 5 % of the time) at the rate of two wavefronts a SIMD, and the tile copies
+// (8 KB a block and wavefront, twice the unshared loops': 10 %).  Copies spread over the chunks with an iteration or more of flight: started together after
+// barrier 1 they took 102 us on the 512 queries below, the form with the sums together 99, this 91.  Prefetching into the L2 gives nothing,
+// operands fetched two products ahead neither.  Measured (us, sums together -> apart): 512 queries on 16384 keys, 32 heads on 8 k/v heads, head dim 128:
+// 98.8 -> 90.6; 128 queries on 8192 keys, head dim 64: 38.4 -> 29.3; 4 heads, 4096 keys, causal, head dim 64: 21.3 -> 17.2; 4 heads, 4096
+// keys, full, head dim 96: 29.2 -> 25.3; 16 heads, 1024 keys, causal, head dim 64: 8.6 -> 8.2.  The lines of the rule: keep_sums_apart.
 #ifndef FA8_SHARED_ROWS_H_
 #define FA8_SHARED_ROWS_H_
 #include <type_traits>
@@ -58,7 +72,7 @@ struct SharedArgs {
 };
 static_assert(sizeof(SharedArgs) == 112, "see above");
 
-template <int D, bool E5M2, bool VT, int R, int W, int STAGES>
+template <int D, bool E5M2, bool VT, int R, int W, int STAGES, bool APART>
 __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2))) void fa8_shared_rows_kernel(
     const uint8_t* k_
 #define FA8_FIELD(type, name) , type name##_
@@ -75,8 +89,11 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
   constexpr int kTileBytes = kKvBlock * DP;
   constexpr int kKSteps = (D + 63) / 64;
   constexpr int kMTiles = D / 32;
-  constexpr int kOwn = (kMTiles + W - 1) / W;     // O^T tiles of a wavefront (the last wavefronts may have one less, or none)
+  constexpr int kOut = (kMTiles + W - 1) / W;     // O^T tiles that a wavefront writes (the last wavefronts may have one less, or none)
+  constexpr int kOwn = APART ? kMTiles : kOut;    // ... and adds products to: tiles kFirst + m * kStep
+  constexpr int kStep = APART ? 1 : W;
   constexpr int kSegs = kTileBytes / 1024;        // 1 KB copy segments per K or V tile, shared by the R wavefronts of a block
+  static_assert(!APART || STAGES == 2, "sums apart: two stages");
   static_assert(kSegs % R == 0, "a block's copy is split evenly over the row tiles");
   constexpr int kPasses = kSegs / R;
   // two stages each, separate objects: the compiler then knows that copies in flight do not alias the reads (see fa8_fwd_kernel)
@@ -84,8 +101,8 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
   __shared__ __attribute__((aligned(1024))) uint8_t k_lds1[STAGES == 2 ? W * kTileBytes : 16];
   __shared__ __attribute__((aligned(1024))) uint8_t v_lds0[W * kTileBytes];
   __shared__ __attribute__((aligned(1024))) uint8_t v_lds1[STAGES == 2 ? W * kTileBytes : 16];
-  __shared__ __attribute__((aligned(1024))) uint8_t p_lds[R * W * 2048];
-  __shared__ float max_lds[R * W * 32];
+  __shared__ __attribute__((aligned(1024))) uint8_t p_lds[APART ? 16 : R * W * 2048];
+  __shared__ float max_lds[(APART ? 2 : 1) * R * W * 32];
   __shared__ float sum_lds[R * W * 64];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -209,7 +226,7 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
   }
   issue_k(w, k_lds0, w < all_blocks, 0, kPasses);
   if constexpr (STAGES == 2) issue_k(w + W, k_lds1, w + W < all_blocks, 0, kPasses);
-  issue_v(w, v_lds0, w < all_blocks, 0, kPasses);
+  if constexpr (!APART) issue_v(w, v_lds0, w < all_blocks, 0, kPasses);
   // ---- LDS read offsets (see fa8_fwd_kernel) ----
   int k_off[kKSteps][2];
 #pragma unroll
@@ -222,17 +239,18 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
   int v_off[VT ? 2 : kOwn];
   if constexpr (VT) {
 #pragma unroll
-    for (int e = 0; e < 2; ++e) v_off[e] = w * kVtTileStride + tile_offset<64, false>(qn, 2 * h + e);
+    for (int e = 0; e < 2; ++e) v_off[e] = w * (APART ? kTileBytes : kVtTileStride) + tile_offset<64, false>(qn, 2 * h + e);
   } else {
 #pragma unroll
-    for (int m = 0; m < kOwn; ++m) v_off[m] = tile_offset<DP, true>(32 * h + tr_j, 2 * min(w + m * W, kMTiles - 1) + tr_g1) + 8 * tr_e;
+    for (int m = 0; m < kOwn; ++m)
+      v_off[m] = (APART ? w * kTileBytes : 0) + tile_offset<DP, true>(32 * h + tr_j, 2 * min((APART ? 0 : w) + m * kStep, kMTiles - 1) + tr_g1) + 8 * tr_e;
   }
   auto load_vf = [&](const uint8_t* v_lds, int i, int m) __attribute__((always_inline)) {
     const uint8_t* vb = v_lds + i * kTileBytes;
     v8i vf;
     if constexpr (VT) {
-      const v4i lo = *LDS_PTR(const v4i, vb + m * W * kVtTileStride + v_off[0]);
-      const v4i hi = *LDS_PTR(const v4i, vb + m * W * kVtTileStride + v_off[VT ? 1 : 0]);
+      const v4i lo = *LDS_PTR(const v4i, vb + m * kStep * kVtTileStride + v_off[0]);
+      const v4i hi = *LDS_PTR(const v4i, vb + m * kStep * kVtTileStride + v_off[VT ? 1 : 0]);
       vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     } else {
 #pragma unroll
@@ -251,17 +269,9 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
 #pragma unroll
     for (int i = 0; i < 16; ++i) o_acc[m][i] = 0.f;
   float m_run = kMaxStart, l_run = 0.f;
-  // rescale factors of the group whose PV products are due, and whether any row of the tile needs them
-  float alpha[W];
-  bool changed[W];
   auto load_kf = [&](const uint8_t* k_lds, int t, int ks) __attribute__((always_inline)) {
     const v4i lo = *LDS_PTR(const v4i, k_lds + t * kSubTileStride + k_off[ks][0]);
     const v4i hi = *LDS_PTR(const v4i, k_lds + t * kSubTileStride + k_off[ks][1]);
-    return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-  };
-  auto load_pf = [&](int i) __attribute__((always_inline)) {
-    const v4i lo = *LDS_PTR(const v4i, p_lds + (r * W + i) * 2048 + lane * 16);
-    const v4i hi = *LDS_PTR(const v4i, p_lds + (r * W + i) * 2048 + 1024 + lane * 16);
     return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
   };
   auto s_product = [&](v16f& acc, int ks, const v8i& kf) __attribute__((always_inline)) {
@@ -274,195 +284,439 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
       acc = mfma_fp8<E5M2>(kf, qf[ks], acc);
     }
   };
-  // brings O and l to the running max after block i of the group and adds the block's row sums
-  auto rescale = [&](int i, float sum) __attribute__((always_inline)) {
-#pragma clang fp contract(off)
-    if (changed[i]) {
-      l_run = l_run * alpha[i];
-      if (alpha[i] != 1.f) {
-#pragma unroll
-        for (int m = 0; m < kOwn; ++m)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) o_acc[m][e] *= alpha[i];
-      }
-    }
-    l_run = l_run + sum;
-  };
-  // Barrier once this wavefront's LDS operations are done and all but its latest `copies` tile copies have landed (vmcnt counts a
-  // lane's loads in issue order).  Bare s_barrier: __syncthreads() would wait for all copies.
-  auto sync = [&](auto copies_c) __attribute__((always_inline)) {
-    constexpr int n = decltype(copies_c)::value * kPasses;
-    static_assert(n < 64, "vmcnt has six bits");
-    __builtin_amdgcn_s_waitcnt(0x0070 | (n & 15) | (n >> 4 << 14));
-    __builtin_amdgcn_s_barrier();
-  };
-  constexpr std::integral_constant<int, 0> none{};
-  constexpr bool kAllOwn = kMTiles % W == 0;  // every wavefront has kOwn tiles of O^T
-  auto owns = [&](int m) __attribute__((always_inline)) { return kAllOwn || w + m * W < kMTiles; };
-  constexpr int kPv = W * kOwn, kS = 2 * kKSteps;  // matrix instructions of an iteration
-  v16f sbuf[2][2];
-  v8i p8;
+  const int groups = (all_blocks + W - 1) / W;
 
-  auto iteration = [&](auto first_c, auto parity_c, int g) __attribute__((always_inline)) {
-    constexpr int PH = decltype(parity_c)::value;
-    v16f(&s)[2] = sbuf[PH];
-    v16f(&sn)[2] = sbuf[PH ^ 1];
-    constexpr bool kTwo = STAGES == 2;
-    uint8_t* const k_this = kTwo && PH ? k_lds1 : k_lds0;
-    uint8_t* const k_next = kTwo && !PH ? k_lds1 : k_lds0;
-    uint8_t* const v_prev = kTwo && !PH ? v_lds1 : v_lds0;
-    constexpr bool kFirst = decltype(first_c)::value;
-    const int j = g * W + w;
-    const bool more = (g + 1) * W < all_blocks;  // workgroup-uniform
-    if (j >= n_plain) {
+  if constexpr (APART) {
+    v16f sbuf[2][2];
+    v8i p8;
+    float m_own = 0.f;              // running max after this wavefront's block of the group: what its weights are taken against
+    float alpha = 1.f, o_alpha = 1.f;  // from m_own of the group before to m_own; of the two groups before, for O
+    bool changed = false, o_changed = false;
+    // logits of keys that a row does not see, then the row max of a block, with all blocks before the group -> LDS
+    auto publish_max = [&](auto parity_c, v16f(&s)[2], int j) __attribute__((always_inline)) {
+      constexpr int PH = decltype(parity_c)::value;
+      if (j >= n_plain) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (j * kKvBlock + 32 * h + 16 * t + i > kv_limit) s[t][i] = -INFINITY;
-    }
-    float mx[4];
-#pragma unroll
-    for (int ch = 0; ch < 4; ++ch) mx[ch] = max3(s[0][4 * ch], s[0][4 * ch + 1], s[0][4 * ch + 2]);
-#pragma unroll
-    for (int ch = 0; ch < 4; ++ch) mx[ch] = max3(mx[ch], s[0][4 * ch + 3], s[1][4 * ch]);
-#pragma unroll
-    for (int ch = 0; ch < 4; ++ch) mx[ch] = max3(mx[ch], s[1][4 * ch + 1], s[1][4 * ch + 2]);
-    const float bm = lane32_max(max3(max3(mx[0], s[1][3], s[1][7]), max3(mx[1], s[1][11], s[1][15]), max3(mx[2], mx[3], m_run)));
-    if (h == 0) max_lds[wave * 32 + qn] = bm;
-    sync(std::integral_constant<int, kTwo || kFirst ? 1 : 0>());  // barrier 1: row maxima; weights, row sums and V of group g - 1; K of group g + 1; K of group g has been read
-    v8i vfrag[kPv], pfrag[W], kfrag[kS];
-    float sums[W], maxima[W];
-#pragma unroll
-    for (int i = 0; i < W; ++i) maxima[i] = max_lds[(r * W + i) * 32 + qn];
-    if constexpr (!kFirst) {
-      pfrag[0] = load_pf(0);
-      if (owns(0)) vfrag[0] = load_vf(v_prev, 0, 0);
-#pragma unroll
-      for (int i = 0; i < W; ++i) sums[i] = sum_lds[(r * W + i) * 64 + lane];
-    }
-    float m_after[W], m_own = m_run;
-#pragma unroll
-    for (int i = 0; i < W; ++i) {
-      m_after[i] = max2(i == 0 ? m_run : m_after[i - 1], maxima[i]);
-      if (i == w) m_own = m_after[i];
-    }
-    const float mc = m_own * c;
-    float sum0, sum1;
-    __builtin_amdgcn_sched_barrier(0);
-    // The softmax of 4 weights a chunk, three stages deep so that no instruction waits for the one before it: exponentials of
-    // chunk u, their arguments for chunk u + 1, row sum and fp8 packing of chunk u - 1.  The scheduling barriers keep that order.
-    float y[2][4], x[2][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) y[0][i] = __builtin_fmaf(s[0][i], c, -mc);
-    auto pack = [&](int u) __attribute__((always_inline)) {
-      int packed = pack4_fp8<E5M2>(x[u & 1][0], x[u & 1][1], x[u & 1][2], x[u & 1][3]);
-      asm volatile("" : "+v"(packed));
-      p8[u] = packed;
-    };
-    auto add = [&](int u, int i) __attribute__((always_inline)) {
-      float& sum = i & 1 ? sum1 : sum0;
-      sum = (u == 0 && i < 2) ? x[u & 1][i] : sum + x[u & 1][i];
-    };
-    auto chunk = [&](int u) __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        x[u & 1][i] = __builtin_amdgcn_exp2f(y[u & 1][i]);
-        if (u < 7) y[(u + 1) & 1][i] = __builtin_fmaf(s[(u + 1) >> 2][4 * ((u + 1) & 3) + i], c, -mc);
-        if (u > 0) add(u - 1, i);
-        __builtin_amdgcn_sched_barrier(0);
+          for (int i = 0; i < 16; ++i)
+            if (j * kKvBlock + 32 * h + 16 * t + i > kv_limit) s[t][i] = -INFINITY;
       }
-      if (u > 0) {
-        pack(u - 1);
-        asm volatile("" : "+v"(sum0), "+v"(sum1));  // keeps the additions in their chunk
-      }
-      if (u == 7) {
+      float mx[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) add(7, i);
-        pack(7);
-      }
-      __builtin_amdgcn_sched_barrier(0);
+      for (int ch = 0; ch < 4; ++ch) mx[ch] = max3(s[0][4 * ch], s[0][4 * ch + 1], s[0][4 * ch + 2]);
+#pragma unroll
+      for (int ch = 0; ch < 4; ++ch) mx[ch] = max3(mx[ch], s[0][4 * ch + 3], s[1][4 * ch]);
+#pragma unroll
+      for (int ch = 0; ch < 4; ++ch) mx[ch] = max3(mx[ch], s[1][4 * ch + 1], s[1][4 * ch + 2]);
+      const float bm = lane32_max(max3(max3(mx[0], s[1][3], s[1][7]), max3(mx[1], s[1][11], s[1][15]), max3(mx[2], mx[3], m_run)));
+      if (h == 0) max_lds[(PH * R * W + wave) * 32 + qn] = bm;
     };
+    float maxima[W];
+    auto read_maxima = [&](auto parity_c) __attribute__((always_inline)) {
+      constexpr int PH = decltype(parity_c)::value;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if constexpr (kTwo)
-        issue_k(j + 2 * W, k_this, j + 2 * W < all_blocks, u * kPasses / 4, (u + 1) * kPasses / 4);
-      else if (u == 0)
-        issue_k(j + W, k_this, more && j + W < all_blocks, 0, kPasses);
-      chunk(u);
-      if constexpr (!kFirst) {
+      for (int i = 0; i < W; ++i) maxima[i] = max_lds[(PH * R * W + r * W + i) * 32 + qn];
+    };
+    // from the maxima of a group: m_own and m_run after it
+    auto follow_max = [&](bool first) __attribute__((always_inline)) {
+      float m = m_run, own = m_run;
 #pragma unroll
-        for (int n = u * kPv / 4; n < (u + 1) * kPv / 4; ++n) {
-          const int i = n / kOwn, m = n % kOwn;
-          if (n + 1 < kPv) {  // operands of the next product
-            if ((n + 1) % kOwn == 0) pfrag[(n + 1) / kOwn] = load_pf((n + 1) / kOwn);
-            if (owns((n + 1) % kOwn)) vfrag[n + 1] = load_vf(v_prev, (n + 1) / kOwn, (n + 1) % kOwn);
-          }
-          if (m == 0) rescale(i, sums[i]);
-          if (owns(m)) o_acc[m] = mfma_fp8<E5M2>(vfrag[n], pfrag[i], o_acc[m]);
+      for (int i = 0; i < W; ++i) {
+        m = max2(m, maxima[i]);
+        own = i <= w ? m : own;
+      }
+      o_alpha = alpha;
+      o_changed = changed;
+      changed = !first && __any(own != m_own);
+      alpha = changed ? __builtin_amdgcn_exp2f((m_own - own) * c) : 1.f;
+      m_own = own;
+      m_run = m;
+    };
+    auto rescale = [&]() __attribute__((always_inline)) {
+      if (o_changed) {
+        if (o_alpha != 1.f) {
+#pragma unroll
+          for (int m = 0; m < kOwn; ++m)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o_acc[m][e] *= o_alpha;
         }
       }
-      if (kTwo && u == 3) kfrag[0] = load_kf(k_next, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    };
+    // Waits until all but the latest `copies` tile copies of this wavefront have landed; barrier: and its LDS operations are done.
+    auto wait_copies = [&](auto copies_c) __attribute__((always_inline)) {
+      constexpr int n = decltype(copies_c)::value * kPasses;
+      static_assert(n < 64, "vmcnt has six bits");
+      __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | (n >> 4 << 14));
+    };
+    auto barrier = [&](auto copies_c) __attribute__((always_inline)) {
+      constexpr int n = decltype(copies_c)::value * kPasses;
+      __builtin_amdgcn_s_waitcnt(0x0070 | (n & 15) | (n >> 4 << 14));
+      __builtin_amdgcn_s_barrier();
+    };
+    constexpr std::integral_constant<int, 0> none{};
+    constexpr std::integral_constant<int, 1> one{};
+    constexpr std::integral_constant<int, 2> two{};
+    constexpr int kS = 2 * kKSteps;
+    constexpr int kCut = 6;  // chunks in front of barrier 1 (512 queries on 16384 keys: 5 92.1 us, 6 90.7, 7 94)
+    auto iteration = [&](auto first_c, auto parity_c, int g) __attribute__((always_inline)) {
+      constexpr int PH = decltype(parity_c)::value;
+      constexpr bool kFirst = decltype(first_c)::value;
+      v16f(&s)[2] = sbuf[PH];
+      v16f(&sn)[2] = sbuf[PH ^ 1];
+      uint8_t* const k_next = PH ? k_lds0 : k_lds1;
+      uint8_t* const v_this = PH ? v_lds1 : v_lds0;
+      uint8_t* const v_prev = PH ? v_lds0 : v_lds1;
+      const int j = g * W + w;
+      const float mc = m_own * c;
+      float sum0, sum1, y[2][4], x[2][4];
+      v8i p8_cur;
 #pragma unroll
-    for (int i = 0; i < W; ++i) {
-      const float before = i == 0 ? m_run : m_after[i - 1];
-      changed[i] = __any(m_after[i] != before);
-      alpha[i] = changed[i] ? __builtin_amdgcn_exp2f((before - m_after[i]) * c) : 1.f;
-    }
-    m_run = m_after[W - 1];
-    // barrier 2: weights, row sums and V of group g - 1 have been read (LDS operations only; one stage: K of group g + 1 has landed)
-    __builtin_amdgcn_s_waitcnt(kTwo ? 0xC07F : 0x0070);
-    __builtin_amdgcn_s_barrier();
-    if constexpr (!kTwo) {
-      if constexpr (!kFirst) issue_v(j, v_prev, j < all_blocks, 0, kPasses);
+      for (int i = 0; i < 4; ++i) y[0][i] = __builtin_fmaf(s[0][i], c, -mc);
+      auto pack = [&](int u) __attribute__((always_inline)) {
+        int packed = pack4_fp8<E5M2>(x[u & 1][0], x[u & 1][1], x[u & 1][2], x[u & 1][3]);
+        asm volatile("" : "+v"(packed));
+        p8_cur[u] = packed;
+      };
+      auto add = [&](int u, int i) __attribute__((always_inline)) {
+        float& sum = i & 1 ? sum1 : sum0;
+        sum = (u == 0 && i < 2) ? x[u & 1][i] : sum + x[u & 1][i];
+      };
+      auto chunk = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          x[u & 1][i] = __builtin_amdgcn_exp2f(y[u & 1][i]);
+          if (u < 7) y[(u + 1) & 1][i] = __builtin_fmaf(s[(u + 1) >> 2][4 * ((u + 1) & 3) + i], c, -mc);
+          if (u > 0) add(u - 1, i);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (u > 0) {
+          pack(u - 1);
+          asm volatile("" : "+v"(sum0), "+v"(sum1));
+        }
+        if (u == 7) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) add(7, i);
+          pack(7);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      v8i kfrag[kS], vfrag[kOwn];
       kfrag[0] = load_kf(k_next, 0, 0);
-    }
-#pragma unroll
-    for (int u = 4; u < 8; ++u) {
-      // (after the last group this is the product of a stale tile: never used)
-#pragma unroll
-      for (int n = ((u - 4) * kS + 3) / 4; n < ((u - 3) * kS + 3) / 4; ++n) {
-        if (n + 1 < kS) kfrag[n + 1] = load_kf(k_next, (n + 1) / kKSteps, (n + 1) % kKSteps);
-        s_product(sn[n / kKSteps], n % kKSteps, kfrag[n]);
-      }
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (kTwo) issue_v(j + W, v_prev, j + W < all_blocks, (u - 4) * kPasses / 4, (u - 3) * kPasses / 4);
-      chunk(u);
-      if (u == 4) *LDS_PTR(v4i, p_lds + wave * 2048 + lane * 16) = v4i{p8[0], p8[1], p8[2], p8[3]};
+#pragma unroll
+      for (int u = 0; u < kCut; ++u) {
+        if (u < 4) {
+#pragma unroll
+          for (int n = (u * kS + 3) / 4; n < ((u + 1) * kS + 3) / 4; ++n) {
+            if (n + 1 < kS) kfrag[n + 1] = load_kf(k_next, (n + 1) / kKSteps, (n + 1) % kKSteps);
+            s_product(sn[n / kKSteps], n % kKSteps, kfrag[n]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          issue_v(j, v_this, j < all_blocks, u * kPasses / 4, (u + 1) * kPasses / 4);
+        }
+        chunk(u);
+      }
+      publish_max(std::integral_constant<int, PH ^ 1>(), sn, j + W);
+      barrier(two);  // barrier 1: row maxima of group g + 1; V of group g - 1 has landed; K of group g + 1 has been read
+      read_maxima(std::integral_constant<int, PH ^ 1>());
+      if constexpr (!kFirst) vfrag[0] = load_vf(v_prev, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!kFirst) rescale();
+#pragma unroll
+      for (int u = kCut; u < 8; ++u) {
+        if constexpr (!kFirst) {
+          constexpr int kIn = 8 - kCut;
+#pragma unroll
+          for (int m = (u - kCut) * kOwn / kIn; m < (u - kCut + 1) * kOwn / kIn; ++m) {
+            if (m + 1 < kOwn) vfrag[m + 1] = load_vf(v_prev, 0, m + 1);
+            o_acc[m] = mfma_fp8<E5M2>(vfrag[m], p8, o_acc[m]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        issue_k(j + 3 * W, k_next, j + 3 * W < all_blocks, (u - kCut) * kPasses / (8 - kCut), (u - kCut + 1) * kPasses / (8 - kCut));
+        chunk(u);
+      }
+      l_run = l_run * alpha + (sum0 + sum1);
+      p8 = p8_cur;
+      follow_max(false);
+      // K of group g + 2 has landed; barrier 2 (a tile that two wavefronts read): for both, and V of group g - 1 has been read
+      if constexpr (R > 1)
+        barrier(two);
+      else
+        wait_copies(two);
+    };
+    using T = std::true_type;
+    using F = std::false_type;
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    // K of group 0 has landed
+    if constexpr (R > 1)
+      barrier(one);
+    else
+      wait_copies(one);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < kKSteps; ++ks) s_product(sbuf[0][t], ks, load_kf(k_lds0, t, ks));
+    publish_max(even, sbuf[0], w);
+    barrier(none);
+    read_maxima(even);
+    issue_k(w + 2 * W, k_lds0, w + 2 * W < all_blocks, 0, kPasses);
+    follow_max(true);
+    iteration(T(), even, 0);
+    int g = 1;
+    for (; g + 1 < groups; g += 2) {
+      iteration(F(), odd, g);
+      iteration(F(), even, g + 1);
     }
-    *LDS_PTR(v4i, p_lds + wave * 2048 + 1024 + lane * 16) = v4i{p8[4], p8[5], p8[6], p8[7]};
-    sum_lds[wave * 64 + lane] = sum0 + sum1;
-  };
+    if (g < groups) iteration(F(), odd, g);
+    barrier(none);
+    // the products of the last group; then m_own is the max over all keys (the group after the last one shows none)
+    rescale();
+#pragma unroll
+    for (int m = 0; m < kOwn; ++m) o_acc[m] = mfma_fp8<E5M2>(load_vf((groups & 1) ? v_lds0 : v_lds1, 0, m), p8, o_acc[m]);
+    o_alpha = alpha;
+    o_changed = changed;
+    rescale();
+    l_run *= alpha;
+    // The wavefronts of a tile add up their O and l, in their order: tiles of 4 KB through the LDS of K and V.
+    constexpr int kUnits = W * kTileBytes / 4096, kObjects = 4;
+    constexpr int kRounds = (R * W * kMTiles + kUnits * kObjects - 1) / (kUnits * kObjects), kT = kMTiles / kRounds;
+    static_assert(kMTiles % kRounds == 0 && (kRounds == 1 || kT % W == 0) && R * W * kT <= kUnits * kObjects, "rounds of whole tiles");
+    auto unit = [&](int u) __attribute__((always_inline)) {
+      const int at = u / kUnits;
+      uint8_t* const base = at == 0 ? k_lds0 : (at == 1 ? v_lds0 : (at == 2 ? k_lds1 : v_lds1));
+      return base + (u - at * kUnits) * 4096 + lane * 16;
+    };
+    sum_lds[wave * 64 + lane] = l_run;
+    v16f total[kOut];
+#pragma unroll
+    for (int n = 0; n < kRounds; ++n) {
+      barrier(none);  // V, or the tiles of the round before, have been read
+#pragma unroll
+      for (int m = 0; m < kT; ++m)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          *LDS_PTR(v4f, unit(wave * kT + m) + e * 1024) = v4f{o_acc[n * kT + m][4 * e], o_acc[n * kT + m][4 * e + 1], o_acc[n * kT + m][4 * e + 2], o_acc[n * kT + m][4 * e + 3]};
+      barrier(none);
+#pragma unroll
+      for (int m = 0; m < (kT + W - 1) / W; ++m) {
+        if (w + m * W >= kT) break;
+#pragma unroll
+        for (int i = 0; i < W; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const v4f part = *LDS_PTR(const v4f, unit((r * W + i) * kT + w + m * W) + e * 1024);
+#pragma unroll
+            for (int b2 = 0; b2 < 4; ++b2)
+              total[n * (kT / W) + m][4 * e + b2] = i == 0 ? part[b2] : total[n * (kT / W) + m][4 * e + b2] + part[b2];
+          }
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < kOut; ++m) o_acc[m] = total[m];
+    l_run = sum_lds[r * W * 64 + lane];
+#pragma unroll
+    for (int i = 1; i < W; ++i) l_run += sum_lds[(r * W + i) * 64 + lane];
+  } else {
+    // rescale factors of the group whose PV products are due, and whether any row of the tile needs them
+    float alpha[W];
+    bool changed[W];
+    auto load_pf = [&](int i) __attribute__((always_inline)) {
+      const v4i lo = *LDS_PTR(const v4i, p_lds + (r * W + i) * 2048 + lane * 16);
+      const v4i hi = *LDS_PTR(const v4i, p_lds + (r * W + i) * 2048 + 1024 + lane * 16);
+      return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    };
+    // brings O and l to the running max after block i of the group and adds the block's row sums
+    auto rescale = [&](int i, float sum) __attribute__((always_inline)) {
+  #pragma clang fp contract(off)
+      if (changed[i]) {
+        l_run = l_run * alpha[i];
+        if (alpha[i] != 1.f) {
+  #pragma unroll
+          for (int m = 0; m < kOwn; ++m)
+  #pragma unroll
+            for (int e = 0; e < 16; ++e) o_acc[m][e] *= alpha[i];
+        }
+      }
+      l_run = l_run + sum;
+    };
+    // Barrier once this wavefront's LDS operations are done and all but its latest `copies` tile copies have landed (vmcnt counts a
+    // lane's loads in issue order).  Bare s_barrier: __syncthreads() would wait for all copies.
+    auto sync = [&](auto copies_c) __attribute__((always_inline)) {
+      constexpr int n = decltype(copies_c)::value * kPasses;
+      static_assert(n < 64, "vmcnt has six bits");
+      __builtin_amdgcn_s_waitcnt(0x0070 | (n & 15) | (n >> 4 << 14));
+      __builtin_amdgcn_s_barrier();
+    };
+    constexpr std::integral_constant<int, 0> none{};
+    constexpr bool kAllOwn = kMTiles % W == 0;  // every wavefront has kOwn tiles of O^T
+    auto owns = [&](int m) __attribute__((always_inline)) { return kAllOwn || w + m * W < kMTiles; };
+    constexpr int kPv = W * kOwn, kS = 2 * kKSteps;  // matrix instructions of an iteration
+    v16f sbuf[2][2];
+    v8i p8;
 
-  using T = std::true_type;
-  using F = std::false_type;
-  constexpr std::integral_constant<int, 0> even{};
-  constexpr std::integral_constant<int, 1> odd{};
-  sync(std::integral_constant<int, STAGES>());  // K of group 0 landed
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int ks = 0; ks < kKSteps; ++ks) s_product(sbuf[0][t], ks, load_kf(k_lds0, t, ks));
-  const int groups = (all_blocks + W - 1) / W;
-  iteration(T(), even, 0);
-  int g = 1;
-  for (; g + 1 < groups; g += 2) {
-    iteration(F(), odd, g);
-    iteration(F(), even, g + 1);
-  }
-  if (g < groups) iteration(F(), odd, g);
-  sync(none);
-  // the PV products of the last group
-#pragma unroll
-  for (int i = 0; i < W; ++i) {
-    if ((groups - 1) * W + i < blocks) {
-      rescale(i, sum_lds[(r * W + i) * 64 + lane]);
-      const v8i pf = load_pf(i);
-#pragma unroll
-      for (int m = 0; m < kOwn; ++m)
-        if (owns(m)) o_acc[m] = mfma_fp8<E5M2>(load_vf(STAGES == 1 || (groups & 1) ? v_lds0 : v_lds1, i, m), pf, o_acc[m]);
+    auto iteration = [&](auto first_c, auto parity_c, int g) __attribute__((always_inline)) {
+      constexpr int PH = decltype(parity_c)::value;
+      v16f(&s)[2] = sbuf[PH];
+      v16f(&sn)[2] = sbuf[PH ^ 1];
+      constexpr bool kTwo = STAGES == 2;
+      uint8_t* const k_this = kTwo && PH ? k_lds1 : k_lds0;
+      uint8_t* const k_next = kTwo && !PH ? k_lds1 : k_lds0;
+      uint8_t* const v_prev = kTwo && !PH ? v_lds1 : v_lds0;
+      constexpr bool kFirst = decltype(first_c)::value;
+      const int j = g * W + w;
+      const bool more = (g + 1) * W < all_blocks;  // workgroup-uniform
+      if (j >= n_plain) {
+  #pragma unroll
+        for (int t = 0; t < 2; ++t)
+  #pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if (j * kKvBlock + 32 * h + 16 * t + i > kv_limit) s[t][i] = -INFINITY;
+      }
+      float mx[4];
+  #pragma unroll
+      for (int ch = 0; ch < 4; ++ch) mx[ch] = max3(s[0][4 * ch], s[0][4 * ch + 1], s[0][4 * ch + 2]);
+  #pragma unroll
+      for (int ch = 0; ch < 4; ++ch) mx[ch] = max3(mx[ch], s[0][4 * ch + 3], s[1][4 * ch]);
+  #pragma unroll
+      for (int ch = 0; ch < 4; ++ch) mx[ch] = max3(mx[ch], s[1][4 * ch + 1], s[1][4 * ch + 2]);
+      const float bm = lane32_max(max3(max3(mx[0], s[1][3], s[1][7]), max3(mx[1], s[1][11], s[1][15]), max3(mx[2], mx[3], m_run)));
+      if (h == 0) max_lds[wave * 32 + qn] = bm;
+      sync(std::integral_constant<int, kTwo || kFirst ? 1 : 0>());  // barrier 1: row maxima; weights, row sums and V of group g - 1; K of group g + 1; K of group g has been read
+      v8i vfrag[kPv], pfrag[W], kfrag[kS];
+      float sums[W], maxima[W];
+  #pragma unroll
+      for (int i = 0; i < W; ++i) maxima[i] = max_lds[(r * W + i) * 32 + qn];
+      if constexpr (!kFirst) {
+        pfrag[0] = load_pf(0);
+        if (owns(0)) vfrag[0] = load_vf(v_prev, 0, 0);
+  #pragma unroll
+        for (int i = 0; i < W; ++i) sums[i] = sum_lds[(r * W + i) * 64 + lane];
+      }
+      float m_after[W], m_own = m_run;
+  #pragma unroll
+      for (int i = 0; i < W; ++i) {
+        m_after[i] = max2(i == 0 ? m_run : m_after[i - 1], maxima[i]);
+        if (i == w) m_own = m_after[i];
+      }
+      const float mc = m_own * c;
+      float sum0, sum1;
+      __builtin_amdgcn_sched_barrier(0);
+      // The softmax of 4 weights a chunk, three stages deep so that no instruction waits for the one before it: exponentials of
+      // chunk u, their arguments for chunk u + 1, row sum and fp8 packing of chunk u - 1.  The scheduling barriers keep that order.
+      float y[2][4], x[2][4];
+  #pragma unroll
+      for (int i = 0; i < 4; ++i) y[0][i] = __builtin_fmaf(s[0][i], c, -mc);
+      auto pack = [&](int u) __attribute__((always_inline)) {
+        int packed = pack4_fp8<E5M2>(x[u & 1][0], x[u & 1][1], x[u & 1][2], x[u & 1][3]);
+        asm volatile("" : "+v"(packed));
+        p8[u] = packed;
+      };
+      auto add = [&](int u, int i) __attribute__((always_inline)) {
+        float& sum = i & 1 ? sum1 : sum0;
+        sum = (u == 0 && i < 2) ? x[u & 1][i] : sum + x[u & 1][i];
+      };
+      auto chunk = [&](int u) __attribute__((always_inline)) {
+  #pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          x[u & 1][i] = __builtin_amdgcn_exp2f(y[u & 1][i]);
+          if (u < 7) y[(u + 1) & 1][i] = __builtin_fmaf(s[(u + 1) >> 2][4 * ((u + 1) & 3) + i], c, -mc);
+          if (u > 0) add(u - 1, i);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (u > 0) {
+          pack(u - 1);
+          asm volatile("" : "+v"(sum0), "+v"(sum1));  // keeps the additions in their chunk
+        }
+        if (u == 7) {
+  #pragma unroll
+          for (int i = 0; i < 4; ++i) add(7, i);
+          pack(7);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+  #pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if constexpr (kTwo)
+          issue_k(j + 2 * W, k_this, j + 2 * W < all_blocks, u * kPasses / 4, (u + 1) * kPasses / 4);
+        else if (u == 0)
+          issue_k(j + W, k_this, more && j + W < all_blocks, 0, kPasses);
+        chunk(u);
+        if constexpr (!kFirst) {
+  #pragma unroll
+          for (int n = u * kPv / 4; n < (u + 1) * kPv / 4; ++n) {
+            const int i = n / kOwn, m = n % kOwn;
+            if (n + 1 < kPv) {  // operands of the next product
+              if ((n + 1) % kOwn == 0) pfrag[(n + 1) / kOwn] = load_pf((n + 1) / kOwn);
+              if (owns((n + 1) % kOwn)) vfrag[n + 1] = load_vf(v_prev, (n + 1) / kOwn, (n + 1) % kOwn);
+            }
+            if (m == 0) rescale(i, sums[i]);
+            if (owns(m)) o_acc[m] = mfma_fp8<E5M2>(vfrag[n], pfrag[i], o_acc[m]);
+          }
+        }
+        if (kTwo && u == 3) kfrag[0] = load_kf(k_next, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+  #pragma unroll
+      for (int i = 0; i < W; ++i) {
+        const float before = i == 0 ? m_run : m_after[i - 1];
+        changed[i] = __any(m_after[i] != before);
+        alpha[i] = changed[i] ? __builtin_amdgcn_exp2f((before - m_after[i]) * c) : 1.f;
+      }
+      m_run = m_after[W - 1];
+      // barrier 2: weights, row sums and V of group g - 1 have been read (LDS operations only; one stage: K of group g + 1 has landed)
+      __builtin_amdgcn_s_waitcnt(kTwo ? 0xC07F : 0x0070);
+      __builtin_amdgcn_s_barrier();
+      if constexpr (!kTwo) {
+        if constexpr (!kFirst) issue_v(j, v_prev, j < all_blocks, 0, kPasses);
+        kfrag[0] = load_kf(k_next, 0, 0);
+      }
+  #pragma unroll
+      for (int u = 4; u < 8; ++u) {
+        // (after the last group this is the product of a stale tile: never used)
+  #pragma unroll
+        for (int n = ((u - 4) * kS + 3) / 4; n < ((u - 3) * kS + 3) / 4; ++n) {
+          if (n + 1 < kS) kfrag[n + 1] = load_kf(k_next, (n + 1) / kKSteps, (n + 1) % kKSteps);
+          s_product(sn[n / kKSteps], n % kKSteps, kfrag[n]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kTwo) issue_v(j + W, v_prev, j + W < all_blocks, (u - 4) * kPasses / 4, (u - 3) * kPasses / 4);
+        chunk(u);
+        if (u == 4) *LDS_PTR(v4i, p_lds + wave * 2048 + lane * 16) = v4i{p8[0], p8[1], p8[2], p8[3]};
+      }
+      *LDS_PTR(v4i, p_lds + wave * 2048 + 1024 + lane * 16) = v4i{p8[4], p8[5], p8[6], p8[7]};
+      sum_lds[wave * 64 + lane] = sum0 + sum1;
+    };
+
+    using T = std::true_type;
+    using F = std::false_type;
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    sync(std::integral_constant<int, STAGES>());  // K of group 0 landed
+  #pragma unroll
+    for (int t = 0; t < 2; ++t)
+  #pragma unroll
+      for (int ks = 0; ks < kKSteps; ++ks) s_product(sbuf[0][t], ks, load_kf(k_lds0, t, ks));
+    iteration(T(), even, 0);
+    int g = 1;
+    for (; g + 1 < groups; g += 2) {
+      iteration(F(), odd, g);
+      iteration(F(), even, g + 1);
+    }
+    if (g < groups) iteration(F(), odd, g);
+    sync(none);
+    // the PV products of the last group
+  #pragma unroll
+    for (int i = 0; i < W; ++i) {
+      if ((groups - 1) * W + i < blocks) {
+        rescale(i, sum_lds[(r * W + i) * 64 + lane]);
+        const v8i pf = load_pf(i);
+  #pragma unroll
+        for (int m = 0; m < kOwn; ++m)
+          if (owns(m)) o_acc[m] = mfma_fp8<E5M2>(load_vf(STAGES == 1 || (groups & 1) ? v_lds0 : v_lds1, i, m), pf, o_acc[m]);
+      }
     }
   }
 
@@ -476,7 +730,7 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
   }
   const unsigned long long o_at = ((unsigned long long)a.o_bs * b + (unsigned long long)a.o_hs * hd + (unsigned long long)a.o_rs * qi) * 4 + 4 * h;
 #pragma unroll
-  for (int m = 0; m < kOwn; ++m) {
+  for (int m = 0; m < kOut; ++m) {
     const int mt = w + m * W;
     if (kMTiles % W != 0 && mt >= kMTiles) break;
     if (!(a.mode & kSharedFp8Out)) {

@@ -8,8 +8,8 @@ using namespace fa8;
 template <int D, int R, int W, int STAGES>
 const void* pick(bool e5m2, bool vt) {
   if (e5m2)
-    return vt ? (const void*)&fa8_shared_rows_kernel<D, true, true, R, W, STAGES> : (const void*)&fa8_shared_rows_kernel<D, true, false, R, W, STAGES>;
-  return vt ? (const void*)&fa8_shared_rows_kernel<D, false, true, R, W, STAGES> : (const void*)&fa8_shared_rows_kernel<D, false, false, R, W, STAGES>;
+    return vt ? (const void*)&fa8_shared_rows_kernel<D, true, true, R, W, STAGES, false> : (const void*)&fa8_shared_rows_kernel<D, true, false, R, W, STAGES, false>;
+  return vt ? (const void*)&fa8_shared_rows_kernel<D, false, true, R, W, STAGES, false> : (const void*)&fa8_shared_rows_kernel<D, false, false, R, W, STAGES, false>;
 }
 template <int D>
 const void* pick_rw(int r, int w, int stages, bool e5m2, bool vt) {
@@ -28,7 +28,7 @@ const void* pick_rw(int r, int w, int stages, bool e5m2, bool vt) {
 
 }  // namespace
 
-int fa8::launch_shared(const Fa8FwdParams* p, int r, int w, int stages, hipStream_t stream) {
+int fa8::launch_shared(const Fa8FwdParams* p, int r, int w, int stages, bool apart, hipStream_t stream) {
   SharedArgs a;
   a.q = (const uint8_t*)p->q;
   a.k = (const uint8_t*)p->k;
@@ -47,8 +47,8 @@ int fa8::launch_shared(const Fa8FwdParams* p, int r, int w, int stages, hipStrea
   a.lse_bs = p->lse_batch_stride; a.lse_hs = p->lse_head_stride;
   const int tiles = (int)(((long long)group * p->seqlen_q + 32 * r - 1) / (32 * r));
   const bool e5m2 = p->in_dtype == FA8_DTYPE_E5M2, vt = p->v_layout == FA8_V_TRANSPOSED;
-  const void* fn = nullptr;
-  switch (p->head_dim) {
+  const void* fn = apart ? apart_kernel(p->head_dim, r, w, e5m2, vt) : nullptr;
+  if (!apart) switch (p->head_dim) {
 #define FA8_HEAD_DIM_CASE(D_) \
   case D_: fn = pick_rw<D_>(r, w, stages, e5m2, vt); break
     FA8_HEAD_DIM_CASE(32);
@@ -70,6 +70,6 @@ int fa8::launch_shared(const Fa8FwdParams* p, int r, int w, int stages, hipStrea
   };
   // Head dim 32, two stages: 32 KB that nothing uses keep a compute unit at two workgroups, for which choose_plan takes them; with a third, 1024 tiles
   // take a round of three a compute unit and one of one (1024 heads, 7297 keys: 105 us, 91 so).
-  const unsigned unused_lds = p->head_dim == 32 && r == 1 && stages == 2 ? 32 * 1024 : 0;
+  const unsigned unused_lds = p->head_dim == 32 && r == 1 && stages == 2 && !apart ? 32 * 1024 : 0;
   return (int)hipLaunchKernel(fn, dim3((unsigned)heads_k, (unsigned)p->batch, (unsigned)tiles), dim3(64 * r * w), argv, unused_lds, stream);
 }

@@ -137,6 +137,16 @@ int fa8_fwd_workspace(const Fa8FwdParams* p, int64_t* bytes);
 int fa8_fwd_ws(const Fa8FwdParams* p, void* workspace, int64_t bytes, void* hip_stream);
 
 /*
+ * fa8_fwd_ws, free to take the fp32 sums over the keys in another order also where that needs no memory (library version 7): launches with few
+ * query rows then keep the sums of the wavefronts that share a row tile apart and add them up at the end.  The weights are the same bit for
+ * bit; the last bits of O and of the log-sum-exp can depend on the whole launch and on the number of compute units, not on anything else.  The
+ * workspace is that of fa8_fwd_workspace, and may be NULL.  fa8_fwd_apart tells whether a call would do so (1 or 0, or the FA8_ERR_* code
+ * fa8_fwd_validate gives; launches nothing).  No counterpart in the reference.
+ */
+int fa8_fwd_any_order(const Fa8FwdParams* p, void* workspace, int64_t bytes, void* hip_stream);
+int fa8_fwd_apart(const Fa8FwdParams* p);
+
+/*
  * fa8_fwd_ws for tests (library version 6).  Where the parts of split keys run in one kernel, each takes the row maxima of the parts before
  * it from the workspace and, after a number of looks, forms those that have not come itself; the parts in late_parts (a bit each) do not
  * hand theirs on.  The results are those of fa8_fwd_ws bit for bit.
@@ -147,8 +157,10 @@ int fa8_fwd_ws_late(const Fa8FwdParams* p, void* workspace, int64_t bytes, uint3
  * How a call would be cut on the current device, for benchmarks and tests (library version 5; nothing is launched): query rows of a workgroup
  * (grouped q heads counted together), wavefronts that share 32 of them (1: one of the main loops of fa8_fwd_schedule; 2 or 4: shared
  * rows, for launches with few of them; a schedule hint always gives 1), and into how many parts the keys of a row are split
- * (more than 1 only with_workspace).  The results of shared and unshared rows are bitwise the same.
+ * (more than 1 only with_workspace).  The results of shared and unshared rows are bitwise the same.  with_workspace: 0 for fa8_fwd, 1 for
+ * fa8_fwd_ws, FA8_PLAN_ANY_ORDER (library version 7) for fa8_fwd_any_order, both with the workspace that they ask for.
  */
+#define FA8_PLAN_ANY_ORDER 2
 int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* rows_per_workgroup, int32_t* wavefronts_per_tile,
                  int32_t* kv_splits);
 
