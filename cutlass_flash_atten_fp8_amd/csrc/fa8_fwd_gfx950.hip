@@ -392,11 +392,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
   // s_barrier: __syncthreads() would also wait for the copy that is meant to stay in flight.
   constexpr int kLoadsPerTile = kSplitPass ? 1 : 2 * kPasses;
   auto stage_sync = [&](bool next_in_flight) __attribute__((always_inline)) {
-    // s_waitcnt immediate (gfx9 layout): vmcnt[3:0], expcnt[6:4] = 7 and lgkmcnt[11:8] = 15 (no wait on those)
+    // s_waitcnt immediate (gfx9 layout): vmcnt[3:0], expcnt[6:4] = 7 (no wait on those), lgkmcnt[11:8] = 0: the reads of block j have returned.  The
+    // compiler may move the last product of a step, and its wait for its operands, behind the barrier; a copy into the stage, one of nothing above
+    // all, could then overtake the read.
     if (next_in_flight)
-      __builtin_amdgcn_s_waitcnt(0x0F70 | kLoadsPerTile);
+      __builtin_amdgcn_s_waitcnt(0x0070 | kLoadsPerTile);
     else
-      __builtin_amdgcn_s_waitcnt(0x0F70);
+      __builtin_amdgcn_s_waitcnt(0x0070);
     __builtin_amdgcn_s_barrier();
   };
   static_assert(kLoadsPerTile < 16, "vmcnt immediate above");
@@ -529,7 +531,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
     auto wait_in_flight = [&](auto tiles_c) __attribute__((always_inline)) {
       constexpr int n = decltype(tiles_c)::value * kPasses;
       static_assert(n < 16, "vmcnt immediate");
-      __builtin_amdgcn_s_waitcnt(0x0F70 | n);
+      __builtin_amdgcn_s_waitcnt(0x0070 | n);  // (and its LDS reads have returned, see stage_sync)
       __builtin_amdgcn_s_barrier();
     };
     using T = std::true_type;
@@ -546,6 +548,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
 #pragma unroll
       for (int ks = 0; ks < kKSteps; ++ks) s[t] = mfma_fp8<E5M2>(load_kf(k_lds0, t, ks), qf[ks], s[t]);
     }
+    __builtin_amdgcn_s_waitcnt(0xC07F);
     __builtin_amdgcn_s_barrier();  // every wavefront has read K(0): step 0 may overwrite its stage
     // One step with compile-time LDS stages (PH = j % 3).
     auto step = [&](auto first_c, auto tail_c, auto ph_c, int j) __attribute__((always_inline)) {
@@ -699,7 +702,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
     auto wait_in_flight = [&](auto tiles_c) __attribute__((always_inline)) {
       constexpr int n = decltype(tiles_c)::value * kPasses;
       static_assert(n < 16, "vmcnt immediate");
-      __builtin_amdgcn_s_waitcnt(0x0F70 | n);
+      __builtin_amdgcn_s_waitcnt(0x0070 | n);  // (and its LDS reads have returned, see stage_sync)
       __builtin_amdgcn_s_barrier();
     };
     // Ends step j: K(j+2) and V(j) must have landed; the copies of steps j-1 and j (K(j+3), V(j+1), K(j+4), V(j+2)) may stay
