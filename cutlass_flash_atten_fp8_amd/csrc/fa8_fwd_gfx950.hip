@@ -858,25 +858,41 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
     const float lse = l_tot > 0.f ? (m_run * c + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f : (l_tot == 0.f ? -INFINITY : l_tot);
     a.lse[b * a.lse_bs + hd * a.lse_hs + q_row] = lse;
   }
-  if (q_row < a.seqlen_q) {
+  // A lane holds pieces of 8 bytes (fp8: 4) of its row, 16 (8) bytes apart: stored as they are, a wavefront's store would touch 32 rows with 16
+  // bytes each, and at the end of a launch whose workgroups all run at once the 16-byte writes are what the L2s wait for.  They go through LDS, 128
+  // bytes of the 32 rows at a time, and leave as whole lines, eight lanes a row, past the L2 (they are not read again).  us, as they are -> whole
+  // lines -> not kept: 2 x 16 heads of 3072 queries, head dim 128, on 64 keys 15.6 -> 11.4 -> 8.2 (37.7 MB, 7.3 at the rate of a copy), on 3072
+  // 93.9 -> 91.0 -> 89.2; 8 x 32 heads, 1024 keys 95.0 -> 89.8 -> 88.0; 4 x 16 heads, 1024 keys, head dim 64 20.9 -> 20.0 -> 19.1; 2 x 32
+  // heads, 4096 keys 295.4 -> 291.0 -> 289.6.  (Without any stores: 90.6, 84.2, 18.2, 291.)
+  __builtin_amdgcn_s_waitcnt(0x0070);  // every wavefront has read its last tiles, and its copies (also those of nothing) have landed
+  __builtin_amdgcn_s_barrier();
+  constexpr int kElem = OUT == FA8_OUT_FP16 ? 2 : 1;
+  constexpr int kRowBytes = D * kElem <= 32 ? 32 : (D * kElem <= 64 ? 64 : 128), kSlab = 32 * kRowBytes;  // of a wavefront
+  constexpr int kChunks = kRowBytes / 16, kRoundTiles = kRowBytes / (32 * kElem), kRounds = (kMTiles + kRoundTiles - 1) / kRoundTiles;
+  constexpr int kPerTile = kTileBytes / kSlab < 4 ? kTileBytes / kSlab : 4;  // slabs that a K or V tile has room for
+  static_assert(kPerTile >= 1 && kStages * kPerTile >= 3, "four slabs in K stages and a V stage");
+  uint8_t* const slab = kPerTile == 4 ? k_lds0 + wave * kSlab
+                        : kPerTile >= 2 ? (wave < 2 ? k_lds0 : k_lds1) + (wave & 1) * kSlab
+                                        : (wave == 0 ? k_lds0 : wave == 1 ? k_lds1 : wave == 2 ? k_lds2 : v_lds0);
+  constexpr int kRowsAtOnce = 64 / kChunks;
+  // 16-byte chunk ch of row r: neighbouring rows start in different banks
+  auto slab_at = [](int r, int ch) __attribute__((always_inline)) { return r * kRowBytes + ((ch ^ (kChunks == 8 ? r & 7 : kChunks == 4 ? (r >> 1) & 3 : (r >> 2) & 1)) << 4); };
+  uint8_t* const op = (uint8_t*)a.o + ((long long)b * a.o_bs + (long long)hd * a.o_hs + (long long)q_wave0 * a.o_rs) * kElem;
+#pragma unroll
+  for (int n = 0; n < kRounds; ++n) {
     // register i = 4a2 + b2 of tile mt is head-dim column 32mt + 8a2 + 4h + b2
-    if constexpr (OUT == FA8_OUT_FP16) {
-      _Float16* op = (_Float16*)a.o + b * a.o_bs + hd * a.o_hs + (long long)q_row * a.o_rs + 4 * h;
 #pragma unroll
-      for (int mt = 0; mt < kMTiles; ++mt)
+    for (int m = 0; m < kRoundTiles; ++m) {
+      const int mt = n * kRoundTiles + m;
+      if (mt >= kMTiles) break;
 #pragma unroll
-        for (int a2 = 0; a2 < 4; ++a2) {
+      for (int a2 = 0; a2 < 4; ++a2) {
+        if constexpr (OUT == FA8_OUT_FP16) {
           v4h w;
 #pragma unroll
           for (int b2 = 0; b2 < 4; ++b2) w[b2] = (_Float16)(o_acc[mt][4 * a2 + b2] * inv);
-          *(v4h*)(op + 32 * mt + 8 * a2) = w;
-        }
-    } else {
-      uint8_t* op = (uint8_t*)a.o + b * a.o_bs + hd * a.o_hs + (long long)q_row * a.o_rs + 4 * h;
-#pragma unroll
-      for (int mt = 0; mt < kMTiles; ++mt)
-#pragma unroll
-        for (int a2 = 0; a2 < 4; ++a2) {
+          *LDS_PTR(v4h, slab + slab_at(qn, 4 * m + a2) + 8 * h) = w;
+        } else {
           float x[4];
           constexpr float kMaxFinite = OUT == FA8_OUT_E5M2 ? 57344.f : 448.f;
 #pragma unroll
@@ -884,8 +900,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
             const float y = o_acc[mt][4 * a2 + b2] * inv;
             x[b2] = (y != y) ? y : fminf(fmaxf(y, -kMaxFinite), kMaxFinite);  // saturate to finite, keep NaN
           }
-          *(int*)(op + 32 * mt + 8 * a2) = pack4_fp8<OUT == FA8_OUT_E5M2>(x[0], x[1], x[2], x[3]);
+          *LDS_PTR(int, slab + slab_at(qn, 2 * m + (a2 >> 1)) + 8 * (a2 & 1) + 4 * h) = pack4_fp8<OUT == FA8_OUT_E5M2>(x[0], x[1], x[2], x[3]);
         }
+      }
+    }
+    const int ch = lane % kChunks;
+#pragma unroll
+    for (int p = 0; p < 32 / kRowsAtOnce; ++p) {
+      const int r = p * kRowsAtOnce + lane / kChunks;
+      const v4i x = *LDS_PTR(const v4i, slab + slab_at(r, ch));
+      if (q_wave0 + r < a.seqlen_q && n * kRowBytes + 16 * ch < D * kElem)
+        __builtin_nontemporal_store(x, (v4i_unaligned*)(op + (long long)r * a.o_rs * kElem + n * kRowBytes + 16 * ch));
     }
   }
 #endif  // __HIP_DEVICE_COMPILE__
