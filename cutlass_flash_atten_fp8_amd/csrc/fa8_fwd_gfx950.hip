@@ -867,6 +867,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
   __builtin_amdgcn_s_waitcnt(0x0070);  // every wavefront has read its last tiles, and its copies (also those of nothing) have landed
   __builtin_amdgcn_s_barrier();
   constexpr int kElem = OUT == FA8_OUT_FP16 ? 2 : 1;
+  // (head dim 256: the lane's number taken anew; with transposed v, keeping it over the loop for these addresses spilled eight registers.  Head dim
+  // 224 spilled ten the other way round.)
+  const int lane_o = D == 256 ? (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) : lane, row_o = lane_o & 31, half_o = lane_o >> 5;
   constexpr int kRowBytes = D * kElem <= 32 ? 32 : (D * kElem <= 64 ? 64 : 128), kSlab = 32 * kRowBytes;  // of a wavefront
   constexpr int kChunks = kRowBytes / 16, kRoundTiles = kRowBytes / (32 * kElem), kRounds = (kMTiles + kRoundTiles - 1) / kRoundTiles;
   constexpr int kPerTile = kTileBytes / kSlab < 4 ? kTileBytes / kSlab : 4;  // slabs that a K or V tile has room for
@@ -891,7 +894,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
           v4h w;
 #pragma unroll
           for (int b2 = 0; b2 < 4; ++b2) w[b2] = (_Float16)(o_acc[mt][4 * a2 + b2] * inv);
-          *LDS_PTR(v4h, slab + slab_at(qn, 4 * m + a2) + 8 * h) = w;
+          *LDS_PTR(v4h, slab + slab_at(row_o, 4 * m + a2) + 8 * half_o) = w;
         } else {
           float x[4];
           constexpr float kMaxFinite = OUT == FA8_OUT_E5M2 ? 57344.f : 448.f;
@@ -900,14 +903,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
             const float y = o_acc[mt][4 * a2 + b2] * inv;
             x[b2] = (y != y) ? y : fminf(fmaxf(y, -kMaxFinite), kMaxFinite);  // saturate to finite, keep NaN
           }
-          *LDS_PTR(int, slab + slab_at(qn, 2 * m + (a2 >> 1)) + 8 * (a2 & 1) + 4 * h) = pack4_fp8<OUT == FA8_OUT_E5M2>(x[0], x[1], x[2], x[3]);
+          *LDS_PTR(int, slab + slab_at(row_o, 2 * m + (a2 >> 1)) + 8 * (a2 & 1) + 4 * half_o) = pack4_fp8<OUT == FA8_OUT_E5M2>(x[0], x[1], x[2], x[3]);
         }
       }
     }
-    const int ch = lane % kChunks;
+    const int ch = lane_o % kChunks;
 #pragma unroll
     for (int p = 0; p < 32 / kRowsAtOnce; ++p) {
-      const int r = p * kRowsAtOnce + lane / kChunks;
+      const int r = p * kRowsAtOnce + lane_o / kChunks;
       const v4i x = *LDS_PTR(const v4i, slab + slab_at(r, ch));
       if (q_wave0 + r < a.seqlen_q && n * kRowBytes + 16 * ch < D * kElem)
         __builtin_nontemporal_store(x, (v4i_unaligned*)(op + (long long)r * a.o_rs * kElem + n * kRowBytes + 16 * ch));
