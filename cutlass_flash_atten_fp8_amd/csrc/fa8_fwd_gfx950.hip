@@ -1097,7 +1097,9 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 //     blocks eight, 64 five), 0.87 - 0.93
 void keep_sums_apart(const Fa8FwdParams* p, long long cus, long long rows, long long tiles, long long pairs, long long longest, bool unequal, Plan& n) {
   const int d = p->head_dim;
-  if (n.splits > 1 || d > 128 || d % 32 != 0) return;
+  // An fp8 output moves by a whole step of its type where the last bit of a sum carries it over a rounding boundary, 2^-9 in the range of the long
+  // averages of small v, a quarter of their size: fp8 outputs keep the order of fa8_fwd, and its bits.
+  if (n.splits > 1 || d > 128 || p->out_dtype != FA8_OUT_FP16) return;
   const bool many_rows = rows > 128;
   bool apart;
   if (n.waves_per_tile == 4 && n.tiles_per_workgroup == 1) {

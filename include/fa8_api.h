@@ -138,7 +138,7 @@ int fa8_fwd_ws(const Fa8FwdParams* p, void* workspace, int64_t bytes, void* hip_
 
 /*
  * fa8_fwd_ws, free to take the fp32 sums over the keys in another order also where that needs no memory (library version 7): launches with few
- * query rows then keep the sums of the wavefronts that share a row tile apart and add them up at the end.  The weights are the same bit for
+ * query rows and an fp16 output then keep the sums of the wavefronts that share a row tile apart and add them up at the end.  The weights are the same bit for
  * bit; the last bits of O and of the log-sum-exp can depend on the whole launch and on the number of compute units, not on anything else.  The
  * workspace is that of fa8_fwd_workspace, and may be NULL.  fa8_fwd_apart tells whether a call would do so (1 or 0, or the FA8_ERR_* code
  * fa8_fwd_validate gives; launches nothing).  No counterpart in the reference.

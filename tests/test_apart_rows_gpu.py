@@ -16,29 +16,30 @@ CASES = [
     # B, H, Hk, Nq, Nk, d, causal, bottom_right, vt, dtype, fp8 out, (rows per workgroup, wavefronts per tile), sums apart
     (1, 2, 2, 100, 704, 64, False, False, False, E4, False, (32, 4), False),     # 11 blocks
     (1, 2, 2, 100, 705, 64, False, False, False, E4, False, (32, 4), True),      # 12, the last with one key
-    (1, 4, 2, 70, 784, 64, True, True, True, E5, True, (32, 4), True),           # 13 blocks: one in the last group; v^T, ragged
+    (1, 4, 2, 70, 784, 64, True, True, True, E5, False, (32, 4), True),           # 13 blocks: one in the last group; v^T, ragged
     (1, 8, 8, 1200, 800, 64, True, True, False, E4, False, (32, 4), True),       # queries that see no key
-    (1, 16, 16, 1024, 1024, 64, True, False, False, E4, True, (32, 4), True),    # two tiles a compute unit
+    (1, 16, 16, 1024, 1024, 64, True, False, False, E4, False, (32, 4), True),   # two tiles a compute unit
+    (1, 16, 16, 1024, 1024, 64, True, False, False, E4, True, (32, 4), False),   # fp8 output: the bits of fa8_fwd
     (2, 6, 2, 11, 900, 32, True, True, False, E4, False, (32, 4), True),         # 33 packed rows, group of 3
-    (1, 4, 4, 90, 1030, 32, False, False, False, E5, True, (32, 4), True),
+    (1, 4, 4, 90, 1030, 32, False, False, False, E5, False, (32, 4), True),
     (1, 8, 4, 40, 1100, 96, True, True, False, E4, False, (32, 4), True),
     (1, 2, 2, 40, 1100, 96, False, False, False, E5, False, (32, 4), True),
     (1, 3, 3, 200, 1216, 128, True, False, True, E4, False, (32, 4), False),     # 19 blocks
-    (1, 3, 3, 200, 1232, 128, False, False, True, E4, True, (32, 4), True),      # 20
+    (1, 3, 3, 200, 1232, 128, False, False, True, E4, False, (32, 4), True),      # 20
     (1, 8, 8, 32, 1300, 128, False, False, False, E4, False, (32, 4), False),    # one tile a k/v head
     (1, 16, 4, 512, 3001, 128, True, True, False, E4, False, (32, 4), True),
     (1, 32, 32, 500, 760, 96, False, False, False, E4, False, (64, 4), True),    # 12 blocks
-    (1, 30, 30, 290, 1330, 96, True, True, False, E5, True, (64, 4), True),      # ten tiles
+    (1, 30, 30, 290, 1330, 96, True, True, False, E5, False, (64, 4), True),      # ten tiles
     (1, 30, 30, 270, 1330, 128, True, True, False, E4, False, (64, 4), True),    # nine: the last workgroup's second one is empty
     (1, 32, 8, 512, 2000, 128, True, True, False, E4, False, (64, 4), True),
-    (1, 11, 11, 1400, 1408, 128, False, False, True, E5, True, (64, 4), True),
+    (1, 11, 11, 1400, 1408, 128, False, False, True, E5, False, (64, 4), True),
     (1, 24, 24, 1300, 1300, 64, False, False, False, E4, False, (64, 2), True),  # two tiles, two wavefronts each; 21 blocks
-    (1, 20, 20, 2100, 2100, 64, True, False, False, E4, True, (64, 2), True),    # 33 blocks, 660 pairs of unequal length
+    (1, 20, 20, 2100, 2100, 64, True, False, False, E4, False, (64, 2), True),    # 33 blocks, 660 pairs of unequal length
     (1, 30, 30, 1500, 1504, 32, False, False, True, E5, False, (64, 2), True),
     (1, 28, 28, 1100, 1100, 96, True, False, False, E4, False, (64, 2), True),
     (1, 45, 45, 705, 705, 96, False, False, False, E4, False, (64, 2), False),   # 540 pairs; two a compute unit run at once
     (3, 30, 10, 250, 2101, 128, False, False, False, E4, False, (64, 2), True),  # instead of unshared rows
-    (1, 20, 20, 1600, 1600, 128, True, False, False, E5, True, (64, 2), True),   # 25 blocks
+    (1, 20, 20, 1600, 1600, 128, True, False, False, E5, False, (64, 2), True),   # 25 blocks
 ]
 
 
