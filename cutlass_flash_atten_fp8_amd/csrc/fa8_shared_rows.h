@@ -474,8 +474,11 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
     barrier(none);
     // the products of the last group; then m_own is the max over all keys (the group after the last one shows none)
     rescale();
+    // (a block behind the tile's last one is one that the workgroup's other tile sees: weights of zero, which an infinity or a NaN in v would turn into NaN)
+    if ((groups - 1) * W + w < blocks) {
 #pragma unroll
-    for (int m = 0; m < kOwn; ++m) o_acc[m] = mfma_fp8<E5M2>(load_vf((groups & 1) ? v_lds0 : v_lds1, 0, m), p8, o_acc[m]);
+      for (int m = 0; m < kOwn; ++m) o_acc[m] = mfma_fp8<E5M2>(load_vf((groups & 1) ? v_lds0 : v_lds1, 0, m), p8, o_acc[m]);
+    }
     o_alpha = alpha;
     o_changed = changed;
     rescale();

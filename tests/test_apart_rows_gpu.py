@@ -124,3 +124,47 @@ def test_strided_tensors_and_guard_bands(vt):
     torch.cuda.synchronize()
     assert torch.equal(o.contiguous(), fa.flash_attention_v2_cutlass(q, k, vv, True, 0.1, v_transposed=vt, causal_bottom_right=True)[0])
     assert (obuf[:, nq:] == 777.0).all()
+
+
+PAIRS = [
+    # B, H, Hk, Nq, Nk, d, (rows per workgroup, wavefronts per tile): shifts of half a block, so that the second tile of a workgroup sees a block more
+    (1, 30, 30, 1504, 1536, 32, (64, 2)),
+    (1, 20, 20, 2080, 2112, 64, (64, 2)),
+    (1, 28, 28, 1088, 1120, 96, (64, 2)),
+    (1, 20, 20, 1600, 1632, 128, (64, 2)),
+    (1, 30, 30, 320, 1376, 96, (64, 4)),
+    (1, 30, 30, 320, 1376, 128, (64, 4)),
+    (1, 32, 8, 512, 2056, 128, (64, 4)),  # group of 4, tiles of 8 queries: every fourth workgroup
+]
+
+
+@pytest.mark.parametrize("shape", PAIRS, ids=lambda s: "B{}H{}k{}Nq{}Nk{}d{}".format(*s[:6]))
+@pytest.mark.parametrize("dt,code", [(E4, 0x7F), (E5, 0x7F), (E5, 0x7C)], ids=["e4m3-nan", "e5m2-nan", "e5m2-inf"])
+@pytest.mark.parametrize("vt", [False, True], ids=["rows", "vt"])
+def test_infinity_and_nan_in_v_stay_out_of_a_tile_that_ends_before_their_block(shape, dt, code, vt):
+    """Two tiles a workgroup, mask aligned to the last key: a block that only the second tile sees holds an infinity or a NaN, its weights in the first
+    are zero.  Rows that fa8_fwd gives finite are finite here too.  Another workgroup in every k/v head, so that the block falls to every wavefront."""
+    B, H, Hk, Nq, Nk, d, cut = shape
+    if vt and Nk % 16:
+        pytest.skip("transposed v has whole chunks of 16 keys")
+    q, k, v = _inputs(7, B, H, Hk, Nq, Nk, d, dt)
+    group, tile = H // Hk, 32 // (H // Hk)
+    pairs = [p for p in range(Nq // (2 * tile)) if (2 * tile * p + tile + Nk - Nq) % 64 == 0]
+    for head in range(Hk):
+        first_key = 2 * tile * pairs[-1 - head % len(pairs)] + tile + Nk - Nq  # the first that the pair's first tile does not see
+        v.view(torch.uint8)[0, head, first_key + (head % 3) * (tile // 2 - 1), 5 * head % d] = code
+    fine_v = torch.where(torch.isfinite(v.float()), v.float(), torch.zeros(()).to(DEV))
+    if vt:
+        v = v.transpose(2, 3).contiguous()
+    kw = dict(v_transposed=vt, return_lse=True, causal_bottom_right=True)
+    got, lse = fa.flash_attention_v2_cutlass(q, k, v, True, d ** -0.5, **kw)
+    want, want_lse = torch.empty_like(got), torch.empty_like(lse)
+    p = fa.make_params(q, k, v, want, True, d ** -0.5, vt, want_lse, True)
+    assert fa.lib().fa8_fwd_apart(ctypes.byref(p)) == 1 and fa.plan(p, fa.FA8_PLAN_ANY_ORDER) == cut + (1,)
+    assert fa.lib().fa8_fwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    torch.cuda.synchronize()
+    fine = torch.isfinite(want)
+    assert 0 < (~fine).sum() < fine.numel() // 2
+    assert torch.equal(torch.isfinite(got), fine) and torch.equal(torch.isnan(got), torch.isnan(want))
+    assert_same_up_to_sum_order(got[fine], want[fine], fine_v, Nk)
+    assert (lse - want_lse).abs().max() <= 5e-6 * max(1.0, want_lse.abs().max().item())
