@@ -12,7 +12,7 @@ namespace fa8 {
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
-typedef int v4i_unaligned __attribute__((ext_vector_type(4), aligned(8)));  // rows of o are 8-byte aligned
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
@@ -72,6 +72,17 @@ inline unsigned pack_mode(const Fa8FwdParams* p) {
   return (p->is_causal ? kSharedCausal : 0) | (p->causal_align == FA8_CAUSAL_BOTTOM_RIGHT ? kSharedBottomRight : 0) |
          (p->out_dtype != FA8_OUT_FP16 ? kSharedFp8Out : 0) | shift << kSharedShift | (unsigned)group << kSharedGroup;
 }
+
+#if defined(__HIP_DEVICE_COMPILE__)
+// 16 bytes of a row of o (8-byte aligned), written through the L2 at once.  Left dirty there they are written back when the kernel ends; asked not to
+// be kept anywhere (non-temporal) they leave the sooner, but the kernel that reads o next finds them in HBM instead of the memory-side cache: its
+// loss is more than the call's gain.  us, dirty -> not kept -> through, the call and the call with a copy of o after it: 8 x 32 heads, 1024 keys, head dim 128, causal
+// 69.2, 89.7 -> 63.7, 93.8 -> 69.0, 88.2; 4 x 16 heads, 1024 keys, head dim 64 20.5, 24.0 -> 19.4, 24.5 -> 19.5, 23.3; 2 x 32 heads, 4096 keys 300.0, 322.7 ->
+// 298.5, 329.0 -> 299.4, 324.0; 16 heads, 2048 keys, head dim 256, causal 38.8, 44.6 -> 37.0, 47.3 -> 38.5, 44.8.
+__device__ __forceinline__ void store_row_chunk(uint8_t* at, v4i x) {
+  __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) v4u*)at, (v4u)x, "agent");
+}
+#endif
 
 // LDS row r (0..63) of a K tile holds kv row kv_of_lds_row(r) of the block.  With this order the 16
 // accumulator registers a lane gets from S^T sub-tile t (rows 8a+4h+b of the 32x32 result, h = lane/32)

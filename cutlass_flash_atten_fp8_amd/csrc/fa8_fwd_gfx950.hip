@@ -860,10 +860,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
   }
   // A lane holds pieces of 8 bytes (fp8: 4) of its row, 16 (8) bytes apart: stored as they are, a wavefront's store would touch 32 rows with 16
   // bytes each, and at the end of a launch whose workgroups all run at once the 16-byte writes are what the L2s wait for.  They go through LDS, 128
-  // bytes of the 32 rows at a time, and leave as whole lines, eight lanes a row, past the L2 (they are not read again).  us, as they are -> whole
-  // lines -> not kept: 2 x 16 heads of 3072 queries, head dim 128, on 64 keys 15.6 -> 11.4 -> 8.2 (37.7 MB, 7.3 at the rate of a copy), on 3072
-  // 93.9 -> 91.0 -> 89.2; 8 x 32 heads, 1024 keys 95.0 -> 89.8 -> 88.0; 4 x 16 heads, 1024 keys, head dim 64 20.9 -> 20.0 -> 19.1; 2 x 32
-  // heads, 4096 keys 295.4 -> 291.0 -> 289.6.  (Without any stores: 90.6, 84.2, 18.2, 291.)
+  // bytes of the 32 rows at a time, and leave as whole lines, eight lanes a row (store_row_chunk).  us, pieces -> lines: 16 x 32 heads, 256 keys, head dim 128,
+  // causal 27.6 -> 22.4; 8 x 32 heads, 1024 keys, causal 77.1 -> 69.0; 4 x 16 heads, 1024 keys, head dim 64 21.3 -> 19.5; 2 x 16 heads, 2999 keys 99.2 -> 95.5;
+  // 2 x 32 heads, 4096 keys 309.3 -> 299.4.
   __builtin_amdgcn_s_waitcnt(0x0070);  // every wavefront has read its last tiles, and its copies (also those of nothing) have landed
   __builtin_amdgcn_s_barrier();
   constexpr int kElem = OUT == FA8_OUT_FP16 ? 2 : 1;
@@ -913,7 +912,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
       const int r = p * kRowsAtOnce + lane_o / kChunks;
       const v4i x = *LDS_PTR(const v4i, slab + slab_at(r, ch));
       if (q_wave0 + r < a.seqlen_q && n * kRowBytes + 16 * ch < D * kElem)
-        __builtin_nontemporal_store(x, (v4i_unaligned*)(op + (long long)r * a.o_rs * kElem + n * kRowBytes + 16 * ch));
+        store_row_chunk(op + (long long)r * a.o_rs * kElem + n * kRowBytes + 16 * ch, x);
     }
   }
 #endif  // __HIP_DEVICE_COMPILE__

@@ -805,7 +805,7 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
           const v4i x = *LDS_PTR(const v4i, tile_lds + chunk_at(rr, ch));
           const int q_of = query_of(row0 + rr), head = hk * group + (row0 + rr - q_of * group);
           const unsigned long long at = ((unsigned long long)a.o_bs * b + (unsigned long long)a.o_hs * head + (unsigned long long)a.o_rs * q_of) * 4 * kElem;
-          __builtin_nontemporal_store(x, (v4i_unaligned*)((uint8_t*)a.o + at + 16 * ch));
+          store_row_chunk((uint8_t*)a.o + at + 16 * ch, x);
         }
       }
     };

@@ -61,3 +61,22 @@ def test_split_keys_in_one_kernel_hold_no_lds_that_their_ranges_do_not_need(tmp_
         d = int(re.search(r"kernelILi(\d+)E", name)[1])
         row = 32 if d <= 32 else 64 if d <= 64 else 128 if d <= 128 else 256
         assert x <= 2 * 4 * 64 * row + 2048, name
+
+
+OBJDUMP = os.path.join(os.path.dirname(READELF), "llvm-objdump")
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="needs llvm-objdump")
+def test_outputs_are_kept_for_the_kernel_that_reads_them(tmp_path):
+    """No store is non-temporal: the reader of O would find it in HBM (a copy right after the call then loses more than the call gains)."""
+    stores = 0
+    for i, blob in enumerate(code_objects(fa.LIBFA8_PATH)):
+        f = tmp_path / f"{i}.o"
+        f.write_bytes(blob)
+        listing = subprocess.Popen([OBJDUMP, "-d", "--no-show-raw-insn", str(f)], stdout=subprocess.PIPE, text=True)
+        for line in listing.stdout:
+            if "global_store_" in line:
+                stores += 1
+                assert " nt" not in line.split("//")[0], line
+        assert listing.wait() == 0
+    assert stores > 0
