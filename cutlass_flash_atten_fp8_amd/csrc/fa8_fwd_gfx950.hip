@@ -866,9 +866,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
   __builtin_amdgcn_s_waitcnt(0x0070);  // every wavefront has read its last tiles, and its copies (also those of nothing) have landed
   __builtin_amdgcn_s_barrier();
   constexpr int kElem = OUT == FA8_OUT_FP16 ? 2 : 1;
-  // (head dim 256: the lane's number taken anew; with transposed v, keeping it over the loop for these addresses spilled eight registers.  Head dim
-  // 224 spilled ten the other way round.)
-  const int lane_o = D == 256 ? (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) : lane, row_o = lane_o & 31, half_o = lane_o >> 5;
+  // (head dims 32 and 256: the lane's number taken anew; with transposed v, keeping it over the loop for these addresses spilled eight registers of
+  // head dim 256 and cost head dim 32 the fifth workgroup of a compute unit.  Head dim 224 spilled ten the other way round.)
+  const int lane_o = D == 32 || D == 256 ? (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) : lane, row_o = lane_o & 31, half_o = lane_o >> 5;
   constexpr int kRowBytes = D * kElem <= 32 ? 32 : (D * kElem <= 64 ? 64 : 128), kSlab = 32 * kRowBytes;  // of a wavefront
   constexpr int kChunks = kRowBytes / 16, kRoundTiles = kRowBytes / (32 * kElem), kRounds = (kMTiles + kRoundTiles - 1) / kRoundTiles;
   constexpr int kPerTile = kTileBytes / kSlab < 4 ? kTileBytes / kSlab : 4;  // slabs that a K or V tile has room for

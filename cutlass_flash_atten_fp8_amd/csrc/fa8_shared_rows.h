@@ -766,6 +766,8 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
     }
   } else {
     static_assert(R <= W, "the rows of the workgroup fit in one K stage");
+    // (the lane's number taken anew: kept over the loop for these addresses it cost head dim 64 the fourth workgroup of a compute unit)
+    const int lane_o = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), row_o = lane_o & 31, half_o = lane_o >> 5;
     auto store = [&](auto elem_c) __attribute__((always_inline)) {
       constexpr int kElem = decltype(elem_c)::value, kChunks = D * kElem / 16;  // 16-byte chunks of a row
       uint8_t* const tile_lds = k_lds0 + r * 32 * D * kElem;
@@ -783,7 +785,7 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
             v4h x;
 #pragma unroll
             for (int b2 = 0; b2 < 4; ++b2) x[b2] = (_Float16)(o_acc[m][4 * a2 + b2] * inv);
-            *LDS_PTR(v4h, tile_lds + chunk_at(qn, 4 * mt + a2) + 8 * h) = x;
+            *LDS_PTR(v4h, tile_lds + chunk_at(row_o, 4 * mt + a2) + 8 * half_o) = x;
           } else {
             constexpr float kMaxFinite = E5M2 ? 57344.f : 448.f;
             float x[4];
@@ -792,7 +794,7 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
               const float y = o_acc[m][4 * a2 + b2] * inv;
               x[b2] = (y != y) ? y : fminf(fmaxf(y, -kMaxFinite), kMaxFinite);
             }
-            *LDS_PTR(int, tile_lds + chunk_at(qn, 2 * mt + (a2 >> 1)) + 8 * (a2 & 1) + 4 * h) = pack4_fp8<E5M2>(x[0], x[1], x[2], x[3]);
+            *LDS_PTR(int, tile_lds + chunk_at(row_o, 2 * mt + (a2 >> 1)) + 8 * (a2 & 1) + 4 * half_o) = pack4_fp8<E5M2>(x[0], x[1], x[2], x[3]);
           }
         }
       }
@@ -800,7 +802,7 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
       __builtin_amdgcn_s_barrier();
 #pragma unroll
       for (int p = 0; p * 64 * W < 32 * kChunks; ++p) {
-        const int unit = (p * W + w) * 64 + lane, rr = unit / kChunks, ch = unit - rr * kChunks;
+        const int unit = (p * W + w) * 64 + lane_o, rr = unit / kChunks, ch = unit - rr * kChunks;
         if (unit < 32 * kChunks && row0 + rr <= last_row) {
           const v4i x = *LDS_PTR(const v4i, tile_lds + chunk_at(rr, ch));
           const int q_of = query_of(row0 + rr), head = hk * group + (row0 + rr - q_of * group);

@@ -52,6 +52,16 @@ def test_no_kernel_spills_vector_registers(tmp_path):
 
 
 @pytest.mark.skipif(not os.path.exists(READELF), reason="needs llvm-readelf")
+def test_registers_leave_room_for_the_workgroups_that_the_plan_counts_on(tmp_path):
+    """Two tiles a workgroup, two wavefronts a tile, head dims 32 and 64, sums together: four workgroups a compute unit, 128 registers a lane (three took up
+    to 1.15 of the time).  Head dim 32 in the unshared loop: five, 96."""
+    kernels = kernel_notes(tmp_path, "vgpr_count")
+    for pattern, count, most in ((r"shared_rows_kernelILi(32|64)ELb[01]ELb[01]ELi2ELi2ELi[12]ELb0E", 12, 128), (r"fwd_kernelILi32E", 16, 96)):
+        found = {n: v for n, v in kernels.items() if re.search(pattern, n)}
+        assert len(found) == count and {n: v for n, v in found.items() if v > most} == {}
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="needs llvm-readelf")
 def test_split_keys_in_one_kernel_hold_no_lds_that_their_ranges_do_not_need(tmp_path):
     """Every workgroup holds its ring of two tiles a wavefront and 2 KB; LDS for the logits is asked for by length at the launch, so that a
     call with short ranges does not need compute units that are empty."""
