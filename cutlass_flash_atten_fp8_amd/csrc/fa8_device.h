@@ -38,6 +38,7 @@ struct KernelArgs {
   int interleave;    // causal: how many heads deal their q blocks alternately (see decode_block)
   int causal_shift;  // key j is visible to query i when j <= i + causal_shift
   float scale_log2;  // softmax_scale * log2(e)
+  int whole_lines;   // O leaves as whole lines
   long long q_bs, q_hs, q_rs;
   long long k_bs, k_hs, k_rs;
   long long v_bs, v_hs, v_rs;
@@ -49,7 +50,7 @@ struct KernelArgs {
 // host (2.75 us up to 112 bytes, 3.4 - 3.6 us from 120 on; an empty kernel in a loop).  Strides are 32-bit, in units of 16 elements
 // (q, k, v) and of 4 elements (o); `mode` holds flags, log2 of the number of q heads per k/v head (31: no power of two) and the number
 // itself.
-constexpr unsigned kSharedCausal = 1, kSharedBottomRight = 2, kSharedFp8Out = 4;
+constexpr unsigned kSharedCausal = 1, kSharedBottomRight = 2, kSharedFp8Out = 4, kSharedLines = 8;
 constexpr unsigned kSharedShift = 8;  // bits 8..12: log2 of the group, 31 if it is no power of two
 constexpr unsigned kSharedGroup = 16;
 

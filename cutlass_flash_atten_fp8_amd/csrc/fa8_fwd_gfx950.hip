@@ -858,17 +858,48 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
     const float lse = l_tot > 0.f ? (m_run * c + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f : (l_tot == 0.f ? -INFINITY : l_tot);
     a.lse[b * a.lse_bs + hd * a.lse_hs + q_row] = lse;
   }
-  // A lane holds pieces of 8 bytes (fp8: 4) of its row, 16 (8) bytes apart: stored as they are, a wavefront's store would touch 32 rows with 16
-  // bytes each, and at the end of a launch whose workgroups all run at once the 16-byte writes are what the L2s wait for.  They go through LDS, 128
+  // A lane holds pieces of 8 bytes (fp8: 4) of its row, 16 (8) bytes apart: stored as they are, a wavefront's store touches 32 rows with 16
+  // bytes each, and at the end of a launch whose workgroups all run at once the 16-byte writes are what the L2s wait for.  There they go through LDS, 128
   // bytes of the 32 rows at a time, and leave as whole lines, eight lanes a row (store_row_chunk).  us, pieces -> lines: 16 x 32 heads, 256 keys, head dim 128,
   // causal 27.6 -> 22.4; 8 x 32 heads, 1024 keys, causal 77.1 -> 69.0; 4 x 16 heads, 1024 keys, head dim 64 21.3 -> 19.5; 2 x 16 heads, 2999 keys 99.2 -> 95.5;
-  // 2 x 32 heads, 4096 keys 309.3 -> 299.4.
-  __builtin_amdgcn_s_waitcnt(0x0070);  // every wavefront has read its last tiles, and its copies (also those of nothing) have landed
-  __builtin_amdgcn_s_barrier();
+  // 2 x 32 heads, 4096 keys 309.3 -> 299.4.  Smaller launches keep the pieces: whole_lines has the line between the two.
   constexpr int kElem = OUT == FA8_OUT_FP16 ? 2 : 1;
+  // register i = 4a2 + b2 of tile mt is head-dim column 32mt + 8a2 + 4h + b2: a lane's piece a2 of tile mt in the output type
+  auto piece = [&](int mt, int a2) __attribute__((always_inline)) {
+    if constexpr (OUT == FA8_OUT_FP16) {
+      v4h x;
+#pragma unroll
+      for (int b2 = 0; b2 < 4; ++b2) x[b2] = (_Float16)(o_acc[mt][4 * a2 + b2] * inv);
+      return x;
+    } else {
+      float x[4];
+      constexpr float kMaxFinite = OUT == FA8_OUT_E5M2 ? 57344.f : 448.f;
+#pragma unroll
+      for (int b2 = 0; b2 < 4; ++b2) {
+        const float y = o_acc[mt][4 * a2 + b2] * inv;
+        x[b2] = (y != y) ? y : fminf(fmaxf(y, -kMaxFinite), kMaxFinite);  // saturate to finite, keep NaN
+      }
+      return pack4_fp8<OUT == FA8_OUT_E5M2>(x[0], x[1], x[2], x[3]);
+    }
+  };
+  using Piece = decltype(piece(0, 0));
+  // (the pieces follow in line: a launch of few workgroups has none of this in the instruction cache, and a jump costs it 0.2 us)
+  if (__builtin_expect(!a.whole_lines, 1)) {
+    if (q_row < a.seqlen_q) {
+      uint8_t* const at = (uint8_t*)a.o + ((long long)b * a.o_bs + (long long)hd * a.o_hs + (long long)q_row * a.o_rs + 4 * h) * kElem;
+#pragma unroll
+      for (int mt = 0; mt < kMTiles; ++mt)
+#pragma unroll
+        for (int a2 = 0; a2 < 4; ++a2) *(Piece*)(at + (32 * mt + 8 * a2) * kElem) = piece(mt, a2);
+    }
+    return;
+  }
   // (head dims 32 and 256: the lane's number taken anew; with transposed v, keeping it over the loop for these addresses spilled eight registers of
   // head dim 256 and cost head dim 32 the fifth workgroup of a compute unit.  Head dim 224 spilled ten the other way round.)
   const int lane_o = D == 32 || D == 256 ? (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) : lane, row_o = lane_o & 31, half_o = lane_o >> 5;
+  uint8_t* const op = (uint8_t*)a.o + ((long long)b * a.o_bs + (long long)hd * a.o_hs + (long long)q_wave0 * a.o_rs) * kElem;
+  __builtin_amdgcn_s_waitcnt(0x0070);  // every wavefront has read its last tiles, and its copies (also those of nothing) have landed
+  __builtin_amdgcn_s_barrier();
   constexpr int kRowBytes = D * kElem <= 32 ? 32 : (D * kElem <= 64 ? 64 : 128), kSlab = 32 * kRowBytes;  // of a wavefront
   constexpr int kChunks = kRowBytes / 16, kRoundTiles = kRowBytes / (32 * kElem), kRounds = (kMTiles + kRoundTiles - 1) / kRoundTiles;
   constexpr int kPerTile = kTileBytes / kSlab < 4 ? kTileBytes / kSlab : 4;  // slabs that a K or V tile has room for
@@ -879,31 +910,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FA8_WA
   constexpr int kRowsAtOnce = 64 / kChunks;
   // 16-byte chunk ch of row r: neighbouring rows start in different banks
   auto slab_at = [](int r, int ch) __attribute__((always_inline)) { return r * kRowBytes + ((ch ^ (kChunks == 8 ? r & 7 : kChunks == 4 ? (r >> 1) & 3 : (r >> 2) & 1)) << 4); };
-  uint8_t* const op = (uint8_t*)a.o + ((long long)b * a.o_bs + (long long)hd * a.o_hs + (long long)q_wave0 * a.o_rs) * kElem;
 #pragma unroll
   for (int n = 0; n < kRounds; ++n) {
-    // register i = 4a2 + b2 of tile mt is head-dim column 32mt + 8a2 + 4h + b2
 #pragma unroll
     for (int m = 0; m < kRoundTiles; ++m) {
-      const int mt = n * kRoundTiles + m;
-      if (mt >= kMTiles) break;
+      if (n * kRoundTiles + m >= kMTiles) break;
 #pragma unroll
       for (int a2 = 0; a2 < 4; ++a2) {
-        if constexpr (OUT == FA8_OUT_FP16) {
-          v4h w;
-#pragma unroll
-          for (int b2 = 0; b2 < 4; ++b2) w[b2] = (_Float16)(o_acc[mt][4 * a2 + b2] * inv);
-          *LDS_PTR(v4h, slab + slab_at(row_o, 4 * m + a2) + 8 * half_o) = w;
-        } else {
-          float x[4];
-          constexpr float kMaxFinite = OUT == FA8_OUT_E5M2 ? 57344.f : 448.f;
-#pragma unroll
-          for (int b2 = 0; b2 < 4; ++b2) {
-            const float y = o_acc[mt][4 * a2 + b2] * inv;
-            x[b2] = (y != y) ? y : fminf(fmaxf(y, -kMaxFinite), kMaxFinite);  // saturate to finite, keep NaN
-          }
-          *LDS_PTR(int, slab + slab_at(row_o, 2 * m + (a2 >> 1)) + 8 * (a2 & 1) + 4 * half_o) = pack4_fp8<OUT == FA8_OUT_E5M2>(x[0], x[1], x[2], x[3]);
-        }
+        const int ch = 2 * kElem * m + (kElem == 2 ? a2 : a2 >> 1), byte = kElem == 2 ? 8 * half_o : 8 * (a2 & 1) + 4 * half_o;
+        *LDS_PTR(Piece, slab + slab_at(row_o, ch) + byte) = piece(n * kRoundTiles + m, a2);
       }
     }
     const int ch = lane_o % kChunks;
@@ -1265,6 +1280,25 @@ extern "C" int fa8_fwd_validate(const Fa8FwdParams* p) {
 
 namespace {
 
+// Whether O leaves as whole lines, through LDS (the epilogues; the same bits either way).  The way costs a workgroup a barrier, an LDS round trip and
+// instructions that are not in the cache yet, the pieces cost the L2s when many rows leave together.  Drawn launches (2 x 1086 - 3700), time of lines / of pieces, median (95th
+// percentile), with 256 compute units:
+//   unshared, rows of O up to 16384: 1.08 (1.17), above: 0.94 (0.99); up to 32 queries: 1.06 (1.10) also above
+//   two tiles a workgroup, rows of 128, 192, 256, 384, 512 bytes: up to 8192 rows 1.04 (1.13), up to 16384 0.975 (1.04), above 0.96 (1.0); a k/v head with no more than 32
+//     rows, that is with one tile: 1.05
+//   fp16 rows of 192 (head dim 96), 320, 448 bytes: up to 8192 rows 1.08, 8193 - 16384 1.0 (1.06), above: 0.98 (1.01); fp8 rows of 64, 96, 160, 224 bytes: 1.0 above
+//   (1.04 - 1.12), 1.02 - 1.07 below; head dim 32: 1.0 - 1.02 above (1.06), 1.07 below
+// (Launches that keep the pieces take 0.99 - 1.01 of the time that they took in a library without lines.)
+bool whole_lines(const Fa8FwdParams* p, bool shared) {
+  const long long cus = compute_units(), rows = (long long)p->batch * p->heads * p->seqlen_q;
+  const int d = p->head_dim;
+  if (!shared) return p->seqlen_q > 32 && rows > 64 * cus;
+  const bool fp16 = p->out_dtype == FA8_OUT_FP16;
+  const long long group = p->heads_k > 0 ? p->heads / p->heads_k : 1;
+  if (d == 32 || group * p->seqlen_q <= 32) return false;
+  return d % 64 == 0 && (fp16 || d >= 128) ? rows > 32 * cus : fp16 && rows > 64 * cus;
+}
+
 // One wavefront per 32 query rows: the kernel of this file.
 int launch_rows(const Fa8FwdParams* p, hipStream_t stream) {
   KernelArgs a;
@@ -1284,6 +1318,7 @@ int launch_rows(const Fa8FwdParams* p, hipStream_t stream) {
   a.interleave = a.bh_total / 8 < 8 ? (a.bh_total / 8 > 0 ? a.bh_total / 8 : 1) : 8;  // causal launches, see decode_block
   if (env_causal_interleave() > 0) a.interleave = env_causal_interleave();
   a.scale_log2 = p->softmax_scale * 1.4426950408889634f;
+  a.whole_lines = whole_lines(p, false);
   a.q_bs = p->q_batch_stride; a.q_hs = p->q_head_stride; a.q_rs = p->q_row_stride;
   a.k_bs = p->k_batch_stride; a.k_hs = p->k_head_stride; a.k_rs = p->k_row_stride;
   a.v_bs = p->v_batch_stride; a.v_hs = p->v_head_stride; a.v_rs = p->v_row_stride;
@@ -1309,7 +1344,8 @@ int run(const Fa8FwdParams* p, void* workspace, long long bytes, unsigned late, 
   Plan n = choose_plan(p, workspace != nullptr, any_order);
   if (n.splits > 1 && bytes < split_workspace(p, n.splits)) n = choose_plan(p, false, any_order);
   if (n.splits > 1) return (uintptr_t)workspace % 16 != 0 ? FA8_ERR_ALIGN : launch_split(p, n.splits, workspace, late, stream);
-  return n.waves_per_tile > 1 ? launch_shared(p, n.tiles_per_workgroup, n.waves_per_tile, n.stages, n.apart, stream) : launch_rows(p, stream);
+  return n.waves_per_tile > 1 ? launch_shared(p, n.tiles_per_workgroup, n.waves_per_tile, n.stages, n.apart, n.tiles_per_workgroup > 1 && whole_lines(p, true), stream)
+                              : launch_rows(p, stream);
 }
 
 }  // namespace

@@ -8,8 +8,8 @@
 namespace fa8 {
 
 // r row tiles of 32 query rows per workgroup, w wavefronts per row tile, one or two LDS stages where both are built, or the sums of the wavefronts
-// apart (fa8_shared_rows.h)
-__attribute__((visibility("hidden"))) int launch_shared(const Fa8FwdParams* p, int r, int w, int stages, bool apart, hipStream_t stream);
+// apart; two tiles: O as whole lines (fa8_shared_rows.h)
+__attribute__((visibility("hidden"))) int launch_shared(const Fa8FwdParams* p, int r, int w, int stages, bool apart, bool whole_lines, hipStream_t stream);
 
 // the kernel with sums apart, nullptr where none is built
 __attribute__((visibility("hidden"))) const void* apart_kernel(int head_dim, int r, int w, bool e5m2, bool vt);

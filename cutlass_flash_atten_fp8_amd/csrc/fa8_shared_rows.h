@@ -725,51 +725,55 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
   }
 
   // ---- epilogue (see fa8_fwd_kernel) ----
-  // Two tiles a workgroup: the rows of a tile meet in LDS, in the first K stage, and leave as whole lines.  One tile: there are fewer rows
-  // to write, and another barrier costs as much as it saves or more.  us, pieces -> lines: two tiles, 32 heads, 1000 keys, head dim 128,
-  // causal 15.4 -> 14.4; 16 heads, 2048 keys, head dim 256, causal 39.8 -> 38.0; 512 queries on 4096 keys 28.6 -> 27.8; one tile, 16 heads, 1024
-  // keys, head dim 64, causal 7.73 -> 8.00; 24 heads, 1000 keys, head dim 32 8.13 -> 8.52.
+  // Two tiles a workgroup: where many rows leave together (whole_lines) the rows of a tile meet in LDS, in the first K stage, and leave as whole lines.
+  // One tile: there are fewer rows to write, and another barrier costs as much as it saves or more (16 heads, 1024 keys, head dim 64, causal
+  // 7.73 -> 8.00 us).  us, pieces -> lines: 32 heads, 1000 keys, head dim 128, causal 15.5 -> 14.9; 16 heads, 2048 keys, head dim 256, causal 39.8 ->
+  // 38.5; 512 queries on 4096 keys, 32 heads on 8 k/v heads 28.7 -> 28.1.
   const float l_tot = lane32_sum(l_run);
   const float inv = (l_tot == 0.f || l_tot != l_tot) ? 1.f : 1.f / l_tot;
   if (a.lse != nullptr && h == 0 && w == 0 && row <= last_row) {
     const float lse = l_tot > 0.f ? (m_run * c + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f : (l_tot == 0.f ? -INFINITY : l_tot);
     a.lse[(unsigned long long)a.lse_bs * b + (unsigned long long)a.lse_hs * hd + qi] = lse;
   }
-  if constexpr (R == 1) {
-    if (row > last_row) return;
-    const unsigned long long o_at = ((unsigned long long)a.o_bs * b + (unsigned long long)a.o_hs * hd + (unsigned long long)a.o_rs * qi) * 4 + 4 * h;
+  auto store = [&](auto elem_c) __attribute__((always_inline)) {
+    constexpr int kElem = decltype(elem_c)::value;
+    auto piece = [&](int m, int a2) __attribute__((always_inline)) {
+      if constexpr (kElem == 2) {
+        v4h x;
 #pragma unroll
-    for (int m = 0; m < kOut; ++m) {
-      const int mt = w + m * W;
-      if (kMTiles % W != 0 && mt >= kMTiles) break;
-      if (!(a.mode & kSharedFp8Out)) {
-#pragma unroll
-        for (int a2 = 0; a2 < 4; ++a2) {
-          v4h x;
-#pragma unroll
-          for (int b2 = 0; b2 < 4; ++b2) x[b2] = (_Float16)(o_acc[m][4 * a2 + b2] * inv);
-          *(v4h*)((_Float16*)a.o + o_at + 32 * mt + 8 * a2) = x;
-        }
+        for (int b2 = 0; b2 < 4; ++b2) x[b2] = (_Float16)(o_acc[m][4 * a2 + b2] * inv);
+        return x;
       } else {
         constexpr float kMaxFinite = E5M2 ? 57344.f : 448.f;
+        float x[4];
 #pragma unroll
-        for (int a2 = 0; a2 < 4; ++a2) {
-          float x[4];
-#pragma unroll
-          for (int b2 = 0; b2 < 4; ++b2) {
-            const float y = o_acc[m][4 * a2 + b2] * inv;
-            x[b2] = (y != y) ? y : fminf(fmaxf(y, -kMaxFinite), kMaxFinite);
-          }
-          *(int*)((uint8_t*)a.o + o_at + 32 * mt + 8 * a2) = pack4_fp8<E5M2>(x[0], x[1], x[2], x[3]);
+        for (int b2 = 0; b2 < 4; ++b2) {
+          const float y = o_acc[m][4 * a2 + b2] * inv;
+          x[b2] = (y != y) ? y : fminf(fmaxf(y, -kMaxFinite), kMaxFinite);
         }
+        return pack4_fp8<E5M2>(x[0], x[1], x[2], x[3]);
       }
+    };
+    using Piece = decltype(piece(0, 0));
+    constexpr bool kLines = R == 2 && (kElem == 2 ? D > 32 : D % 64 == 0 && D >= 128);
+    if (__builtin_expect(!kLines || !(a.mode & kSharedLines), 1)) {
+      if (row > last_row) return;
+      uint8_t* const at =
+          (uint8_t*)a.o + (((unsigned long long)a.o_bs * b + (unsigned long long)a.o_hs * hd + (unsigned long long)a.o_rs * qi) * 4 + 4 * h) * kElem;
+#pragma unroll
+      for (int m = 0; m < kOut; ++m) {
+        const int mt = w + m * W;
+        if (kMTiles % W != 0 && mt >= kMTiles) break;
+#pragma unroll
+        for (int a2 = 0; a2 < 4; ++a2) *(Piece*)(at + (32 * mt + 8 * a2) * kElem) = piece(m, a2);
+      }
+      return;
     }
-  } else {
-    static_assert(R <= W, "the rows of the workgroup fit in one K stage");
-    // (the lane's number taken anew: kept over the loop for these addresses it cost head dim 64 the fourth workgroup of a compute unit)
-    const int lane_o = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), row_o = lane_o & 31, half_o = lane_o >> 5;
-    auto store = [&](auto elem_c) __attribute__((always_inline)) {
-      constexpr int kElem = decltype(elem_c)::value, kChunks = D * kElem / 16;  // 16-byte chunks of a row
+    if constexpr (kLines) {
+      // (the lane's number taken anew; kept over the loop for these addresses it cost head dim 64 the fourth workgroup of a compute unit)
+      const int lane_o = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), row_o = lane_o & 31, half_o = lane_o >> 5;
+      static_assert(R <= W, "the rows of the workgroup fit in one K stage");
+      constexpr int kChunks = D * kElem / 16;  // 16-byte chunks of a row
       uint8_t* const tile_lds = k_lds0 + r * 32 * D * kElem;
       auto chunk_at = [](int rr, int ch) __attribute__((always_inline)) {  // neighbouring rows start in different banks
         const int key = kChunks % 8 == 0 ? rr & 7 : (kChunks % 4 == 0 ? (rr >> 1) & 3 : (rr >> 2) & 1);
@@ -781,21 +785,8 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
         if (kMTiles % W != 0 && mt >= kMTiles) break;
 #pragma unroll
         for (int a2 = 0; a2 < 4; ++a2) {
-          if constexpr (kElem == 2) {
-            v4h x;
-#pragma unroll
-            for (int b2 = 0; b2 < 4; ++b2) x[b2] = (_Float16)(o_acc[m][4 * a2 + b2] * inv);
-            *LDS_PTR(v4h, tile_lds + chunk_at(row_o, 4 * mt + a2) + 8 * half_o) = x;
-          } else {
-            constexpr float kMaxFinite = E5M2 ? 57344.f : 448.f;
-            float x[4];
-#pragma unroll
-            for (int b2 = 0; b2 < 4; ++b2) {
-              const float y = o_acc[m][4 * a2 + b2] * inv;
-              x[b2] = (y != y) ? y : fminf(fmaxf(y, -kMaxFinite), kMaxFinite);
-            }
-            *LDS_PTR(int, tile_lds + chunk_at(row_o, 2 * mt + (a2 >> 1)) + 8 * (a2 & 1) + 4 * half_o) = pack4_fp8<E5M2>(x[0], x[1], x[2], x[3]);
-          }
+          const int ch = 2 * kElem * mt + (kElem == 2 ? a2 : a2 >> 1), byte = kElem == 2 ? 8 * half_o : 8 * (a2 & 1) + 4 * half_o;
+          *LDS_PTR(Piece, tile_lds + chunk_at(row_o, ch) + byte) = piece(m, a2);
         }
       }
       __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -810,12 +801,12 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
           store_row_chunk((uint8_t*)a.o + at + 16 * ch, x);
         }
       }
-    };
-    if (a.mode & kSharedFp8Out)
-      store(std::integral_constant<int, 1>());
-    else
-      store(std::integral_constant<int, 2>());
-  }
+    }
+  };
+  if (!(a.mode & kSharedFp8Out))
+    store(std::integral_constant<int, 2>());
+  else
+    store(std::integral_constant<int, 1>());
 #endif
 }
 

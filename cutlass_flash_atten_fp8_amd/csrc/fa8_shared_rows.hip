@@ -28,7 +28,7 @@ const void* pick_rw(int r, int w, int stages, bool e5m2, bool vt) {
 
 }  // namespace
 
-int fa8::launch_shared(const Fa8FwdParams* p, int r, int w, int stages, bool apart, hipStream_t stream) {
+int fa8::launch_shared(const Fa8FwdParams* p, int r, int w, int stages, bool apart, bool whole_lines, hipStream_t stream) {
   SharedArgs a;
   a.q = (const uint8_t*)p->q;
   a.k = (const uint8_t*)p->k;
@@ -39,7 +39,7 @@ int fa8::launch_shared(const Fa8FwdParams* p, int r, int w, int stages, bool apa
   a.seqlen_q = p->seqlen_q;
   a.seqlen_k = p->seqlen_k;
   const int heads_k = p->heads_k > 0 ? p->heads_k : p->heads, group = p->heads / heads_k;
-  a.mode = pack_mode(p);
+  a.mode = pack_mode(p) | (whole_lines ? kSharedLines : 0);
   a.q_bs = p->q_batch_stride / 16; a.q_hs = p->q_head_stride / 16; a.q_rs = p->q_row_stride / 16;
   a.k_bs = p->k_batch_stride / 16; a.k_hs = p->k_head_stride / 16; a.k_rs = p->k_row_stride / 16;
   a.v_bs = p->v_batch_stride / 16; a.v_hs = p->v_head_stride / 16; a.v_rs = p->v_row_stride / 16;
