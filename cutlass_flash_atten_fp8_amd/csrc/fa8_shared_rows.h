@@ -343,15 +343,15 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
         }
       }
     };
-    // Waits until all but the latest `copies` tile copies of this wavefront have landed; barrier: and its LDS operations are done.
-    auto wait_copies = [&](auto copies_c) __attribute__((always_inline)) {
+    // Waits until all but the latest `copies` tile copies of this wavefront have landed and its LDS operations are done: with one tile a workgroup K and V of
+    // a block are the wavefront's own, and its next copy may go where it has just read.
+    auto wait = [&](auto copies_c) __attribute__((always_inline)) {
       constexpr int n = decltype(copies_c)::value * kPasses;
       static_assert(n < 64, "vmcnt has six bits");
-      __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | (n >> 4 << 14));
+      __builtin_amdgcn_s_waitcnt(0x0070 | (n & 15) | (n >> 4 << 14));
     };
     auto barrier = [&](auto copies_c) __attribute__((always_inline)) {
-      constexpr int n = decltype(copies_c)::value * kPasses;
-      __builtin_amdgcn_s_waitcnt(0x0070 | (n & 15) | (n >> 4 << 14));
+      wait(copies_c);
       __builtin_amdgcn_s_barrier();
     };
     constexpr std::integral_constant<int, 0> none{};
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
       if constexpr (R > 1)
         barrier(two);
       else
-        wait_copies(two);
+        wait(two);
     };
     using T = std::true_type;
     using F = std::false_type;
@@ -454,7 +454,7 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
     if constexpr (R > 1)
       barrier(one);
     else
-      wait_copies(one);
+      wait(one);
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
