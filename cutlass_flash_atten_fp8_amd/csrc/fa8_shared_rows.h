@@ -484,45 +484,37 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
     rescale();
     l_run *= alpha;
     // The wavefronts of a tile add up their O and l, in their order: tiles of 4 KB through the LDS of K and V.
-    constexpr int kUnits = W * kTileBytes / 4096, kObjects = 4;
-    constexpr int kRounds = (R * W * kMTiles + kUnits * kObjects - 1) / (kUnits * kObjects), kT = kMTiles / kRounds;
-    static_assert(kMTiles % kRounds == 0 && (kRounds == 1 || kT % W == 0) && R * W * kT <= kUnits * kObjects, "rounds of whole tiles");
+    constexpr int kUnits = W * kTileBytes / 4096;
+    static_assert(R * W * kMTiles <= 4 * kUnits, "all tiles of O at once");
     auto unit = [&](int u) __attribute__((always_inline)) {
       const int at = u / kUnits;
       uint8_t* const base = at == 0 ? k_lds0 : (at == 1 ? v_lds0 : (at == 2 ? k_lds1 : v_lds1));
       return base + (u - at * kUnits) * 4096 + lane * 16;
     };
     sum_lds[wave * 64 + lane] = l_run;
-    v16f total[kOut];
+    barrier(none);  // V has been read
 #pragma unroll
-    for (int n = 0; n < kRounds; ++n) {
-      barrier(none);  // V, or the tiles of the round before, have been read
+    for (int m = 0; m < kMTiles; ++m)
 #pragma unroll
-      for (int m = 0; m < kT; ++m)
+      for (int e = 0; e < 4; ++e)
+        *LDS_PTR(v4f, unit(wave * kMTiles + m) + e * 1024) = v4f{o_acc[m][4 * e], o_acc[m][4 * e + 1], o_acc[m][4 * e + 2], o_acc[m][4 * e + 3]};
+    barrier(none);
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          *LDS_PTR(v4f, unit(wave * kT + m) + e * 1024) = v4f{o_acc[n * kT + m][4 * e], o_acc[n * kT + m][4 * e + 1], o_acc[n * kT + m][4 * e + 2], o_acc[n * kT + m][4 * e + 3]};
-      barrier(none);
+    for (int m = 0; m < kOut; ++m) {
+      if (w + m * W >= kMTiles) break;
 #pragma unroll
-      for (int m = 0; m < (kT + W - 1) / W; ++m) {
-        if (w + m * W >= kT) break;
+      for (int i = 0; i < W; ++i)
 #pragma unroll
-        for (int i = 0; i < W; ++i)
+        for (int e = 0; e < 4; ++e) {
+          const v4f part = *LDS_PTR(const v4f, unit((r * W + i) * kMTiles + w + m * W) + e * 1024);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const v4f part = *LDS_PTR(const v4f, unit((r * W + i) * kT + w + m * W) + e * 1024);
-#pragma unroll
-            for (int b2 = 0; b2 < 4; ++b2)
-              total[n * (kT / W) + m][4 * e + b2] = i == 0 ? part[b2] : total[n * (kT / W) + m][4 * e + b2] + part[b2];
-          }
-      }
+          for (int b2 = 0; b2 < 4; ++b2) o_acc[m][4 * e + b2] = i == 0 ? part[b2] : o_acc[m][4 * e + b2] + part[b2];
+        }
     }
-#pragma unroll
-    for (int m = 0; m < kOut; ++m) o_acc[m] = total[m];
     l_run = sum_lds[r * W * 64 + lane];
 #pragma unroll
     for (int i = 1; i < W; ++i) l_run += sum_lds[(r * W + i) * 64 + lane];
-    if constexpr (R == 2) barrier(none);  // the parts have been read
+    if constexpr (R == 2 && D > 32) barrier(none);  // the parts have been read, O's lines may go there
   } else {
     // rescale factors of the group whose PV products are due, and whether any row of the tile needs them
     float alpha[W];
@@ -803,7 +795,7 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
       }
     }
   };
-  if (!(a.mode & kSharedFp8Out))
+  if (APART || !(a.mode & kSharedFp8Out))  // (keep_sums_apart takes fp16 outputs only)
     store(std::integral_constant<int, 2>());
   else
     store(std::integral_constant<int, 1>());
