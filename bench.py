@@ -241,11 +241,11 @@ MAIN_LOOPS = {1: "rolling", 2: "pipelined", 3: "dense"}  # FA8_SCHEDULE_* (inclu
 
 def loop_name(fa, p):
     """What the library runs for a call through the binding: split keys, shared rows, or one of the three main loops."""
-    _, waves, splits = fa.plan(p)
+    _, waves, splits = fa.plan(p, fa.FA8_PLAN_ANY_ORDER)
     if splits > 1:
         return f"split keys ({splits} parts)"
     if waves > 1:
-        return f"shared rows ({waves} wavefronts)"
+        return f"shared rows ({waves} wavefronts{', sums apart' if fa.lib().fa8_fwd_apart(ctypes.byref(p)) == 1 else ''})"
     loop = fa.lib().fa8_fwd_schedule(ctypes.byref(p))
     return MAIN_LOOPS.get(loop, f"error {loop}")
 

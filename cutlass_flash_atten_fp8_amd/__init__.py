@@ -101,7 +101,8 @@ def query(what):
 
 
 def plan(p, with_workspace=True):
-    """(query rows per workgroup, wavefronts per 32 rows, parts the keys are split into) of a call with these parameters."""
+    """(query rows per workgroup, wavefronts per 32 rows, parts the keys are split into) of a call with these parameters: fa8_fwd_ws (with_workspace
+    True), fa8_fwd (False) or fa8_fwd_any_order, which both bindings call (FA8_PLAN_ANY_ORDER)."""
     v = [ctypes.c_int32() for _ in range(3)]
     rc = lib().fa8_fwd_plan(ctypes.byref(p), int(with_workspace), *(ctypes.byref(x) for x in v))
     if rc != 0:
@@ -110,7 +111,7 @@ def plan(p, with_workspace=True):
 
 
 def form(p, with_workspace=True):
-    """(LDS stages of shared rows or 0, kernels launched) of a call with these parameters."""
+    """(LDS stages of shared rows or 0, kernels launched) of a call with these parameters; with_workspace as in plan."""
     v = [ctypes.c_int32() for _ in range(2)]
     rc = lib().fa8_fwd_form(ctypes.byref(p), int(with_workspace), *(ctypes.byref(x) for x in v))
     if rc != 0:

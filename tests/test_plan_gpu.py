@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 UNSHARED = (128, 1, 1)
 
 
-def plan_of(B, H, Hk, Nq, Nk, d, causal=False, bottom_right=False, vt=False, with_workspace=True):
+def params_of(B, H, Hk, Nq, Nk, d, causal=False, bottom_right=False, vt=False):
     """Nothing is launched: the parameters of tiny tensors with other sizes and contiguous strides."""
     t = torch.zeros((1, 1, 1, 256), dtype=torch.float8_e4m3fn, device="cuda:0")
     p = fa.make_params(t, t, t, torch.zeros((1, 1, 1, 256), dtype=torch.float16, device="cuda:0"), causal, d ** -0.5, vt, None, bottom_right)
@@ -18,7 +18,11 @@ def plan_of(B, H, Hk, Nq, Nk, d, causal=False, bottom_right=False, vt=False, wit
         setattr(p, name + "_row_stride", cols)
         setattr(p, name + "_head_stride", rows * cols)
         setattr(p, name + "_batch_stride", heads * rows * cols)
-    return fa.plan(p, with_workspace)
+    return p
+
+
+def plan_of(*shape, with_workspace=True):
+    return fa.plan(params_of(*shape), with_workspace)
 
 
 @pytest.mark.parametrize("shape", [
@@ -81,3 +85,15 @@ def test_many_keys_are_split(shape):
 def test_head_counts_beyond_32_bit_products():
     """65535 sequences of 1024 heads on one k/v head: 40 * batch * heads does not fit 32 bits; one query each leaves 127 of 128 rows idle."""
     assert plan_of(65535, 1024, 1, 1, 1, 128) == (64, 2, 1)
+
+
+@pytest.mark.parametrize("shape,name", [
+    ((1, 20, 20, 1600, 1632, 128, True, True), "shared rows (2 wavefronts, sums apart)"),  # where fa8_fwd_ws runs a main loop
+    ((1, 16, 16, 1024, 1024, 64, True), "shared rows (4 wavefronts, sums apart)"),
+    ((1, 16, 16, 128, 128, 64), "shared rows (4 wavefronts)"),
+    ((1, 32, 8, 1, 32768, 128, True, True), "split keys (32 parts)"),
+    ((2, 32, 32, 4096, 4096, 128), "dense"),
+], ids=lambda s: "B{}H{}k{}Nq{}Nk{}d{}".format(*s[:6]) if isinstance(s, tuple) else "")
+def test_the_benchmark_names_what_a_call_through_the_binding_runs(shape, name):
+    import bench
+    assert bench.loop_name(fa, params_of(*shape)) == name
