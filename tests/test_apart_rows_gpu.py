@@ -8,6 +8,9 @@ import pytest
 import torch
 
 import cutlass_flash_atten_fp8_amd as fa
+from oracle import fa8_oracle as fo
+from oracle.parity_gate import assert_parity
+from test_parity_gpu import sample_rows
 from test_split_kv_gpu import DEV, E4, E5, _inputs, assert_same_up_to_sum_order
 
 pytestmark = pytest.mark.gpu
@@ -40,6 +43,22 @@ CASES = [
     (1, 45, 45, 705, 705, 96, False, False, False, E4, False, (64, 2), False),   # 540 pairs; two a compute unit run at once
     (3, 30, 10, 250, 2101, 128, False, False, False, E4, False, (64, 2), True),  # instead of unshared rows
     (1, 20, 20, 1600, 1600, 128, True, False, False, E5, False, (64, 2), True),   # 25 blocks
+    # tiles of unequal length, more pairs than the first line lets through: both sides of blocks and of pairs a compute unit
+    (1, 40, 40, 1536, 1536, 32, True, False, False, E4, False, (64, 2), True),    # 24 blocks, 960 pairs
+    (1, 40, 40, 1472, 1472, 32, True, False, False, E4, False, (64, 2), False),   # 23
+    (1, 86, 86, 1536, 1536, 32, True, False, False, E4, False, (64, 2), False),   # 2064 pairs: more than eight
+    (1, 20, 20, 3072, 3072, 64, True, False, True, E4, False, (64, 2), True),     # 48, 960
+    (1, 20, 20, 3008, 3008, 64, True, False, False, E4, False, (64, 2), False),   # 47
+    (1, 27, 27, 3072, 3072, 64, True, False, False, E4, False, (64, 2), False),   # 1296: more than five
+    (1, 12, 12, 3072, 3072, 96, True, False, False, E5, False, (64, 2), True),    # 48, 576
+    (1, 12, 12, 3008, 3008, 96, True, False, False, E4, False, (64, 2), False),   # 47
+    (1, 12, 12, 3072, 3072, 128, True, False, True, E4, False, (64, 2), True),
+    (1, 12, 12, 3008, 3008, 128, True, False, False, E4, False, (64, 2), False),
+    (1, 17, 17, 3072, 3072, 128, True, False, False, E4, False, (64, 2), False),  # 816: more than three
+    # one tile a workgroup, two to three of them a compute unit
+    (1, 20, 20, 1056, 1056, 32, False, False, False, E4, False, (32, 4), True),   # 660 tiles
+    (1, 7, 7, 3072, 3072, 64, False, False, False, E4, False, (32, 4), True),     # 672, 48 blocks
+    (1, 7, 7, 3008, 3008, 64, False, False, True, E5, False, (32, 4), False),     # 47
 ]
 
 
@@ -168,3 +187,29 @@ def test_infinity_and_nan_in_v_stay_out_of_a_tile_that_ends_before_their_block(s
     assert torch.equal(torch.isfinite(got), fine) and torch.equal(torch.isnan(got), torch.isnan(want))
     assert_same_up_to_sum_order(got[fine], want[fine], fine_v, Nk)
     assert (lse - want_lse).abs().max() <= 5e-6 * max(1.0, want_lse.abs().max().item())
+
+
+@pytest.mark.parametrize("shape,causal,br,vt,dt,rows", [
+    ((1, 2, 2, 100, 705, 64), False, False, False, E4, None),
+    ((1, 4, 2, 70, 784, 64), True, True, True, E5, None),
+    ((2, 6, 2, 11, 900, 32), True, True, False, E4, None),
+    ((1, 8, 4, 40, 1100, 96), True, True, False, E4, None),
+    ((1, 3, 3, 200, 1232, 128), False, False, True, E4, None),
+    ((1, 32, 32, 500, 760, 96), False, False, False, E4, 48),   # two tiles, four wavefronts
+    ((1, 30, 30, 270, 1330, 128), True, True, False, E4, 48),
+    ((1, 24, 24, 1300, 1300, 64), False, False, False, E4, 48),  # two tiles, two wavefronts
+    ((1, 28, 28, 1088, 1120, 96), True, True, True, E5, 48),
+    ((1, 20, 20, 1600, 1632, 128), True, True, False, E4, 48),
+], ids=lambda x: "B{}H{}k{}Nq{}Nk{}d{}".format(*x) if isinstance(x, tuple) else "")
+def test_sums_apart_against_the_oracle(shape, causal, br, vt, dt, rows):
+    """The gate of every GPU parity test (max-abs 2e-2 a row, mean-abs 2e-3 against the oracle in the device's arithmetic), through the binding."""
+    q, k, v = _inputs(shape[3] + shape[4], *shape, dt)
+    vv = v.transpose(2, 3).contiguous() if vt else v
+    scale = shape[5] ** -0.5
+    o, lse = fa.load_extension().flash_attention_v2_cutlass(q, k, vv, causal, scale, v_transposed=vt, return_lse=True, causal_bottom_right=br)
+    assert fa.lib().fa8_fwd_apart(ctypes.byref(fa.make_params(q, k, vv, o, causal, scale, vt, lse, br))) == 1
+    at = None if rows is None else sample_rows(shape[3], rows)
+    got, got_lse = o.float().cpu().numpy(), lse.cpu().numpy()
+    _, want_lse = assert_parity(got if at is None else got[:, :, at], *(t.view(torch.uint8).cpu().numpy() for t in (q, k, v)), scale, causal=causal, rows=at,
+                                kv_block=fa.query(fa.FA8_QUERY_KV_BLOCK), in_dtype=fo.E5M2 if dt == E5 else fo.E4M3, causal_bottom_right=br, label=f"apart {shape}")
+    assert abs((got_lse if at is None else got_lse[:, :, at]) - want_lse).max() <= 5e-6 * max(1.0, abs(want_lse).max())
