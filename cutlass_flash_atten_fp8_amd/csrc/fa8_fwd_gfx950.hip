@@ -1281,22 +1281,24 @@ extern "C" int fa8_fwd_validate(const Fa8FwdParams* p) {
 namespace {
 
 // Whether O leaves as whole lines, through LDS (the epilogues; the same bits either way).  The way costs a workgroup a barrier, an LDS round trip and
-// instructions that are not in the cache yet, the pieces cost the L2s when many rows leave together.  Drawn launches (2 x 1086 - 3700), time of lines / of pieces, median (95th
-// percentile), with 256 compute units:
-//   unshared, rows of O up to 16384: 1.08 (1.17), above: 0.94 (0.99); up to 32 queries: 1.06 (1.10) also above
-//   two tiles a workgroup, rows of 128, 192, 256, 384, 512 bytes: up to 8192 rows 1.04 (1.13), up to 16384 0.975 (1.04), above 0.96 (1.0); a k/v head with no more than 32
-//     rows, that is with one tile: 1.05
-//   fp16 rows of 192 (head dim 96), 320, 448 bytes: up to 8192 rows 1.08, 8193 - 16384 1.0 (1.06), above: 0.98 (1.01); fp8 rows of 64, 96, 160, 224 bytes: 1.0 above
-//   (1.04 - 1.12), 1.02 - 1.07 below; head dim 32: 1.0 - 1.02 above (1.06), 1.07 below
+// instructions that are not in the cache yet, the pieces cost the L2s when many rows leave together.  2049 unshared and 3685 two-tile launches, drawn; time of lines / of
+// pieces, median (95th percentile), with 256 compute units:
+//   unshared, O above 1.8 MB: 0.94 (0.995), below: 1.07 (1.17); up to 32 queries: 1.06 (1.10) also above
+//   two tiles a workgroup: a k/v head with no more than 32 rows, that is with one tile: 1.05
+//     head dims 192 and 256 0.967 (1.013) whatever the size
+//     128, and fp16 of 64: 0.964 (0.997) above 8192 rows, 1.06 (1.12) below
+//     fp16 of 96, 160 and 224: 0.98 (1.01) above 16384 rows, 1.0 (1.06) from 8192 on, 1.08 below
+//     fp8 of 64, 96, 160 and 224: 1.0 (1.04 - 1.12) above, 1.02 - 1.07 below; head dim 32: 1.0 - 1.02 (1.06) above, 1.07 below
 // (Launches that keep the pieces take 0.99 - 1.01 of the time that they took in a library without lines.)
 bool whole_lines(const Fa8FwdParams* p, bool shared) {
-  const long long cus = compute_units(), rows = (long long)p->batch * p->heads * p->seqlen_q;
-  const int d = p->head_dim;
-  if (!shared) return p->seqlen_q > 32 && rows > 64 * cus;
   const bool fp16 = p->out_dtype == FA8_OUT_FP16;
-  const long long group = p->heads_k > 0 ? p->heads / p->heads_k : 1;
-  if (d == 32 || group * p->seqlen_q <= 32) return false;
-  return d % 64 == 0 && (fp16 || d >= 128) ? rows > 32 * cus : fp16 && rows > 64 * cus;
+  const long long cus = compute_units(), rows = (long long)p->batch * p->heads * p->seqlen_q;
+  const int d = p->head_dim, group = p->heads_k > 0 ? p->heads / p->heads_k : 1;
+  if (!shared) return p->seqlen_q > 32 && rows * d * (fp16 ? 2 : 1) > 7168 * cus;
+  if ((long long)group * p->seqlen_q <= 32) return false;
+  if (d == 192 || d == 256) return true;
+  if (d == 128 || (d == 64 && fp16)) return rows > 32 * cus;
+  return fp16 && d > 32 && rows > 64 * cus;
 }
 
 // One wavefront per 32 query rows: the kernel of this file.

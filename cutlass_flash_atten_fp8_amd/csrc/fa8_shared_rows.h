@@ -727,78 +727,82 @@ __global__ __launch_bounds__(64 * R * W) __attribute__((amdgpu_waves_per_eu(2)))
     const float lse = l_tot > 0.f ? (m_run * c + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f : (l_tot == 0.f ? -INFINITY : l_tot);
     a.lse[(unsigned long long)a.lse_bs * b + (unsigned long long)a.lse_hs * hd + qi] = lse;
   }
-  auto store = [&](auto elem_c) __attribute__((always_inline)) {
-    constexpr int kElem = decltype(elem_c)::value;
-    auto piece = [&](int m, int a2) __attribute__((always_inline)) {
-      if constexpr (kElem == 2) {
-        v4h x;
+  // a lane's piece a2 of its m-th O^T tile, 4 columns in the output type
+  auto piece = [&](auto elem_c, int m, int a2) __attribute__((always_inline)) {
+    if constexpr (decltype(elem_c)::value == 2) {
+      v4h x;
 #pragma unroll
-        for (int b2 = 0; b2 < 4; ++b2) x[b2] = (_Float16)(o_acc[m][4 * a2 + b2] * inv);
-        return x;
-      } else {
-        constexpr float kMaxFinite = E5M2 ? 57344.f : 448.f;
-        float x[4];
+      for (int b2 = 0; b2 < 4; ++b2) x[b2] = (_Float16)(o_acc[m][4 * a2 + b2] * inv);
+      return x;
+    } else {
+      constexpr float kMaxFinite = E5M2 ? 57344.f : 448.f;
+      float x[4];
 #pragma unroll
-        for (int b2 = 0; b2 < 4; ++b2) {
-          const float y = o_acc[m][4 * a2 + b2] * inv;
-          x[b2] = (y != y) ? y : fminf(fmaxf(y, -kMaxFinite), kMaxFinite);
-        }
-        return pack4_fp8<E5M2>(x[0], x[1], x[2], x[3]);
+      for (int b2 = 0; b2 < 4; ++b2) {
+        const float y = o_acc[m][4 * a2 + b2] * inv;
+        x[b2] = (y != y) ? y : fminf(fmaxf(y, -kMaxFinite), kMaxFinite);
       }
-    };
-    using Piece = decltype(piece(0, 0));
-    constexpr bool kLines = R == 2 && (kElem == 2 ? D > 32 : D % 64 == 0 && D >= 128);
-    if (__builtin_expect(!kLines || !(a.mode & kSharedLines), 1)) {
-      if (row > last_row) return;
-      uint8_t* const at =
-          (uint8_t*)a.o + (((unsigned long long)a.o_bs * b + (unsigned long long)a.o_hs * hd + (unsigned long long)a.o_rs * qi) * 4 + 4 * h) * kElem;
-#pragma unroll
-      for (int m = 0; m < kOut; ++m) {
-        const int mt = w + m * W;
-        if (kMTiles % W != 0 && mt >= kMTiles) break;
-#pragma unroll
-        for (int a2 = 0; a2 < 4; ++a2) *(Piece*)(at + (32 * mt + 8 * a2) * kElem) = piece(m, a2);
-      }
-      return;
+      return pack4_fp8<E5M2>(x[0], x[1], x[2], x[3]);
     }
-    if constexpr (kLines) {
-      // (the lane's number taken anew; kept over the loop for these addresses it cost head dim 64 the fourth workgroup of a compute unit)
-      const int lane_o = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), row_o = lane_o & 31, half_o = lane_o >> 5;
-      static_assert(R <= W, "the rows of the workgroup fit in one K stage");
-      constexpr int kChunks = D * kElem / 16;  // 16-byte chunks of a row
-      uint8_t* const tile_lds = k_lds0 + r * 32 * D * kElem;
-      auto chunk_at = [](int rr, int ch) __attribute__((always_inline)) {  // neighbouring rows start in different banks
-        const int key = kChunks % 8 == 0 ? rr & 7 : (kChunks % 4 == 0 ? (rr >> 1) & 3 : (rr >> 2) & 1);
-        return rr * D * kElem + ((ch ^ key) << 4);
-      };
+  };
+  constexpr std::integral_constant<int, 1> fp8{};
+  constexpr std::integral_constant<int, 2> fp16{};
+  const bool fp8_out = !APART && (a.mode & kSharedFp8Out);  // (keep_sums_apart takes fp16 outputs only)
+  constexpr bool kLines16 = R == 2 && D > 32, kLines8 = R == 2 && !APART && D % 64 == 0 && D >= 128;
+  if (__builtin_expect(!kLines16 || !(a.mode & kSharedLines), D != 192 && D != 256)) {  // (what most calls take follows in line)
+    if (row > last_row) return;
+    const unsigned long long o_at = ((unsigned long long)a.o_bs * b + (unsigned long long)a.o_hs * hd + (unsigned long long)a.o_rs * qi) * 4 + 4 * h;
 #pragma unroll
-      for (int m = 0; m < kOut; ++m) {
-        const int mt = w + m * W;
-        if (kMTiles % W != 0 && mt >= kMTiles) break;
+    for (int m = 0; m < kOut; ++m) {
+      const int mt = w + m * W;
+      if (kMTiles % W != 0 && mt >= kMTiles) break;
+      if (!fp8_out) {
 #pragma unroll
-        for (int a2 = 0; a2 < 4; ++a2) {
-          const int ch = 2 * kElem * mt + (kElem == 2 ? a2 : a2 >> 1), byte = kElem == 2 ? 8 * half_o : 8 * (a2 & 1) + 4 * half_o;
-          *LDS_PTR(Piece, tile_lds + chunk_at(row_o, ch) + byte) = piece(m, a2);
-        }
+        for (int a2 = 0; a2 < 4; ++a2) *(v4h*)((_Float16*)a.o + o_at + 32 * mt + 8 * a2) = piece(fp16, m, a2);
+      } else {
+#pragma unroll
+        for (int a2 = 0; a2 < 4; ++a2) *(int*)((uint8_t*)a.o + o_at + 32 * mt + 8 * a2) = piece(fp8, m, a2);
       }
-      __builtin_amdgcn_s_waitcnt(0xC07F);
-      __builtin_amdgcn_s_barrier();
+    }
+    return;
+  }
+  auto lines = [&](auto elem_c) __attribute__((always_inline)) {
+    static_assert(R <= W, "the rows of the workgroup fit in one K stage");
+    constexpr int kElem = decltype(elem_c)::value, kChunks = D * kElem / 16;  // 16-byte chunks of a row
+    using Piece = decltype(piece(elem_c, 0, 0));
+    // (the lane's number taken anew; kept over the loop for these addresses it cost head dim 64 the fourth workgroup of a compute unit)
+    const int lane_o = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), row_o = lane_o & 31, half_o = lane_o >> 5;
+    uint8_t* const tile_lds = k_lds0 + r * 32 * D * kElem;
+    auto chunk_at = [](int rr, int ch) __attribute__((always_inline)) {  // neighbouring rows start in different banks
+      const int key = kChunks % 8 == 0 ? rr & 7 : (kChunks % 4 == 0 ? (rr >> 1) & 3 : (rr >> 2) & 1);
+      return rr * D * kElem + ((ch ^ key) << 4);
+    };
 #pragma unroll
-      for (int p = 0; p * 64 * W < 32 * kChunks; ++p) {
-        const int unit = (p * W + w) * 64 + lane_o, rr = unit / kChunks, ch = unit - rr * kChunks;
-        if (unit < 32 * kChunks && row0 + rr <= last_row) {
-          const v4i x = *LDS_PTR(const v4i, tile_lds + chunk_at(rr, ch));
-          const int q_of = query_of(row0 + rr), head = hk * group + (row0 + rr - q_of * group);
-          const unsigned long long at = ((unsigned long long)a.o_bs * b + (unsigned long long)a.o_hs * head + (unsigned long long)a.o_rs * q_of) * 4 * kElem;
-          store_row_chunk((uint8_t*)a.o + at + 16 * ch, x);
-        }
+    for (int m = 0; m < kOut; ++m) {
+      const int mt = w + m * W;
+      if (kMTiles % W != 0 && mt >= kMTiles) break;
+#pragma unroll
+      for (int a2 = 0; a2 < 4; ++a2) {
+        const int ch = 2 * kElem * mt + (kElem == 2 ? a2 : a2 >> 1), byte = kElem == 2 ? 8 * half_o : 8 * (a2 & 1) + 4 * half_o;
+        *LDS_PTR(Piece, tile_lds + chunk_at(row_o, ch) + byte) = piece(elem_c, m, a2);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int p = 0; p * 64 * W < 32 * kChunks; ++p) {
+      const int unit = (p * W + w) * 64 + lane_o, rr = unit / kChunks, ch = unit - rr * kChunks;
+      if (unit < 32 * kChunks && row0 + rr <= last_row) {
+        const v4i x = *LDS_PTR(const v4i, tile_lds + chunk_at(rr, ch));
+        const int q_of = query_of(row0 + rr), head = hk * group + (row0 + rr - q_of * group);
+        const unsigned long long at = ((unsigned long long)a.o_bs * b + (unsigned long long)a.o_hs * head + (unsigned long long)a.o_rs * q_of) * 4 * kElem;
+        store_row_chunk((uint8_t*)a.o + at + 16 * ch, x);
       }
     }
   };
-  if (APART || !(a.mode & kSharedFp8Out))  // (keep_sums_apart takes fp16 outputs only)
-    store(std::integral_constant<int, 2>());
-  else
-    store(std::integral_constant<int, 1>());
+  if constexpr (kLines8)
+    if (fp8_out) return lines(fp8);
+  if constexpr (kLines16) lines(fp16);
 #endif
 }
 

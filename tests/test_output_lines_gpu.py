@@ -1,5 +1,5 @@
 """O leaves the kernels in pieces of 4 - 8 bytes a lane where few rows are written, and as whole lines through LDS where many are (whole_lines in the library).
-Same bits: every head of a call with lines is also run by itself, in pieces.  Every head dim and both output types, a last tile that is not full, rows of O that are 8-byte
+Same bits: heads of a call with lines are also run by themselves, in pieces.  Every head dim and both output types, a last tile that is not full, rows of O that are 8-byte
 aligned only and apart, with guard bands; query counts on both sides of the line."""
 import ctypes
 
@@ -22,7 +22,7 @@ def _call(q, k, v, o, causal, lse, rows_schedule):
 
 @pytest.mark.parametrize("d", [32, 64, 96, 128, 160, 192, 224, 256])
 @pytest.mark.parametrize("out8", [False, True], ids=["fp16", "fp8"])
-@pytest.mark.parametrize("heads,n,shared", [(41, 400, False), (40, 409, False), (513, 33, False), (33, 250, True), (33, 248, True), (20, 900, True)],
+@pytest.mark.parametrize("heads,n,shared", [(180, 330, False), (24, 150, False), (513, 33, False), (600, 32, False), (33, 250, True), (33, 248, True), (20, 900, True)],
                          ids=lambda x: str(x))
 def test_lines_and_pieces_give_the_same_bits(d, out8, heads, n, shared):
     g = torch.Generator().manual_seed(d + n)
@@ -38,11 +38,11 @@ def test_lines_and_pieces_give_the_same_bits(d, out8, heads, n, shared):
     if shared:
         if fa.plan(p, False)[0] == 32:
             pytest.skip("one tile a workgroup")
-    for at in range(0, heads, 7):
-        few = slice(at, min(heads, at + 7))
+    for at in range(0, heads, 1 + heads // 15):  # at most 1.4 MB of O, in the rolling loop: pieces
+        few = slice(at, min(heads, at + 3))
         part = torch.empty((1, few.stop - at, n, d), dtype=out, device=DEV)
         part_lse = torch.empty((1, few.stop - at, n), dtype=torch.float32, device=DEV)
-        _call(q[:, few].contiguous(), k[:, few].contiguous(), v[:, few].contiguous(), part, True, part_lse, not shared)
+        _call(q[:, few].contiguous(), k[:, few].contiguous(), v[:, few].contiguous(), part, True, part_lse, True)
         assert torch.equal(o[:, few].contiguous().view(torch.uint8), part.view(torch.uint8)), at
         assert torch.equal(lse[:, few], part_lse)
     before[:, :n, :, :d] = buf[:, :n, :, :d]
