@@ -1107,7 +1107,7 @@ constexpr long long kMaxWorkspace = 256LL << 20;  // bytes that a call may ask f
 //   two wavefronts a tile, two tiles, instead of the same with sums together or of the unshared loops: head dim 32 0.90, 0.97 and 0.80, 0.92 (12 blocks, unequal
 //     tiles 24; up to three pairs a CU); head dim 64 0.94, 0.99 instead of the former alone (16 blocks up to two pairs a CU, 32 up to three); head
 //     dim 96 0.86, 0.95 and 0.87, 0.96 (12 blocks), 128 0.92, 0.98 and 0.90, 1.0 (24 blocks, instead of the unshared loops 32), up to the two pairs a CU that run
-//     at once, k/v heads of more than 128 rows (fewer: up to 1.23, bytes); unequal tiles, 48 blocks: up to three pairs (head dim 32 from 12
+//     at once, k/v heads of more than 128 rows (fewer: up to 1.23, bytes); unequal tiles, 48 blocks: up to three pairs (head dim 32 from 24
 //     blocks eight, 64 five), 0.87 - 0.93
 void keep_sums_apart(const Fa8FwdParams* p, long long cus, long long rows, long long tiles, long long pairs, long long longest, bool unequal, Plan& n) {
   const int d = p->head_dim;
@@ -1245,7 +1245,7 @@ extern "C" int fa8_fwd_validate(const Fa8FwdParams* p) {
   if (!span_ok(p->k_row_stride, d) || !span_ok(p->k_head_stride, 1) || !span_ok(p->k_batch_stride, 1)) return FA8_ERR_STRIDE;
   if (!span_ok(p->v_row_stride, v_cols) || !span_ok(p->v_head_stride, 1) || !span_ok(p->v_batch_stride, 1)) return FA8_ERR_STRIDE;
   if (!span_ok(p->o_row_stride, d) || !span_ok(p->o_head_stride, 1) || !span_ok(p->o_batch_stride, 1)) return FA8_ERR_STRIDE;
-  // 16-byte vector loads of q/k/v rows, 8-byte (fp16) or 4-byte (fp8) vector stores of o
+  // 16-byte vector loads of q/k/v rows; o is stored in pieces of 8 (fp8: 4) bytes or in 16-byte chunks that need no more than this alignment
   const long long in_strides[] = {p->q_batch_stride, p->q_head_stride, p->q_row_stride, p->k_batch_stride, p->k_head_stride,
                                   p->k_row_stride,   p->v_batch_stride, p->v_head_stride, p->v_row_stride};
   for (long long s : in_strides)

@@ -42,9 +42,9 @@
 // the rescaling of O, needed in two thirds of the groups, four blocks apart: 5 % of the time) at the rate of two wavefronts a SIMD, and the tile copies
 // (8 KB a block and wavefront, twice the unshared loops': 10 %).  Copies spread over the chunks with an iteration or more of flight: started together after
 // barrier 1 they took 102 us on the 512 queries below, the form with the sums together 99, this 91.  Prefetching into the L2 gives nothing,
-// operands fetched two products ahead neither.  Measured (us, sums together -> apart): 512 queries on 16384 keys, 32 heads on 8 k/v heads, head dim 128:
-// 98.8 -> 90.6 (87.4 with the rows stored as whole lines); 128 queries on 8192 keys, head dim 64: 38.4 -> 29.3; 4 heads, 4096 keys, causal, head dim 64: 21.3 -> 17.2; 4 heads, 4096
-// keys, full, head dim 96: 29.2 -> 25.3; 16 heads, 1024 keys, causal, head dim 64: 8.6 -> 7.7.  The lines of the rule: keep_sums_apart.
+// operands fetched two products ahead neither.  Measured (us, sums together -> apart, calls in a captured graph over rotating inputs): 512 queries on 16384 keys, 32 heads on 8 k/v heads, head
+// dim 128: 98.8 -> 89.4; on 4096 keys 29.2 -> 27.0; 64 heads, 128 queries on 8192 keys, head dim 64: 39.4 -> 29.8; 4 heads, 4096 keys, causal, head dim 64: 21.5 -> 16.9; 4 heads,
+// 4096 keys, full, head dim 96: 29.3 -> 25.7; 16 heads, 1024 keys, causal, head dim 64: 8.7 -> 7.8.  The lines of the rule: keep_sums_apart.
 #ifndef FA8_SHARED_ROWS_H_
 #define FA8_SHARED_ROWS_H_
 #include <type_traits>

@@ -39,8 +39,9 @@ extern "C" {
 #define FA8_CAUSAL_BOTTOM_RIGHT 1 /* key j <= i + seqlen_k - seqlen_q: the last query sees every key (decode, chunked prefill) */
 
 /* which main loop the kernel runs: a performance hint.  The three loops and shared rows (fa8_fwd_plan) give bitwise the same results.
- *   AUTO      the library chooses from the shape of the launch.  The only value with which fa8_fwd_ws may split the keys of a call, and
- *             so sum in another order (fa8_fwd_plan tells); any hint, and any call without a workspace, keeps the unsplit order
+ *   AUTO      the library chooses from the shape of the launch.  The only value with which fa8_fwd_ws and fa8_fwd_any_order may split the keys
+ *             of a call and fa8_fwd_any_order may keep sums apart, and so sum in another order (fa8_fwd_plan, fa8_fwd_apart tell); any hint, and
+ *             fa8_fwd, keep the one order
  *   ROLLING   one KV block after the other, three wavefronts per SIMD: for masked launches that fill the chip
  *   PIPELINED software-pipelined over neighbouring KV blocks, two wavefronts per SIMD: for small masked launches
  *   DENSE     the same pipeline in three wavefronts per SIMD, for full (non-causal) attention; asked for under a mask, the library
@@ -139,8 +140,8 @@ int fa8_fwd_ws(const Fa8FwdParams* p, void* workspace, int64_t bytes, void* hip_
 /*
  * fa8_fwd_ws, free to take the fp32 sums over the keys in another order also where that needs no memory (library version 7): launches with few
  * query rows and an fp16 output then keep the sums of the wavefronts that share a row tile apart and add them up at the end.  The weights are the same bit for
- * bit; the last bits of O and of the log-sum-exp can depend on the whole launch and on the number of compute units, not on anything else.  The
- * workspace is that of fa8_fwd_workspace, and may be NULL.  fa8_fwd_apart tells whether a call would do so (1 or 0, or the FA8_ERR_* code
+ * bit; the last bits of O and of the log-sum-exp can depend on the whole launch, on the number of compute units and on whether there is a workspace, not on
+ * anything else.  The workspace is that of fa8_fwd_workspace, and may be NULL.  fa8_fwd_apart tells whether a call would do so (1 or 0, or the FA8_ERR_* code
  * fa8_fwd_validate gives; launches nothing).  No counterpart in the reference.
  */
 int fa8_fwd_any_order(const Fa8FwdParams* p, void* workspace, int64_t bytes, void* hip_stream);
@@ -157,8 +158,9 @@ int fa8_fwd_ws_late(const Fa8FwdParams* p, void* workspace, int64_t bytes, uint3
  * How a call would be cut on the current device, for benchmarks and tests (library version 5; nothing is launched): query rows of a workgroup
  * (grouped q heads counted together), wavefronts that share 32 of them (1: one of the main loops of fa8_fwd_schedule; 2 or 4: shared
  * rows, for launches with few of them; a schedule hint always gives 1), and into how many parts the keys of a row are split
- * (more than 1 only with_workspace).  The results of shared and unshared rows are bitwise the same.  with_workspace: 0 for fa8_fwd, 1 for
- * fa8_fwd_ws, FA8_PLAN_ANY_ORDER (library version 7) for fa8_fwd_any_order, both with the workspace that they ask for.
+ * (more than 1 only with_workspace).  The results of shared and unshared rows are bitwise the same, but for calls whose sums are apart
+ * (fa8_fwd_apart).  with_workspace: 0 for fa8_fwd, 1 (or any other number) for fa8_fwd_ws, FA8_PLAN_ANY_ORDER (library version 7) for
+ * fa8_fwd_any_order, both with the workspace that they ask for.
  */
 #define FA8_PLAN_ANY_ORDER 2
 int fa8_fwd_plan(const Fa8FwdParams* p, int with_workspace, int32_t* rows_per_workgroup, int32_t* wavefronts_per_tile,
