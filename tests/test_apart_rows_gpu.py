@@ -153,7 +153,7 @@ PAIRS = [
     (1, 20, 20, 1600, 1632, 128, (64, 2)),
     (1, 30, 30, 320, 1376, 96, (64, 4)),
     (1, 30, 30, 320, 1376, 128, (64, 4)),
-    (1, 32, 8, 512, 2056, 128, (64, 4)),  # group of 4, tiles of 8 queries: every fourth workgroup
+    (1, 32, 8, 504, 2048, 128, (64, 4)),  # group of 4, tiles of 8 queries: every fourth workgroup
 ]
 
 
@@ -164,8 +164,6 @@ def test_infinity_and_nan_in_v_stay_out_of_a_tile_that_ends_before_their_block(s
     """Two tiles a workgroup, mask aligned to the last key: a block that only the second tile sees holds an infinity or a NaN, its weights in the first
     are zero.  Rows that fa8_fwd gives finite are finite here too.  Another workgroup in every k/v head, so that the block falls to every wavefront."""
     B, H, Hk, Nq, Nk, d, cut = shape
-    if vt and Nk % 16:
-        pytest.skip("transposed v has whole chunks of 16 keys")
     q, k, v = _inputs(7, B, H, Hk, Nq, Nk, d, dt)
     group, tile = H // Hk, 32 // (H // Hk)
     pairs = [p for p in range(Nq // (2 * tile)) if (2 * tile * p + tile + Nk - Nq) % 64 == 0]

@@ -17,7 +17,6 @@ def _call(q, k, v, o, causal, lse, rows_schedule):
     p = fa.make_params(q, k, v, o, causal, q.shape[3] ** -0.5, False, lse)
     p.schedule = fa.FA8_SCHEDULE_ROLLING if rows_schedule else fa.FA8_SCHEDULE_AUTO
     assert fa.lib().fa8_fwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
-    return p
 
 
 @pytest.mark.parametrize("d", [32, 64, 96, 128, 160, 192, 224, 256])
@@ -34,10 +33,7 @@ def test_lines_and_pieces_give_the_same_bits(d, out8, heads, n, shared):
     before = buf.clone()
     o = buf[:, :n, :, :d].permute(0, 2, 1, 3)
     lse = torch.empty((1, heads, n), dtype=torch.float32, device=DEV)
-    p = _call(q, k, v, o, True, lse, not shared)
-    if shared:
-        if fa.plan(p, False)[0] == 32:
-            pytest.skip("one tile a workgroup")
+    _call(q, k, v, o, True, lse, not shared)
     for at in range(0, heads, 1 + heads // 15):  # at most 1.4 MB of O, in the rolling loop: pieces
         few = slice(at, min(heads, at + 3))
         part = torch.empty((1, few.stop - at, n, d), dtype=out, device=DEV)
